@@ -77,7 +77,7 @@ def measure_config(torch, np, hs, G, index, N, steps, warmup, mode=0, matrix=Non
     t = (main_ms + fix_ms) * 1e-3
     out = {"workload": "configs[%d]: %s, N=%d" % (index, cfg["name"], N),
            "dtype": "f16 in, f32 accumulate" if A["dtype"] == hs.FP16 else "f32 (tf32 variant)",
-           "kernel": KERNELS.get(info["last_kernel_family"], "none"),
+           "kernel": kernel_name(info),
            "kernel_ms": main_ms, "fixup_kernel_ms": fix_ms,
            "tflops": flops / t / 1e12, "algorithmic_bytes": bytes_alg,
            "bound": BOUND.get((index, N), "hbm"),
@@ -166,6 +166,13 @@ def kernel_sources_digest():
             with open(path, "rb") as f:
                 h.update(f.read())
     return h.hexdigest()
+
+
+def kernel_name(info):
+    """The main kernel of the last launch: the gather family without matrix instructions is the entry kernels."""
+    if info["last_kernel_family"] == 2 and info["last_mfma_kind"] == 0:
+        return "spmm_entries_kernel"
+    return KERNELS.get(info["last_kernel_family"], "none")
 
 
 def info_family(plan):
@@ -326,7 +333,7 @@ def main():
                      "unit": "GB/s", "frac": bytes_alg / (kernels_ms * 1e-3) / 1e9 / HBM_PEAK_GBPS,
                      # counter figures stored with the rocprofv3 summary they come from (not measured in this run)
                      "traffic": traffic,
-                     "kernel": KERNELS.get(info["last_kernel_family"], "none"),
+                     "kernel": kernel_name(info),
                      "kernel_ms": main_ms, "fixup_kernel_ms": fix_ms,
                      "algorithmic_bytes": bytes_alg, "gather_bytes": bytes_gather,
                      # every gathered B row counted every time it is gathered, for comparison with the HBM peak

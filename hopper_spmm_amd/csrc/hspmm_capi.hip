@@ -253,6 +253,7 @@ void hspmm_destroy(hspmm_plan *p)
     (void)hipFree(p->panel.d_unitRow);
     (void)hipFree(p->panel.d_step_panel);
     (void)hipFree(p->panel.d_masks); (void)hipFree(p->panel.d_vals); (void)hipFree(p->panel.d_step_voff);
+    (void)hipFree(p->entries.d_stream);
     (void)hipFree(p->bm.d_header); (void)hipFree(p->bm.d_vals);
     for (auto &b : p->buffers) { (void)hipFree(b.d_scratch); (void)hipFree(b.d_arrive); (void)hipFree(b.d_vector); }
     for (void *old : p->retired) (void)hipFree(old);

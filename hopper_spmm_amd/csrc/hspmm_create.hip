@@ -490,6 +490,27 @@ uint32_t bitmap_header_from_caller(uint32_t T, uint32_t elem, const BitmapSource
     return first_bad.load();
 }
 
+// Stored entries per real tile column, from 256 groups of 64 tiles spread over the matrix (every tile of a small one).
+double entries_per_column(uint32_t T, uint32_t cw, uint32_t elem, const uint32_t *tcA2B, const void *data, const BitmapSource *bitmap)
+{
+    const uint32_t group = 64u, groups = std::min(256u, (T + group - 1u) / group);
+    uint64_t stored = 0, columns = 0;
+    for (uint32_t g = 0; g < groups; ++g) {
+        const uint32_t t0 = uint32_t(uint64_t(T) * g / groups), t1 = std::min(T, t0 + group);
+        for (size_t i = size_t(t0) * cw; i < size_t(t1) * cw; ++i) columns += tcA2B[i] != HSPMM_IDX_MAX;
+        if (bitmap) {
+            stored += bitmap->nnzOffset[t1] - bitmap->nnzOffset[t0];
+        } else if (elem == 2u) {
+            const uint16_t *v = static_cast<const uint16_t *>(data);
+            for (size_t i = size_t(t0) * 8u * cw; i < size_t(t1) * 8u * cw; ++i) stored += v[i] != 0;
+        } else {
+            const uint32_t *v = static_cast<const uint32_t *>(data);
+            for (size_t i = size_t(t0) * 8u * cw; i < size_t(t1) * 8u * cw; ++i) stored += v[i] != 0;
+        }
+    }
+    return columns ? double(stored) / double(columns) : 8.0;
+}
+
 // hspmm_create; with `bitmap` (data == nullptr) the tiles come as the caller's bitmap arrays,
 // which are uploaded as they are, kept as the gather kernels' bitmap stream and expanded on the device for the
 // kernels that read plain tiles.  Returns kNeedsPlainTiles when the plan would need the tiles on the host
@@ -652,6 +673,12 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
             HSPMM_HIP_OR(hipStreamSynchronize(nullptr), bail);
         }
         timer.mark("bitmap tiles");
+        p->per_column = entries_per_column(total_tiles, cw, elem, tcA2B, data, bitmap);
+        {
+            uint32_t longest = 0;
+            for (size_t u = 0; u + 1 < st.unitOffset.size(); ++u) longest = std::max(longest, st.unitOffset[u + 1] - st.unitOffset[u]);
+            p->even_windows = uint64_t(longest) * p->n_units <= uint64_t(p->n_steps) * 8u;
+        }
         p->h_unitOffset = st.unitOffset;
         p->h_unitRow = st.unitRow;
         if (st.G != 1) {

@@ -104,6 +104,38 @@ struct PanelArgs {
 // packed: its tiles are stored without their zeros (tall streams only).
 hipError_t launch_spmm_panel(int dtype, int G, bool split, bool tall, bool packed, const PanelArgs &pa, const KernelArgs &ka,
                              int units, hipStream_t s, hipEvent_t mid);
+
+// Entry kernels for narrow feature dimensions (spmm_entries.hip): stored entries in units of four (the last unit of a
+// row filled up with zeros), rows sorted by length.  A class is the rows of 2^(c+1) + 1 .. 2^(c+2) units (c = 0: 1 .. 4);
+// rows above kEntryPieceUnits are cut into pieces of that many.
+constexpr uint32_t kEntryPieceUnits = 512u, kEntryClassesByLength = 8u, kEntryBins = 2u + 4u * kEntryClassesByLength;
+constexpr uint32_t kEntryChunkTiles = 64u, kEntryClasses = 2u + kEntryClassesByLength;
+struct EntryClass { uint32_t group_begin, slot_begin, slot_end, log2g; };    // first workgroup; slots; log2 subgroups per row
+struct EntryArgs {
+    const uint32_t *desc;        // per slot three words: first unit, units, matrix row (pieces: number of the piece)
+    const uint32_t *ids;         // per unit four column ids
+    const void     *vals;        // per unit four values
+    const uint32_t *pieces;      // per piece three words: matrix row, the row's first piece, its number of pieces
+    float          *scratch;     // sums of pieces [piece][lane][features of a lane]
+    uint32_t       *arrive;      // [first piece of a row]: pieces that have left their sums (zero between launches)
+    const void     *B;
+    void           *C;
+    uint32_t ld;                 // elements from one row of B (and of C) to the next
+    uint32_t block_bytes, n_feat_blocks, xcd_split;  // bytes of a row one subgroup covers; blocks side by side; != 0: on XCDs of their own
+    uint32_t n_groups;           // workgroups of one block
+    uint32_t n_pieces, n_classes;
+    EntryClass cls[kEntryClasses];   // pieces first where there are any, then from the longest rows to the empty ones
+};
+// lane_bytes (2, 4, 8, 16) x lanes (1 .. 32): how a row of B is shared out; at least lane_bytes long
+hipError_t launch_spmm_entries(int dtype, const EntryArgs &ea, uint32_t lane_bytes, uint32_t lanes, hipStream_t s);
+// The three steps that make the stream (hspmm_entries.hip); chunks: {first tile, tiles, first matrix row, window} each.
+hipError_t launch_entry_count(int elem, const void *tiles, const uint32_t *chunks, uint32_t n_chunks, uint32_t *counts, hipStream_t s);
+hipError_t launch_entry_rows(const uint32_t *rowIdx, const uint32_t *first_chunk, uint32_t n_windows, uint32_t rows, uint32_t *counts,
+                             uint32_t *row_len, uint32_t *totals, hipStream_t s);
+hipError_t launch_entry_fill(int elem, const void *tiles, const uint32_t *a2b, const uint32_t *chunks, uint32_t n_chunks,
+                             const uint32_t *positions, const uint32_t *row_len, uint32_t rows, const uint32_t *places,
+                             uint32_t *cursors, uint32_t *desc, uint32_t *pieces, uint32_t *row_first, uint32_t *ids, void *vals,
+                             hipStream_t s);
 hipError_t launch_fill_zero(void *dst, size_t bytes, hipStream_t s);
 // bitmap tiles (header, stored elements: see KernelArgs::bm_header and, for 32-bit elements, launch_bitmap_header
 // below) -> plain tiles (8 x 16 of 16-bit elements, 8 x 8 of 32-bit elements)

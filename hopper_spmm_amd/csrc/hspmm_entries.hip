@@ -1,0 +1,224 @@
+// Host side of the entry kernels (spmm_entries.hip): which launches they take, the stream they walk, the launch.
+#include "hspmm_plan.hpp"
+
+using namespace hspmm_host;
+
+namespace {
+
+// How a row of B of `bytes` bytes is shared out over the lanes of a subgroup: the widest load the row can fill.
+struct RowShare { uint32_t lane_bytes, lanes; };
+RowShare share_row(uint32_t bytes)
+{
+    if (bytes < 4u) return {2u, 1u};
+    if (bytes < 8u) return {4u, bytes > 4u ? 2u : 1u};
+    if (bytes < 16u) return {8u, bytes > 8u ? 2u : 1u};
+    uint32_t lanes = 1;
+    while (lanes * 16u < bytes) lanes <<= 1;
+    return {16u, lanes};
+}
+
+// Device memory that a failed or finished build gives back.
+struct Temporary {
+    void *p = nullptr;
+    ~Temporary() { (void)hipFree(p); }
+};
+
+// Most units of a row of bin b (see entry_bin in spmm_entries.hip).
+uint32_t bin_units(uint32_t b)
+{
+    if (b == 0u || b == hspmm::kEntryBins - 1u) return 0u;
+    const uint32_t c = hspmm::kEntryClassesByLength - 1u - (b - 1u) / 4u, step = 3u - (b - 1u) % 4u;
+    return c == 0u ? step + 1u : (2u << c) + (step + 1u) * (1u << (c - 1u));
+}
+
+// Makes the entry stream from the uploaded tiles.  Called with the plan's mutex held; waits for the device.
+int build_entries(hspmm_plan *p, hipStream_t s)
+{
+    using namespace hspmm;
+    const std::vector<uint32_t> &offset = p->G == 1 ? p->h_unitOffset : p->h_winOffset;
+    std::vector<uint32_t> chunks, first_chunk(size_t(p->W) + 1u);
+    for (uint32_t w = 0; w < p->W; ++w) {
+        first_chunk[w] = uint32_t(chunks.size() / 4u);
+        for (uint32_t t = offset[w]; t < offset[w + 1]; t += kEntryChunkTiles) {
+            chunks.push_back(t);
+            chunks.push_back(std::min(kEntryChunkTiles, offset[w + 1] - t));
+            chunks.push_back(p->G == 1 ? p->h_unitRow[w] : p->h_winRow[w]);
+            chunks.push_back(w);
+        }
+    }
+    const uint32_t n_chunks = uint32_t(chunks.size() / 4u);
+    first_chunk[p->W] = n_chunks;
+    // one allocation for what only the build needs: chunks, their windows, counts, row lengths and places, totals
+    const size_t words = chunks.size() + first_chunk.size() + size_t(n_chunks) * 8u + size_t(p->rows) * 2u + 3u * (kEntryBins + 1u) + 3u * kEntryBins;
+    Temporary tmp;
+    HSPMM_HIP(hipMalloc(&tmp.p, words * 4u));
+    uint32_t *d_chunks = static_cast<uint32_t *>(tmp.p), *d_first_chunk = d_chunks + chunks.size();
+    uint32_t *d_counts = d_first_chunk + first_chunk.size(), *d_len = d_counts + size_t(n_chunks) * 8u, *d_first = d_len + p->rows;
+    uint32_t *d_totals = d_first + p->rows, *d_cursors = d_totals + kEntryBins + 1u, *d_places = d_cursors + kEntryBins + 1u;
+    HSPMM_HIP(hipMemcpyAsync(d_chunks, chunks.data(), chunks.size() * 4u, hipMemcpyHostToDevice, s));
+    HSPMM_HIP(hipMemcpyAsync(d_first_chunk, first_chunk.data(), first_chunk.size() * 4u, hipMemcpyHostToDevice, s));
+    HSPMM_HIP(launch_fill_zero(d_totals, 2u * (kEntryBins + 1u) * 4u, s));
+    HSPMM_HIP(launch_entry_count(int(p->elem), p->d_data, d_chunks, n_chunks, d_counts, s));
+    HSPMM_HIP(launch_entry_rows(p->d_rowIdx, d_first_chunk, p->W, p->rows, d_counts, d_len, d_totals, s));
+    uint32_t totals[kEntryBins + 1u];
+    HSPMM_HIP(hipMemcpyAsync(totals, d_totals, sizeof totals, hipMemcpyDeviceToHost, s));
+    HSPMM_HIP(hipStreamSynchronize(s));
+    uint32_t places[3u * kEntryBins];
+    uint64_t slot = 0, unit = 0;
+    for (uint32_t b = 0; b < kEntryBins; ++b) {
+        const uint32_t width = bin_units(b);
+        places[3u * b] = uint32_t(slot); places[3u * b + 1u] = uint32_t(unit); places[3u * b + 2u] = width;
+        slot += totals[b];
+        unit += b == 0u ? uint64_t(totals[kEntryBins]) : uint64_t(totals[b]) * width;
+    }
+    if (slot > 0xFFFFFFFFull || unit > 0xFFFFFFFFull) return fail(HSPMM_ERR_UNSUPPORTED, "the entry stream exceeds 32-bit positions");
+    // the stream in one allocation (each takes about 0.1 ms): ids, values, descriptors, pieces
+    const size_t units_kept = size_t(unit ? unit : 1u), ids_bytes = units_kept * 16u, vals_bytes = units_kept * 4u * p->elem;
+    const size_t desc_bytes = size_t(slot) * 12u, bytes = ids_bytes + vals_bytes + desc_bytes + size_t(totals[0]) * 12u;
+    Temporary stream;
+    HSPMM_HIP(hipMalloc(&stream.p, bytes));
+    char *at = static_cast<char *>(stream.p);
+    uint32_t *ids = reinterpret_cast<uint32_t *>(at), *desc = reinterpret_cast<uint32_t *>(at + ids_bytes + vals_bytes);
+    uint32_t *pieces = reinterpret_cast<uint32_t *>(at + ids_bytes + vals_bytes + desc_bytes);
+    HSPMM_HIP(hipMemcpyAsync(d_places, places, sizeof places, hipMemcpyHostToDevice, s));
+    HSPMM_HIP(launch_entry_fill(int(p->elem), p->d_data, p->d_a2b_raw, d_chunks, n_chunks, d_counts, d_len, p->rows, d_places,
+                                d_cursors, desc, pieces, d_first, ids, at + ids_bytes, s));
+    HSPMM_HIP(hipStreamSynchronize(s));         // (launches on other streams may follow at once)
+    hspmm_plan::Entries &e = p->entries;
+    std::copy(totals, totals + kEntryBins, e.slots);
+    e.n_pieces = totals[0];
+    e.long_rows = unit >= 64u * uint64_t(slot - totals[kEntryBins - 1u]);
+    e.d_stream = stream.p;
+    e.d_ids = ids; e.d_vals = at + ids_bytes; e.d_desc = desc; e.d_pieces = pieces;
+    stream.p = nullptr;
+    p->fixed_bytes += bytes;
+    e.built = true;
+    return HSPMM_OK;
+}
+
+// The classes of a launch; returns the number of workgroups.  A subgroup gets at most 4 << shift units.
+uint32_t fill_classes(const hspmm_plan *p, uint32_t lanes, int shift, hspmm::EntryArgs *ea)
+{
+    using namespace hspmm;
+    const uint32_t subgroups = 256u / lanes;                 // of a workgroup
+    uint32_t most = 0;
+    while ((2u << most) <= subgroups) ++most;
+    uint32_t group = 0, slot = 0;
+    ea->n_classes = 0;
+    auto add = [&](uint32_t slots, int wanted) {
+        if (!slots) return;
+        const uint32_t log2g = std::min(uint32_t(std::max(wanted, 0)), most);
+        ea->cls[ea->n_classes++] = {group, slot, slot + slots, log2g};
+        const uint32_t per_group = subgroups >> log2g;
+        group += (slots + per_group - 1u) / per_group;
+        slot += slots;
+    };
+    const uint32_t *n = p->entries.slots;
+    const uint32_t top = kEntryClassesByLength - 1u;
+    add(n[0], int(top) - shift);
+    for (uint32_t c = top;; --c) {
+        const uint32_t *bins = n + 1u + (top - c) * 4u;
+        add(bins[0] + bins[1] + bins[2] + bins[3], int(c) - shift);
+        if (c == 0u) break;
+    }
+    add(n[kEntryBins - 1u], 0);
+    return group;
+}
+
+}  // namespace
+
+namespace hspmm_host {
+
+constexpr uint32_t kEntryMaxRowBytes = 512;        // 32 lanes of 16 bytes
+
+// Feature blocks of 128 bytes resp. half a row on XCDs of their own (see spmm_mfma_kernel.hpp), here for rows of 256 bytes
+// (fp32 storage: also 512): pays where B is far larger than an L2 and no row of it is hot (uniform 65536^2, 16 per row:
+// fp16 N = 128 34 -> 29 us, fp32 N = 64 34 -> 30 us); with the hot rows of a power-law graph it only adds passes over
+// the entries (2^20 vertices, N = 128: 474 -> 510 us).
+static bool entries_by_xcd(const hspmm_plan *p, uint64_t row_bytes)
+{
+    return p->even_windows && (row_bytes == 256u || (row_bytes == 512u && p->elem == 4u)) &&
+           uint64_t(p->cols) * row_bytes >= (uint64_t(8) << 20);
+}
+
+// What an entry costs here is the lines of its row of B, what a tile column costs in the MFMA kernels does not depend
+// on how many of its eight elements are stored nor, up to a block of 32 features (16 of fp32 storage), on N.  So the line goes by
+// the bytes of a row of B and by the stored entries per tile column (per_column: 1.0 for graphs, 1.4 for weights
+// pruned to 10 %, 1.9 to 20 %, 8 for blocks).  Measured (entry / other kernels, us):
+//   16 bits, graph 2^18 N = 1 / 16 / 64: 14.5 / 45, 26 / 41, 44 / 53;  N = 100: 85 / 134, N = 200: 174 / 214 (there the
+//   other kernels lack the word-load layout), N = 128: 95 / 87, N = 192: 144 / 136;  uniform 8192^2 at 2 %, N = 256: 35 / 51
+//   16 bits, 4096^2 pruned to 10 % N = 8 / 16: 5.8 / 10.3, 7 / 10.4; 4096 x 11008 N = 32: 24.6 / 22.5; to 30 % N = 8 / 16:
+//   10 / 15.3, 16 / 15.3
+//   fp32, graph of 150001 N = 16 / 64 / 128: 18 / 39, 43 / 68, 92 / 126; 4096^2 pruned to 10 % N = 8 / 32 / 64: 6 / 19.5,
+//   12 / 19.5, 21 / 19.4; to 30 % N = 12 / 16: 24 / 29.7, 24 / 21; graph of 691333 (B of 354 MB) N = 128: 326 / 300
+bool entries_serve(const hspmm_plan *p, uint32_t N)
+{
+    const Config &c = p->cfg;
+    // (the caller's own settings are settings of the gather kernels)
+    if (c.kernel_mode != 0 || c.entries == 0 || c.fused_fixup >= 0 || c.buffer_stage || c.consumer_warp_num || c.producer_warp_group_num)
+        return false;
+    if (!p->caller_cuts.empty() || p->rows >= (1u << 31)) return false;
+    const uint64_t row = uint64_t(N) * p->elem, all = uint64_t(p->cols) * row;
+    if (row > kEntryMaxRowBytes) return false;
+    if (c.entries > 0) return true;
+    const double per_column = p->per_column, weight = double(row) * (per_column - 0.8);
+    if (p->G != 1 || per_column > 3.5) return false;
+    const bool sparse = per_column <= 1.25;
+    if (p->elem == 4u) {
+        if (weight <= 100.0) return true;
+        return sparse && !p->panel.built && (row <= 256u || all <= (uint64_t(256) << 20));
+    }
+    if (weight <= 42.0 || (sparse && row <= 128u)) return true;
+    if (!sparse) return false;
+    return (N % 64u != 0u && row <= 400u) || (per_column <= 1.15 && all <= (uint64_t(6) << 20)) || entries_by_xcd(p, row);
+}
+
+int run_entries(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode, bool *taken)
+{
+    const uint32_t row_bytes = N * p->elem;
+    const bool by_xcd = entries_by_xcd(p, row_bytes);
+    const uint32_t blocks = by_xcd ? 2u : 1u, block_bytes = row_bytes / blocks;
+    const RowShare share = share_row(block_bytes);
+    hspmm::EntryArgs ea{};
+    hspmm_plan::Entries &e = p->entries;
+    *taken = false;
+    {
+        std::lock_guard<std::mutex> lk(p->mu);
+        if (!e.built) {
+            if (mode == RunMode::kStatic)
+                return fail(HSPMM_ERR_UNSUPPORTED, "hspmm_run_static: the entry stream of narrow feature dimensions is not built yet; "
+                            "call hspmm_prepare(plan, N) or hspmm_run once with this N first");
+            hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+            if (mode == RunMode::kLaunch && s && (hipStreamIsCapturing(s, &status) != hipSuccess || status != hipStreamCaptureStatusNone))
+                return HSPMM_OK;                // (nothing can be built under capture: the gather kernels take it)
+            if (const int rc = build_entries(p, s)) return rc;
+        }
+        // Units per subgroup: long chains need few waves and add few sums (all rows long: 4096 x 11008 at 10 %, N = 8:
+        // 17.4 -> 13.0 us from 4 to 16), but where rows are short a launch takes as long as its longest chain
+        // (graph of 2^18, N = 16: 30 us at 8, 26 at 4) unless it has waves for several rounds.
+        if (e.long_rows) ea.n_groups = fill_classes(p, share.lanes, 2, &ea);
+        else if ((ea.n_groups = fill_classes(p, share.lanes, 1, &ea)) < uint32_t(p->compute_units) * 16u)
+            ea.n_groups = fill_classes(p, share.lanes, 0, &ea);
+        ea.n_pieces = e.n_pieces;
+        if (e.n_pieces) {
+            // sums of the pieces, and behind them, where nothing may be allocated, their counters
+            const size_t sums = size_t(e.n_pieces) * blocks * share.lanes * share.lane_bytes / p->elem * 4u;
+            if (const int rc = scratch_for(p, s, mode == RunMode::kStatic ? sums + size_t(e.n_pieces) * blocks * 4u : sums, mode, &ea.scratch)) return rc;
+            if (mode == RunMode::kStatic) {
+                ea.arrive = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(ea.scratch) + sums);
+                HSPMM_HIP(hspmm::launch_fill_zero(ea.arrive, size_t(e.n_pieces) * blocks * 4u, s));
+            } else if (const int rc = ensure_arrive(p, s, size_t(e.n_pieces) * blocks, mode, &ea.arrive)) {
+                return rc;
+            }
+        }
+    }
+    *taken = true;
+    if (mode == RunMode::kPrepare) return HSPMM_OK;
+    ea.desc = e.d_desc; ea.ids = e.d_ids; ea.vals = e.d_vals; ea.pieces = e.d_pieces;
+    ea.B = dB; ea.C = dC; ea.ld = N; ea.block_bytes = block_bytes; ea.n_feat_blocks = blocks; ea.xcd_split = by_xcd;
+    p->note_launch(2, 0, 0);
+    HSPMM_HIP(hspmm::launch_spmm_entries(p->dtype, ea, share.lane_bytes, share.lanes, s));
+    return HSPMM_OK;
+}
+
+}  // namespace hspmm_host

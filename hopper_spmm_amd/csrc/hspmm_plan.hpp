@@ -61,6 +61,7 @@ struct Config {
     int panel_max_windows = 0;          // 2 or 4: windows per unit of the panel stream (0: by matrix size)
     int aligned_small = -1;             // small matrices: waves per unit of the one-workgroup-per-unit partition (-1: by size; 0, 4, 8)
     int gather_bitmap = -1;             // gather kernels read single 16-bit windows as bitmap + stored elements (-1: by fill)
+    int entries = -1;                   // entry kernels for narrow feature dimensions (-1: by width, 0 never, 1 wherever they can)
     int xcd_split = -1;                 // gather kernels: two feature blocks dealt out by XCD half (-1: by matrix, 0 never, 1 always)
     // (set through hspmm_set_panel_stream; builds with HSPMM_EXPERIMENTAL only)
     int panel_tall = 0;                 // LDS-panel waves with two units each
@@ -75,6 +76,7 @@ struct Config {
         if (const char *e = std::getenv("HSPMM_PANEL_CHUNKS")) panel_chunks = std::max(1, std::atoi(e));
         if (const char *e = std::getenv("HSPMM_PANEL_MAX_WINDOWS")) panel_max_windows = std::atoi(e) >= 4 ? 4 : 2;
         if (const char *e = std::getenv("HSPMM_XCD_SPLIT")) xcd_split = std::atoi(e) != 0;
+        if (const char *e = std::getenv("HSPMM_ENTRIES")) entries = std::atoi(e) != 0;
         if (const char *e = std::getenv("HSPMM_GATHER_BITMAP")) gather_bitmap = std::atoi(e) != 0;
         if (const char *e = std::getenv("HSPMM_ALIGNED_SMALL")) { const int v = std::atoi(e); aligned_small = v == 4 || v == 8 ? v : 0; }
         if (const char *e = std::getenv("HSPMM_PANEL_UNITS_PER_GROUP")) panel_units_per_group = std::max(1, std::atoi(e));
@@ -161,6 +163,19 @@ struct hspmm_plan {
         uint64_t stored = 0;
         bool from_caller = false;     // header and elements are the caller's tcBit / nnzOffset / data, uploaded as they came
     } bm;
+    // Stored entries, rows sorted by length, for narrow feature dimensions (spmm_entries.hip): made from the tiles on the
+    // device by the first launch (or hspmm_prepare) that wants it
+    struct Entries {
+        bool built = false;
+        void *d_stream = nullptr;                                // one allocation for the four below
+        const uint32_t *d_desc = nullptr, *d_ids = nullptr, *d_pieces = nullptr;
+        const void *d_vals = nullptr;
+        uint32_t slots[hspmm::kEntryBins] = {};                  // rows per bin (bin 0: pieces)
+        uint32_t n_pieces = 0;
+        bool long_rows = false;                                  // 64 units and more in a row on average
+    } entries;
+    double per_column = 8.0;            // stored entries per tile column, from a sample of the tiles
+    bool even_windows = false;          // no unit has over eight times the average number of steps
     // What launches write besides C, one set per stream that has launched this plan (launches on different
     // streams may overlap in time): the first stream seen gets set 0, every other stream a set of its own at its
     // first launch - except a stream that is being captured (no allocation under capture) and streams beyond
@@ -238,6 +253,13 @@ int validate_format(uint32_t rows, uint32_t cols, uint32_t W, uint32_t T, uint32
                     bool *canonical = nullptr);
 int choose_ranges(const hspmm_plan *p);
 int build_and_upload_partition(hspmm_plan *p, int level, uint32_t group = 1, bool aligned = false);
+
+// hspmm_run.hip: memory a launch writes besides C (called with the plan's mutex held)
+int ensure_arrive(hspmm_plan *p, hipStream_t s, size_t words, RunMode mode, uint32_t **out);
+int scratch_for(hspmm_plan *p, hipStream_t s, size_t bytes, RunMode mode, float **out);
+// hspmm_entries.hip: whether the entry kernels take this launch, and the launch
+bool entries_serve(const hspmm_plan *p, uint32_t N);
+int run_entries(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode, bool *taken);
 
 // hspmm_run.hip: the address of the device's fixed scratch array (hspmm_run_static); `device` must be current
 int static_scratch_address(int device, float **out);

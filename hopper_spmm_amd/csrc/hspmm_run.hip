@@ -137,6 +137,10 @@ std::vector<hspmm_plan::StreamBuffers *> sets_for(hspmm_plan *p, hipStream_t s, 
     return sets;
 }
 
+}  // namespace
+
+namespace hspmm_host {
+
 // Arrival counters of the in-kernel reduction (never used by hspmm_run_static).
 // Called with the plan's mutex held.
 int ensure_arrive(hspmm_plan *p, hipStream_t s, size_t words, RunMode mode, uint32_t **out)
@@ -190,7 +194,7 @@ int scratch_for(hspmm_plan *p, hipStream_t s, size_t bytes, RunMode mode, float 
     return HSPMM_OK;
 }
 
-}  // namespace
+}  // namespace hspmm_host
 
 static int run_impl(hspmm_plan *p, const void *dB, void *dC, uint32_t N, void *stream, hipEvent_t mid, RunMode mode);
 
@@ -402,6 +406,11 @@ static int run_impl(hspmm_plan *p, const void *dB, void *dC, uint32_t N, void *s
         p->note_launch(4, 0, 0);
         HSPMM_HIP(hspmm::launch_fill_zero(dC, size_t(p->rows) * N * p->elem, s));
         return HSPMM_OK;
+    }
+    if (entries_serve(p, N)) {
+        bool taken = false;
+        const int rc = run_entries(p, dB, dC, N, s, mode, &taken);
+        if (rc || taken) return rc;
     }
     if (panel_serves(p, N)) return run_panel(p, dB, dC, N, s, mid, mode);
     // A feature dimension that no wide load divides (16-bit types: N not a multiple of 8, fp32 storage: of 4) would

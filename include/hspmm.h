@@ -77,7 +77,9 @@ int hspmm_create(hspmm_plan **plan, int dtype, uint32_t rows, uint32_t cols,
  * hipStream_t, NULL = default stream).
  * Host side: a plan is immutable after hspmm_create except for what the first
  * launch with a new N, or on a new stream, may add under the plan's own mutex -
- * a work partition for that width and buffers for what a launch writes besides C
+ * a work partition for that width or, for narrow feature dimensions, the matrix
+ * once more entry by entry (made on the device, which that launch waits for; not
+ * made under stream capture, where such a launch takes other kernels), and buffers for what a launch writes besides C
  * (partial sums of cut windows, their arrival counters; older buffers stay
  * allocated until hspmm_destroy, so launches recorded earlier, e.g. in a HIP
  * graph, stay valid whatever N is run afterwards).  hspmm_run may therefore be
@@ -259,8 +261,8 @@ typedef struct {
     uint32_t n_panel_units;     /* units of that stream: groups of up to four adjacent windows that share, or were given, one column list */
     uint32_t n_panel_paired_units;  /* of those: units of two or more windows */
     uint32_t n_panel_wide_units;    /* of those: units of three or four windows */
-    uint32_t last_kernel_family;    /* what the last hspmm_run launched: 0 nothing yet, 1 all-shapes kernel, 2 gather (MFMA) kernels,
-                                       3 LDS-staging kernels, 4 clear only (matrix without entries) */
+    uint32_t last_kernel_family;    /* what the last hspmm_run launched: 0 nothing yet, 1 all-shapes kernel, 2 gather kernels (MFMA, or entry
+                                       by entry for narrow feature dimensions: last_mfma_kind 0 then), 3 LDS-staging kernels, 4 clear only (matrix without entries) */
     uint32_t gather_bitmap;         /* 1: the gather kernels read this plan's tiles as bitmap + stored elements (single
                                      * windows with few stored elements per tile), 0: as uncompressed tiles */
     uint32_t bitmap_from_caller;    /* 1: the plan was made from bitmap tiles (hspmm_create_bitmap / _grouped) and uploaded them as they
