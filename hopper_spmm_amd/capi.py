@@ -133,6 +133,9 @@ def load_library():
     L.hspmm_btcf_fill.argtypes = [i, u32, vp, vp, vp, i, vp, vp, vp, vp]
     L.hspmm_btcf_sizes_cw.argtypes = [i, u32, u32, vp, vp, C.POINTER(u32), C.POINTER(u32)]
     L.hspmm_btcf_fill_cw.argtypes = [i, u32, u32, vp, vp, vp, i, vp, vp, vp, vp]
+    L.hspmm_count_tiles.argtypes = [i, u32, u32, vp, vp, vp, C.POINTER(u32), C.POINTER(u32)]
+    L.hspmm_btcf_fill_counted.argtypes = [i, u32, u32, vp, vp, vp, i, vp, vp, vp, vp, vp]
+    L.hspmm_bitmap_fill_counted.argtypes = [i, u32, vp, vp, vp, i, i, vp, vp, vp, vp, vp, vp, vp]
     L.hspmm_bitmap_sizes.argtypes = [i, u32, vp, vp, C.POINTER(u32), C.POINTER(u32), C.POINTER(u32)]
     L.hspmm_bitmap_fill.argtypes = [i, u32, vp, vp, vp, i, i, vp, vp, vp, vp, vp, vp]
     L.hspmm_bitmap_expand.argtypes = [i, u32, vp, vp, vp, vp]
@@ -249,14 +252,15 @@ def csr_to_btcf(rows, cols, row_ptr, col_idx, values, dtype, transpose=False, cw
     if row_ptr.size != rows + 1:
         raise ValueError("row_ptr must have rows + 1 entries")
     W, T = C.c_uint32(), C.c_uint32()
-    _check(L.hspmm_btcf_sizes_cw(dtype, cw, rows, _p(row_ptr), _p(col_idx), C.byref(W), C.byref(T)))
+    window_tiles = np.empty(max(1, (rows + ROW_WINDOW - 1) // ROW_WINDOW), np.uint32)
+    _check(L.hspmm_count_tiles(dtype, cw, rows, _p(row_ptr), _p(col_idx), _p(window_tiles), C.byref(W), C.byref(T)))
     W, T = W.value, T.value
     rowOffset = np.zeros(W + 1, np.uint32)
     tcA2B = np.empty(T * cw, np.uint32)
     data = np.empty(T * ROW_WINDOW * cw, vt)
     rowIdx = np.empty(W, np.uint32)
-    _check(L.hspmm_btcf_fill_cw(dtype, cw, rows, _p(row_ptr), _p(col_idx), _p(values), int(transpose),
-                                _p(rowOffset), _p(tcA2B), _p(data), _p(rowIdx)))
+    _check(L.hspmm_btcf_fill_counted(dtype, cw, rows, _p(row_ptr), _p(col_idx), _p(values), int(transpose), _p(window_tiles),
+                                     _p(rowOffset), _p(tcA2B), _p(data), _p(rowIdx)))
     return dict(rows=rows, cols=cols, nnzs=int(col_idx.size), dtype=dtype, cw=cw, transposed=bool(transpose),
                 total_row_windows=(rows + ROW_WINDOW - 1) // ROW_WINDOW, eff_row_windows=W,
                 total_tiles=T, rowOffset=rowOffset, tcA2B=tcA2B, data=data, rowIdx=rowIdx)
@@ -307,17 +311,18 @@ def csr_to_bitmap(rows, cols, row_ptr, col_idx, values, dtype, transpose=False, 
     values = np.ascontiguousarray(values, vt)
     if row_ptr.size != rows + 1:
         raise ValueError("row_ptr must have rows + 1 entries")
-    W, T, S = C.c_uint32(), C.c_uint32(), C.c_uint32()
-    _check(L.hspmm_bitmap_sizes(dtype, rows, _p(row_ptr), _p(col_idx), C.byref(W), C.byref(T), C.byref(S)))
-    W, T, S = W.value, T.value, S.value
+    W, T, S = C.c_uint32(), C.c_uint32(), int(row_ptr[rows])        # every CSR entry is stored
+    window_tiles = np.empty(max(1, (rows + ROW_WINDOW - 1) // ROW_WINDOW), np.uint32)
+    _check(L.hspmm_count_tiles(dtype, cw, rows, _p(row_ptr), _p(col_idx), _p(window_tiles), C.byref(W), C.byref(T)))
+    W, T = W.value, T.value
     rowOffset = np.zeros(W + 1, np.uint32)
     nnzOffset = np.zeros(T + 1, np.uint32)
     tcA2B = np.empty(T * cw, np.uint32)
     tcBit = np.empty(T * words, np.uint64)
     data = np.empty(S, vt)
     rowIdx = np.empty(W, np.uint32)
-    _check(L.hspmm_bitmap_fill(dtype, rows, _p(row_ptr), _p(col_idx), _p(values), int(transpose), int(bit_layout),
-                               rowOffset.ctypes.data_as(C.c_void_p), nnzOffset.ctypes.data_as(C.c_void_p),
+    _check(L.hspmm_bitmap_fill_counted(dtype, rows, _p(row_ptr), _p(col_idx), _p(values), int(transpose), int(bit_layout),
+                               _p(window_tiles), rowOffset.ctypes.data_as(C.c_void_p), nnzOffset.ctypes.data_as(C.c_void_p),
                                _p(tcA2B), _p(tcBit), _p(data), _p(rowIdx)))
     return dict(rows=rows, cols=cols, nnzs=int(col_idx.size), dtype=dtype, cw=cw,
                 total_row_windows=(rows + ROW_WINDOW - 1) // ROW_WINDOW, eff_row_windows=W,
@@ -443,6 +448,7 @@ class Plan:
         (it has "tcBit") or bitmap_to_grouped (it has "groupOffset")."""
         L = load_library()
         self._h = C.c_void_p()
+        self._run = L.hspmm_run          # (bound once: a run's host time is what small operators are made of)
         self.dtype = btcf["dtype"]
         self.rows, self.cols = int(btcf["rows"]), int(btcf["cols"])
         vt = _val_dtype(self.dtype)
@@ -480,7 +486,9 @@ class Plan:
 
     def run(self, dB_ptr, dC_ptr, N, stream=0):
         """dB_ptr / dC_ptr: integer device addresses (e.g. torch tensor .data_ptr())."""
-        _check(load_library().hspmm_run(self._h, C.c_void_p(dB_ptr), C.c_void_p(dC_ptr), N, C.c_void_p(stream)))
+        rc = self._run(self._h, dB_ptr, dC_ptr, N, stream)
+        if rc:
+            _check(rc)
 
     def run_static(self, dB_ptr, dC_ptr, N, stream=0):
         """hspmm_run_static: the same launch with its partial sums in the library's fixed device array

@@ -35,16 +35,17 @@ void parallel_chunks(size_t n, size_t chunk, F &&fn, unsigned workers = 0)
     std::atomic<size_t> next{0};
     std::vector<std::thread> th;
     std::vector<std::exception_ptr> err(nw);
-    th.reserve(nw);
-    for (unsigned i = 0; i < nw; ++i)
-        th.emplace_back([&fn, &err, &next, i, n, chunk] {
-            try {
-                for (size_t b = next.fetch_add(chunk); b < n; b = next.fetch_add(chunk)) fn(b, std::min(n, b + chunk));
-            } catch (...) {
-                err[i] = std::current_exception();
-                next.store(n);                        // the others stop at their next chunk
-            }
-        });
+    th.reserve(nw - 1);
+    auto work = [&fn, &err, &next, n, chunk](unsigned i) {
+        try {
+            for (size_t b = next.fetch_add(chunk); b < n; b = next.fetch_add(chunk)) fn(b, std::min(n, b + chunk));
+        } catch (...) {
+            err[i] = std::current_exception();
+            next.store(n);                            // the others stop at their next chunk
+        }
+    };
+    for (unsigned i = 1; i < nw; ++i) th.emplace_back(work, i);
+    work(0);                                          // (the calling thread is one of the workers)
     for (auto &t : th) t.join();
     for (auto &e : err) if (e) std::rethrow_exception(e);
 }

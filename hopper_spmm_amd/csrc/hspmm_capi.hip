@@ -245,16 +245,8 @@ int hspmm_panel_units_preview(int dtype, uint32_t rows, uint32_t cols, uint32_t 
 void hspmm_destroy(hspmm_plan *p)
 {
     if (!p) return;
-    (void)hipFree(p->d_rowOffset); (void)hipFree(p->d_rowIdx); (void)hipFree(p->d_a2b_raw);
-    if (p->d_tiles != p->d_data) (void)hipFree(p->d_tiles);
-    (void)hipFree(p->d_data); (void)hipFree(p->d_unitOffset); (void)hipFree(p->d_unitRow); (void)hipFree(p->d_ids);
-    for (auto &dp : p->parts) { (void)hipFree(dp.d_ranges); (void)hipFree(dp.d_split); (void)hipFree(dp.d_fix_slots); }
-    (void)hipFree(p->panel.d_poff); (void)hipFree(p->panel.d_ids); (void)hipFree(p->panel.d_tiles);
-    (void)hipFree(p->panel.d_unitRow);
-    (void)hipFree(p->panel.d_step_panel);
-    (void)hipFree(p->panel.d_masks); (void)hipFree(p->panel.d_vals); (void)hipFree(p->panel.d_step_voff);
+    for (void *mine : p->owned) (void)hipFree(mine);
     (void)hipFree(p->entries.d_stream);
-    (void)hipFree(p->bm.d_header); (void)hipFree(p->bm.d_vals);
     for (auto &b : p->buffers) { (void)hipFree(b.d_scratch); (void)hipFree(b.d_arrive); (void)hipFree(b.d_vector); }
     for (void *old : p->retired) (void)hipFree(old);
     delete p;

@@ -3,6 +3,7 @@
 // work partition.  Everything the reference's fp16_spmm does before its first launch (reference
 // src/fp16.cu:221-254), done once per matrix.
 #include "hspmm_plan.hpp"
+#include "hspmm_pack.hpp"
 
 using namespace hspmm_host;
 
@@ -12,7 +13,7 @@ namespace hspmm_host {
 // the window's last column, as the reference's converter writes them (src/utils/convert.h:166-181).
 int validate_format(uint32_t rows, uint32_t cols, uint32_t W, uint32_t T, uint32_t cw,
                     const uint32_t *rowOffset, const uint32_t *tcA2B, const void *data, const uint32_t *rowIdx,
-                    bool *canonical)
+                    bool *canonical, uint32_t *header, uint32_t *window_stored)
 {
     if (canonical) *canonical = true;
     if (W == 0) {
@@ -47,35 +48,69 @@ int validate_format(uint32_t rows, uint32_t cols, uint32_t W, uint32_t T, uint32
         }
         return false;
     };
+    // (one pass on all cores for the ids, their order and, where asked for, what the tiles store)
     std::atomic<uint32_t> first_bad{T};
-    hspmm_host::parallel_blocks(T, 65536, [&](size_t tb, size_t te) {
-        if (tb >= first_bad.load(std::memory_order_relaxed)) return;
-        for (size_t t = tb; t < te; ++t)
+    std::atomic<bool> ordered{true};
+    const size_t windows = std::max<size_t>(1, (size_t(1) << 13) / std::max<uint32_t>(1u, T / W));
+    hspmm_host::parallel_blocks(W, windows, [&](size_t wb, size_t we) {
+        for (size_t t = rowOffset[wb], e = rowOffset[we]; t < e; ++t)
             if (tile_error(uint32_t(t), false)) {
                 uint32_t seen = first_bad.load(std::memory_order_relaxed);
                 while (uint32_t(t) < seen && !first_bad.compare_exchange_weak(seen, uint32_t(t), std::memory_order_relaxed)) {}
                 return;
             }
+        for (size_t w = wb; canonical && w < we && ordered.load(std::memory_order_relaxed); ++w) {
+            const uint32_t *c = tcA2B + size_t(rowOffset[w]) * cw;
+            const size_t n = size_t(rowOffset[w + 1] - rowOffset[w]) * cw;
+            size_t real = n;
+            while (real && c[real - 1] == HSPMM_IDX_MAX) --real;
+            bool good = n - real < cw;                      // padding only in the window's last tile
+            for (size_t i = 1; i < real && good; ++i) good = c[i] != HSPMM_IDX_MAX && c[i] > c[i - 1];
+            if (!good) ordered.store(false, std::memory_order_relaxed);
+        }
+        for (size_t w = wb; header && w < we; ++w)
+            window_stored[w] = uint32_t(hspmm_host::tile_masks(static_cast<const char *>(data) + size_t(rowOffset[w]) * 256u,
+                                                               rowOffset[w + 1] - rowOffset[w], cw == 16u ? 2u : 4u,
+                                                               header + size_t(rowOffset[w]) * (cw == 16u ? 8u : 4u)));
     });
     if (first_bad.load() < T) { tile_error(first_bad.load(), true); return HSPMM_ERR_INVALID; }
-    if (canonical) {
-        std::atomic<bool> ok{true};
-        hspmm_host::parallel_blocks(W, 4096, [&](size_t wb, size_t we) {
-            for (size_t w = wb; w < we && ok.load(std::memory_order_relaxed); ++w) {
-                const uint32_t *c = tcA2B + size_t(rowOffset[w]) * cw;
-                const size_t n = size_t(rowOffset[w + 1] - rowOffset[w]) * cw;
-                size_t real = n;
-                while (real && c[real - 1] == HSPMM_IDX_MAX) --real;
-                bool good = n - real < cw;                      // padding only in the window's last tile
-                for (size_t i = 1; i < real && good; ++i) good = c[i] != HSPMM_IDX_MAX && c[i] > c[i - 1];
-                if (!good) ok.store(false, std::memory_order_relaxed);
-            }
-        });
-        *canonical = ok.load();
-    }
+    if (canonical) *canonical = ordered.load();
     return HSPMM_OK;
 }
 
+int plan_reserve(hspmm_plan *p, size_t bytes)
+{
+    void *fresh = nullptr;
+    HSPMM_HIP(hipMalloc(&fresh, bytes));
+    p->owned.push_back(fresh);
+    p->block = static_cast<char *>(fresh);
+    p->block_left = bytes;
+    return HSPMM_OK;
+}
+
+int plan_alloc(hspmm_plan *p, size_t bytes, void **out)
+{
+    const size_t rounded = (bytes + 255u) & ~size_t(255);
+    if (rounded <= p->block_left) {
+        *out = p->block;
+        p->block += rounded;
+        p->block_left -= rounded;
+    } else {
+        HSPMM_HIP(hipMalloc(out, bytes));
+        p->owned.push_back(*out);
+    }
+    p->fixed_bytes += bytes;
+    return HSPMM_OK;
+}
+
+void plan_release(hspmm_plan *p, const void *ptr, size_t bytes)
+{
+    const auto it = std::find(p->owned.begin(), p->owned.end(), ptr);
+    if (it == p->owned.end()) return;           // (part of the reserved block)
+    (void)hipFree(*it);
+    p->owned.erase(it);
+    p->fixed_bytes -= bytes;
+}
 
 int choose_ranges(const hspmm_plan *p)
 {
@@ -113,9 +148,9 @@ int build_and_upload_partition(hspmm_plan *p, int level, uint32_t group, bool al
         d[0] = part.split[i].window; d[1] = part.split[i].slot_begin; d[2] = part.split[i].slot_count;
     }
     int rc;
-    if ((rc = upload(&dp.d_ranges, rw.data(), rw.size(), &p->fixed_bytes))) return rc;
-    if ((rc = upload(&dp.d_split, sw.data(), sw.size(), &p->fixed_bytes))) return rc;
-    if ((rc = upload(&dp.d_fix_slots, part.fix_slots.data(), part.fix_slots.size(), &p->fixed_bytes))) return rc;
+    if ((rc = upload(p, &dp.d_ranges, rw.data(), rw.size()))) return rc;
+    if ((rc = upload(p, &dp.d_split, sw.data(), sw.size()))) return rc;
+    if ((rc = upload(p, &dp.d_fix_slots, part.fix_slots.data(), part.fix_slots.size()))) return rc;
     dp.built = true;
     return HSPMM_OK;
 }
@@ -123,42 +158,6 @@ int build_and_upload_partition(hspmm_plan *p, int level, uint32_t group, bool al
 }  // namespace hspmm_host
 
 namespace {
-
-// The bitmap stream of the gather kernels (Fp16TileDWB in spmm_mfma_kernel.hpp) from the uncompressed 8 x 16 tiles
-// of a 16-bit matrix, made on the device from the tiles already uploaded (p->d_data): per tile the bitmap of the
-// reference's CSR2BTCF (bit 16 r + k for element (r, k), reference src/utils/convert.h:83-101; an element is stored
-// when its bit pattern is not +0) as four 32-bit words, the bit counts of words 0, 0..1 and 0..2 in bytes 1..3 of
-// word 4, and in word 5 the position of the tile's first stored element in `vals` (the reference's nnzOffset),
-// where the stored elements follow tile after tile in bit order.  Leaves p->bm.built false when the positions
-// would not fit 31 bits.  (On the host this took 29 ms for the 257 MB of tiles of the 2^20 power-law graph.)
-int bitmap_from_uploaded_tiles(hspmm_plan *p, uint32_t T)
-{
-    const uint32_t n_blocks = hspmm::bitmap_scan_blocks(T);
-    const size_t header_bytes = size_t(T) * (p->elem == 2u ? 32u : 16u);     // fp32 tiles (8 x 8): two mask words, position, count
-    const size_t spare = 8u / p->elem;                                        // a lane may read 8 bytes from the last element on
-    uint64_t *d_sums = nullptr;
-    HSPMM_HIP(hipMalloc(reinterpret_cast<void **>(&p->bm.d_header), header_bytes));        // (released by hspmm_destroy)
-    HSPMM_HIP(hipMalloc(reinterpret_cast<void **>(&d_sums), (size_t(n_blocks) + 1u) * sizeof(uint64_t)));
-    auto done = [&](int code) { (void)hipFree(d_sums); return code; };
-    HSPMM_HIP_OR(hspmm::launch_bitmap_header(int(p->elem), p->d_data, p->bm.d_header, T, d_sums, nullptr), done);
-    uint64_t stored = 0;
-    HSPMM_HIP_OR(hipMemcpy(&stored, d_sums + n_blocks, sizeof(stored), hipMemcpyDeviceToHost), done);
-    if (stored + spare >= (uint64_t(1) << 31)) {                // positions are 32-bit
-        (void)hipFree(p->bm.d_header);
-        p->bm.d_header = nullptr;
-        return done(HSPMM_OK);
-    }
-    char *dv = nullptr;
-    HSPMM_HIP_OR(hipMalloc(reinterpret_cast<void **>(&dv), (size_t(stored) + spare) * p->elem), done);
-    p->bm.d_vals = dv;
-    HSPMM_HIP_OR(hipMemset(dv + size_t(stored) * p->elem, 0, spare * p->elem), done);
-    HSPMM_HIP_OR(hspmm::launch_bitmap_pack(int(p->elem), p->d_data, p->bm.d_header, dv, T, d_sums, nullptr), done);
-    HSPMM_HIP_OR(hipStreamSynchronize(nullptr), done);
-    p->bm.stored = stored;
-    p->bm.built = true;
-    p->fixed_bytes += header_bytes + (size_t(stored) + spare) * p->elem;
-    return done(HSPMM_OK);
-}
 
 // Re-tiles the matrix panel by panel for the LDS-panel kernels (spmm_panel_kernel.hpp):
 // inside every window the columns of one panel of kPanelRows columns get tiles of
@@ -409,9 +408,9 @@ bool build_panel_stream(hspmm_plan *p, const StepStream &gather_st, const uint32
         merge_unit_pairs(U, NP, tile_words, ps.unitOffset, poff, step_panel, ids, tiles);
         packed = p->cfg.panel_packed > 0;
     }
-    if ((rc = upload(&pl.d_poff, poff.data(), poff.size(), &p->fixed_bytes))) { *rc_out = rc; return false; }
-    if ((rc = upload(&pl.d_step_panel, step_panel.data(), step_panel.size(), &p->fixed_bytes))) { *rc_out = rc; return false; }
-    if ((rc = upload(&pl.d_ids, ids.data(), ids.size(), &p->fixed_bytes))) { *rc_out = rc; return false; }
+    if ((rc = upload(p, &pl.d_poff, poff.data(), poff.size()))) { *rc_out = rc; return false; }
+    if ((rc = upload(p, &pl.d_step_panel, step_panel.data(), step_panel.size()))) { *rc_out = rc; return false; }
+    if ((rc = upload(p, &pl.d_ids, ids.data(), ids.size()))) { *rc_out = rc; return false; }
     if (packed) {
         std::vector<uint64_t> masks;
         std::vector<uint8_t> vals;
@@ -420,15 +419,15 @@ bool build_panel_stream(hspmm_plan *p, const StepStream &gather_st, const uint32
         if (vals.size() >= (size_t(1) << 32)) packed = false;        // positions are 32-bit byte offsets in the kernel
         else {
             uint8_t *dv = nullptr;
-            if ((rc = upload(&pl.d_masks, masks.data(), masks.size(), &p->fixed_bytes))) { *rc_out = rc; return false; }
-            if ((rc = upload(&dv, vals.data(), vals.size(), &p->fixed_bytes))) { *rc_out = rc; return false; }
+            if ((rc = upload(p, &pl.d_masks, masks.data(), masks.size()))) { *rc_out = rc; return false; }
+            if ((rc = upload(p, &dv, vals.data(), vals.size()))) { *rc_out = rc; return false; }
             pl.d_vals = dv;
-            if ((rc = upload(&pl.d_step_voff, step_voff.data(), step_voff.size(), &p->fixed_bytes))) { *rc_out = rc; return false; }
+            if ((rc = upload(p, &pl.d_step_voff, step_voff.data(), step_voff.size()))) { *rc_out = rc; return false; }
         }
     }
     if (!packed) {
         uint32_t *dt = nullptr;
-        if ((rc = upload(&dt, tiles.data(), tiles.size(), &p->fixed_bytes))) { *rc_out = rc; return false; }
+        if ((rc = upload(p, &dt, tiles.data(), tiles.size()))) { *rc_out = rc; return false; }
         pl.d_tiles = dt;
     }
     pl.tall = tall; pl.packed = packed;
@@ -440,7 +439,7 @@ bool build_panel_stream(hspmm_plan *p, const StepStream &gather_st, const uint32
                                                  : double(tiles.size()) * 4.0 / double(std::max<uint32_t>(ps.n_steps, 1u)));
         pl.unit_lines = step_bytes * double(ps.n_steps) / (double(U) * double(NP)) / 128.0;
     }
-    if ((rc = upload(&pl.d_unitRow, st.unitRow.data(), st.unitRow.size(), &p->fixed_bytes))) { *rc_out = rc; return false; }
+    if ((rc = upload(p, &pl.d_unitRow, st.unitRow.data(), st.unitRow.size()))) { *rc_out = rc; return false; }
     pl.n_units = U; pl.G = st.G; pl.n_paired = st.n_paired; pl.n_wide = st.n_wide;
     pl.n_panels = NP; pl.n_steps = ps.n_steps; pl.quad = quad; pl.split = split; pl.density = density; pl.built = true;
     timer.mark("  panel: upload");
@@ -491,7 +490,9 @@ uint32_t bitmap_header_from_caller(uint32_t T, uint32_t elem, const BitmapSource
 }
 
 // Stored entries per real tile column, from 256 groups of 64 tiles spread over the matrix (every tile of a small one).
-double entries_per_column(uint32_t T, uint32_t cw, uint32_t elem, const uint32_t *tcA2B, const void *data, const BitmapSource *bitmap)
+// header: their masks, where they are known.
+double entries_per_column(uint32_t T, uint32_t cw, uint32_t elem, const uint32_t *tcA2B, const void *data, const BitmapSource *bitmap,
+                          const uint32_t *header)
 {
     const uint32_t group = 64u, groups = std::min(256u, (T + group - 1u) / group);
     uint64_t stored = 0, columns = 0;
@@ -500,6 +501,10 @@ double entries_per_column(uint32_t T, uint32_t cw, uint32_t elem, const uint32_t
         for (size_t i = size_t(t0) * cw; i < size_t(t1) * cw; ++i) columns += tcA2B[i] != HSPMM_IDX_MAX;
         if (bitmap) {
             stored += bitmap->nnzOffset[t1] - bitmap->nnzOffset[t0];
+        } else if (header) {
+            const uint32_t words = elem == 2u ? 8u : 4u, masks = words / 2u;
+            for (size_t t = t0; t < t1; ++t)
+                for (uint32_t q = 0; q < masks; ++q) stored += uint32_t(__builtin_popcount(header[t * words + q]));
         } else if (elem == 2u) {
             const uint16_t *v = static_cast<const uint16_t *>(data);
             for (size_t i = size_t(t0) * 8u * cw; i < size_t(t1) * 8u * cw; ++i) stored += v[i] != 0;
@@ -509,6 +514,24 @@ double entries_per_column(uint32_t T, uint32_t cw, uint32_t elem, const uint32_t
         }
     }
     return columns ? double(stored) / double(columns) : 8.0;
+}
+
+// Whether the gather kernels of a plan would read these plain tiles (single windows) as bitmap + stored elements:
+// 32 + 2 e bytes against 256 per tile with e stored elements (16 + 4 e for fp32) - worth it below about a third full, and
+// where the tile stream is large enough to be traffic at all (a matrix whose tiles sit in the L2s only pays the longer
+// dependent chain: 4096 x 4096 at 1 %, 2.7 MB of tiles: 6.8 -> 7.5 us).  From 64 groups of 64 tiles spread over the matrix.
+bool tiles_look_sparse(const Config &cfg, uint32_t T, uint32_t elem, const void *data)
+{
+    if (cfg.gather_bitmap >= 0) return cfg.gather_bitmap > 0;
+    if (size_t(T) * 256u < (size_t(8) << 20)) return false;
+    std::vector<uint32_t> header(64u * 8u);
+    uint64_t stored = 0, seen = 0;
+    for (uint32_t g = 0; g < 64u; ++g) {
+        const size_t t0 = size_t(uint64_t(T) * g / 64u), n = std::min<size_t>(64u, T - t0);
+        stored += hspmm_host::tile_masks(static_cast<const char *>(data) + t0 * 256u, n, elem, header.data());
+        seen += n * (256u / elem);
+    }
+    return stored * 3u < seen;
 }
 
 // hspmm_create; with `bitmap` (data == nullptr) the tiles come as the caller's bitmap arrays,
@@ -526,9 +549,23 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
     const uint32_t cw = dtype == HSPMM_TF32 ? 8u : 16u;
     const uint32_t elem = dtype == HSPMM_TF32 ? 4u : 2u;
     PhaseTimer timer;
+    Config cfg;
+    { std::lock_guard<std::mutex> lk(g_cfg_mutex); cfg = g_cfg; }
+    cfg.read_environment();                         // tuning overrides, once per plan
     bool canonical = true;
+    // Tiles that are mostly zeros go to the device as bitmap + stored elements and are expanded there: the gather kernels
+    // read that stream, and a graph of 2^18 vertices is 24 MB to send instead of 77.
+    hspmm_host::ZeroedBuffer<uint32_t> header;
+    std::vector<uint32_t> window_stored;
+    bool sparse_tiles = !bitmap && data && eff_row_windows && total_tiles && tiles_look_sparse(cfg, total_tiles, elem, data);
+    try {
+        if (sparse_tiles) {
+            header = hspmm_host::ZeroedBuffer<uint32_t>(size_t(total_tiles) * (elem == 2u ? 8u : 4u));
+            window_stored.assign(size_t(eff_row_windows) + 1u, 0u);
+        }
+    } catch (const std::bad_alloc &) { return fail(HSPMM_ERR_ALLOC, "out of host memory"); }
     int rc = validate_format(rows, cols, eff_row_windows, total_tiles, cw, rowOffset, tcA2B, bitmap ? bitmap->data : data, rowIdx,
-                             &canonical);
+                             &canonical, sparse_tiles ? header.data() : nullptr, window_stored.data());
     if (rc) return rc;
     timer.mark("validate");
 
@@ -536,8 +573,7 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
     if (!p) return fail(HSPMM_ERR_ALLOC, "out of host memory");
     p->dtype = dtype; p->rows = rows; p->cols = cols; p->W = eff_row_windows; p->T = total_tiles;
     p->cw = cw; p->elem = elem; p->canonical = canonical;
-    { std::lock_guard<std::mutex> lk(g_cfg_mutex); p->cfg = g_cfg; }
-    p->cfg.read_environment();                      // tuning overrides, once per plan
+    p->cfg = cfg;
 
     auto bail = [&](int code) { hspmm_destroy(p); return code; };
     hipError_t e = hipGetDevice(&p->device);
@@ -557,65 +593,89 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
 
     // (a host allocation that fails anywhere below ends the call with HSPMM_ERR_ALLOC)
     if (p->W) try {
-        const size_t n_ids = size_t(total_tiles) * cw;
-        if ((rc = upload(&p->d_rowOffset, rowOffset, size_t(p->W) + 1, &p->fixed_bytes))) return bail(rc);
-        if ((rc = upload(&p->d_rowIdx, rowIdx, size_t(p->W), &p->fixed_bytes))) return bail(rc);
-        if ((rc = upload(&p->d_a2b_raw, tcA2B, n_ids, &p->fixed_bytes))) return bail(rc);
-        if (!bitmap) {
-            uint8_t *dd = nullptr;
-            if ((rc = upload(&dd, static_cast<const uint8_t *>(data), size_t(total_tiles) * 8u * cw * elem,
-                             &p->fixed_bytes)))
-                return bail(rc);
-            p->d_data = dd;
-        } else {
-            // the caller's bitmap tiles: header from tcBit / nnzOffset, the stored elements as they are (and four
-            // more: a lane of the gather kernels reads 8 bytes from its first element), plain tiles by a kernel
-            hspmm_host::ZeroedBuffer<uint32_t> header;
-            const uint32_t bad = bitmap_header_from_caller(total_tiles, elem, *bitmap, header);
-            if (bad != HSPMM_IDX_MAX)
-                return bail(fail(HSPMM_ERR_INVALID, "tile %u: %s", bad, "the bit count of tcBit differs from the nnzOffset span"));
-            const size_t stored = bitmap->nnzOffset[total_tiles], spare = 8u / elem;
-            if (stored + spare >= (size_t(1) << 31)) return bail(kNeedsPlainTiles);      // positions are 32-bit
-            if ((rc = upload(&p->bm.d_header, header.data(), header.size(), &p->fixed_bytes))) return bail(rc);
-            char *dv = nullptr;
-            HSPMM_HIP_OR(hipMalloc(reinterpret_cast<void **>(&dv), (stored + spare) * elem), bail);
-            p->bm.d_vals = dv; p->bm.stored = stored; p->fixed_bytes += (stored + spare) * elem;
-            if (stored) HSPMM_HIP_OR(hipMemcpy(dv, bitmap->data, stored * elem, hipMemcpyHostToDevice), bail);
-            HSPMM_HIP_OR(hipMemset(dv + stored * elem, 0, 8), bail);
-            uint8_t *dd = nullptr;
-            HSPMM_HIP_OR(hipMalloc(reinterpret_cast<void **>(&dd), size_t(total_tiles) * 256u), bail);
-            p->d_data = dd; p->fixed_bytes += size_t(total_tiles) * 256u;
-            HSPMM_HIP_OR(hspmm::launch_expand_bitmap(int(elem), p->bm.d_header, dv, dd, total_tiles, nullptr), bail);
-            HSPMM_HIP_OR(hipStreamSynchronize(nullptr), bail);
-            p->bm.from_caller = true;
-        }
-        timer.mark("upload format arrays");
-        // padding ids -> the real id in front of them (the tile column is all zero)
-        // (padding trails a window's real ids, of which every window has one at least)
-        hspmm_host::ZeroedBuffer<uint32_t> clean_ids;
-        try { clean_ids = hspmm_host::ZeroedBuffer<uint32_t>(n_ids); }
-        catch (const std::bad_alloc &) { return bail(fail(HSPMM_ERR_ALLOC, "out of host memory")); }
-        uint32_t *clean = clean_ids.data();
-        hspmm_host::parallel_blocks(p->W, 1024, [&](size_t wb, size_t we) {
-            for (size_t i = size_t(rowOffset[wb]) * cw, e = size_t(rowOffset[we]) * cw; i < e; ++i)
-                clean[i] = (tcA2B[i] == HSPMM_IDX_MAX && i) ? clean[i - 1] : tcA2B[i];
-        });
-        timer.mark("ids without padding");
-        const StepStream st = build_units(p->W, cw, rowOffset, rowIdx, clean, p->cfg.pairing);
-        timer.mark("units");
+        const size_t n_ids = size_t(total_tiles) * cw, tile_bytes = size_t(total_tiles) * 256u;
+        const StepStream st = build_units(p->W, cw, rowOffset, rowIdx, tcA2B, p->cfg.pairing);
         if (bitmap && st.G != 1) return bail(kNeedsPlainTiles);         // paired windows: their tiles are re-laid out on the host
         p->G = st.G;
         p->n_units = uint32_t(st.unitRow.size());
         p->n_paired = st.n_paired;
         p->n_steps = st.n_steps;
-        if ((rc = upload(&p->d_unitOffset, st.unitOffset.data(), st.unitOffset.size(), &p->fixed_bytes))) return bail(rc);
-        if ((rc = upload(&p->d_unitRow, st.unitRow.data(), st.unitRow.size(), &p->fixed_bytes))) return bail(rc);
-        if (dtype != HSPMM_TF32 && st.G == 1) {
-            // single 16-bit windows: the steps are the caller's tiles in the caller's order, their ids these
-            if ((rc = upload(&p->d_ids, clean, n_ids, &p->fixed_bytes))) return bail(rc);
+        timer.mark("units");
+        const size_t spare = 8u / elem;                                 // a lane may read 8 bytes from the last element on
+        uint64_t stored = 0;
+        for (uint32_t w = 0; sparse_tiles && w < p->W; ++w) stored += window_stored[w];
+        sparse_tiles = sparse_tiles && st.G == 1 && stored + spare < (uint64_t(1) << 31) &&
+                       (p->cfg.gather_bitmap > 0 || stored * 3u < uint64_t(total_tiles) * 8u * cw);
+        // one block for everything whose size is known here, and a megabyte for the partitions
+        if ((rc = plan_reserve(p, (size_t(p->W) * 4u + 2u) * 4u + n_ids * 8u + tile_bytes + header.size() * 4u +
+                                      (sparse_tiles ? (size_t(stored) + spare) * elem : 0u) + (size_t(1) << 20))))
+            return bail(rc);
+        if ((rc = upload(p, &p->d_rowOffset, rowOffset, size_t(p->W) + 1))) return bail(rc);
+        if ((rc = upload(p, &p->d_rowIdx, rowIdx, size_t(p->W)))) return bail(rc);
+        if ((rc = upload(p, &p->d_a2b_raw, tcA2B, n_ids))) return bail(rc);
+        void *room = nullptr;
+        if (sparse_tiles) {
+            hspmm_host::ZeroedBuffer<uint8_t> vals((size_t(stored) + spare) * elem);
+            uint64_t at = 0;
+            std::vector<uint64_t> first(p->W);
+            for (uint32_t w = 0; w < p->W; ++w) { first[w] = at; at += window_stored[w]; }
+            const size_t windows = std::max<size_t>(1, (size_t(1) << 13) / std::max<uint32_t>(1u, total_tiles / p->W));
+            hspmm_host::parallel_blocks(p->W, windows, [&](size_t wb, size_t we) {
+                const uint32_t t0 = rowOffset[wb];
+                hspmm_host::pack_tiles(static_cast<const char *>(data) + size_t(t0) * 256u, rowOffset[we] - t0, elem,
+                                       header.data() + size_t(t0) * (elem == 2u ? 8u : 4u), first[wb], vals.data());
+            });
+            timer.mark("bitmap tiles");
+            uint8_t *dv = nullptr;
+            if ((rc = upload(p, &p->bm.d_header, header.data(), header.size()))) return bail(rc);
+            if ((rc = upload(p, &dv, vals.data(), vals.size()))) return bail(rc);
+            p->bm.d_vals = dv; p->bm.stored = stored; p->bm.built = true;
+            if ((rc = plan_alloc(p, tile_bytes, &room))) return bail(rc);
+            p->d_data = room;
+            HSPMM_HIP_OR(hspmm::launch_expand_bitmap(int(elem), p->bm.d_header, dv, room, total_tiles, nullptr), bail);
+        } else if (!bitmap) {
+            uint8_t *dd = nullptr;
+            if ((rc = upload(p, &dd, static_cast<const uint8_t *>(data), tile_bytes))) return bail(rc);
+            p->d_data = dd;
         } else {
+            // the caller's bitmap tiles: header from tcBit / nnzOffset, the stored elements as they are (and four
+            // more: a lane of the gather kernels reads 8 bytes from its first element), plain tiles by a kernel
+            const uint32_t bad = bitmap_header_from_caller(total_tiles, elem, *bitmap, header);
+            if (bad != HSPMM_IDX_MAX)
+                return bail(fail(HSPMM_ERR_INVALID, "tile %u: %s", bad, "the bit count of tcBit differs from the nnzOffset span"));
+            stored = bitmap->nnzOffset[total_tiles];
+            if (stored + spare >= (uint64_t(1) << 31)) return bail(kNeedsPlainTiles);    // positions are 32-bit
+            if ((rc = plan_alloc(p, tile_bytes, &room))) return bail(rc);
+            p->d_data = room;
+            if ((rc = upload(p, &p->bm.d_header, header.data(), header.size()))) return bail(rc);
+            const size_t vals_bytes = (size_t(stored) + spare) * elem;
+            if ((rc = plan_alloc(p, vals_bytes, &room))) return bail(rc);
+            char *dv = static_cast<char *>(room);
+            p->bm.d_vals = dv; p->bm.stored = stored;
+            if (stored) HSPMM_HIP_OR(hipMemcpy(dv, bitmap->data, size_t(stored) * elem, hipMemcpyHostToDevice), bail);
+            HSPMM_HIP_OR(hipMemset(dv + size_t(stored) * elem, 0, 8), bail);
+            HSPMM_HIP_OR(hspmm::launch_expand_bitmap(int(elem), p->bm.d_header, dv, p->d_data, total_tiles, nullptr), bail);
+            HSPMM_HIP_OR(hipStreamSynchronize(nullptr), bail);
+            p->bm.from_caller = true;
+        }
+        timer.mark("upload format arrays");
+        if ((rc = upload(p, &p->d_unitOffset, st.unitOffset.data(), st.unitOffset.size()))) return bail(rc);
+        if ((rc = upload(p, &p->d_unitRow, st.unitRow.data(), st.unitRow.size()))) return bail(rc);
+        // padding ids -> the real id in front of them (the tile column is all zero; no tile starts with padding)
+        if (st.G == 1) {
+            // single windows: the steps are the caller's tiles in the caller's order
+            if ((rc = plan_alloc(p, n_ids * 4u, &room))) return bail(rc);
+            p->d_ids = static_cast<uint32_t *>(room);
+            HSPMM_HIP_OR(hspmm::launch_step_ids(int(elem), p->d_a2b_raw, p->d_ids, total_tiles, nullptr), bail);
+        } else {
+            hspmm_host::ZeroedBuffer<uint32_t> clean_ids(n_ids);
+            uint32_t *clean = clean_ids.data();
+            hspmm_host::parallel_blocks(p->W, 1024, [&](size_t wb, size_t we) {
+                for (size_t i = size_t(rowOffset[wb]) * cw, e = size_t(rowOffset[we]) * cw; i < e; ++i)
+                    clean[i] = (tcA2B[i] == HSPMM_IDX_MAX && i) ? clean[i - 1] : tcA2B[i];
+            });
             const hspmm_host::ZeroedBuffer<uint32_t> ids = lane_order_ids(st, dtype, rowOffset, clean);
-            if ((rc = upload(&p->d_ids, ids.data(), ids.size(), &p->fixed_bytes))) return bail(rc);
+            if ((rc = upload(p, &p->d_ids, ids.data(), ids.size()))) return bail(rc);
         }
         // (single fp32 windows: decided below, once it is known whether the gather kernels of this plan read
         // bitmap tiles - then nothing reads tiles in lane order)
@@ -625,55 +685,31 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
         } else if (!lane_tiles_later) {
             const hspmm_host::ZeroedBuffer<uint32_t> tiles = lane_order_tiles(st, dtype, rowOffset, data);
             uint32_t *dt = nullptr;
-            if ((rc = upload(&dt, tiles.data(), tiles.size(), &p->fixed_bytes))) return bail(rc);
+            if ((rc = upload(p, &dt, tiles.data(), tiles.size()))) return bail(rc);
             p->d_tiles = dt;
         }
         timer.mark("step stream (ids, tiles)");
-        // Single 16-bit windows with few stored elements per tile (graphs: 16 of 128): the gather kernels read the
-        // tiles as bitmap + stored elements, 32 + 2 x 16 bytes per tile instead of 256 (power-law graph 2^20 at
-        // N = 128, where the stream is read once per XCD half: 0.64 -> 0.19 GB per launch).
+        // Single windows with few stored elements per tile (graphs: 16 of 128): the gather kernels read the tiles as
+        // bitmap + stored elements, 32 + 2 x 16 bytes per tile instead of 256 (power-law graph 2^20 at N = 128, where
+        // the stream is read once per XCD half: 0.64 -> 0.19 GB per launch).
         if (bitmap) {
-            // (same rule as below, with the exact number of stored elements)
-            const size_t stored = size_t(p->bm.stored);
+            // (the rule of tiles_look_sparse, with the exact number of stored elements)
             p->bm.built = total_tiles && p->cfg.gather_bitmap != 0 &&
                           (p->cfg.gather_bitmap > 0 ||
-                           (stored * 3u < size_t(total_tiles) * 8u * cw && size_t(total_tiles) * 256u >= (size_t(8) << 20)));
+                           (stored * 3u < uint64_t(total_tiles) * 8u * cw && tile_bytes >= (size_t(8) << 20)));
             if (!p->bm.built) {
-                (void)hipFree(p->bm.d_header); (void)hipFree(p->bm.d_vals);
+                plan_release(p, p->bm.d_header, header.size() * 4u);
+                plan_release(p, p->bm.d_vals, (size_t(stored) + spare) * elem);
                 p->bm.d_header = nullptr; p->bm.d_vals = nullptr;
-            }
-        } else if (st.G == 1 && p->cfg.gather_bitmap != 0 && total_tiles) {
-            const size_t n = size_t(total_tiles) * 8u * cw;                 // tile elements
-            size_t stored = 0;
-            if (p->cfg.gather_bitmap < 0) {
-                const size_t sample = std::min<size_t>(n, size_t(1) << 22);
-                if (elem == 2u) {
-                    const uint16_t *hv = static_cast<const uint16_t *>(data);
-                    for (size_t i = 0; i < sample; ++i) stored += hv[i] != 0;
-                } else {
-                    const uint32_t *wv = static_cast<const uint32_t *>(data);
-                    for (size_t i = 0; i < sample; ++i) stored += wv[i] != 0;
-                }
-                stored = size_t(double(stored) * double(n) / double(sample));
-            }
-            // 32 + 2 e bytes against 256 per tile with e stored elements (16 + 4 e for fp32): worth it below about a
-            // third full, and where the tile stream is large enough to be traffic at all (a matrix whose tiles sit
-            // in the L2s only pays the longer dependent chain: 4096 x 4096 at 1 %, 2.7 MB of tiles: 6.8 -> 7.5 us)
-            if (p->cfg.gather_bitmap > 0 ||
-                (stored * 3u < n && size_t(total_tiles) * 256u >= (size_t(8) << 20))) {
-                if ((rc = bitmap_from_uploaded_tiles(p, total_tiles))) return bail(rc);
             }
         }
         if (lane_tiles_later && total_tiles && !(p->bm.built && (p->cfg.kernel_mode == 0 || p->cfg.kernel_mode == 3))) {
             // single fp32 windows: steps are the caller's tiles in the caller's order; a kernel re-orders each for the lanes
-            void *dt = nullptr;
-            HSPMM_HIP_OR(hipMalloc(&dt, size_t(total_tiles) * 256u), bail);
-            p->d_tiles = dt; p->fixed_bytes += size_t(total_tiles) * 256u;
-            HSPMM_HIP_OR(hspmm::launch_lane_order32(p->d_data, dt, total_tiles, nullptr), bail);
-            HSPMM_HIP_OR(hipStreamSynchronize(nullptr), bail);
+            if ((rc = plan_alloc(p, tile_bytes, &room))) return bail(rc);
+            p->d_tiles = room;
+            HSPMM_HIP_OR(hspmm::launch_lane_order32(p->d_data, room, total_tiles, nullptr), bail);
         }
-        timer.mark("bitmap tiles");
-        p->per_column = entries_per_column(total_tiles, cw, elem, tcA2B, data, bitmap);
+        p->per_column = entries_per_column(total_tiles, cw, elem, tcA2B, data, bitmap, sparse_tiles ? header.data() : nullptr);
         {
             uint32_t longest = 0;
             for (size_t u = 0; u + 1 < st.unitOffset.size(); ++u) longest = std::max(longest, st.unitOffset[u + 1] - st.unitOffset[u]);
@@ -723,6 +759,7 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
             if (prc) return bail(prc);
             timer.mark("LDS-panel stream");
         }
+        HSPMM_HIP_OR(hipStreamSynchronize(nullptr), bail);              // (any stream may launch now)
     } catch (const std::bad_alloc &) {
         return bail(fail(HSPMM_ERR_ALLOC, "out of host memory"));
     }

@@ -137,8 +137,8 @@ hipError_t launch_entry_fill(int elem, const void *tiles, const uint32_t *a2b, c
                              uint32_t *cursors, uint32_t *desc, uint32_t *pieces, uint32_t *row_first, uint32_t *ids, void *vals,
                              hipStream_t s);
 hipError_t launch_fill_zero(void *dst, size_t bytes, hipStream_t s);
-// bitmap tiles (header, stored elements: see KernelArgs::bm_header and, for 32-bit elements, launch_bitmap_header
-// below) -> plain tiles (8 x 16 of 16-bit elements, 8 x 8 of 32-bit elements)
+// bitmap tiles -> plain tiles.  8 x 16 tiles of 16-bit elements: header as KernelArgs::bm_header; 8 x 8 tiles of 32-bit
+// elements: 4 header words per tile - rows 0..3, rows 4..7, position of the first stored element, number of stored elements
 hipError_t launch_expand_bitmap(int elem_bytes, const uint32_t *header, const void *vals, void *tiles, uint32_t n_tiles,
                                 hipStream_t s);
 // n 16-bit elements -> n words with the element in the low half (launch_widen_halves), and back (launch_narrow_words):
@@ -147,17 +147,8 @@ hipError_t launch_widen_halves(const void *src, void *dst, size_t n, hipStream_t
 hipError_t launch_narrow_words(const void *src, void *dst, size_t n, hipStream_t s);
 // plain 8 x 8 tiles of 32-bit elements, single windows -> the order the lanes of the fp32 gather kernels read them in
 hipError_t launch_lane_order32(const void *tiles, void *out, uint32_t n_tiles, hipStream_t s);
-// plain tiles -> bitmap tiles (8 x 16 tiles of 16-bit elements, elem_bytes = 2: 8 header words per tile, see
-// KernelArgs::bm_header; 8 x 8 tiles of 32-bit elements, elem_bytes = 4: 4 header words - rows 0..3, rows 4..7,
-// position of the first stored element, number of stored elements), in two steps with the host in between (it
-// sizes `vals`): launch_bitmap_header writes the masks and the tiles' counts, and leaves in block_sums
-// (bitmap_scan_blocks(n_tiles) + 1 words of 64 bits) the exclusive sums per 2048 tiles and, last, the number of
-// stored elements; launch_bitmap_pack writes the positions and the stored elements.
-uint32_t bitmap_scan_blocks(uint32_t n_tiles);
-hipError_t launch_bitmap_header(int elem_bytes, const void *tiles, uint32_t *header, uint32_t n_tiles, uint64_t *block_sums,
-                                hipStream_t s);
-hipError_t launch_bitmap_pack(int elem_bytes, const void *tiles, uint32_t *header, void *vals, uint32_t n_tiles,
-                              const uint64_t *block_sums, hipStream_t s);
+// column ids of single windows -> without padding, in the order the lanes of the gather kernels read them in
+hipError_t launch_step_ids(int elem_bytes, const uint32_t *raw, uint32_t *out, uint32_t n_tiles, hipStream_t s);
 // Measurement only (gather_rate_kernel in hspmm_kernels.hip): loads part_bytes (128 or 256) of row ids[i] of B for
 // every i < n_ids; parts > 1: `parts` parts of part_bytes each, dealt out by XCD, every part walking all ids.
 hipError_t launch_gather_rate(const uint32_t *ids, uint64_t n_ids, const void *B, uint32_t row_bytes, uint32_t part_bytes,

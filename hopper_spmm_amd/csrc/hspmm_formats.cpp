@@ -19,6 +19,7 @@
 #include <cstring>
 #include <string>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/hspmm.h"
@@ -393,26 +394,34 @@ public:
     const std::vector<uint32_t> &list(const uint32_t *col, size_t n)
     {
         if (sorted_) { list_sorted(col, n); return columns_; }
-        for (uint32_t w : used_) words_[w] = 0;
-        used_.clear(); columns_.clear();
+        for (uint32_t i = 0; i < n_used_; ++i) words_[used_[i]] = 0;
+        if (used_.size() < std::min(n, words_.size())) used_.resize(std::min(n, words_.size()));
+        columns_.resize(n);                                 // (room; cut below)
+        uint64_t *words = words_.data(), *mids = mids_.data(), *tops = tops_.data();
         for (size_t i = 0; i < n; ++i) {
-            const uint32_t w = col[i] >> 6;
-            if (!words_[w]) { mids_[w >> 6] |= uint64_t(1) << (w & 63u); tops_[w >> 12] |= uint64_t(1) << ((w >> 6) & 63u); }
-            words_[w] |= uint64_t(1) << (col[i] & 63u);
+            const uint32_t c = col[i], w = c >> 6;
+            mids[w >> 6] |= uint64_t(1) << (w & 63u);
+            tops[w >> 12] |= uint64_t(1) << ((w >> 6) & 63u);
+            words[w] |= uint64_t(1) << (c & 63u);
         }
+        uint32_t *used = used_.data(), *columns = columns_.data(), *ranks = rank_.data();
+        uint32_t n_used = 0, n_columns = 0;
         for (size_t t = 0; t < tops_.size(); ++t) {
-            for (uint64_t top = tops_[t]; top; top &= top - 1) {
+            for (uint64_t top = tops[t]; top; top &= top - 1) {
                 const size_t m = t * 64 + size_t(__builtin_ctzll(top));
-                for (uint64_t mid = mids_[m]; mid; mid &= mid - 1) {
+                for (uint64_t mid = mids[m]; mid; mid &= mid - 1) {
                     const uint32_t w = uint32_t(m * 64 + size_t(__builtin_ctzll(mid)));
-                    used_.push_back(w);
-                    rank_[w] = uint32_t(columns_.size());
-                    for (uint64_t word = words_[w]; word; word &= word - 1) columns_.push_back(w * 64u + uint32_t(__builtin_ctzll(word)));
+                    used[n_used++] = w;
+                    ranks[w] = n_columns;
+                    uint64_t word = words[w];               // (never 0)
+                    do columns[n_columns++] = w * 64u + uint32_t(__builtin_ctzll(word)); while (word &= word - 1);
                 }
-                mids_[m] = 0;
+                mids[m] = 0;
             }
-            tops_[t] = 0;
+            tops[t] = 0;
         }
+        n_used_ = n_used;
+        columns_.resize(n_columns);
         return columns_;
     }
     uint32_t rank(uint32_t column) const
@@ -430,6 +439,7 @@ private:
         columns_.erase(std::unique(columns_.begin(), columns_.end()), columns_.end());
     }
     bool sorted_;
+    uint32_t n_used_ = 0;
     std::vector<uint64_t> words_, mids_, tops_;
     std::vector<uint32_t> rank_, used_, columns_;          // rank_: of a word's first column, where the word holds one
 };
@@ -456,12 +466,14 @@ static size_t windows_per_worker(size_t nwin, size_t nnz)
     return std::max<size_t>(1, std::min<size_t>(2048, (size_t(1) << 14) / std::max<size_t>(1, per_window)));
 }
 
+static size_t window_count(uint32_t rows) { return (size_t(rows) + HSPMM_ROW_WINDOW - 1) / HSPMM_ROW_WINDOW; }
+
 // tiles[w] = number of tiles of window w (0 for a window without entries).
 static void count_tiles(uint32_t rows, const uint32_t *row_ptr, const uint32_t *col_idx, uint32_t cw,
-                        uint32_t n_columns, std::vector<uint32_t> &tiles)
+                        uint32_t n_columns, uint32_t *tiles)
 {
-    const size_t nwin = (size_t(rows) + HSPMM_ROW_WINDOW - 1) / HSPMM_ROW_WINDOW;
-    tiles.assign(nwin, 0u);
+    const size_t nwin = window_count(rows);
+    std::fill(tiles, tiles + nwin, 0u);
     parallel_chunks(nwin, windows_per_worker(nwin, row_ptr[rows]), [&](size_t wb, size_t we) {
         ColumnSet set(n_columns, row_ptr[rows]);
         for (size_t w = wb; w < we; ++w) {
@@ -472,6 +484,56 @@ static void count_tiles(uint32_t rows, const uint32_t *row_ptr, const uint32_t *
             tiles[w] = (u + cw - 1) / cw;                                   // convert.h:178-185
         }
     });
+}
+
+// Where fill_tiles writes, and the scans that say where a window's part begins.
+struct TileArrays {
+    uint32_t *rowOffset, *tcA2B;
+    void *data;
+    uint32_t *rowIdx;
+    const uint32_t *eff_index, *first_tile;
+};
+
+// The tiles of every window.  Element type and tile width are constants of the build: an entry costs one rank, a shift, a
+// mask and one store (with the width and the element size as variables, a division and a call of memcpy more: graph of
+// 2^18 vertices, 8 cores: 12.3 -> 6.5 ms).
+// Returns whether every window needs as many tiles as `tiles` says (one that does not is left out).
+template <class V, uint32_t CW>
+static bool fill_tiles(uint32_t rows, uint32_t n_columns, const uint32_t *row_ptr, const uint32_t *col_idx, const void *values,
+                       bool transpose, const std::vector<uint32_t> &tiles, const TileArrays &out)
+{
+    constexpr size_t kTile = size_t(HSPMM_ROW_WINDOW) * CW;
+    const size_t nwin = tiles.size();
+    const V *from = static_cast<const V *>(values);
+    std::atomic<bool> as_counted{true};
+    parallel_chunks(nwin, windows_per_worker(nwin, row_ptr[rows]), [&](size_t wb, size_t we) {
+        ColumnSet set(n_columns, row_ptr[rows]);
+        for (size_t w = wb; w < we; ++w) {
+            if (!tiles[w] && row_ptr[std::min<size_t>((w + 1) * HSPMM_ROW_WINDOW, rows)] == row_ptr[w * HSPMM_ROW_WINDOW]) continue;
+            const uint32_t r0 = uint32_t(w * HSPMM_ROW_WINDOW);
+            const uint32_t r1 = std::min<uint64_t>(uint64_t(r0) + HSPMM_ROW_WINDOW, rows);
+            const std::vector<uint32_t> &uniq = set.list(col_idx + row_ptr[r0], row_ptr[r1] - row_ptr[r0]);
+            const uint32_t u = uint32_t(uniq.size());
+            const uint32_t ew = out.eff_index[w], ft = out.first_tile[w], nt = tiles[w];
+            if ((u + CW - 1) / CW != nt) { as_counted.store(false); continue; }
+            out.rowOffset[ew + 1] = ft + nt;                                 // convert.h:186
+            out.rowIdx[ew] = r0;                                             // convert.h:187
+            uint32_t *ids = out.tcA2B + size_t(ft) * CW;
+            std::memcpy(ids, uniq.data(), size_t(u) * 4);                    // convert.h:178-184
+            for (uint32_t i = u; i < nt * CW; ++i) ids[i] = HSPMM_IDX_MAX;
+            V *win = static_cast<V *>(out.data) + size_t(ft) * kTile;
+            std::memset(win, 0, size_t(nt) * kTile * sizeof(V));             // convert.h:191-193
+            const uint32_t row_step = transpose ? 1u : CW, col_step = transpose ? HSPMM_ROW_WINDOW : 1u;   // convert.h:209, :212
+            for (uint32_t r = r0; r < r1; ++r) {
+                V *row = win + size_t(r - r0) * row_step;
+                for (uint32_t id = row_ptr[r]; id < row_ptr[r + 1]; ++id) {  // stored order: a later duplicate wins
+                    const uint32_t rank = set.rank(col_idx[id]);
+                    row[size_t(rank / CW) * kTile + (rank % CW) * col_step] = from[id];
+                }
+            }
+        }
+    });
+    return as_counted.load();
 }
 
 }  // namespace hspmm_host
@@ -490,23 +552,29 @@ static uint32_t tile_width(int dtype, uint32_t col_window)
     return 0;
 }
 
-int hspmm_btcf_sizes_cw(int dtype, uint32_t col_window, uint32_t rows, const uint32_t *row_ptr, const uint32_t *col_idx,
-                        uint32_t *eff_row_windows, uint32_t *total_tiles)
+int hspmm_count_tiles(int dtype, uint32_t col_window, uint32_t rows, const uint32_t *row_ptr, const uint32_t *col_idx,
+                      uint32_t *window_tiles, uint32_t *eff_row_windows, uint32_t *total_tiles)
 {
     const uint32_t cw = tile_width(dtype, col_window);
     if (!cw) return HSPMM_ERR_INVALID;
-    if (!row_ptr || !eff_row_windows || !total_tiles || (!col_idx && row_ptr[rows])) {
+    if (!row_ptr || !window_tiles || !eff_row_windows || !total_tiles || (!col_idx && row_ptr[rows])) {
         set_error("null argument");
         return HSPMM_ERR_INVALID;
     }
-    std::vector<uint32_t> tiles;
-    count_tiles(rows, row_ptr, col_idx, cw, column_count(col_idx, row_ptr[rows]), tiles);
+    count_tiles(rows, row_ptr, col_idx, cw, column_count(col_idx, row_ptr[rows]), window_tiles);
     uint64_t W = 0, T = 0;
-    for (uint32_t t : tiles) { W += t != 0; T += t; }
+    for (size_t w = 0, n = window_count(rows); w < n; ++w) { W += window_tiles[w] != 0; T += window_tiles[w]; }
     if (T > 0xFFFFFFFFull) { set_error("tile count exceeds 32 bits"); return HSPMM_ERR_UNSUPPORTED; }
     *eff_row_windows = uint32_t(W);
     *total_tiles = uint32_t(T);
     return HSPMM_OK;
+}
+
+int hspmm_btcf_sizes_cw(int dtype, uint32_t col_window, uint32_t rows, const uint32_t *row_ptr, const uint32_t *col_idx,
+                        uint32_t *eff_row_windows, uint32_t *total_tiles)
+{
+    std::vector<uint32_t> tiles(window_count(rows) + 1);
+    return hspmm_count_tiles(dtype, col_window, rows, row_ptr, col_idx, tiles.data(), eff_row_windows, total_tiles);
 }
 
 int hspmm_btcf_sizes(int dtype, uint32_t rows, const uint32_t *row_ptr, const uint32_t *col_idx,
@@ -526,16 +594,23 @@ int hspmm_btcf_fill_cw(int dtype, uint32_t col_window, uint32_t rows, const uint
                        const void *values, int transpose, uint32_t *rowOffset, uint32_t *tcA2B, void *data,
                        uint32_t *rowIdx)
 {
+    return hspmm_btcf_fill_counted(dtype, col_window, rows, row_ptr, col_idx, values, transpose, nullptr, rowOffset, tcA2B, data,
+                                   rowIdx);
+}
+
+int hspmm_btcf_fill_counted(int dtype, uint32_t col_window, uint32_t rows, const uint32_t *row_ptr, const uint32_t *col_idx,
+                            const void *values, int transpose, const uint32_t *window_tiles, uint32_t *rowOffset,
+                            uint32_t *tcA2B, void *data, uint32_t *rowIdx)
+{
     const uint32_t cw = tile_width(dtype, col_window);
     if (!cw) return HSPMM_ERR_INVALID;
     if (!row_ptr || !rowOffset) { set_error("null argument"); return HSPMM_ERR_INVALID; }
-    const size_t es = dtype == HSPMM_TF32 ? 4 : 2;
-    const size_t tile_elems = size_t(HSPMM_ROW_WINDOW) * cw;
     if (!col_idx && row_ptr[rows]) { set_error("null argument"); return HSPMM_ERR_INVALID; }
     const uint32_t n_columns = column_count(col_idx, row_ptr[rows]);
-    std::vector<uint32_t> tiles;
-    count_tiles(rows, row_ptr, col_idx, cw, n_columns, tiles);
-    const size_t nwin = tiles.size();
+    const size_t nwin = window_count(rows);
+    std::vector<uint32_t> tiles(nwin);
+    if (window_tiles) std::copy(window_tiles, window_tiles + nwin, tiles.begin());
+    else count_tiles(rows, row_ptr, col_idx, cw, n_columns, tiles.data());
     // exclusive scans: effective-window index and first tile of every window
     std::vector<uint32_t> eff_index(nwin + 1, 0u), first_tile(nwin + 1, 0u);
     for (size_t w = 0; w < nwin; ++w) {
@@ -547,32 +622,12 @@ int hspmm_btcf_fill_cw(int dtype, uint32_t col_window, uint32_t rows, const uint
         set_error("null argument");
         return HSPMM_ERR_INVALID;
     }
-    parallel_chunks(nwin, windows_per_worker(nwin, row_ptr[rows]), [&](size_t wb, size_t we) {
-        ColumnSet set(n_columns, row_ptr[rows]);
-        for (size_t w = wb; w < we; ++w) {
-            if (!tiles[w]) continue;
-            const uint32_t r0 = uint32_t(w * HSPMM_ROW_WINDOW);
-            const uint32_t r1 = std::min<uint64_t>(uint64_t(r0) + HSPMM_ROW_WINDOW, rows);
-            const std::vector<uint32_t> &uniq = set.list(col_idx + row_ptr[r0], row_ptr[r1] - row_ptr[r0]);
-            const uint32_t u = uint32_t(uniq.size());
-            const uint32_t ew = eff_index[w], ft = first_tile[w], nt = tiles[w];
-            rowOffset[ew + 1] = ft + nt;                                     // convert.h:186
-            rowIdx[ew] = r0;                                                 // convert.h:187
-            uint32_t *ids = tcA2B + size_t(ft) * cw;
-            for (uint32_t i = 0; i < nt * cw; ++i) ids[i] = i < u ? uniq[i] : HSPMM_IDX_MAX;   // convert.h:178-184
-            unsigned char *win = static_cast<unsigned char *>(data) + size_t(ft) * tile_elems * es;
-            std::memset(win, 0, size_t(nt) * tile_elems * es);               // convert.h:191-193
-            for (uint32_t r = r0; r < r1; ++r)
-                for (uint32_t id = row_ptr[r]; id < row_ptr[r + 1]; ++id) {  // stored order: a later duplicate wins
-                    const uint32_t rank = set.rank(col_idx[id]);
-                    const uint32_t tc = rank / cw, lc = rank % cw, lr = r % HSPMM_ROW_WINDOW;
-                    const size_t off = transpose ? size_t(lc) * HSPMM_ROW_WINDOW + lr       // convert.h:209
-                                                 : size_t(lr) * cw + lc;                    // convert.h:212
-                    std::memcpy(win + (size_t(tc) * tile_elems + off) * es,
-                                static_cast<const unsigned char *>(values) + size_t(id) * es, es);
-                }
-        }
-    });
+    const TileArrays out{rowOffset, tcA2B, data, rowIdx, eff_index.data(), first_tile.data()};
+    auto fill = cw == 16 ? fill_tiles<uint16_t, 16> : cw == 8 ? fill_tiles<uint32_t, 8> : fill_tiles<uint32_t, 4>;
+    if (!fill(rows, n_columns, row_ptr, col_idx, values, transpose != 0, tiles, out)) {
+        set_error("window_tiles does not belong to this matrix");
+        return HSPMM_ERR_INVALID;
+    }
     return HSPMM_OK;
 }
 
@@ -597,6 +652,15 @@ int hspmm_bitmap_fill(int dtype, uint32_t rows, const uint32_t *row_ptr, const u
                       uint32_t *rowOffset, uint32_t *nnzOffset, uint32_t *tcA2B, uint64_t *tcBit,
                       void *data, uint32_t *rowIdx)
 {
+    return hspmm_bitmap_fill_counted(dtype, rows, row_ptr, col_idx, values, transpose, bit_layout, nullptr, rowOffset, nnzOffset,
+                                     tcA2B, tcBit, data, rowIdx);
+}
+
+int hspmm_bitmap_fill_counted(int dtype, uint32_t rows, const uint32_t *row_ptr, const uint32_t *col_idx,
+                              const void *values, int transpose, int bit_layout, const uint32_t *window_tiles,
+                              uint32_t *rowOffset, uint32_t *nnzOffset, uint32_t *tcA2B, uint64_t *tcBit,
+                              void *data, uint32_t *rowIdx)
+{
     using namespace hspmm_host;
     if (dtype != HSPMM_FP16 && dtype != HSPMM_TF32 && dtype != HSPMM_BF16) { set_error("unknown dtype"); return HSPMM_ERR_INVALID; }
     if (bit_layout != HSPMM_BITS_PER_TILE && bit_layout != HSPMM_BITS_AS_REFERENCE) {
@@ -606,12 +670,12 @@ int hspmm_bitmap_fill(int dtype, uint32_t rows, const uint32_t *row_ptr, const u
     if (!row_ptr || !rowOffset || !nnzOffset) { set_error("null argument"); return HSPMM_ERR_INVALID; }
     const uint32_t cw = dtype == HSPMM_TF32 ? 8u : 16u;
     const uint32_t wpt = HSPMM_BITMAP_WORDS(dtype);
-    const size_t es = dtype == HSPMM_TF32 ? 4 : 2;
     if (!col_idx && row_ptr[rows]) { set_error("null argument"); return HSPMM_ERR_INVALID; }
     const uint32_t n_columns = column_count(col_idx, row_ptr[rows]);
-    std::vector<uint32_t> tiles;
-    count_tiles(rows, row_ptr, col_idx, cw, n_columns, tiles);
-    const size_t nwin = tiles.size();
+    const size_t nwin = window_count(rows);
+    std::vector<uint32_t> tiles(nwin);
+    if (window_tiles) std::copy(window_tiles, window_tiles + nwin, tiles.begin());
+    else count_tiles(rows, row_ptr, col_idx, cw, n_columns, tiles.data());
     std::vector<uint32_t> eff_index(nwin + 1, 0u), first_tile(nwin + 1, 0u);
     for (size_t w = 0; w < nwin; ++w) {
         eff_index[w + 1] = eff_index[w] + (tiles[w] != 0);
@@ -624,33 +688,41 @@ int hspmm_bitmap_fill(int dtype, uint32_t rows, const uint32_t *row_ptr, const u
         set_error("null argument");
         return HSPMM_ERR_INVALID;
     }
-    if (T) std::memset(tcBit, 0, size_t(T) * wpt * 8);                       // convert.h:67
     // The reference's word index for 8 x 16 tiles lets neighbouring tiles, and so
     // neighbouring windows, share a word: that layout is filled by one thread.
     const bool shared_words = bit_layout == HSPMM_BITS_AS_REFERENCE && wpt == 2;
-    auto convert_windows = [&](size_t wb, size_t we) {
+    if (shared_words) std::memset(tcBit, 0, size_t(T) * wpt * 8);
+    // (width and element type are constants of the instance, as in fill_tiles)
+    std::atomic<bool> as_counted{true};
+    auto convert_windows = [&](auto width, auto element, size_t wb, size_t we) {
+        constexpr uint32_t CW = decltype(width)::value;
+        typedef decltype(element) V;
+        const V *from = static_cast<const V *>(values);
+        V *to = static_cast<V *>(data);
         ColumnSet set(n_columns, row_ptr[rows]);
         std::vector<uint32_t> start, cursor;
         for (size_t w = wb; w < we; ++w) {
-            if (!tiles[w]) continue;
+            if (!tiles[w] && row_ptr[std::min<size_t>((w + 1) * HSPMM_ROW_WINDOW, rows)] == row_ptr[w * HSPMM_ROW_WINDOW]) continue;
             const uint32_t r0 = uint32_t(w * HSPMM_ROW_WINDOW);
             const uint32_t r1 = std::min<uint64_t>(uint64_t(r0) + HSPMM_ROW_WINDOW, rows);
             const std::vector<uint32_t> &uniq = set.list(col_idx + row_ptr[r0], row_ptr[r1] - row_ptr[r0]);
             const uint32_t u = uint32_t(uniq.size());
             const uint32_t ew = eff_index[w], ft = first_tile[w], nt = tiles[w];
+            if ((u + CW - 1) / CW != nt) { as_counted.store(false); continue; }
             rowOffset[ew + 1] = ft + nt;                                     // convert.h:58
             rowIdx[ew] = r0;                                                 // convert.h:68
-            uint32_t *ids = tcA2B + size_t(ft) * cw;
-            for (uint32_t i = 0; i < nt * cw; ++i) ids[i] = i < u ? uniq[i] : HSPMM_IDX_MAX;   // convert.h:50-56
+            if (!shared_words) std::memset(tcBit + size_t(ft) * wpt, 0, size_t(nt) * wpt * 8);  // convert.h:67
+            uint32_t *ids = tcA2B + size_t(ft) * CW;
+            for (uint32_t i = 0; i < nt * CW; ++i) ids[i] = i < u ? uniq[i] : HSPMM_IDX_MAX;   // convert.h:50-56
             // Stored entries are grouped by tile, and inside a tile by (row, position in
             // the row) - or by (tile column, row) with `transpose` (convert.h:114-133).  Count
             // per sub-bucket, scan, place.  All entries of earlier windows come first, so
             // the window's part of `data` starts at row_ptr[r0].
-            const uint32_t sub = transpose ? cw : 1u;
+            const uint32_t sub = transpose ? CW : 1u;
             start.assign(size_t(nt) * sub + 1, 0u);
             for (uint32_t id = row_ptr[r0]; id < row_ptr[r1]; ++id) {
                 const uint32_t rank = set.rank(col_idx[id]);
-                ++start[size_t(rank / cw) * sub + (transpose ? rank % cw : 0u) + 1];
+                ++start[size_t(rank / CW) * sub + (transpose ? rank % CW : 0u) + 1];
             }
             for (size_t i = 0; i < size_t(nt) * sub; ++i) start[i + 1] += start[i];
             for (uint32_t t = 0; t < nt; ++t)
@@ -659,20 +731,24 @@ int hspmm_bitmap_fill(int dtype, uint32_t rows, const uint32_t *row_ptr, const u
             for (uint32_t r = r0; r < r1; ++r)
                 for (uint32_t id = row_ptr[r]; id < row_ptr[r + 1]; ++id) {
                     const uint32_t rank = set.rank(col_idx[id]);
-                    const uint32_t tc = rank / cw, lc = rank % cw, lr = r % HSPMM_ROW_WINDOW;
+                    const uint32_t tc = rank / CW, lc = rank % CW, lr = r % HSPMM_ROW_WINDOW;
                     const uint32_t bit = transpose ? lc * HSPMM_ROW_WINDOW + lr              // convert.h:90
-                                                   : lr * cw + lc;                           // convert.h:93
+                                                   : lr * CW + lc;                           // convert.h:93
                     const size_t word = shared_words ? size_t(ft + tc) + bit / 64u           // convert.h:97-101
                                                      : size_t(ft + tc) * wpt + bit / 64u;
                     tcBit[word] |= uint64_t(1) << (bit % 64u);
                     const uint32_t pos = row_ptr[r0] + cursor[size_t(tc) * sub + (transpose ? lc : 0u)]++;
-                    std::memcpy(static_cast<unsigned char *>(data) + size_t(pos) * es,
-                                static_cast<const unsigned char *>(values) + size_t(id) * es, es);
+                    to[pos] = from[id];
                 }
         }
     };
-    if (shared_words) convert_windows(0, nwin);
-    else parallel_chunks(nwin, windows_per_worker(nwin, row_ptr[rows]), convert_windows);
+    auto convert = [&](size_t wb, size_t we) {
+        if (cw == 16) convert_windows(std::integral_constant<uint32_t, 16>{}, uint16_t{}, wb, we);
+        else convert_windows(std::integral_constant<uint32_t, 8>{}, uint32_t{}, wb, we);
+    };
+    if (shared_words) convert(0, nwin);
+    else parallel_chunks(nwin, windows_per_worker(nwin, row_ptr[rows]), convert);
+    if (!as_counted.load()) { set_error("window_tiles does not belong to this matrix"); return HSPMM_ERR_INVALID; }
     return HSPMM_OK;
 }
 

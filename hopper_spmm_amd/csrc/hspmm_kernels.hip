@@ -139,211 +139,28 @@ hipError_t launch_lane_order32(const void *tiles, void *out, uint32_t n_tiles, h
     return hipGetLastError();
 }
 
-// Plain 8 x 16 tiles of 16-bit elements -> bitmap tiles, on the device: what hspmm_create does for a matrix of
-// sparse tiles once the plain tiles are uploaded (the reverse of the kernel above; the bitmap is the reference's,
-// src/utils/convert.h:83-101: bit 16 r + k for element (r, k), stored when its bit pattern is not +0).  Three
-// passes: the four mask words, their running bit counts and the tile's count (header words 0..4 and 6); an
-// exclusive sum of the counts over all tiles (header word 5, the reference's nnzOffset); the stored elements
-// written tile after tile in bit order.
-typedef uint32_t bm_u32x4 __attribute__((ext_vector_type(4)));
-constexpr uint32_t kScanTilesPerBlock = 2048;          // 256 threads x 8 tiles
-
-// the 32 elements of word `word` of tile t as a mask (four consecutive lanes take the four words of one tile)
-__device__ __forceinline__ uint32_t tile_word_mask(const uint16_t *tiles, uint32_t t, uint32_t word)
-{
-    const bm_u32x4 *src = reinterpret_cast<const bm_u32x4 *>(tiles + size_t(t) * 128u + word * 32u);
-    uint32_t mask = 0;
-#pragma unroll
-    for (uint32_t q = 0; q < 4; ++q) {
-        const bm_u32x4 v = src[q];
-#pragma unroll
-        for (uint32_t e = 0; e < 4; ++e) {
-            mask |= ((v[e] & 0xFFFFu) ? 1u : 0u) << (q * 8u + 2u * e);
-            mask |= ((v[e] >> 16) ? 1u : 0u) << (q * 8u + 2u * e + 1u);
-        }
-    }
-    return mask;
-}
-
-__global__ __launch_bounds__(256) void bitmap_header_kernel(const uint16_t *__restrict__ tiles, uint32_t *__restrict__ header,
-                                                            uint32_t n_tiles)
+// Column ids of single windows as the gather kernels read them: a padding id becomes the real id in front of it (its tile
+// column is all zero, and no tile starts with padding), and 8 x 8 tiles of 32-bit elements get the lane order [g][2] =
+// (id g, id g + 4).  One thread per id.
+template <uint32_t CW>
+__global__ __launch_bounds__(256) void step_ids_kernel(const uint32_t *__restrict__ raw, uint32_t *__restrict__ out, uint32_t n_tiles)
 {
     const uint64_t i = uint64_t(blockIdx.x) * 256u + threadIdx.x;
-    const uint32_t t = uint32_t(i >> 2), word = uint32_t(i & 3u), lane = threadIdx.x & 63u;
-    const bool active = i < uint64_t(n_tiles) * 4u;
-    const uint32_t mask = active ? tile_word_mask(tiles, t, word) : 0u;
-    const uint32_t c = uint32_t(__builtin_popcount(mask)), first = lane & ~3u;
-    const uint32_t c0 = __shfl(c, first), c1 = c0 + __shfl(c, first + 1u), c2 = c1 + __shfl(c, first + 2u),
-                   c3 = c2 + __shfl(c, first + 3u);
-    if (!active) return;
-    uint32_t *hd = header + size_t(t) * 8u;
-    hd[word] = mask;
-    if (word == 0u) { hd[4] = c0 << 8 | c1 << 16 | c2 << 24; hd[6] = c3; hd[7] = 0u; }
+    if (i >= uint64_t(n_tiles) * CW) return;
+    const uint32_t o = uint32_t(i % CW);
+    uint32_t k = CW == 8u ? (o >> 1) + 4u * (o & 1u) : o;
+    const uint32_t *tile = raw + (i - o);
+    while (k && tile[k] == kIdxMax) --k;
+    out[i] = tile[k];
 }
 
-// sum of a value over the 256 threads of a workgroup, and the sum over the threads in front of this one
-__device__ __forceinline__ uint32_t block_exclusive_sum(uint32_t v, uint32_t *total)
-{
-    __shared__ uint32_t wave_sum[4];
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    uint32_t x = v;
-#pragma unroll
-    for (uint32_t d = 1; d < 64u; d <<= 1) {
-        const uint32_t y = __shfl_up(x, d);
-        if (lane >= d) x += y;
-    }
-    __syncthreads();                       // (a second call must not overwrite sums still being read)
-    if (lane == 63u) wave_sum[wave] = x;
-    __syncthreads();
-    uint32_t before = 0, all = 0;
-#pragma unroll
-    for (uint32_t w = 0; w < 4u; ++w) { if (w < wave) before += wave_sum[w]; all += wave_sum[w]; }
-    *total = all;
-    return before + x - v;
-}
-
-// (words: header words per tile; at_count / at_first: where a tile's count is and where its position goes)
-__global__ __launch_bounds__(256) void bitmap_block_sums_kernel(const uint32_t *__restrict__ header, uint32_t n_tiles,
-                                                                uint64_t *__restrict__ block_sums, uint32_t words,
-                                                                uint32_t at_count)
-{
-    const uint64_t t0 = uint64_t(blockIdx.x) * kScanTilesPerBlock + threadIdx.x * 8u;
-    uint32_t s = 0;
-    for (uint32_t k = 0; k < 8u; ++k)
-        if (t0 + k < n_tiles) s += header[(t0 + k) * words + at_count];
-    uint32_t total;
-    (void)block_exclusive_sum(s, &total);
-    if (threadIdx.x == 0) block_sums[blockIdx.x] = total;
-}
-
-// exclusive sums of block_sums in place (one workgroup; a chunk of 256 block sums is below 2^26), the total behind them
-__global__ __launch_bounds__(256) void bitmap_scan_sums_kernel(uint64_t *block_sums, uint32_t n_blocks)
-{
-    uint64_t carry = 0;
-    for (uint32_t base = 0; base < n_blocks; base += 256u) {
-        const uint32_t i = base + threadIdx.x;
-        const uint32_t v = i < n_blocks ? uint32_t(block_sums[i]) : 0u;
-        uint32_t total;
-        const uint32_t before = block_exclusive_sum(v, &total);
-        if (i < n_blocks) block_sums[i] = carry + before;
-        carry += total;
-    }
-    if (threadIdx.x == 0) block_sums[n_blocks] = carry;
-}
-
-__global__ __launch_bounds__(256) void bitmap_offsets_kernel(uint32_t *__restrict__ header, uint32_t n_tiles,
-                                                             const uint64_t *__restrict__ block_sums, uint32_t words,
-                                                             uint32_t at_count, uint32_t at_first)
-{
-    const uint64_t t0 = uint64_t(blockIdx.x) * kScanTilesPerBlock + threadIdx.x * 8u;
-    uint32_t count[8], s = 0;
-    for (uint32_t k = 0; k < 8u; ++k) {
-        count[k] = t0 + k < n_tiles ? header[(t0 + k) * words + at_count] : 0u;
-        s += count[k];
-    }
-    uint32_t total;
-    uint64_t at = block_sums[blockIdx.x] + block_exclusive_sum(s, &total);
-    for (uint32_t k = 0; k < 8u; ++k)
-        if (t0 + k < n_tiles) { header[(t0 + k) * words + at_first] = uint32_t(at); at += count[k]; }
-}
-
-// The same for 8 x 8 tiles of 32-bit elements (Fp32TileB in spmm_mfma_kernel.hpp): header words {rows 0..3, rows
-// 4..7, position of the first stored element, number of stored elements}; four consecutive lanes take two rows each.
-__global__ __launch_bounds__(256) void bitmap_header32_kernel(const uint32_t *__restrict__ tiles, uint32_t *__restrict__ header,
-                                                              uint32_t n_tiles)
-{
-    const uint64_t i = uint64_t(blockIdx.x) * 256u + threadIdx.x;
-    const uint32_t t = uint32_t(i >> 2), quarter = uint32_t(i & 3u), lane = threadIdx.x & 63u;
-    const bool active = i < uint64_t(n_tiles) * 4u;
-    uint32_t mask = 0;
-    if (active) {
-        const bm_u32x4 *src = reinterpret_cast<const bm_u32x4 *>(tiles + size_t(t) * 64u + quarter * 16u);
-#pragma unroll
-        for (uint32_t q = 0; q < 4; ++q) {
-            const bm_u32x4 v = src[q];
-#pragma unroll
-            for (uint32_t e = 0; e < 4; ++e) mask |= (v[e] ? 1u : 0u) << (q * 4u + e);
-        }
-    }
-    const uint32_t first = lane & ~3u;
-    const uint32_t m0 = __shfl(mask, first), m1 = __shfl(mask, first + 1u), m2 = __shfl(mask, first + 2u),
-                   m3 = __shfl(mask, first + 3u);
-    if (!active || quarter != 0u) return;
-    uint32_t *hd = header + size_t(t) * 4u;
-    const uint32_t lo = m0 | m1 << 16, hi = m2 | m3 << 16;
-    hd[0] = lo; hd[1] = hi; hd[2] = 0u;
-    hd[3] = uint32_t(__builtin_popcount(lo)) + uint32_t(__builtin_popcount(hi));
-}
-
-__global__ __launch_bounds__(256) void bitmap_pack32_kernel(const uint32_t *__restrict__ tiles, const uint32_t *__restrict__ header,
-                                                            uint32_t *__restrict__ vals, uint32_t n_tiles)
-{
-    const uint64_t i = uint64_t(blockIdx.x) * 256u + threadIdx.x;
-    if (i >= uint64_t(n_tiles) * 4u) return;
-    const uint32_t t = uint32_t(i >> 2), quarter = uint32_t(i & 3u);
-    const uint32_t *hd = header + size_t(t) * 4u;
-    const uint32_t w = (quarter & 2u) ? hd[1] : hd[0], sh = 16u * (quarter & 1u);
-    uint32_t mask = (w >> sh) & 0xFFFFu;
-    size_t at = size_t(hd[2]) + ((quarter & 2u) ? uint32_t(__builtin_popcount(hd[0])) : 0u) +
-                uint32_t(__builtin_popcount(w & ((1u << sh) - 1u)));
-    const uint32_t *src = tiles + size_t(t) * 64u + quarter * 16u;
-    while (mask) {
-        const uint32_t b = uint32_t(__builtin_ctz(mask));
-        vals[at++] = src[b];
-        mask &= mask - 1u;
-    }
-}
-
-__global__ __launch_bounds__(256) void bitmap_pack_kernel(const uint16_t *__restrict__ tiles, const uint32_t *__restrict__ header,
-                                                          uint16_t *__restrict__ vals, uint32_t n_tiles)
-{
-    const uint64_t i = uint64_t(blockIdx.x) * 256u + threadIdx.x;
-    if (i >= uint64_t(n_tiles) * 4u) return;
-    const uint32_t t = uint32_t(i >> 2), word = uint32_t(i & 3u);
-    const uint32_t *hd = header + size_t(t) * 8u;
-    uint32_t mask = hd[word];
-    size_t at = size_t(hd[5]) + ((hd[4] >> (8u * word)) & 0xFFu);
-    const uint16_t *src = tiles + size_t(t) * 128u + word * 32u;
-    while (mask) {
-        const uint32_t b = uint32_t(__builtin_ctz(mask));
-        vals[at++] = src[b];
-        mask &= mask - 1u;
-    }
-}
-
-hipError_t launch_bitmap_header(int elem_bytes, const void *tiles, uint32_t *header, uint32_t n_tiles, uint64_t *block_sums,
-                                hipStream_t s)
+hipError_t launch_step_ids(int elem_bytes, const uint32_t *raw, uint32_t *out, uint32_t n_tiles, hipStream_t s)
 {
     if (!n_tiles) return hipSuccess;
-    const uint32_t word_blocks = uint32_t((uint64_t(n_tiles) * 4u + 255u) / 256u);
-    const uint32_t n_blocks = (n_tiles + kScanTilesPerBlock - 1u) / kScanTilesPerBlock;
-    if (elem_bytes == 2) {
-        bitmap_header_kernel<<<dim3(word_blocks), 256, 0, s>>>(static_cast<const uint16_t *>(tiles), header, n_tiles);
-        bitmap_block_sums_kernel<<<dim3(n_blocks), 256, 0, s>>>(header, n_tiles, block_sums, 8u, 6u);
-    } else {
-        bitmap_header32_kernel<<<dim3(word_blocks), 256, 0, s>>>(static_cast<const uint32_t *>(tiles), header, n_tiles);
-        bitmap_block_sums_kernel<<<dim3(n_blocks), 256, 0, s>>>(header, n_tiles, block_sums, 4u, 3u);
-    }
-    bitmap_scan_sums_kernel<<<dim3(1), 256, 0, s>>>(block_sums, n_blocks);
-    return hipGetLastError();
-}
-
-uint32_t bitmap_scan_blocks(uint32_t n_tiles) { return (n_tiles + kScanTilesPerBlock - 1u) / kScanTilesPerBlock; }
-
-hipError_t launch_bitmap_pack(int elem_bytes, const void *tiles, uint32_t *header, void *vals, uint32_t n_tiles,
-                              const uint64_t *block_sums, hipStream_t s)
-{
-    if (!n_tiles) return hipSuccess;
-    const uint32_t word_blocks = uint32_t((uint64_t(n_tiles) * 4u + 255u) / 256u);
-    if (elem_bytes == 2) {
-        bitmap_offsets_kernel<<<dim3(bitmap_scan_blocks(n_tiles)), 256, 0, s>>>(header, n_tiles, block_sums, 8u, 6u, 5u);
-        bitmap_pack_kernel<<<dim3(word_blocks), 256, 0, s>>>(static_cast<const uint16_t *>(tiles), header,
-                                                            static_cast<uint16_t *>(vals), n_tiles);
-    } else {
-        bitmap_offsets_kernel<<<dim3(bitmap_scan_blocks(n_tiles)), 256, 0, s>>>(header, n_tiles, block_sums, 4u, 3u, 2u);
-        bitmap_pack32_kernel<<<dim3(word_blocks), 256, 0, s>>>(static_cast<const uint32_t *>(tiles), header,
-                                                              static_cast<uint32_t *>(vals), n_tiles);
-    }
+    const uint32_t cw = elem_bytes == 4 ? 8u : 16u;
+    const dim3 grid(uint32_t((uint64_t(n_tiles) * cw + 255u) / 256u));
+    if (elem_bytes == 4) step_ids_kernel<8><<<grid, 256, 0, s>>>(raw, out, n_tiles);
+    else step_ids_kernel<16><<<grid, 256, 0, s>>>(raw, out, n_tiles);
     return hipGetLastError();
 }
 

@@ -193,6 +193,9 @@ struct hspmm_plan {
     static constexpr size_t kMaxStreamBuffers = 16;
     std::vector<StreamBuffers> buffers;
     size_t fixed_bytes = 0;
+    std::vector<void *> owned;              // allocations of plan_reserve / plan_alloc
+    char *block = nullptr;                  // what is left of the reserved block
+    size_t block_left = 0;
     // Every real column list strictly ascending and padding only behind a window's last column: what the
     // reference's converters write (reference src/utils/convert.h:166-181).  The gather and all-shapes
     // kernels take any list; merging windows and the LDS-panel stream need this order.
@@ -231,13 +234,20 @@ struct PhaseTimer {
     }
 };
 
+// Device memory of a plan, all of it given back by hspmm_destroy (hspmm_create.hip).  plan_reserve allocates one block
+// that later plan_alloc calls are served from as long as they fit (an allocation takes 50 to 100 us, and freeing one as
+// long again); what does not fit gets an allocation of its own, which plan_release can give back early.
+int plan_reserve(hspmm_plan *p, size_t bytes);
+int plan_alloc(hspmm_plan *p, size_t bytes, void **out);
+void plan_release(hspmm_plan *p, const void *ptr, size_t bytes);
+
 template <typename T>
-int upload(T **dst, const T *src, size_t n, size_t *acc_bytes)
+int upload(hspmm_plan *p, T **dst, const T *src, size_t n)
 {
-    const size_t bytes = (n ? n : 1) * sizeof(T);
-    HSPMM_HIP(hipMalloc(reinterpret_cast<void **>(dst), bytes));
+    void *fresh = nullptr;
+    if (int rc = plan_alloc(p, (n ? n : 1) * sizeof(T), &fresh)) return rc;
+    *dst = static_cast<T *>(fresh);
     if (n) HSPMM_HIP(hipMemcpy(*dst, src, n * sizeof(T), hipMemcpyHostToDevice));
-    *acc_bytes += bytes;
     return HSPMM_OK;
 }
 
@@ -250,7 +260,7 @@ enum class RunMode { kLaunch, kPrepare, kStatic };
 // hspmm_create.hip
 int validate_format(uint32_t rows, uint32_t cols, uint32_t W, uint32_t T, uint32_t cw,
                     const uint32_t *rowOffset, const uint32_t *tcA2B, const void *data, const uint32_t *rowIdx,
-                    bool *canonical = nullptr);
+                    bool *canonical = nullptr, uint32_t *header = nullptr, uint32_t *window_stored = nullptr);
 int choose_ranges(const hspmm_plan *p);
 int build_and_upload_partition(hspmm_plan *p, int level, uint32_t group = 1, bool aligned = false);
 

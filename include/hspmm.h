@@ -371,6 +371,19 @@ int hspmm_btcf_fill_cw(int dtype, uint32_t col_window, uint32_t rows, const uint
                        const void *values, int transpose,
                        uint32_t *rowOffset, uint32_t *tcA2B, void *data, uint32_t *rowIdx);
 
+/* The same converters without counting the tiles twice: hspmm_count_tiles leaves the tiles of every window (rows / 8,
+ * rounded up, words; 0 for a window without entries) in window_tiles, the fills take it from there - same matrix, same
+ * width.  null: counted again.  A count that does not fit the matrix is an error. */
+int hspmm_count_tiles(int dtype, uint32_t col_window, uint32_t rows, const uint32_t *row_ptr, const uint32_t *col_idx,
+                      uint32_t *window_tiles, uint32_t *eff_row_windows, uint32_t *total_tiles);
+int hspmm_btcf_fill_counted(int dtype, uint32_t col_window, uint32_t rows, const uint32_t *row_ptr, const uint32_t *col_idx,
+                            const void *values, int transpose, const uint32_t *window_tiles,
+                            uint32_t *rowOffset, uint32_t *tcA2B, void *data, uint32_t *rowIdx);
+int hspmm_bitmap_fill_counted(int dtype, uint32_t rows, const uint32_t *row_ptr, const uint32_t *col_idx,
+                              const void *values, int transpose, int bit_layout, const uint32_t *window_tiles,
+                              uint32_t *rowOffset, uint32_t *nnzOffset, uint32_t *tcA2B, uint64_t *tcBit,
+                              void *data, uint32_t *rowIdx);
+
 /* ---- bitmap-compressed and grouped formats ------------------------------ */
 
 /* Words of tcBit per tile: one 64-bit word for 8 x 8 tiles (HSPMM_TF32), two
