@@ -610,9 +610,11 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
         if ((rc = plan_reserve(p, (size_t(p->W) * 4u + 2u) * 4u + n_ids * 8u + tile_bytes + header.size() * 4u +
                                       (sparse_tiles ? (size_t(stored) + spare) * elem : 0u) + (size_t(1) << 20))))
             return bail(rc);
+        timer.mark("device memory");
         if ((rc = upload(p, &p->d_rowOffset, rowOffset, size_t(p->W) + 1))) return bail(rc);
         if ((rc = upload(p, &p->d_rowIdx, rowIdx, size_t(p->W)))) return bail(rc);
         if ((rc = upload(p, &p->d_a2b_raw, tcA2B, n_ids))) return bail(rc);
+        timer.mark("upload ids");
         void *room = nullptr;
         if (sparse_tiles) {
             hspmm_host::ZeroedBuffer<uint8_t> vals((size_t(stored) + spare) * elem);
@@ -759,6 +761,8 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
             if (prc) return bail(prc);
             timer.mark("LDS-panel stream");
         }
+        if ((rc = build_tile_stream(p))) return bail(rc);
+        timer.mark("full-tile stream");
         HSPMM_HIP_OR(hipStreamSynchronize(nullptr), bail);              // (any stream may launch now)
     } catch (const std::bad_alloc &) {
         return bail(fail(HSPMM_ERR_ALLOC, "out of host memory"));

@@ -136,6 +136,28 @@ hipError_t launch_entry_fill(int elem, const void *tiles, const uint32_t *a2b, c
                              const uint32_t *positions, const uint32_t *row_len, uint32_t rows, const uint32_t *places,
                              uint32_t *cursors, uint32_t *desc, uint32_t *pieces, uint32_t *row_first, uint32_t *ids, void *vals,
                              hipStream_t s);
+// Full-tile kernels (spmm_tile_kernel.hip): stored entries in blocks of 128 rows x tile_block_columns() columns, in units of
+// four: positions inside the block's LDS image (16 bits) and values (fp32 storage: hi | lo parts).
+constexpr uint32_t kTileBlockRows = 128u, kTileMaxBlocks = 4096u;     // blocks of a row block at most
+constexpr uint32_t kTileSpareUnits = 512u;                            // behind the last unit (read and not used)
+uint32_t tile_block_columns(int dtype);
+struct TileArgs {
+    const uint32_t *blocks;      // per row block and block: its first unit (n_row_blocks x n_blocks + 1)
+    const void     *pos, *vals;
+    const void     *B;
+    void           *C;
+    float          *scratch;     // sums of the parts of cut C tiles: part g + t for workgroup g and tile t
+    uint32_t       *arrive;      // per C tile: parts that have left their sums (zero between launches)
+    uint32_t rows, cols, N;
+    uint32_t n_row_blocks, n_chunks, n_feat_tiles;               // chunks: blocks of columns
+    uint32_t share, rest;        // items (chunks of C tiles) of a workgroup; the first `rest` have one more
+};
+// nt: features of a C tile (16, 32, 64)
+hipError_t launch_spmm_tile(int dtype, const TileArgs &ta, uint32_t nt, uint32_t groups, hipStream_t s);
+struct TileSource { const uint32_t *rowOffset, *rowIdx, *a2b; const void *tiles; uint32_t n_windows, cols; };   // the format arrays
+hipError_t launch_tile_count(int dtype, const TileSource &src, uint32_t n_row_blocks, uint32_t n_blocks, uint32_t *counts, uint32_t *blocks, hipStream_t s);
+hipError_t launch_tile_fill(int dtype, const TileSource &src, uint32_t n_row_blocks, uint32_t n_blocks, const uint32_t *counts,
+                            const uint32_t *blocks, void *pos, void *vals, hipStream_t s);
 hipError_t launch_fill_zero(void *dst, size_t bytes, hipStream_t s);
 // bitmap tiles -> plain tiles.  8 x 16 tiles of 16-bit elements: header as KernelArgs::bm_header; 8 x 8 tiles of 32-bit
 // elements: 4 header words per tile - rows 0..3, rows 4..7, position of the first stored element, number of stored elements

@@ -62,6 +62,7 @@ struct Config {
     int aligned_small = -1;             // small matrices: waves per unit of the one-workgroup-per-unit partition (-1: by size; 0, 4, 8)
     int gather_bitmap = -1;             // gather kernels read single 16-bit windows as bitmap + stored elements (-1: by fill)
     int entries = -1;                   // entry kernels for narrow feature dimensions (-1: by width, 0 never, 1 wherever they can)
+    int tile = -1;                      // full-tile kernels (-1: by density and width, 0 never, 1 wherever they can)
     int xcd_split = -1;                 // gather kernels: two feature blocks dealt out by XCD half (-1: by matrix, 0 never, 1 always)
     // (set through hspmm_set_panel_stream; builds with HSPMM_EXPERIMENTAL only)
     int panel_tall = 0;                 // LDS-panel waves with two units each
@@ -77,6 +78,7 @@ struct Config {
         if (const char *e = std::getenv("HSPMM_PANEL_MAX_WINDOWS")) panel_max_windows = std::atoi(e) >= 4 ? 4 : 2;
         if (const char *e = std::getenv("HSPMM_XCD_SPLIT")) xcd_split = std::atoi(e) != 0;
         if (const char *e = std::getenv("HSPMM_ENTRIES")) entries = std::atoi(e) != 0;
+        if (const char *e = std::getenv("HSPMM_TILE")) tile = std::atoi(e) != 0;
         if (const char *e = std::getenv("HSPMM_GATHER_BITMAP")) gather_bitmap = std::atoi(e) != 0;
         if (const char *e = std::getenv("HSPMM_ALIGNED_SMALL")) { const int v = std::atoi(e); aligned_small = v == 4 || v == 8 ? v : 0; }
         if (const char *e = std::getenv("HSPMM_PANEL_UNITS_PER_GROUP")) panel_units_per_group = std::max(1, std::atoi(e));
@@ -174,6 +176,15 @@ struct hspmm_plan {
         uint32_t n_pieces = 0;
         bool long_rows = false;                                  // 64 units and more in a row on average
     } entries;
+    // Stored entries by blocks of 128 rows x 64 (fp32 storage: 32) columns, for matrices that are dense to a workgroup
+    // (spmm_tile_kernel.hip): made from the tiles on the device by hspmm_create
+    struct Tile {
+        bool built = false;
+        const uint32_t *d_blocks = nullptr;
+        const void *d_pos = nullptr, *d_vals = nullptr;
+        uint32_t n_row_blocks = 0, n_blocks = 0;
+        uint64_t entries = 0;                                    // stored entries, blocks rounded up to four
+    } tile;
     double per_column = 8.0;            // stored entries per tile column, from a sample of the tiles
     bool even_windows = false;          // no unit has over eight times the average number of steps
     // What launches write besides C, one set per stream that has launched this plan (launches on different
@@ -270,6 +281,11 @@ int scratch_for(hspmm_plan *p, hipStream_t s, size_t bytes, RunMode mode, float 
 // hspmm_entries.hip: whether the entry kernels take this launch, and the launch
 bool entries_serve(const hspmm_plan *p, uint32_t N);
 int run_entries(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode, bool *taken);
+
+// hspmm_tile.hip: the full-tile kernels' stream, whether they take this launch, and the launch
+int build_tile_stream(hspmm_plan *p);
+bool tile_serves(const hspmm_plan *p, uint32_t N);
+int run_tile(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode, bool *taken);
 
 // hspmm_run.hip: the address of the device's fixed scratch array (hspmm_run_static); `device` must be current
 int static_scratch_address(int device, float **out);

@@ -1,0 +1,126 @@
+// Host side of the full-tile kernels (spmm_tile_kernel.hip): which plans carry their stream, which launches they take, the
+// launch.
+#include "hspmm_plan.hpp"
+
+using namespace hspmm_host;
+
+namespace {
+
+// Features of a C tile: the narrowest that covers N, else 64.
+uint32_t tile_features(uint32_t N) { return N <= 16u ? 16u : N <= 32u ? 32u : 64u; }
+
+struct TileShape { uint32_t nt, n_feat_tiles, n_chunks, n_tiles, groups; size_t part_bytes; };
+
+TileShape choose_tile_shape(const hspmm_plan *p, uint32_t N)
+{
+    const hspmm_plan::Tile &t = p->tile;
+    TileShape sh;
+    sh.nt = tile_features(N);
+    sh.n_feat_tiles = (N + sh.nt - 1u) / sh.nt;
+    sh.n_chunks = t.n_blocks;
+    sh.n_tiles = t.n_row_blocks * sh.n_feat_tiles;
+    // Workgroups: one per compute unit while they are short - a workgroup more is a part more to add up, through memory -
+    // and from about 9 chunks each (20 of the longer ones of 64 features) more, up to what is resident at a time
+    // (pruned to 20 %, 11008 x 4096, N = 16: 256 / 512 / 688 workgroups 16.8 / 14.5 / 14.9 us; 4096 x 4096: 10.9 / 13.6).
+    const uint64_t items = uint64_t(sh.n_tiles) * sh.n_chunks, cu = uint64_t(p->compute_units), most = 3u;
+    const uint64_t per_cu = std::min<uint64_t>(most, std::max<uint64_t>(1u, items / (cu * (sh.nt >= 64u ? 20u : 9u))));
+    sh.groups = uint32_t(std::max<uint64_t>(1u, std::min(cu * per_cu, items / 4u)));
+    sh.part_bytes = size_t(sh.nt) * hspmm::kTileBlockRows * 4u;
+    return sh;
+}
+
+}  // namespace
+
+namespace hspmm_host {
+
+// Made where some feature dimension would take it (tile_serves) by the stored entries as estimated from a sample.
+// Block-clustered weights (over four of a column's eight elements stored) stay with kernels that read whole tiles.
+int build_tile_stream(hspmm_plan *p)
+{
+    using namespace hspmm;
+    hspmm_plan::Tile &t = p->tile;
+    const double entries = double(p->T) * p->cw * p->per_column, most_features = p->elem == 4u ? 47.0 : 127.0;
+    if (p->cfg.tile == 0 || !p->canonical || p->cfg.kernel_mode != 0) return HSPMM_OK;
+    if (p->cfg.tile < 0 && (p->G != 1 || p->per_column > 4.0 || entries * most_features < 65e6 ||
+                            entries < 0.04 * double(p->rows) * p->cols)) return HSPMM_OK;
+    const uint32_t kk = tile_block_columns(p->dtype), n_blocks = (p->cols + kk - 1u) / kk, n_row_blocks = (p->rows + kTileBlockRows - 1u) / kTileBlockRows;
+    const uint64_t cells = uint64_t(n_blocks) * n_row_blocks;
+    if (p->cols < kk || n_blocks > kTileMaxBlocks || cells >= (1u << 26)) return HSPMM_OK;
+    const TileSource src{p->d_rowOffset, p->d_rowIdx, p->d_a2b_raw, p->d_data, p->W, p->cols};
+    void *room = nullptr;
+    if (int rc = plan_alloc(p, (size_t(cells) + 1u) * 4u, &room)) return rc;
+    uint32_t *blocks = static_cast<uint32_t *>(room);
+    struct Temporary { void *p = nullptr; ~Temporary() { (void)hipFree(p); } } counts;
+    HSPMM_HIP(hipMalloc(&counts.p, size_t(cells) * 4u));
+    HSPMM_HIP(launch_tile_count(p->dtype, src, n_row_blocks, n_blocks, static_cast<uint32_t *>(counts.p), blocks, nullptr));
+    uint32_t units = 0;
+    HSPMM_HIP(hipMemcpy(&units, blocks + cells, 4, hipMemcpyDeviceToHost));
+    if (units >= (1u << 30)) return HSPMM_OK;
+    void *pos = nullptr, *vals = nullptr;
+    if (int rc = plan_alloc(p, (size_t(units) + kTileSpareUnits) * 8u, &pos)) return rc;
+    if (int rc = plan_alloc(p, (size_t(units) + kTileSpareUnits) * 4u * p->elem, &vals)) return rc;
+    HSPMM_HIP(launch_tile_fill(p->dtype, src, n_row_blocks, n_blocks, static_cast<uint32_t *>(counts.p), blocks, pos, vals, nullptr));
+    HSPMM_HIP(hipStreamSynchronize(nullptr));
+    t.d_blocks = blocks; t.d_pos = pos; t.d_vals = vals;
+    t.entries = uint64_t(units) * 4u;
+    t.n_blocks = n_blocks; t.n_row_blocks = n_row_blocks;
+    t.built = true;
+    return HSPMM_OK;
+}
+
+// Narrower than what the LDS-panel kernels take, wider than what the entry kernels are best at.  A chunk costs the same
+// whatever it stores, an entry of the other kernels a row of B, so the line goes by entries x N, and by the density for
+// large matrices.  Measured (this / the kernels otherwise chosen, us):
+//   bf16, 11008 x 4096 at 20 %: N = 8 15 / 18, 16 14.5 / 29, 32 16 / 34, 64 23 / 53;  4096 x 11008 at 10 %: N = 8 18 / 13,
+//   16 17 / 21, 32 19.5 / 27, 64 24 / 36;  5003 x 3001 at 20 %: N = 16 10.5 / 10.6, 32 11.7 / 15.2, 64 14.2 / 22;  4096^2 at 10 %:
+//   N = 32 12.4 / 8.8, 64 14.5 / 15.4;  fp32, 11008 x 4096 at 20 %: N = 8 24 / 29, 16 24 / 42, 32 28 / 35, 64 36 / 35;
+//   4096 x 11008 at 10 %: N = 16 25.7 / 26.6, 32 29 / 34.  N = 256 and more: the LDS-panel kernels by a fifth.
+bool tile_serves(const hspmm_plan *p, uint32_t N)
+{
+    const Config &c = p->cfg;
+    if (!p->tile.built || c.kernel_mode != 0 || uint64_t(N) * p->elem < 16u) return false;
+    if (c.buffer_stage || c.consumer_warp_num || c.producer_warp_group_num || c.fused_fixup >= 0) return false;     // (settings of other kernels)
+    const TileShape sh = choose_tile_shape(p, N);
+    if (uint64_t(sh.n_tiles) * sh.n_chunks >= (1u << 31) || uint64_t(N) * p->elem >= (1u << 24)) return false;
+    if (c.tile > 0) return true;
+    const bool wide = p->elem == 4u;
+    const double work = double(p->tile.entries) * N, fill = double(p->tile.entries) / (double(p->rows) * p->cols);
+    return N >= 8u && N < (wide ? 48u : 128u) && work >= (wide ? 75e6 : 65e6) && fill >= 0.04 && fill * N >= 1.5;
+}
+
+int run_tile(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode, bool *taken)
+{
+    const hspmm_plan::Tile &t = p->tile;
+    const TileShape sh = choose_tile_shape(p, N);
+    const uint32_t items = sh.n_tiles * sh.n_chunks;
+    hspmm::TileArgs ta{};
+    *taken = false;
+    ta.share = items / sh.groups; ta.rest = items % sh.groups;
+    // sums of cut tiles (see TileArgs::scratch)
+    const bool cut = sh.n_tiles % sh.groups != 0 || ta.rest || ta.share % sh.n_chunks;
+    if (cut) {
+        const size_t sums = (size_t(sh.groups) + sh.n_tiles) * sh.part_bytes;
+        std::lock_guard<std::mutex> lk(p->mu);
+        if (mode == RunMode::kStatic) {
+            // (what does not fit the fixed array is left to the kernels that need less)
+            if (sums + size_t(sh.n_tiles) * 4u > HSPMM_STATIC_SCRATCH_BYTES) return HSPMM_OK;
+            if (const int rc = scratch_for(p, s, sums, mode, &ta.scratch)) return rc;
+            ta.arrive = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(ta.scratch) + sums);
+            HSPMM_HIP(hspmm::launch_fill_zero(ta.arrive, size_t(sh.n_tiles) * 4u, s));
+        } else {
+            if (const int rc = scratch_for(p, s, sums, mode, &ta.scratch)) return rc;
+            if (const int rc = ensure_arrive(p, s, sh.n_tiles, mode, &ta.arrive)) return rc;
+        }
+    }
+    *taken = true;
+    if (mode == RunMode::kPrepare) return HSPMM_OK;
+    ta.blocks = t.d_blocks; ta.pos = t.d_pos; ta.vals = t.d_vals;
+    ta.B = dB; ta.C = dC; ta.rows = p->rows; ta.cols = p->cols; ta.N = N;
+    ta.n_row_blocks = t.n_row_blocks; ta.n_chunks = sh.n_chunks; ta.n_feat_tiles = sh.n_feat_tiles;
+    const uint32_t kind = p->dtype == HSPMM_FP16 ? 1u : 2u;
+    p->note_launch(3, kind, uint64_t(items) * (sh.nt / 16u) * 8u * (p->dtype == HSPMM_TF32 ? 3u : 2u));
+    HSPMM_HIP(hspmm::launch_spmm_tile(p->dtype, ta, sh.nt, sh.groups, s));
+    return HSPMM_OK;
+}
+
+}  // namespace hspmm_host
