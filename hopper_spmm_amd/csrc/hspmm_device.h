@@ -110,14 +110,14 @@ hipError_t launch_spmm_panel(int dtype, int G, bool split, bool tall, bool packe
 // rows above kEntryPieceUnits are cut into pieces of that many.
 constexpr uint32_t kEntryPieceUnits = 512u, kEntryClassesByLength = 8u, kEntryBins = 2u + 4u * kEntryClassesByLength;
 constexpr uint32_t kEntryChunkTiles = 64u, kEntryClasses = 2u + kEntryClassesByLength;
-struct EntryClass { uint32_t group_begin, slot_begin, slot_end, log2g; };    // first workgroup; slots; log2 subgroups per row
+struct EntryClass { uint32_t group_begin, slot_begin, slot_end, logs; };    // first workgroup; slots; log2 subgroups per row or part | log2 parts of a row << 8
 struct EntryArgs {
     const uint32_t *desc;        // per slot three words: first unit, units, matrix row (pieces: number of the piece)
     const uint32_t *ids;         // per unit four column ids
     const void     *vals;        // per unit four values
     const uint32_t *pieces;      // per piece three words: matrix row, the row's first piece, its number of pieces
-    float          *scratch;     // sums of pieces [piece][lane][features of a lane]
-    uint32_t       *arrive;      // [first piece of a row]: pieces that have left their sums (zero between launches)
+    float          *scratch;     // sums of pieces and parts [part][lane][features of a lane]
+    uint32_t       *arrive;      // [first part of a row]: parts that have left their sums (zero between launches)
     const void     *B;
     void           *C;
     uint32_t ld;                 // elements from one row of B (and of C) to the next
@@ -125,6 +125,7 @@ struct EntryArgs {
     uint32_t n_groups;           // workgroups of one block
     uint32_t n_pieces, n_classes;
     EntryClass cls[kEntryClasses];   // pieces first where there are any, then from the longest rows to the empty ones
+    uint32_t part_begin[kEntryClasses], n_parts;     // number of a class's first part
 };
 // lane_bytes (2, 4, 8, 16) x lanes (1 .. 32): how a row of B is shared out; at least lane_bytes long
 hipError_t launch_spmm_entries(int dtype, const EntryArgs &ea, uint32_t lane_bytes, uint32_t lanes, hipStream_t s);

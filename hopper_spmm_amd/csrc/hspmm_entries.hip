@@ -1,5 +1,6 @@
 // Host side of the entry kernels (spmm_entries.hip): which launches they take, the stream they walk, the launch.
 #include "hspmm_plan.hpp"
+#include <cmath>
 
 using namespace hspmm_host;
 
@@ -96,40 +97,62 @@ int build_entries(hspmm_plan *p, hipStream_t s)
     return HSPMM_OK;
 }
 
-// The classes of a launch; returns the number of workgroups.  A subgroup gets at most 4 << shift units.
-uint32_t fill_classes(const hspmm_plan *p, uint32_t lanes, int shift, hspmm::EntryArgs *ea)
+// The classes of a launch; returns the number of workgroups.  A subgroup gets at most 4 << shift units where a workgroup has
+// subgroups enough; chain: rows that would still leave a subgroup more units than that are cut into parts (0: never).
+uint32_t fill_classes(const hspmm_plan *p, uint32_t lanes, int shift, uint32_t chain, hspmm::EntryArgs *ea)
 {
     using namespace hspmm;
     const uint32_t subgroups = 256u / lanes;                 // of a workgroup
     uint32_t most = 0;
     while ((2u << most) <= subgroups) ++most;
-    uint32_t group = 0, slot = 0;
+    const uint32_t *n = p->entries.slots;
+    uint32_t group = 0, slot = 0, part = 0;
     ea->n_classes = 0;
-    auto add = [&](uint32_t slots, int wanted) {
+    auto add = [&](uint32_t slots, int wanted, uint32_t units) {
         if (!slots) return;
         const uint32_t log2g = std::min(uint32_t(std::max(wanted, 0)), most);
-        ea->cls[ea->n_classes++] = {group, slot, slot + slots, log2g};
+        uint32_t log2parts = 0;
+        while (chain && (units >> log2g >> log2parts) > chain) ++log2parts;
+        ea->part_begin[ea->n_classes] = part;
+        ea->cls[ea->n_classes++] = {group, slot, slot + slots, log2g | log2parts << 8};
         const uint32_t per_group = subgroups >> log2g;
-        group += (slots + per_group - 1u) / per_group;
+        group += ((slots << log2parts) + per_group - 1u) / per_group;
         slot += slots;
+        if (log2parts || (slot == slots && n[0])) part += slots << log2parts;       // (pieces are parts in any case)
     };
-    const uint32_t *n = p->entries.slots;
     const uint32_t top = kEntryClassesByLength - 1u;
-    add(n[0], int(top) - shift);
+    add(n[0], int(top) - shift, kEntryPieceUnits);
     for (uint32_t c = top;; --c) {
         const uint32_t *bins = n + 1u + (top - c) * 4u;
-        add(bins[0] + bins[1] + bins[2] + bins[3], int(c) - shift);
+        add(bins[0] + bins[1] + bins[2] + bins[3], int(c) - shift, 4u << c);
         if (c == 0u) break;
     }
-    add(n[kEntryBins - 1u], 0);
+    add(n[kEntryBins - 1u], 0, 0u);
+    ea->n_parts = part;
     return group;
+}
+
+// Units per subgroup: long chains need few waves and add few sums (all rows long: 4096 x 11008 at 10 %, N = 8: 17.4 -> 13.0 us
+// from 4 to 16), but where rows are short a launch takes as long as its longest chain (graph of 2^18, N = 16: 30 us at 8, 26
+// at 4) unless it has waves for several rounds.
+// A launch of few rounds also cuts rows that a workgroup's subgroups cannot bring down to 8 units each into parts (24894 vertices,
+// fp16, N = 88: 20.9 us uncut, 15.2 / 14.5 / 16.7 at 16 / 8 / 4 units; 12288, fp32, N = 128: 20.2 -> 10.2; rows all long, 4096 x
+// 11008 at 10 %, N = 8: 12.9 uncut, 19.9 at 8).  The line lies at four rounds of workgroups: graph of 40000, fp16, N = 200 (2.4
+// rounds) 37.1 -> 25.4 us, of 73838, N = 128 (2.3) 27.9 -> 29.6, of 100000 (3.1) 24.0 -> 21.0, of 73838, N = 200 (4.6) 50.8 -> 59.9.
+void choose_classes(const hspmm_plan *p, uint32_t lanes, hspmm::EntryArgs *ea)
+{
+    const uint32_t round = uint32_t(p->compute_units) * 8u;
+    int shift = 2;
+    if (!p->entries.long_rows) shift = fill_classes(p, lanes, 1, 0, ea) < 2u * round ? 0 : 1;
+    ea->n_groups = fill_classes(p, lanes, shift, 0, ea);
+    if (!p->entries.long_rows && ea->n_groups < 4u * round) ea->n_groups = fill_classes(p, lanes, shift, 8, ea);
 }
 
 }  // namespace
 
 namespace hspmm_host {
 
-constexpr uint32_t kEntryMaxRowBytes = 512;        // 32 lanes of 16 bytes
+constexpr uint32_t kEntryMaxBlockBytes = 512, kEntryMaxRowBytes = 2048;        // 32 lanes of 16 bytes; four blocks
 
 // Feature blocks of 128 bytes resp. half a row on XCDs of their own (see spmm_mfma_kernel.hpp), here for rows of 256 bytes
 // (fp32 storage: also 512): pays where B is far larger than an L2 and no row of it is hot (uniform 65536^2, 16 per row:
@@ -141,16 +164,46 @@ static bool entries_by_xcd(const hspmm_plan *p, uint64_t row_bytes)
            uint64_t(p->cols) * row_bytes >= (uint64_t(8) << 20);
 }
 
+// Bytes of a block: whole 16-byte pieces (the last block is moved back to end with the row).
+static uint32_t entry_block_bytes(uint32_t row_bytes, uint32_t blocks)
+{
+    return blocks == 1u ? row_bytes : ((row_bytes + blocks - 1u) / blocks + 15u) & ~15u;
+}
+
+// Blocks a row of B is cut into, which are passes over the entries one after the other: as few lanes as possible (a block's
+// are a power of two) and few passes; blocks of 512 bytes are behind those of 256 where B is large, and where no row is hot a
+// pass is faster the more of its part of B an L2 holds.  Measured (1 / 2 / 4 or, where in brackets, other blocks, us):
+//   fp16, graph of 40000, N = 181: 38 / 37 (3) 33, N = 256: 28 / 28 / 31; of 73838, N = 336: (2) 126 (3) 96 (6) 121, N = 512:
+//   (2) 128 (4) 113 (8) 130;  of 262144, bf16, N = 256: 147 / 126 / 128;  uniform 61181 columns, N = 256: 141 / 121 / 102, 18432
+//   columns: 133 / 95 / 95;  fp32, uniform 17544 columns, N = 224: (2) 39 (4) 40 (7) 29
+static uint32_t row_blocks(const hspmm_plan *p, uint32_t row_bytes)
+{
+    uint32_t best = 1;
+    double least = 0.0;
+    for (uint32_t b = (row_bytes + kEntryMaxBlockBytes - 1u) / kEntryMaxBlockBytes; b <= 16u && (b == 1u || row_bytes / b >= 96u); ++b) {
+        const uint32_t bytes = entry_block_bytes(row_bytes, b);
+        const RowShare share = share_row(bytes);
+        double cost = double(b * share.lanes) * (1.0 + 0.05 * double(b - 1u));
+        const double part = double(p->cols) * bytes;
+        if (bytes >= 448u && double(p->cols) * row_bytes > 16e6) cost *= 1.06;
+        if (p->even_windows && part > 3e6) cost *= 1.0 + 0.15 * std::log2(part / 3e6);
+        if (least == 0.0 || cost < least) { least = cost; best = b; }
+    }
+    return best;
+}
+
 // What an entry costs here is the lines of its row of B, what a tile column costs in the MFMA kernels does not depend
 // on how many of its eight elements are stored nor, up to a block of 32 features (16 of fp32 storage), on N.  So the line goes by
 // the bytes of a row of B and by the stored entries per tile column (per_column: 1.0 for graphs, 1.4 for weights
 // pruned to 10 %, 1.9 to 20 %, 8 for blocks).  Measured (entry / other kernels, us):
-//   16 bits, graph 2^18 N = 1 / 16 / 64: 14.5 / 45, 26 / 41, 44 / 53;  N = 100: 85 / 134, N = 200: 174 / 214 (there the
-//   other kernels lack the word-load layout), N = 128: 95 / 87, N = 192: 144 / 136;  uniform 8192^2 at 2 %, N = 256: 35 / 51
+//   16 bits, graph 2^18 N = 1 / 16 / 64: 14.5 / 45, 26 / 41, 44 / 58;  11610 vertices N = 128 / 333 / 512 / 1000: 7.6 / 14, 17 / 36,
+//   16 / 13, 26 / 25;  40000 N = 128 / 512: 16 / 24, 50 / 60;  73838 N = 128 / 336 / 512: 31 / 45, 96 / 113, 113 / 148;  2^18, 8 per
+//   vertex, N = 128 / 200 / 256: 62 / 64, 116 / 135, 126 / 119;  2^20 N = 128: 510 / 474;  uniform 8192^2 at 2 %, N = 256: 35 / 51
 //   16 bits, 4096^2 pruned to 10 % N = 8 / 16: 5.8 / 10.3, 7 / 10.4; 4096 x 11008 N = 32: 24.6 / 22.5; to 30 % N = 8 / 16:
-//   10 / 15.3, 16 / 15.3
-//   fp32, graph of 150001 N = 16 / 64 / 128: 18 / 39, 43 / 68, 92 / 126; 4096^2 pruned to 10 % N = 8 / 32 / 64: 6 / 19.5,
-//   12 / 19.5, 21 / 19.4; to 30 % N = 12 / 16: 24 / 29.7, 24 / 21; graph of 691333 (B of 354 MB) N = 128: 326 / 300
+//   10 / 15.3, 16 / 15.3;  5376 x 3328 pruned to 3 %, N = 126 / 208 / 387: 12 / 18, 18 / 21, 54 / 26 (LDS-panel kernels)
+//   fp32, graph of 150001 N = 16 / 64 / 128: 18 / 39, 43 / 68, 88 / 126;  12288 N = 128 / 256 / 500: 10 / 20, 16 / 26, 28 / 38;
+//   4096^2 pruned to 10 % N = 8 / 32 / 64: 6 / 19.5, 12 / 19.5, 21 / 19.4; to 30 % N = 12 / 16: 24 / 29.7, 24 / 21;  graph of 691333
+//   (B of 354 MB) N = 128: 326 / 300
 bool entries_serve(const hspmm_plan *p, uint32_t N)
 {
     const Config &c = p->cfg;
@@ -169,15 +222,18 @@ bool entries_serve(const hspmm_plan *p, uint32_t N)
         return sparse && !p->panel.built && (row <= 256u || all <= (uint64_t(256) << 20));
     }
     if (weight <= 42.0 || (sparse && row <= 128u)) return true;
-    if (!sparse) return false;
-    return (N % 64u != 0u && row <= 400u) || (per_column <= 1.15 && all <= (uint64_t(6) << 20)) || entries_by_xcd(p, row);
+    if (!sparse || panel_serves(p, N)) return false;
+    // (N a multiple of 64, where the other kernels load words: ahead on a B beyond the L2s' reach, and in eight blocks on a small
+    // one.  Of 8, where they load 16 bytes: on a small B with very many rows, uniform 34816 x 3575, 4 per row, N = 480: 18.7 / 16.1)
+    if (N % 64u != 0u) return !(N % 8u == 0u && row >= 896u && all <= (uint64_t(20) << 20) && p->rows > 16384u);
+    return entries_by_xcd(p, row) || (all <= (uint64_t(64) << 20) && !(row >= 1024u && all <= (uint64_t(16) << 20)));
 }
 
 int run_entries(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode, bool *taken)
 {
     const uint32_t row_bytes = N * p->elem;
     const bool by_xcd = entries_by_xcd(p, row_bytes);
-    const uint32_t blocks = by_xcd ? 2u : 1u, block_bytes = row_bytes / blocks;
+    const uint32_t blocks = by_xcd ? 2u : row_blocks(p, row_bytes), block_bytes = entry_block_bytes(row_bytes, blocks);
     const RowShare share = share_row(block_bytes);
     hspmm::EntryArgs ea{};
     hspmm_plan::Entries &e = p->entries;
@@ -193,21 +249,18 @@ int run_entries(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t
                 return HSPMM_OK;                // (nothing can be built under capture: the gather kernels take it)
             if (const int rc = build_entries(p, s)) return rc;
         }
-        // Units per subgroup: long chains need few waves and add few sums (all rows long: 4096 x 11008 at 10 %, N = 8:
-        // 17.4 -> 13.0 us from 4 to 16), but where rows are short a launch takes as long as its longest chain
-        // (graph of 2^18, N = 16: 30 us at 8, 26 at 4) unless it has waves for several rounds.
-        if (e.long_rows) ea.n_groups = fill_classes(p, share.lanes, 2, &ea);
-        else if ((ea.n_groups = fill_classes(p, share.lanes, 1, &ea)) < uint32_t(p->compute_units) * 16u)
-            ea.n_groups = fill_classes(p, share.lanes, 0, &ea);
+        hspmm::EntryArgs &classes = e.classes[__builtin_ctz(share.lanes)];
+        if (!classes.n_classes) choose_classes(p, share.lanes, &classes);
+        ea = classes;
         ea.n_pieces = e.n_pieces;
-        if (e.n_pieces) {
-            // sums of the pieces, and behind them, where nothing may be allocated, their counters
-            const size_t sums = size_t(e.n_pieces) * blocks * share.lanes * share.lane_bytes / p->elem * 4u;
-            if (const int rc = scratch_for(p, s, mode == RunMode::kStatic ? sums + size_t(e.n_pieces) * blocks * 4u : sums, mode, &ea.scratch)) return rc;
+        if (ea.n_parts) {
+            // sums of the parts, and behind them, where nothing may be allocated, their counters
+            const size_t sums = size_t(ea.n_parts) * blocks * share.lanes * share.lane_bytes / p->elem * 4u;
+            if (const int rc = scratch_for(p, s, mode == RunMode::kStatic ? sums + size_t(ea.n_parts) * blocks * 4u : sums, mode, &ea.scratch)) return rc;
             if (mode == RunMode::kStatic) {
                 ea.arrive = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(ea.scratch) + sums);
-                HSPMM_HIP(hspmm::launch_fill_zero(ea.arrive, size_t(e.n_pieces) * blocks * 4u, s));
-            } else if (const int rc = ensure_arrive(p, s, size_t(e.n_pieces) * blocks, mode, &ea.arrive)) {
+                HSPMM_HIP(hspmm::launch_fill_zero(ea.arrive, size_t(ea.n_parts) * blocks * 4u, s));
+            } else if (const int rc = ensure_arrive(p, s, size_t(ea.n_parts) * blocks, mode, &ea.arrive)) {
                 return rc;
             }
         }

@@ -175,6 +175,7 @@ struct hspmm_plan {
         uint32_t slots[hspmm::kEntryBins] = {};                  // rows per bin (bin 0: pieces)
         uint32_t n_pieces = 0;
         bool long_rows = false;                                  // 64 units and more in a row on average
+        hspmm::EntryArgs classes[6] = {};                        // by log2 lanes of a row, once a launch has asked for it
     } entries;
     // Stored entries by blocks of 128 rows x 64 (fp32 storage: 32) columns, for matrices that are dense to a workgroup
     // (spmm_tile_kernel.hip): made from the tiles on the device by hspmm_create
@@ -282,6 +283,8 @@ int scratch_for(hspmm_plan *p, hipStream_t s, size_t bytes, RunMode mode, float 
 bool entries_serve(const hspmm_plan *p, uint32_t N);
 int run_entries(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode, bool *taken);
 
+// hspmm_run.hip: whether the LDS-panel kernels serve feature dimension N
+bool panel_serves(const hspmm_plan *p, uint32_t N);
 // hspmm_tile.hip: the full-tile kernels' stream, whether they take this launch, and the launch
 int build_tile_stream(hspmm_plan *p);
 bool tile_serves(const hspmm_plan *p, uint32_t N);

@@ -358,7 +358,7 @@ static int run_panel(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStr
 
 // Whether the LDS-panel kernels serve feature dimension N (a workgroup covers 256 bytes of every B row with
 // 16-byte accesses).
-static bool panel_serves(const hspmm_plan *p, uint32_t N)
+bool hspmm_host::panel_serves(const hspmm_plan *p, uint32_t N)
 {
     if (!p->panel.built || !(p->cfg.kernel_mode == 0 || p->cfg.kernel_mode >= 4)) return false;
     const uint32_t block_feat = hspmm::kPanelRowBytes / p->elem;

@@ -109,7 +109,7 @@ __device__ __forceinline__ Piece<VB> round_sums(const float (&acc)[NF])
 // What bounds it: the gathers.  A wave keeps four rows of B per subgroup in flight and has no other loads to wait
 // for than the next unit's, so with eight waves per SIMD (64 registers) latency is covered and the L1s' and L2s'
 // line rate is what remains.
-template <class E, int VB, int L, int U>
+template <class E, int VB, int L, int U, bool Cut>
 __global__ __launch_bounds__(256)
 void spmm_entries_kernel(const EntryArgs ea)
 {
@@ -128,13 +128,23 @@ void spmm_entries_kernel(const EntryArgs ea)
     }
     uint32_t c = 0;
     while (c + 1u < ea.n_classes && group >= ea.cls[c + 1u].group_begin) ++c;
-    const uint32_t log2g = ea.cls[c].log2g, g = 1u << log2g;
+    const uint32_t logs = ea.cls[c].logs, log2g = logs & 0xFFu, log2parts = Cut ? logs >> 8 : 0u, g = 1u << log2g;
     const uint32_t sub = threadIdx.x / L, lane = threadIdx.x % L;
-    const uint32_t slot = ea.cls[c].slot_begin + (group - ea.cls[c].group_begin) * ((4u * S) >> log2g) + (sub >> log2g);
+    // (Cut: a class may cut its rows into 2^log2parts parts, each a subgroup group of its own.  An instance of its own: where
+    // no class does, the arithmetic for it is 1 - 3 % of a launch)
+    const uint32_t nth = (group - ea.cls[c].group_begin) * ((4u * S) >> log2g) + (sub >> log2g);
+    const uint32_t slot = ea.cls[c].slot_begin + (nth >> log2parts);
     const bool exists = slot < ea.cls[c].slot_end;
     const uint32_t member = sub & (g - 1u);
     const uint32_t *d = ea.desc + size_t(exists ? slot : ea.cls[c].slot_begin) * 3u;
-    const uint32_t first = d[0], units = exists ? d[1] : 0u, row = d[2];
+    uint32_t first = d[0], units = exists ? d[1] : 0u, part = 0;
+    const uint32_t row = d[2];
+    if (Cut && log2parts) {
+        part = nth & ((1u << log2parts) - 1u);
+        const uint32_t of_part = (units + (1u << log2parts) - 1u) >> log2parts, skip = part * of_part;
+        first += skip;
+        units = units > skip ? umin_e(of_part, units - skip) : 0u;
+    }
 
     // bytes of a row this block covers, and where: a last block that would reach past the row is moved back to end with it
     const uint32_t row_len = ea.block_bytes;
@@ -209,14 +219,18 @@ void spmm_entries_kernel(const EntryArgs ea)
     }
     if (!exists || member != 0u) return;
     uint32_t row_out = row;
-    if (c == 0u && ea.n_pieces) {
-        // A piece of a row longer than kEntryPieceUnits: its sums go to memory, and the subgroup that brings the
-        // row's last piece adds all of them, in order.  They cross the L2s of different XCDs: device-scope accesses,
+    const bool piece = c == 0u && ea.n_pieces;
+    if (piece || (Cut && log2parts)) {
+        // A piece of a row longer than kEntryPieceUnits, or a part of either: its sums go to memory, and the subgroup that
+        // brings the row's last part adds all of them, in order.  They cross the L2s of different XCDs: device-scope accesses,
         // and the writes are acknowledged before the arrival is counted (lanes of one subgroup are in one wave).
-        const uint32_t *pc = ea.pieces + size_t(row) * 3u;
-        const uint32_t head = pc[1], count = pc[2];
-        row_out = pc[0];
-        float *out = ea.scratch + ((size_t(row) * ea.n_feat_blocks + fb) * L + lane) * NF;
+        uint32_t mine = ea.part_begin[c] + nth, head = ea.part_begin[c] + (nth - part), count = 1u << log2parts;
+        if (piece) {
+            const uint32_t *pc = ea.pieces + size_t(row) * 3u;
+            mine = (row << log2parts) + part; head = pc[1] << log2parts; count = pc[2] << log2parts;
+            row_out = pc[0];
+        }
+        float *out = ea.scratch + ((size_t(mine) * ea.n_feat_blocks + fb) * L + lane) * NF;
 #pragma unroll
         for (int i = 0; i < NF; ++i) __hip_atomic_store(out + i, acc[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -238,13 +252,13 @@ void spmm_entries_kernel(const EntryArgs ea)
     round_sums<E, VB, NF>(acc).store(reinterpret_cast<char *>(ea.C) + size_t(row_out) * pitch + block + off);
 }
 
-template <class E>
+template <class E, bool Cut>
 static hipError_t launch_entries_e(const EntryArgs &ea, uint32_t lane_bytes, uint32_t lanes, hipStream_t s)
 {
     const uint32_t sets = ea.xcd_split ? 8u / ea.n_feat_blocks : 1u;      // workgroups of one feature block in a round over the XCDs
     const uint32_t grid = ea.xcd_split ? 8u * ((ea.n_groups + sets - 1u) / sets) : ea.n_groups * ea.n_feat_blocks;
 #define HSPMM_ENTRIES(VB, L) \
-    if (lane_bytes == VB && lanes == L) { spmm_entries_kernel<E, VB, L, (E::kElem == 2 && VB * L <= 128) ? 2 : 1><<<dim3(grid), 256, 0, s>>>(ea); return hipGetLastError(); }
+    if (lane_bytes == VB && lanes == L) { spmm_entries_kernel<E, VB, L, (E::kElem == 2 && VB * L <= 128) ? 2 : 1, Cut><<<dim3(grid), 256, 0, s>>>(ea); return hipGetLastError(); }
     if constexpr (E::kElem == 2) { HSPMM_ENTRIES(2, 1) }
     HSPMM_ENTRIES(4, 1) HSPMM_ENTRIES(4, 2) HSPMM_ENTRIES(8, 1) HSPMM_ENTRIES(8, 2)
     HSPMM_ENTRIES(16, 1) HSPMM_ENTRIES(16, 2) HSPMM_ENTRIES(16, 4) HSPMM_ENTRIES(16, 8) HSPMM_ENTRIES(16, 16) HSPMM_ENTRIES(16, 32)
@@ -260,9 +274,13 @@ hipError_t launch_spmm_entries(int dtype, const EntryArgs &ea, uint32_t lane_byt
     if (ea.block_bytes < lane_bytes || ea.block_bytes > lane_bytes * lanes || ea.n_feat_blocks < 1u ||
         uint64_t(ea.ld) * (dtype == kDtypeF32 ? 4u : 2u) < ea.block_bytes)
         return hipErrorInvalidValue;
-    if (dtype == kDtypeF32) return launch_entries_e<EntryF32>(ea, lane_bytes, lanes, s);
-    if (dtype == kDtypeBf16) return launch_entries_e<EntryBf16>(ea, lane_bytes, lanes, s);
-    return launch_entries_e<EntryF16>(ea, lane_bytes, lanes, s);
+    bool cut = false;
+    for (uint32_t c = 0; c < ea.n_classes; ++c) cut |= (ea.cls[c].logs >> 8) != 0u;
+#define HSPMM_ENTRIES_OF(E) (cut ? launch_entries_e<E, true>(ea, lane_bytes, lanes, s) : launch_entries_e<E, false>(ea, lane_bytes, lanes, s))
+    if (dtype == kDtypeF32) return HSPMM_ENTRIES_OF(EntryF32);
+    if (dtype == kDtypeBf16) return HSPMM_ENTRIES_OF(EntryBf16);
+    return HSPMM_ENTRIES_OF(EntryF16);
+#undef HSPMM_ENTRIES_OF
 }
 
 // ---------------------------------------------------------------------------

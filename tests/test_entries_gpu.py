@@ -63,6 +63,21 @@ def test_every_width_and_class_of_lengths(torch_cuda, hs, oracle, dtype):
     plan.close()
 
 
+@pytest.mark.parametrize("dtype", [0, 1, 2])
+def test_rows_cut_into_parts_and_wide_rows_in_blocks(torch_cuda, hs, oracle, dtype):
+    torch = torch_cuda
+    rng = np.random.default_rng(405 + dtype)
+    # mostly short rows; the others on both sides of the lengths at which one, two, four ... parts are taken, and of a piece
+    lengths = [2] * 1500 + [0, 32, 33, 64, 65, 128, 129, 257, 511, 513, 1025, 2048, 2049, 2500]
+    A = _rows_of_lengths(rng, lengths, 2600, dtype)
+    plan = _plan(hs, A)
+    for N in (130, 135, 257, 260, 376, 512) + (() if dtype == 1 else (513, 720, 1023, 1024)):
+        B = make_b(rng, A["cols"], N, dtype)
+        ref, mag = oracle_spmm(oracle, A, B, N)
+        _check_guarded(torch, plan, A, B, N, dtype, ref, mag, "N=%d" % N)
+    plan.close()
+
+
 @pytest.mark.parametrize("dtype,cols,N", [(0, 40000, 128), (1, 40000, 64), (1, 20000, 128)])
 def test_blocks_on_xcds_of_their_own(torch_cuda, hs, oracle, dtype, cols, N):
     torch = torch_cuda
