@@ -51,8 +51,7 @@ int validate_format(uint32_t rows, uint32_t cols, uint32_t W, uint32_t T, uint32
     // (one pass on all cores for the ids, their order and, where asked for, what the tiles store)
     std::atomic<uint32_t> first_bad{T};
     std::atomic<bool> ordered{true};
-    const size_t windows = std::max<size_t>(1, (size_t(1) << 13) / std::max<uint32_t>(1u, T / W));
-    hspmm_host::parallel_blocks(W, windows, [&](size_t wb, size_t we) {
+    hspmm_host::parallel_weighted(W, size_t(1) << 13, [=](size_t w) { return rowOffset[w]; }, [&](size_t wb, size_t we) {
         for (size_t t = rowOffset[wb], e = rowOffset[we]; t < e; ++t)
             if (tile_error(uint32_t(t), false)) {
                 uint32_t seen = first_bad.load(std::memory_order_relaxed);
@@ -621,8 +620,7 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
             uint64_t at = 0;
             std::vector<uint64_t> first(p->W);
             for (uint32_t w = 0; w < p->W; ++w) { first[w] = at; at += window_stored[w]; }
-            const size_t windows = std::max<size_t>(1, (size_t(1) << 13) / std::max<uint32_t>(1u, total_tiles / p->W));
-            hspmm_host::parallel_blocks(p->W, windows, [&](size_t wb, size_t we) {
+            hspmm_host::parallel_weighted(p->W, size_t(1) << 13, [=](size_t w) { return rowOffset[w]; }, [&](size_t wb, size_t we) {
                 const uint32_t t0 = rowOffset[wb];
                 hspmm_host::pack_tiles(static_cast<const char *>(data) + size_t(t0) * 256u, rowOffset[we] - t0, elem,
                                        header.data() + size_t(t0) * (elem == 2u ? 8u : 4u), first[wb], vals.data());

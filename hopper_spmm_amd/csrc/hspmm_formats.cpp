@@ -18,9 +18,11 @@
 #include <cstdlib>
 #include <cstring>
 #include <string>
-#include <thread>
 #include <type_traits>
 #include <vector>
+#if defined(__BMI__)
+#include <immintrin.h>
+#endif
 
 #include "../../include/hspmm.h"
 #include "host_parallel.hpp"
@@ -268,12 +270,7 @@ static int read_triples(const char *path, Triples &t, std::string &err)
             p = pe;
         }
     };
-    if (nw <= 1) work(0);
-    else {
-        std::vector<std::thread> th;
-        for (unsigned i = 0; i < nw; ++i) th.emplace_back(work, i);
-        for (auto &x : th) x.join();
-    }
+    parallel_chunks(nw, 1, [&](size_t b, size_t e) { for (; b < e; ++b) work(unsigned(b)); }, nw);
     // the reference stops reading once the declared number of entries is there (load.h:215)
     size_t total = 0;
     for (const Triples &o : part) total += o.r.size();
@@ -391,38 +388,49 @@ public:
         return u;
     }
     // lists the distinct columns among the n at `col`; rank() then holds for them until the next list()
-    const std::vector<uint32_t> &list(const uint32_t *col, size_t n)
+    struct List {
+        const uint32_t *first;
+        uint32_t n;
+        const uint32_t *data() const { return first; }
+        uint32_t size() const { return n; }
+        uint32_t operator[](uint32_t i) const { return first[i]; }
+    };
+    List list(const uint32_t *col, size_t n)
     {
-        if (sorted_) { list_sorted(col, n); return columns_; }
+        if (sorted_) { list_sorted(col, n); return {columns_.data(), uint32_t(columns_.size())}; }
         for (uint32_t i = 0; i < n_used_; ++i) words_[used_[i]] = 0;
-        if (used_.size() < std::min(n, words_.size())) used_.resize(std::min(n, words_.size()));
-        columns_.resize(n);                                 // (room; cut below)
+        if (used_.size() < std::min(n, words_.size()) + 4u) used_.resize(std::min(n, words_.size()) + 4u);
+        if (columns_.size() < n + 4u) columns_.resize(n + 4u);     // (see list_bits)
         uint64_t *words = words_.data(), *mids = mids_.data(), *tops = tops_.data();
+        // (where the entries are as many as the words of the middle level, those are all looked at instead of keeping the top
+        // level: 9 -> 5 ms of one core for the graph above)
+        const bool all_mids = n >= mids_.size();
         for (size_t i = 0; i < n; ++i) {
             const uint32_t c = col[i], w = c >> 6;
             mids[w >> 6] |= uint64_t(1) << (w & 63u);
-            tops[w >> 12] |= uint64_t(1) << ((w >> 6) & 63u);
             words[w] |= uint64_t(1) << (c & 63u);
         }
+        for (size_t i = 0; i < n && !all_mids; ++i) tops[col[i] >> 18] |= uint64_t(1) << ((col[i] >> 12) & 63u);
+        // (most words hold one to three bits, and where a loop over bits ends cannot be foretold: the first four are written in
+        // any case and those that were there are counted: 28 -> 14 ms of one core for the graph above)
         uint32_t *used = used_.data(), *columns = columns_.data(), *ranks = rank_.data();
         uint32_t n_used = 0, n_columns = 0;
-        for (size_t t = 0; t < tops_.size(); ++t) {
-            for (uint64_t top = tops[t]; top; top &= top - 1) {
-                const size_t m = t * 64 + size_t(__builtin_ctzll(top));
-                for (uint64_t mid = mids[m]; mid; mid &= mid - 1) {
-                    const uint32_t w = uint32_t(m * 64 + size_t(__builtin_ctzll(mid)));
-                    used[n_used++] = w;
-                    ranks[w] = n_columns;
-                    uint64_t word = words[w];               // (never 0)
-                    do columns[n_columns++] = w * 64u + uint32_t(__builtin_ctzll(word)); while (word &= word - 1);
-                }
-                mids[m] = 0;
-            }
+        auto list_mid = [&](size_t m) {
+            n_used += list_bits(mids[m], uint32_t(m * 64), used + n_used);
+            mids[m] = 0;
+        };
+        for (size_t m = 0; m < mids_.size() && all_mids; ++m) list_mid(m);
+        for (size_t t = 0; t < tops_.size() && !all_mids; ++t) {
+            for (uint64_t top = tops[t]; top; top &= top - 1) list_mid(t * 64 + size_t(__builtin_ctzll(top)));
             tops[t] = 0;
         }
+        for (uint32_t i = 0; i < n_used; ++i) {
+            const uint32_t w = used[i];
+            ranks[w] = n_columns;
+            n_columns += list_bits(words[w], w * 64u, columns + n_columns);
+        }
         n_used_ = n_used;
-        columns_.resize(n_columns);
-        return columns_;
+        return {columns, n_columns};
     }
     uint32_t rank(uint32_t column) const
     {
@@ -432,6 +440,22 @@ public:
     }
 
 private:
+    // base + the number of every bit of `bits`, lowest first; returns how many.  Writes four numbers in any case.
+    static uint32_t list_bits(uint64_t bits, uint32_t base, uint32_t *out)
+    {
+        const uint32_t n = uint32_t(__builtin_popcountll(bits));
+        for (uint32_t i = 0; i < 4; ++i, bits &= bits - 1) out[i] = base + lowest(bits);
+        for (uint32_t i = 4; bits; ++i, bits &= bits - 1) out[i] = base + lowest(bits);
+        return n;
+    }
+    static uint32_t lowest(uint64_t bits)                  // (0 has none: any number will do)
+    {
+#if defined(__BMI__)
+        return uint32_t(_tzcnt_u64(bits));
+#else
+        return bits ? uint32_t(__builtin_ctzll(bits)) : 0u;
+#endif
+    }
     void list_sorted(const uint32_t *col, size_t n)
     {
         columns_.assign(col, col + n);
@@ -457,16 +481,15 @@ static uint32_t column_count(const uint32_t *col, size_t n)
     return largest.load() == 0xFFFFFFFFu ? 0xFFFFFFFFu : largest.load() + 1u;
 }
 
-// Windows a worker takes at a time: what holds about 16 K stored entries (a matrix of few wide
-// windows, like block-clustered weights, still spreads over the cores).
-static size_t windows_per_worker(size_t nwin, size_t nnz)
-{
-    if (nnz == 0 || nwin == 0) return 2048;
-    const size_t per_window = (nnz + nwin - 1) / nwin;
-    return std::max<size_t>(1, std::min<size_t>(2048, (size_t(1) << 14) / std::max<size_t>(1, per_window)));
-}
-
 static size_t window_count(uint32_t rows) { return (size_t(rows) + HSPMM_ROW_WINDOW - 1) / HSPMM_ROW_WINDOW; }
+
+// fn(first, end) on runs of windows with about the same number of stored entries, 16 K and more per worker.
+template <class F>
+static void parallel_windows(uint32_t rows, const uint32_t *row_ptr, F &&fn)
+{
+    parallel_weighted(window_count(rows), size_t(1) << 14,
+                      [=](size_t w) { return row_ptr[std::min<size_t>(w * HSPMM_ROW_WINDOW, rows)]; }, fn);
+}
 
 // tiles[w] = number of tiles of window w (0 for a window without entries).
 static void count_tiles(uint32_t rows, const uint32_t *row_ptr, const uint32_t *col_idx, uint32_t cw,
@@ -474,7 +497,7 @@ static void count_tiles(uint32_t rows, const uint32_t *row_ptr, const uint32_t *
 {
     const size_t nwin = window_count(rows);
     std::fill(tiles, tiles + nwin, 0u);
-    parallel_chunks(nwin, windows_per_worker(nwin, row_ptr[rows]), [&](size_t wb, size_t we) {
+    parallel_windows(rows, row_ptr, [&](size_t wb, size_t we) {
         ColumnSet set(n_columns, row_ptr[rows]);
         for (size_t w = wb; w < we; ++w) {
             const uint32_t r0 = uint32_t(w * HSPMM_ROW_WINDOW);
@@ -503,16 +526,15 @@ static bool fill_tiles(uint32_t rows, uint32_t n_columns, const uint32_t *row_pt
                        bool transpose, const std::vector<uint32_t> &tiles, const TileArrays &out)
 {
     constexpr size_t kTile = size_t(HSPMM_ROW_WINDOW) * CW;
-    const size_t nwin = tiles.size();
     const V *from = static_cast<const V *>(values);
     std::atomic<bool> as_counted{true};
-    parallel_chunks(nwin, windows_per_worker(nwin, row_ptr[rows]), [&](size_t wb, size_t we) {
+    parallel_windows(rows, row_ptr, [&](size_t wb, size_t we) {
         ColumnSet set(n_columns, row_ptr[rows]);
         for (size_t w = wb; w < we; ++w) {
             if (!tiles[w] && row_ptr[std::min<size_t>((w + 1) * HSPMM_ROW_WINDOW, rows)] == row_ptr[w * HSPMM_ROW_WINDOW]) continue;
             const uint32_t r0 = uint32_t(w * HSPMM_ROW_WINDOW);
             const uint32_t r1 = std::min<uint64_t>(uint64_t(r0) + HSPMM_ROW_WINDOW, rows);
-            const std::vector<uint32_t> &uniq = set.list(col_idx + row_ptr[r0], row_ptr[r1] - row_ptr[r0]);
+            const ColumnSet::List uniq = set.list(col_idx + row_ptr[r0], row_ptr[r1] - row_ptr[r0]);
             const uint32_t u = uint32_t(uniq.size());
             const uint32_t ew = out.eff_index[w], ft = out.first_tile[w], nt = tiles[w];
             if ((u + CW - 1) / CW != nt) { as_counted.store(false); continue; }
@@ -705,7 +727,7 @@ int hspmm_bitmap_fill_counted(int dtype, uint32_t rows, const uint32_t *row_ptr,
             if (!tiles[w] && row_ptr[std::min<size_t>((w + 1) * HSPMM_ROW_WINDOW, rows)] == row_ptr[w * HSPMM_ROW_WINDOW]) continue;
             const uint32_t r0 = uint32_t(w * HSPMM_ROW_WINDOW);
             const uint32_t r1 = std::min<uint64_t>(uint64_t(r0) + HSPMM_ROW_WINDOW, rows);
-            const std::vector<uint32_t> &uniq = set.list(col_idx + row_ptr[r0], row_ptr[r1] - row_ptr[r0]);
+            const ColumnSet::List uniq = set.list(col_idx + row_ptr[r0], row_ptr[r1] - row_ptr[r0]);
             const uint32_t u = uint32_t(uniq.size());
             const uint32_t ew = eff_index[w], ft = first_tile[w], nt = tiles[w];
             if ((u + CW - 1) / CW != nt) { as_counted.store(false); continue; }
@@ -747,7 +769,7 @@ int hspmm_bitmap_fill_counted(int dtype, uint32_t rows, const uint32_t *row_ptr,
         else convert_windows(std::integral_constant<uint32_t, 8>{}, uint32_t{}, wb, we);
     };
     if (shared_words) convert(0, nwin);
-    else parallel_chunks(nwin, windows_per_worker(nwin, row_ptr[rows]), convert);
+    else parallel_windows(rows, row_ptr, convert);
     if (!as_counted.load()) { set_error("window_tiles does not belong to this matrix"); return HSPMM_ERR_INVALID; }
     return HSPMM_OK;
 }
@@ -789,12 +811,7 @@ int hspmm_bitmap_expand(int dtype, uint32_t total_tiles, const uint32_t *nnzOffs
             }
         }
     };
-    if (nw <= 1) work(0);
-    else {
-        std::vector<std::thread> th;
-        for (unsigned i = 0; i < nw; ++i) th.emplace_back(work, i);
-        for (auto &t : th) t.join();
-    }
+    parallel_chunks(nw, 1, [&](size_t b, size_t e) { for (; b < e; ++b) work(unsigned(b)); }, nw);
     for (uint32_t b : bad_per_block) if (b < first_bad) first_bad = b;
     if (first_bad != HSPMM_IDX_MAX) {
         set_error("tile " + std::to_string(first_bad) + ": the number of set bits differs from its nnzOffset span");
