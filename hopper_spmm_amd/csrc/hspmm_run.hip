@@ -270,24 +270,38 @@ static int choose_panel_shape(const hspmm_plan *p, uint32_t N, PanelShape *out)
     const uint32_t wave_units = pl.tall ? (pl.n_units + 1u) / 2u : pl.n_units;
     if (forced_units) forced_units = std::min(forced_units, max_units);
     const uint64_t slots = uint64_t(p->compute_units) * (pl.quad ? 2u : 1u);     // workgroups resident at a time
-    // Units per workgroup and chunks of panels: the workgroups should fill the compute units in whole
-    // rounds.  Cost of a shape = rounds x panels per chunk x (units + 3: a panel costs its LDS reads and
-    // MFMAs, which go with the units, plus its copy and barrier), plus what chunk sums cost.
+    // Units per workgroup and chunks of panels, of all shapes the one expected to be fastest.  What binds is bytes moving into a
+    // compute unit, about 60 KB a microsecond: per panel its 64 KB of B and every unit's tiles of that panel (1 KB a step, 2 KB
+    // for units of four windows and fp32 storage in bf16 parts, which cost 1.6 times as much); more chunks fill more compute units
+    // and cost their sums' way through memory.  The constants are a fit to 650 measured shapes - four to twelve units, one to six
+    // chunks, pruned matrices at 5 to 20 % and block-clustered ones, all types - with a mean error of 9 %; the shape it picks is
+    // within 1.4 % of the fastest on average, where whole rounds of workgroups and ppc * (units + 3) were 7.5 % behind (5003 x
+    // 3001 at 20 %, bf16, N = 128: 18.8 -> 15.8 us; 4096 x 11008 at 10 %, fp16, N = 128: 34.8 -> 26.8).
+    const size_t wide_rows = pl.G == 4 ? 2u : 1u;
+    sh.acc_per_unit = pl.quad ? 2u : pl.split ? 4u * wide_rows : p->dtype != HSPMM_TF32 ? 8u * wide_rows : 4u * size_t(pl.G);
+    const double steps = double(pl.n_steps) / (double(std::max<uint32_t>(pl.n_units, 1u)) * double(pl.n_panels));
+    const double step_cost = 0.017 * steps * (pl.split || pl.G == 4 ? 1.63 : 1.0);
+    const double sum_cost = 0.56 * double(pl.n_units) * sh.n_feat_blocks * double(sh.acc_per_unit) / 1024.0;
     uint64_t chunks = 1;
     int best_units = max_units;
     double best_cost = 0.0;
-    for (int nc = forced_units ? forced_units : std::max(4, max_units / 2); nc <= (forced_units ? forced_units : max_units); ++nc) {
+    for (int nc = forced_units ? forced_units : 4; nc <= (forced_units ? forced_units : max_units); ++nc) {
         const uint64_t rbs = (uint64_t(wave_units) + nc - 1) / nc, base = rbs * sh.n_feat_blocks;
-        uint64_t ch = base >= slots ? 1 : std::min<uint64_t>(slots / base, pl.n_panels);
-        const uint64_t ppc = (pl.n_panels + ch - 1) / ch;
-        ch = (pl.n_panels + ppc - 1) / ppc;
-        const uint64_t rounds = (base * ch + slots - 1) / slots;
-        // (streams with two units per wave: the same in 128-byte lines - per panel its copy and every unit's
-        // tiles and ids - which is what those streams were measured with)
-        const double cost = pl.tall ? double(rounds) * double(ppc) * (512.0 + 2.0 * double(nc) * pl.unit_lines) +
-                                          (ch > 1 ? 2500.0 + 300.0 * double(ch) : 0.0)
-                                    : double(rounds) * double(ppc) * (double(nc) + 3.0) + (ch > 1 ? 80.0 : 0.0);
-        if (best_cost == 0.0 || cost < best_cost) { best_cost = cost; best_units = nc; chunks = ch; }
+        // (the fp32 products and streams with two units per wave: as many chunks as one round of workgroups has room for)
+        const uint64_t fill = std::min<uint64_t>(pl.n_panels, std::max<uint64_t>(1u, slots / base));
+        const bool fitted = wide && !pl.tall;
+        for (uint64_t ask = fitted ? 1u : fill, most = fitted ? std::min<uint64_t>(pl.n_panels, 2u * fill) : fill; ask <= most; ++ask) {
+            const uint64_t ppc = (pl.n_panels + ask - 1) / ask, ch = (pl.n_panels + ppc - 1) / ppc;
+            const uint64_t rounds = (base * ch + slots - 1) / slots;
+            // (streams with two units per wave: in 128-byte lines - per panel its copy and every unit's tiles and ids - which is
+            // what those streams were measured with)
+            const double cost = pl.tall ? double(rounds) * double(ppc) * (512.0 + 2.0 * double(nc) * pl.unit_lines) +
+                                              (ch > 1 ? 2500.0 + 300.0 * double(ch) : 0.0)
+                                : !fitted ? double(rounds) * double(ppc) * (double(nc) + 3.0) + (ch > 1 ? 80.0 : 0.0)
+                                        : double(rounds) * double(ppc) * (1.02 + step_cost * double(nc)) +
+                                              (ch > 1 ? 0.5 * double(ch) - 1.07 + sum_cost * double(ch) : 0.0);
+            if (best_cost == 0.0 || cost < best_cost) { best_cost = cost; best_units = nc; chunks = ch; }
+        }
     }
     sh.units = units;
     sh.units_per_group = uint32_t(best_units);
@@ -302,8 +316,6 @@ static int choose_panel_shape(const hspmm_plan *p, uint32_t N, PanelShape *out)
         return fail(HSPMM_ERR_UNSUPPORTED, "feature dimension %u needs too many workgroups", N);
     if (uint64_t(pl.n_units) * sh.n_chunks > 0xFFFFFFFFull)
         return fail(HSPMM_ERR_UNSUPPORTED, "feature dimension %u needs too many partial sums", N);
-    const size_t wide_rows = pl.G == 4 ? 2u : 1u;
-    sh.acc_per_unit = pl.quad ? 2u : pl.split ? 4u * wide_rows : p->dtype != HSPMM_TF32 ? 8u * wide_rows : 4u * size_t(pl.G);
     // matrix instructions per step and feature block (PanelOps<...>::mma_half in spmm_panel_kernel.hpp)
     sh.mfma_kind = pl.quad ? 4u : (p->dtype == HSPMM_TF32 && !pl.split) ? 3u : (p->dtype == HSPMM_FP16 ? 1u : 2u);
     const uint64_t per_step = pl.quad ? 16u : pl.split ? 12u * wide_rows : p->dtype != HSPMM_TF32 ? 8u * wide_rows : 8u * uint64_t(pl.G);
