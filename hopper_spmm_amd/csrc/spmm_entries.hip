@@ -20,6 +20,7 @@ typedef uint32_t e_u32x4 __attribute__((ext_vector_type(4)));
 struct EntryF16 {
     static constexpr uint32_t kElem = 2;
     typedef e_u32x2 Vals;
+    __device__ static __forceinline__ bool stored(const Vals v, int i) { return (v[i >> 1] & ((i & 1) ? 0xFFFF0000u : 0xFFFFu)) != 0u; }
     __device__ static __forceinline__ float value(const Vals v, int i)
     {
         const uint32_t w = v[i >> 1];
@@ -32,6 +33,7 @@ struct EntryF16 {
 struct EntryBf16 {
     static constexpr uint32_t kElem = 2;
     typedef e_u32x2 Vals;
+    __device__ static __forceinline__ bool stored(const Vals v, int i) { return (v[i >> 1] & ((i & 1) ? 0xFFFF0000u : 0xFFFFu)) != 0u; }
     __device__ static __forceinline__ float value(const Vals v, int i)
     {
         const uint32_t w = v[i >> 1];
@@ -44,6 +46,7 @@ struct EntryBf16 {
 struct EntryF32 {
     static constexpr uint32_t kElem = 4;
     typedef e_u32x4 Vals;
+    __device__ static __forceinline__ bool stored(const Vals v, int i) { return v[i] != 0u; }
     __device__ static __forceinline__ float value(const Vals v, int i)
     {
         const uint32_t w = v[i];
@@ -193,6 +196,26 @@ void spmm_entries_kernel(const EntryArgs ea)
                 }
             if (next >= units) break;
             u = next;
+        }
+        // What fills a row's last unit up (+0, which no stored value is, at the row's last column) counts for nothing, unless that
+        // row of B is not finite there: then once more, the stored entries alone, in the same order.
+        float met = 0.f;
+#pragma unroll
+        for (int i = 0; i < NF; ++i) met = __builtin_fmaf(acc[i], 0.f, met);
+        if (met != 0.f) {
+#pragma unroll
+            for (int i = 0; i < NF; ++i) acc[i] = 0.f;
+            for (u = member; u < units; u += g) {
+                const e_u32x4 at = *reinterpret_cast<const e_u32x4 *>(ids + size_t(u) * 4u);
+                const typename E::Vals a = vals[u];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (E::stored(a, i)) {
+                        Piece<VB> b;
+                        b.load(B + size_t(at[i]) * pitch);
+                        multiply_in<E, VB, NF>(acc, b, E::value(a, i));
+                    }
+            }
         }
     }
     // the subgroups of one wave, then those of the waves of the workgroup
