@@ -142,6 +142,7 @@ hipError_t launch_entry_fill(int elem, const void *tiles, const uint32_t *a2b, c
 constexpr uint32_t kTileBlockRows = 128u, kTileMaxBlocks = 4096u;     // blocks of a row block at most
 constexpr uint32_t kTileSpareUnits = 512u;                            // behind the last unit (read and not used)
 uint32_t tile_block_columns(int dtype);
+struct TileSource { const uint32_t *rowOffset, *rowIdx, *a2b; const void *tiles; uint32_t n_windows, cols; };   // the format arrays
 struct TileArgs {
     const uint32_t *blocks;      // per row block and block: its first unit (n_row_blocks x n_blocks + 1)
     const void     *pos, *vals;
@@ -152,10 +153,10 @@ struct TileArgs {
     uint32_t rows, cols, N;
     uint32_t n_row_blocks, n_chunks, n_feat_tiles;               // chunks: blocks of columns
     uint32_t share, rest;        // items (chunks of C tiles) of a workgroup; the first `rest` have one more
+    const TileSource *src;       // in device memory (read where B is not finite)
 };
 // nt: features of a C tile (16, 32, 64)
 hipError_t launch_spmm_tile(int dtype, const TileArgs &ta, uint32_t nt, uint32_t groups, hipStream_t s);
-struct TileSource { const uint32_t *rowOffset, *rowIdx, *a2b; const void *tiles; uint32_t n_windows, cols; };   // the format arrays
 hipError_t launch_tile_count(int dtype, const TileSource &src, uint32_t n_row_blocks, uint32_t n_blocks, uint32_t *counts, uint32_t *blocks, hipStream_t s);
 hipError_t launch_tile_fill(int dtype, const TileSource &src, uint32_t n_row_blocks, uint32_t n_blocks, const uint32_t *counts,
                             const uint32_t *blocks, void *pos, void *vals, hipStream_t s);

@@ -183,6 +183,7 @@ struct hspmm_plan {
         bool built = false;
         const uint32_t *d_blocks = nullptr;
         const void *d_pos = nullptr, *d_vals = nullptr;
+        hspmm::TileSource *d_source = nullptr;                   // where the tiles are
         uint32_t n_row_blocks = 0, n_blocks = 0;
         uint64_t entries = 0;                                    // stored entries, blocks rounded up to four
     } tile;

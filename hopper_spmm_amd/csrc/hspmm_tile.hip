@@ -60,6 +60,7 @@ int build_tile_stream(hspmm_plan *p)
     if (int rc = plan_alloc(p, (size_t(units) + kTileSpareUnits) * 8u, &pos)) return rc;
     if (int rc = plan_alloc(p, (size_t(units) + kTileSpareUnits) * 4u * p->elem, &vals)) return rc;
     HSPMM_HIP(launch_tile_fill(p->dtype, src, n_row_blocks, n_blocks, static_cast<uint32_t *>(counts.p), blocks, pos, vals, nullptr));
+    if (int rc = upload(p, &t.d_source, &src, 1)) return rc;
     HSPMM_HIP(hipStreamSynchronize(nullptr));
     t.d_blocks = blocks; t.d_pos = pos; t.d_vals = vals;
     t.entries = uint64_t(units) * 4u;
@@ -116,6 +117,7 @@ int run_tile(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s,
     if (mode == RunMode::kPrepare) return HSPMM_OK;
     ta.blocks = t.d_blocks; ta.pos = t.d_pos; ta.vals = t.d_vals;
     ta.B = dB; ta.C = dC; ta.rows = p->rows; ta.cols = p->cols; ta.N = N;
+    ta.src = t.d_source;
     ta.n_row_blocks = t.n_row_blocks; ta.n_chunks = sh.n_chunks; ta.n_feat_tiles = sh.n_feat_tiles;
     const uint32_t kind = p->dtype == HSPMM_FP16 ? 1u : 2u;
     p->note_launch(3, kind, uint64_t(items) * (sh.nt / 16u) * 8u * (p->dtype == HSPMM_TF32 ? 3u : 2u));
