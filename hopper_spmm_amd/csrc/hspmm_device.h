@@ -148,13 +148,17 @@ struct TileArgs {
     const void     *pos, *vals;
     const void     *B;
     void           *C;
-    float          *scratch;     // sums of the parts of cut C tiles: part g + t for workgroup g and tile t
-    uint32_t       *arrive;      // per C tile: parts that have left their sums (zero between launches)
+    float          *scratch;     // sums of the parts of cut C tiles (tile_parts of them)
+    uint32_t       *arrive;      // per workgroup: parts of the cut C tile it has the first part of that have left their sums
+                                 // (zero between launches; of no two cut tiles a workgroup has the first part)
     uint32_t rows, cols, N;
     uint32_t n_row_blocks, n_chunks, n_feat_tiles;               // chunks: blocks of columns
     uint32_t share, rest;        // items (chunks of C tiles) of a workgroup; the first `rest` have one more
     const TileSource *src;       // in device memory (read where B is not finite)
 };
+// Places for the parts of cut C tiles: a workgroup has two at most, of its first and of its last tile (part 2 g + 0 or 1); with
+// no more tiles than workgroups a tile's parts overlap the next one's in one place less (part g + t).
+inline uint64_t tile_parts(uint32_t groups, uint32_t n_tiles) { return uint64_t(groups) + (groups < n_tiles ? groups : n_tiles); }
 // nt: features of a C tile (16, 32, 64)
 hipError_t launch_spmm_tile(int dtype, const TileArgs &ta, uint32_t nt, uint32_t groups, hipStream_t s);
 hipError_t launch_tile_count(int dtype, const TileSource &src, uint32_t n_row_blocks, uint32_t n_blocks, uint32_t *counts, uint32_t *blocks, hipStream_t s);

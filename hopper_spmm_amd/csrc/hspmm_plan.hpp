@@ -289,7 +289,7 @@ bool panel_serves(const hspmm_plan *p, uint32_t N);
 // hspmm_tile.hip: the full-tile kernels' stream, whether they take this launch, and the launch
 int build_tile_stream(hspmm_plan *p);
 bool tile_serves(const hspmm_plan *p, uint32_t N);
-int run_tile(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode, bool *taken);
+int run_tile(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode);
 
 // hspmm_run.hip: the address of the device's fixed scratch array (hspmm_run_static); `device` must be current
 int static_scratch_address(int device, float **out);

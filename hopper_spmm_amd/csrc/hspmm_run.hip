@@ -419,11 +419,7 @@ static int run_impl(hspmm_plan *p, const void *dB, void *dC, uint32_t N, void *s
         HSPMM_HIP(hspmm::launch_fill_zero(dC, size_t(p->rows) * N * p->elem, s));
         return HSPMM_OK;
     }
-    if (tile_serves(p, N)) {
-        bool taken = false;
-        const int rc = run_tile(p, dB, dC, N, s, mode, &taken);
-        if (rc || taken) return rc;
-    }
+    if (tile_serves(p, N)) return run_tile(p, dB, dC, N, s, mode);
     if (entries_serve(p, N)) {
         bool taken = false;
         const int rc = run_entries(p, dB, dC, N, s, mode, &taken);

@@ -9,7 +9,11 @@ namespace {
 // Features of a C tile: the narrowest that covers N, else 64.
 uint32_t tile_features(uint32_t N) { return N <= 16u ? 16u : N <= 32u ? 32u : 64u; }
 
-struct TileShape { uint32_t nt, n_feat_tiles, n_chunks, n_tiles, groups; size_t part_bytes; };
+struct TileShape {
+    uint32_t nt, n_feat_tiles, n_chunks, n_tiles, groups, share, rest;
+    bool cut;                           // C tiles shared by workgroups
+    size_t sums_bytes;                  // of their parts
+};
 
 TileShape choose_tile_shape(const hspmm_plan *p, uint32_t N)
 {
@@ -25,7 +29,18 @@ TileShape choose_tile_shape(const hspmm_plan *p, uint32_t N)
     const uint64_t items = uint64_t(sh.n_tiles) * sh.n_chunks, cu = uint64_t(p->compute_units), most = 3u;
     const uint64_t per_cu = std::min<uint64_t>(most, std::max<uint64_t>(1u, items / (cu * (sh.nt >= 64u ? 20u : 9u))));
     sh.groups = uint32_t(std::max<uint64_t>(1u, std::min(cu * per_cu, items / 4u)));
-    sh.part_bytes = size_t(sh.nt) * hspmm::kTileBlockRows * 4u;
+    // Every mode of launching has the same shape, and its parts and counters fit what hspmm_run_static has: the limit is met
+    // from 16257 rows on at N = 65 .. 127 (767 workgroups instead of 768) and stays at 511, two per compute unit, for any more.
+    const size_t part_bytes = size_t(sh.nt) * hspmm::kTileBlockRows * 4u;
+    for (;;) {
+        sh.share = uint32_t(items / sh.groups);
+        sh.rest = uint32_t(items % sh.groups);
+        sh.cut = sh.rest || sh.share % sh.n_chunks;
+        sh.sums_bytes = sh.cut ? size_t(hspmm::tile_parts(sh.groups, sh.n_tiles)) * part_bytes : 0u;
+        if (sh.sums_bytes + size_t(sh.groups) * 4u <= HSPMM_STATIC_SCRATCH_BYTES) break;
+        const size_t any = HSPMM_STATIC_SCRATCH_BYTES / (2u * part_bytes + 4u), few = HSPMM_STATIC_SCRATCH_BYTES / (part_bytes + 4u);
+        sh.groups = uint32_t(std::max(any, few > sh.n_tiles ? few - sh.n_tiles : size_t(0)));
+    }
     return sh;
 }
 
@@ -89,38 +104,31 @@ bool tile_serves(const hspmm_plan *p, uint32_t N)
     return N >= 8u && N < (wide ? 48u : 128u) && work >= (wide ? 75e6 : 65e6) && fill >= 0.04 && fill * N >= 1.5;
 }
 
-int run_tile(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode, bool *taken)
+int run_tile(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode)
 {
     const hspmm_plan::Tile &t = p->tile;
     const TileShape sh = choose_tile_shape(p, N);
-    const uint32_t items = sh.n_tiles * sh.n_chunks;
     hspmm::TileArgs ta{};
-    *taken = false;
-    ta.share = items / sh.groups; ta.rest = items % sh.groups;
-    // sums of cut tiles (see TileArgs::scratch)
-    const bool cut = sh.n_tiles % sh.groups != 0 || ta.rest || ta.share % sh.n_chunks;
-    if (cut) {
-        const size_t sums = (size_t(sh.groups) + sh.n_tiles) * sh.part_bytes;
+    ta.share = sh.share; ta.rest = sh.rest;
+    if (sh.cut) {
+        const size_t counters = size_t(sh.groups) * 4u;
         std::lock_guard<std::mutex> lk(p->mu);
         if (mode == RunMode::kStatic) {
-            // (what does not fit the fixed array is left to the kernels that need less)
-            if (sums + size_t(sh.n_tiles) * 4u > HSPMM_STATIC_SCRATCH_BYTES) return HSPMM_OK;
-            if (const int rc = scratch_for(p, s, sums, mode, &ta.scratch)) return rc;
-            ta.arrive = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(ta.scratch) + sums);
-            HSPMM_HIP(hspmm::launch_fill_zero(ta.arrive, size_t(sh.n_tiles) * 4u, s));
+            if (const int rc = scratch_for(p, s, sh.sums_bytes + counters, mode, &ta.scratch)) return rc;
+            ta.arrive = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(ta.scratch) + sh.sums_bytes);
+            HSPMM_HIP(hspmm::launch_fill_zero(ta.arrive, counters, s));
         } else {
-            if (const int rc = scratch_for(p, s, sums, mode, &ta.scratch)) return rc;
-            if (const int rc = ensure_arrive(p, s, sh.n_tiles, mode, &ta.arrive)) return rc;
+            if (const int rc = scratch_for(p, s, sh.sums_bytes, mode, &ta.scratch)) return rc;
+            if (const int rc = ensure_arrive(p, s, sh.groups, mode, &ta.arrive)) return rc;
         }
     }
-    *taken = true;
     if (mode == RunMode::kPrepare) return HSPMM_OK;
     ta.blocks = t.d_blocks; ta.pos = t.d_pos; ta.vals = t.d_vals;
     ta.B = dB; ta.C = dC; ta.rows = p->rows; ta.cols = p->cols; ta.N = N;
     ta.src = t.d_source;
     ta.n_row_blocks = t.n_row_blocks; ta.n_chunks = sh.n_chunks; ta.n_feat_tiles = sh.n_feat_tiles;
     const uint32_t kind = p->dtype == HSPMM_FP16 ? 1u : 2u;
-    p->note_launch(3, kind, uint64_t(items) * (sh.nt / 16u) * 8u * (p->dtype == HSPMM_TF32 ? 3u : 2u));
+    p->note_launch(3, kind, uint64_t(sh.n_tiles) * sh.n_chunks * (sh.nt / 16u) * 8u * (p->dtype == HSPMM_TF32 ? 3u : 2u));
     HSPMM_HIP(hspmm::launch_spmm_tile(p->dtype, ta, sh.nt, sh.groups, s));
     return HSPMM_OK;
 }

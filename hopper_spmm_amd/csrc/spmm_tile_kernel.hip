@@ -399,6 +399,11 @@ void spmm_tile_kernel(const TileArgs ta)
         const uint32_t longer = ta.rest * (ta.share + 1u);
         return i < longer ? i / (ta.share + 1u) : ta.rest + (i - longer) / ta.share;
     };
+    // Where the sums of workgroup g's part of tile t go (see tile_parts).
+    auto part = [&](uint32_t g, uint32_t t) __attribute__((always_inline)) -> uint32_t {
+        if (ta.n_row_blocks * ta.n_feat_tiles <= n_groups) return g + t;
+        return 2u * g + (g * ta.share + umin32(g, ta.rest) < t * n_chunks ? 1u : 0u);
+    };
     // The first to the last C tile whose sums this wave has found not finite (it has finished all between them: only the first
     // and the last tile of a workgroup may be another's to finish).
     uint32_t again_begin = 0, again_end = 0;
@@ -407,17 +412,16 @@ void spmm_tile_kernel(const TileArgs ta)
             constexpr uint32_t kSums = RF * CF * 4096u;             // bytes of a part
             const uint32_t first = owner(now.tile * n_chunks), count = owner((now.tile + 1u) * n_chunks - 1u) - first + 1u;
             {
-                // (part of group g of tile t: number g + t, which grows from part to part)
-                const __amdgpu_buffer_rsrc_t out = device_scope_buffer(reinterpret_cast<char *>(ta.scratch) + size_t(group + now.tile) * kSums);
+                const __amdgpu_buffer_rsrc_t out = device_scope_buffer(reinterpret_cast<char *>(ta.scratch) + size_t(part(group, now.tile)) * kSums);
 #pragma unroll
                 for (int i = 0; i < RF * CF; ++i) store_device_scope(out, uint32_t(i) * 4096u + tid * 16u, acc[i / CF][i % CF]);
             }
             wait_stores_acknowledged();
             __syncthreads();
             if (tid == 0u) {
-                const uint32_t old = __hip_atomic_fetch_add(ta.arrive + now.tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const uint32_t old = __hip_atomic_fetch_add(ta.arrive + first, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 last_part = old + 1u == count;
-                if (old + 1u == count) __hip_atomic_store(ta.arrive + now.tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (old + 1u == count) __hip_atomic_store(ta.arrive + first, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
             __syncthreads();
             asm volatile("" ::: "memory");
@@ -425,7 +429,7 @@ void spmm_tile_kernel(const TileArgs ta)
 #pragma unroll
             for (int i = 0; i < RF * CF; ++i) acc[i / CF][i % CF] = f32x4{0.f, 0.f, 0.f, 0.f};
             for (uint32_t s = 0; s < count; ++s) {
-                const __amdgpu_buffer_rsrc_t in = device_scope_buffer(reinterpret_cast<const char *>(ta.scratch) + size_t(first + s + now.tile) * kSums);
+                const __amdgpu_buffer_rsrc_t in = device_scope_buffer(reinterpret_cast<const char *>(ta.scratch) + size_t(part(first + s, now.tile)) * kSums);
 #pragma unroll
                 for (int i = 0; i < RF * CF; ++i) acc[i / CF][i % CF] += load_device_scope(in, uint32_t(i) * 4096u + tid * 16u);
             }

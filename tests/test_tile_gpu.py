@@ -78,3 +78,39 @@ def test_chosen_for_wide_enough_launches_of_dense_enough_matrices(torch_cuda, hs
     assert np.array_equal(dC.cpu().numpy().view(np.uint8), want.view(np.uint8))
     assert plan.info()["last_kernel_family"] == 3
     plan.close()
+
+
+def _sampled_csr(rng, rows, cols, per_row, dtype, values):
+    """per_row entries in every row, at columns without any order to them; values(n) gives them."""
+    step = cols // per_row
+    col_idx = (np.arange(per_row, dtype=np.int64)[None, :] * step + rng.integers(0, step, (rows, per_row))).astype(np.uint32)
+    return dict(rows=rows, cols=cols, nnzs=rows * per_row, dtype=dtype, row_ptr=(np.arange(rows + 1, dtype=np.int64) * per_row).astype(np.uint32),
+                col_idx=col_idx.reshape(-1), values=encode(values(rows * per_row).astype(np.float32), dtype))
+
+
+def _random_operand(torch, rng, cols, N, dtype):
+    B = encode(rng.normal(size=(cols, N)).astype(np.float32), dtype)
+    return B, torch.from_numpy(B if dtype == 1 else B.view(np.int16)).cuda()
+
+
+# (17000 rows at N = 96: three workgroups per compute unit leave more sums than the fixed array holds; 70000: more C tiles
+# than workgroups)
+@pytest.mark.parametrize("dtype,rows,cols,per_row,N", [(2, 17000, 4096, 200, 96), (0, 70000, 1024, 60, 64), (1, 9000, 4096, 455, 20)])
+def test_entry_point_that_allocates_nothing_runs_what_hspmm_run_does(torch_cuda, hs, dtype, rows, cols, per_row, N):
+    torch = torch_cuda
+    rng = np.random.default_rng(90 + dtype)
+    A = _sampled_csr(rng, rows, cols, per_row, dtype, lambda n: rng.normal(size=n))
+    plan = hs.Plan(convert(hs, A))
+    _, dB = _random_operand(torch, rng, cols, N, dtype)
+    outs = [torch.full((rows, N), 7, dtype=dB.dtype, device="cuda") for _ in range(3)]
+    stream = torch.cuda.current_stream().cuda_stream
+    plan.prepare(N)
+    plan.run_static(dB.data_ptr(), outs[0].data_ptr(), N, stream)
+    assert plan.info()["last_kernel_family"] == 3
+    plan.run(dB.data_ptr(), outs[1].data_ptr(), N, stream)
+    assert plan.info()["last_kernel_family"] == 3
+    plan.run_static(dB.data_ptr(), outs[2].data_ptr(), N, stream)
+    torch.cuda.synchronize()
+    bits = [o.view(torch.int32 if dtype == 1 else torch.int16) for o in outs]
+    assert torch.equal(bits[0], bits[1]) and torch.equal(bits[0], bits[2])
+    plan.close()
