@@ -139,13 +139,13 @@ uint32_t fill_classes(const hspmm_plan *p, uint32_t lanes, int shift, uint32_t c
 // fp16, N = 88: 20.9 us uncut, 15.2 / 14.5 / 16.7 at 16 / 8 / 4 units; 12288, fp32, N = 128: 20.2 -> 10.2; rows all long, 4096 x
 // 11008 at 10 %, N = 8: 12.9 uncut, 19.9 at 8).  The line lies at four rounds of workgroups: graph of 40000, fp16, N = 200 (2.4
 // rounds) 37.1 -> 25.4 us, of 73838, N = 128 (2.3) 27.9 -> 29.6, of 100000 (3.1) 24.0 -> 21.0, of 73838, N = 200 (4.6) 50.8 -> 59.9.
-void choose_classes(const hspmm_plan *p, uint32_t lanes, hspmm::EntryArgs *ea)
+void choose_classes(const hspmm_plan *p, uint32_t lanes, bool may_cut, hspmm::EntryArgs *ea)
 {
     const uint32_t round = uint32_t(p->compute_units) * 8u;
     int shift = 2;
     if (!p->entries.long_rows) shift = fill_classes(p, lanes, 1, 0, ea) < 2u * round ? 0 : 1;
     ea->n_groups = fill_classes(p, lanes, shift, 0, ea);
-    if (!p->entries.long_rows && ea->n_groups < 4u * round) ea->n_groups = fill_classes(p, lanes, shift, 8, ea);
+    if (may_cut && !p->entries.long_rows && ea->n_groups < 4u * round) ea->n_groups = fill_classes(p, lanes, shift, 8, ea);
 }
 
 }  // namespace
@@ -250,17 +250,23 @@ int run_entries(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t
             if (const int rc = build_entries(p, s)) return rc;
         }
         hspmm::EntryArgs &classes = e.classes[__builtin_ctz(share.lanes)];
-        if (!classes.n_classes) choose_classes(p, share.lanes, &classes);
+        if (!classes.n_classes) choose_classes(p, share.lanes, true, &classes);
         ea = classes;
+        // Sums of the parts and behind them their counters: what hspmm_run_static has a fixed array for.  The shape is the same
+        // however it is launched: where they do not fit, no rows are cut, and where the pieces of long rows alone do not, this is
+        // a launch for the other kernels.
+        const size_t sums_of_part = size_t(blocks) * share.lanes * share.lane_bytes / p->elem * 4u, counters_of_part = size_t(blocks) * 4u;
+        auto fits = [&]() { return size_t(ea.n_parts) * (sums_of_part + counters_of_part) <= HSPMM_STATIC_SCRATCH_BYTES; };
+        if (!fits()) choose_classes(p, share.lanes, false, &ea);
+        if (!fits()) return HSPMM_OK;
         ea.n_pieces = e.n_pieces;
         if (ea.n_parts) {
-            // sums of the parts, and behind them, where nothing may be allocated, their counters
-            const size_t sums = size_t(ea.n_parts) * blocks * share.lanes * share.lane_bytes / p->elem * 4u;
-            if (const int rc = scratch_for(p, s, mode == RunMode::kStatic ? sums + size_t(ea.n_parts) * blocks * 4u : sums, mode, &ea.scratch)) return rc;
+            const size_t sums = ea.n_parts * sums_of_part, counters = ea.n_parts * counters_of_part;
+            if (const int rc = scratch_for(p, s, mode == RunMode::kStatic ? sums + counters : sums, mode, &ea.scratch)) return rc;
             if (mode == RunMode::kStatic) {
                 ea.arrive = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(ea.scratch) + sums);
-                HSPMM_HIP(hspmm::launch_fill_zero(ea.arrive, size_t(ea.n_parts) * blocks * 4u, s));
-            } else if (const int rc = ensure_arrive(p, s, size_t(ea.n_parts) * blocks, mode, &ea.arrive)) {
+                HSPMM_HIP(hspmm::launch_fill_zero(ea.arrive, counters, s));
+            } else if (const int rc = ensure_arrive(p, s, counters / 4u, mode, &ea.arrive)) {
                 return rc;
             }
         }

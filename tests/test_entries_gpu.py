@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from test_spmm_gpu import assert_parity, convert, gpu_spmm, make_b, oracle_spmm, torch_cuda  # noqa: F401
-from util import encode
+from util import decode, encode
 
 pytestmark = pytest.mark.gpu
 
@@ -133,4 +133,38 @@ def test_paired_windows_static_entry_point_and_capture(torch_cuda, hs, oracle, d
         torch.cuda.synchronize()
         assert np.array_equal(dC.cpu().numpy().view(np.uint8), np.ascontiguousarray(want).view(np.uint8))
     del graph
+    plan.close()
+
+
+@pytest.mark.parametrize("N,lengths,cols,family", [
+    (1024, [2001] * 1150 + [1] * 10500, 4001, 2),       # parts of cut rows: 36 MiB of sums; uncut rows leave none
+    (1024, [2100] * 5400, 2200, 3),                     # pieces of rows above 2048 entries: 42 MiB in any case
+])
+def test_sums_that_do_not_fit_the_fixed_array_choose_another_shape(torch_cuda, hs, N, lengths, cols, family):
+    """hspmm_run_static serves what hspmm_prepare has prepared, and its results are those of hspmm_run."""
+    torch = torch_cuda
+    rng = np.random.default_rng(95)
+    n = np.asarray(lengths)
+    start = np.concatenate([[0], np.cumsum(n)]).astype(np.int64)
+    place = np.arange(start[-1]) - np.repeat(start[:-1], n)
+    col_idx = (place * (cols // np.repeat(n, n)) + np.repeat(rng.integers(0, 2, n.size) * (cols % 2), n)) % cols
+    A = dict(rows=n.size, cols=cols, nnzs=int(start[-1]), dtype=0, row_ptr=start.astype(np.uint32), col_idx=col_idx.astype(np.uint32),
+             values=encode(rng.integers(1, 4, int(start[-1])).astype(np.float32), 0))
+    plan = _plan(hs, A)
+    B = rng.integers(-1, 2, (cols, N)).astype(np.float32)
+    dB = torch.from_numpy(encode(B, 0).view(np.int16)).cuda()
+    outs = [torch.full((n.size, N), 7, dtype=torch.int16, device="cuda") for _ in range(2)]
+    stream = torch.cuda.current_stream().cuda_stream
+    plan.prepare(N)
+    plan.run_static(dB.data_ptr(), outs[0].data_ptr(), N, stream)
+    plan.run(dB.data_ptr(), outs[1].data_ptr(), N, stream)
+    torch.cuda.synchronize()
+    assert plan.info()["last_kernel_family"] == family
+    assert torch.equal(outs[0], outs[1])
+    rows = np.concatenate([np.arange(4), rng.integers(0, n.size, 20), [n.size - 1]])
+    got = outs[0].cpu().numpy().view(np.float16)
+    for r in rows:
+        s = slice(start[r], start[r + 1])
+        want = (decode(A["values"][s], 0)[:, None] * B[col_idx[s]]).sum(0)
+        assert np.array_equal(got[r].astype(np.float64), want.astype(np.float16).astype(np.float64)), "row %d" % r
     plan.close()
