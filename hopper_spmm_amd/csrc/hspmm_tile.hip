@@ -57,7 +57,8 @@ int build_tile_stream(hspmm_plan *p)
     const double entries = double(p->T) * p->cw * p->per_column, most_features = p->elem == 4u ? 47.0 : 127.0;
     if (p->cfg.tile == 0 || !p->canonical || p->cfg.kernel_mode != 0) return HSPMM_OK;
     if (p->cfg.tile < 0 && (p->G != 1 || p->per_column > 4.0 || entries * most_features < 65e6 ||
-                            entries < 0.04 * double(p->rows) * p->cols)) return HSPMM_OK;
+                            entries < 0.04 * double(p->rows) * p->cols ||
+                            (p->elem == 4u && !(p->panel.built && p->panel.split)))) return HSPMM_OK;
     const uint32_t kk = tile_block_columns(p->dtype), n_blocks = (p->cols + kk - 1u) / kk, n_row_blocks = (p->rows + kTileBlockRows - 1u) / kTileBlockRows;
     const uint64_t cells = uint64_t(n_blocks) * n_row_blocks;
     if (p->cols < kk || n_blocks > kTileMaxBlocks || cells >= (1u << 26)) return HSPMM_OK;
@@ -89,8 +90,10 @@ int build_tile_stream(hspmm_plan *p)
 // large matrices.  Measured (this / the kernels otherwise chosen, us):
 //   bf16, 11008 x 4096 at 20 %: N = 8 15 / 18, 16 14.5 / 29, 32 16 / 34, 64 23 / 53;  4096 x 11008 at 10 %: N = 8 18 / 13,
 //   16 17 / 21, 32 19.5 / 27, 64 24 / 36;  5003 x 3001 at 20 %: N = 16 10.5 / 10.6, 32 11.7 / 15.2, 64 14.2 / 22;  4096^2 at 10 %:
-//   N = 32 12.4 / 8.8, 64 14.5 / 15.4;  fp32, 11008 x 4096 at 20 %: N = 8 24 / 29, 16 24 / 42, 32 28 / 35, 64 36 / 35;
+//   N = 32 12.4 / 8.8, 64 14.5 / 15.4;  fp32, 11008 x 4096 at 20 %: N = 16 24 / 42, 32 28 / 35, 64 36 / 35;
 //   4096 x 11008 at 10 %: N = 16 25.7 / 26.6, 32 29 / 34.  N = 256 and more: the LDS-panel kernels by a fifth.
+// fp32 storage is multiplied in bf16 parts here: only where the LDS-panel kernels would do the same (panel.split; N from 16 on,
+// in rows of whole 16-byte pieces).  Other N keep the fp32 products of the entry and gather kernels.
 bool tile_serves(const hspmm_plan *p, uint32_t N)
 {
     const Config &c = p->cfg;
@@ -101,6 +104,7 @@ bool tile_serves(const hspmm_plan *p, uint32_t N)
     if (c.tile > 0) return true;
     const bool wide = p->elem == 4u;
     const double work = double(p->tile.entries) * N, fill = double(p->tile.entries) / (double(p->rows) * p->cols);
+    if (wide && !(p->panel.split && panel_serves(p, N))) return false;
     return N >= 8u && N < (wide ? 48u : 128u) && work >= (wide ? 75e6 : 65e6) && fill >= 0.04 && fill * N >= 1.5;
 }
 
