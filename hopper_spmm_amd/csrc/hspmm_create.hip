@@ -606,7 +606,7 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
         sparse_tiles = sparse_tiles && st.G == 1 && stored + spare < (uint64_t(1) << 31) &&
                        (p->cfg.gather_bitmap > 0 || stored * 3u < uint64_t(total_tiles) * 8u * cw);
         // one block for everything whose size is known here, and a megabyte for the partitions
-        if ((rc = plan_reserve(p, (size_t(p->W) * 4u + 2u) * 4u + n_ids * 8u + tile_bytes + header.size() * 4u +
+        if ((rc = plan_reserve(p, entries_count_bytes(p) + (size_t(p->W) * 4u + 2u) * 4u + n_ids * 8u + tile_bytes + header.size() * 4u +
                                       (sparse_tiles ? (size_t(stored) + spare) * elem : 0u) + (size_t(1) << 20))))
             return bail(rc);
         timer.mark("device memory");
@@ -710,6 +710,8 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
             HSPMM_HIP_OR(hspmm::launch_lane_order32(p->d_data, room, total_tiles, nullptr), bail);
         }
         p->per_column = entries_per_column(total_tiles, cw, elem, tcA2B, data, bitmap, sparse_tiles ? header.data() : nullptr);
+        // single windows walked tile by tile: the caller's tile numbers are the stream's, its cuts can be kept
+        if (cuts && p->cfg.group_cuts && st.G == 1) p->caller_cuts.assign(cuts->offsets, cuts->offsets + size_t(cuts->n_groups) + 1u);
         {
             uint32_t longest = 0;
             for (size_t u = 0; u + 1 < st.unitOffset.size(); ++u) longest = std::max(longest, st.unitOffset[u + 1] - st.unitOffset[u]);
@@ -721,9 +723,8 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
             p->h_winOffset.assign(rowOffset, rowOffset + size_t(p->W) + 1u);
             p->h_winRow.assign(rowIdx, rowIdx + size_t(p->W));
         }
-        // single windows walked tile by tile: the caller's tile numbers are the stream's, its cuts can be kept
-        if (cuts && p->cfg.group_cuts && st.G == 1) p->caller_cuts.assign(cuts->offsets, cuts->offsets + size_t(cuts->n_groups) + 1u);
         if ((rc = build_and_upload_partition(p, 0))) return bail(rc);
+        if ((rc = count_entries(p))) return bail(rc);                   // (behind the last of the small uploads, which would wait for it)
         timer.mark("partition");
         {
             // all units long, and so long that the balanced partition cuts each of them several ways:
@@ -761,7 +762,7 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
         }
         if ((rc = build_tile_stream(p))) return bail(rc);
         timer.mark("full-tile stream");
-        HSPMM_HIP_OR(hipStreamSynchronize(nullptr), bail);              // (any stream may launch now)
+        if ((rc = entries_counted(p))) return bail(rc);                 // (any stream may launch now)
     } catch (const std::bad_alloc &) {
         return bail(fail(HSPMM_ERR_ALLOC, "out of host memory"));
     }

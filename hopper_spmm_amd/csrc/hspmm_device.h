@@ -129,14 +129,16 @@ struct EntryArgs {
 };
 // lane_bytes (2, 4, 8, 16) x lanes (1 .. 32): how a row of B is shared out; at least lane_bytes long
 hipError_t launch_spmm_entries(int dtype, const EntryArgs &ea, uint32_t lane_bytes, uint32_t lanes, hipStream_t s);
-// The three steps that make the stream (hspmm_entries.hip); chunks: {first tile, tiles, first matrix row, window} each.
-hipError_t launch_entry_count(int elem, const void *tiles, const uint32_t *chunks, uint32_t n_chunks, uint32_t *counts, hipStream_t s);
-hipError_t launch_entry_rows(const uint32_t *rowIdx, const uint32_t *first_chunk, uint32_t n_windows, uint32_t rows, uint32_t *counts,
-                             uint32_t *row_len, uint32_t *totals, hipStream_t s);
-hipError_t launch_entry_fill(int elem, const void *tiles, const uint32_t *a2b, const uint32_t *chunks, uint32_t n_chunks,
-                             const uint32_t *positions, const uint32_t *row_len, uint32_t rows, const uint32_t *places,
-                             uint32_t *cursors, uint32_t *desc, uint32_t *pieces, uint32_t *row_first, uint32_t *ids, void *vals,
-                             hipStream_t s);
+// The stream from the format arrays, in two steps: count (chunks of up to kEntryChunkTiles tiles of a window, at most most_chunks;
+// stored entries per chunk and row, which become positions inside the row; row lengths; totals: rows per bin - bin 0:
+// pieces - and behind them the units of the rows cut into pieces, then as many cursors) and fill (which uses the cursors up).
+struct EntrySource { const uint32_t *rowOffset, *rowIdx, *a2b, *first_chunk, *chunk_window; const void *tiles; uint32_t n_windows; };
+struct EntryPlaces { uint32_t places[3u * kEntryBins]; };      // per bin: first slot, first unit, units of a slot's place
+hipError_t launch_entry_count(int elem, const EntrySource &src, uint32_t most_chunks, uint32_t rows, uint32_t *first_chunk, uint32_t *chunk_window,
+                              uint32_t *counts, uint32_t *row_len, uint32_t *totals, hipStream_t s);
+hipError_t launch_entry_fill(int elem, const EntrySource &src, uint32_t most_chunks, const uint32_t *positions, const uint32_t *row_len,
+                             uint32_t rows, const EntryPlaces &places, uint32_t *cursors, uint32_t *desc, uint32_t *pieces,
+                             uint32_t *row_first, uint32_t *ids, void *vals, hipStream_t s);
 // Full-tile kernels (spmm_tile_kernel.hip): stored entries in blocks of 128 rows x tile_block_columns() columns, in units of
 // four: positions inside the block's LDS image (16 bits) and values (fp32 storage: hi | lo parts).
 constexpr uint32_t kTileBlockRows = 128u, kTileMaxBlocks = 4096u;     // blocks of a row block at most

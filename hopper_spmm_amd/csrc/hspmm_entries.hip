@@ -18,12 +18,6 @@ RowShare share_row(uint32_t bytes)
     return {16u, lanes};
 }
 
-// Device memory that a failed or finished build gives back.
-struct Temporary {
-    void *p = nullptr;
-    ~Temporary() { (void)hipFree(p); }
-};
-
 // Most units of a row of bin b (see entry_bin in spmm_entries.hip).
 uint32_t bin_units(uint32_t b)
 {
@@ -32,67 +26,44 @@ uint32_t bin_units(uint32_t b)
     return c == 0u ? step + 1u : (2u << c) + (step + 1u) * (1u << (c - 1u));
 }
 
-// Makes the entry stream from the uploaded tiles.  Called with the plan's mutex held; waits for the device.
+hspmm::EntrySource entry_source(const hspmm_plan *p)
+{
+    const hspmm_plan::Entries &e = p->entries;
+    return {p->d_rowOffset, p->d_rowIdx, p->d_a2b_raw, e.d_first_chunk, e.d_chunk_window, p->d_data, p->W};
+}
+
+// Makes the entry stream from the uploaded tiles: one allocation, two kernels.  Called with the plan's mutex held; waits for
+// the stream, because launches on other streams, and under capture, may follow at once.
 int build_entries(hspmm_plan *p, hipStream_t s)
 {
     using namespace hspmm;
-    const std::vector<uint32_t> &offset = p->G == 1 ? p->h_unitOffset : p->h_winOffset;
-    std::vector<uint32_t> chunks, first_chunk(size_t(p->W) + 1u);
-    for (uint32_t w = 0; w < p->W; ++w) {
-        first_chunk[w] = uint32_t(chunks.size() / 4u);
-        for (uint32_t t = offset[w]; t < offset[w + 1]; t += kEntryChunkTiles) {
-            chunks.push_back(t);
-            chunks.push_back(std::min(kEntryChunkTiles, offset[w + 1] - t));
-            chunks.push_back(p->G == 1 ? p->h_unitRow[w] : p->h_winRow[w]);
-            chunks.push_back(w);
-        }
-    }
-    const uint32_t n_chunks = uint32_t(chunks.size() / 4u);
-    first_chunk[p->W] = n_chunks;
-    // one allocation for what only the build needs: chunks, their windows, counts, row lengths and places, totals
-    const size_t words = chunks.size() + first_chunk.size() + size_t(n_chunks) * 8u + size_t(p->rows) * 2u + 3u * (kEntryBins + 1u) + 3u * kEntryBins;
-    Temporary tmp;
-    HSPMM_HIP(hipMalloc(&tmp.p, words * 4u));
-    uint32_t *d_chunks = static_cast<uint32_t *>(tmp.p), *d_first_chunk = d_chunks + chunks.size();
-    uint32_t *d_counts = d_first_chunk + first_chunk.size(), *d_len = d_counts + size_t(n_chunks) * 8u, *d_first = d_len + p->rows;
-    uint32_t *d_totals = d_first + p->rows, *d_cursors = d_totals + kEntryBins + 1u, *d_places = d_cursors + kEntryBins + 1u;
-    HSPMM_HIP(hipMemcpyAsync(d_chunks, chunks.data(), chunks.size() * 4u, hipMemcpyHostToDevice, s));
-    HSPMM_HIP(hipMemcpyAsync(d_first_chunk, first_chunk.data(), first_chunk.size() * 4u, hipMemcpyHostToDevice, s));
-    HSPMM_HIP(launch_fill_zero(d_totals, 2u * (kEntryBins + 1u) * 4u, s));
-    HSPMM_HIP(launch_entry_count(int(p->elem), p->d_data, d_chunks, n_chunks, d_counts, s));
-    HSPMM_HIP(launch_entry_rows(p->d_rowIdx, d_first_chunk, p->W, p->rows, d_counts, d_len, d_totals, s));
-    uint32_t totals[kEntryBins + 1u];
-    HSPMM_HIP(hipMemcpyAsync(totals, d_totals, sizeof totals, hipMemcpyDeviceToHost, s));
-    HSPMM_HIP(hipStreamSynchronize(s));
-    uint32_t places[3u * kEntryBins];
+    hspmm_plan::Entries &e = p->entries;
+    EntryPlaces at;
     uint64_t slot = 0, unit = 0;
     for (uint32_t b = 0; b < kEntryBins; ++b) {
         const uint32_t width = bin_units(b);
-        places[3u * b] = uint32_t(slot); places[3u * b + 1u] = uint32_t(unit); places[3u * b + 2u] = width;
-        slot += totals[b];
-        unit += b == 0u ? uint64_t(totals[kEntryBins]) : uint64_t(totals[b]) * width;
+        at.places[3u * b] = uint32_t(slot); at.places[3u * b + 1u] = uint32_t(unit); at.places[3u * b + 2u] = width;
+        slot += e.totals[b];
+        unit += b == 0u ? uint64_t(e.totals[kEntryBins]) : uint64_t(e.totals[b]) * width;
     }
-    if (slot > 0xFFFFFFFFull || unit > 0xFFFFFFFFull) return fail(HSPMM_ERR_UNSUPPORTED, "the entry stream exceeds 32-bit positions");
-    // the stream in one allocation (each takes about 0.1 ms): ids, values, descriptors, pieces
+    // ids, values, descriptors, pieces
     const size_t units_kept = size_t(unit ? unit : 1u), ids_bytes = units_kept * 16u, vals_bytes = units_kept * 4u * p->elem;
-    const size_t desc_bytes = size_t(slot) * 12u, bytes = ids_bytes + vals_bytes + desc_bytes + size_t(totals[0]) * 12u;
-    Temporary stream;
-    HSPMM_HIP(hipMalloc(&stream.p, bytes));
-    char *at = static_cast<char *>(stream.p);
-    uint32_t *ids = reinterpret_cast<uint32_t *>(at), *desc = reinterpret_cast<uint32_t *>(at + ids_bytes + vals_bytes);
-    uint32_t *pieces = reinterpret_cast<uint32_t *>(at + ids_bytes + vals_bytes + desc_bytes);
-    HSPMM_HIP(hipMemcpyAsync(d_places, places, sizeof places, hipMemcpyHostToDevice, s));
-    HSPMM_HIP(launch_entry_fill(int(p->elem), p->d_data, p->d_a2b_raw, d_chunks, n_chunks, d_counts, d_len, p->rows, d_places,
-                                d_cursors, desc, pieces, d_first, ids, at + ids_bytes, s));
-    HSPMM_HIP(hipStreamSynchronize(s));         // (launches on other streams may follow at once)
-    hspmm_plan::Entries &e = p->entries;
-    std::copy(totals, totals + kEntryBins, e.slots);
-    e.n_pieces = totals[0];
-    e.long_rows = unit >= 64u * uint64_t(slot - totals[kEntryBins - 1u]);
-    e.d_stream = stream.p;
-    e.d_ids = ids; e.d_vals = at + ids_bytes; e.d_desc = desc; e.d_pieces = pieces;
-    stream.p = nullptr;
+    const size_t desc_bytes = size_t(slot) * 12u, bytes = ids_bytes + vals_bytes + desc_bytes + size_t(e.totals[0]) * 12u;
+    void *stream = nullptr;
+    e.unavailable = true;                       // (what has failed once is not tried again)
+    if (slot > 0xFFFFFFFFull || unit > 0xFFFFFFFFull) return HSPMM_OK;
+    if (hipMalloc(&stream, bytes) != hipSuccess) { (void)hipGetLastError(); return HSPMM_OK; }
+    e.d_stream = stream;
     p->fixed_bytes += bytes;
+    char *base = static_cast<char *>(stream);
+    uint32_t *ids = reinterpret_cast<uint32_t *>(base), *desc = reinterpret_cast<uint32_t *>(base + ids_bytes + vals_bytes);
+    uint32_t *pieces = reinterpret_cast<uint32_t *>(base + ids_bytes + vals_bytes + desc_bytes);
+    HSPMM_HIP(launch_entry_fill(int(p->elem), entry_source(p), e.most_chunks, e.d_positions, e.d_row_len, p->rows, at,
+                                e.d_totals + kEntryBins + 1u, desc, pieces, e.d_row_first, ids, base + ids_bytes, s));
+    HSPMM_HIP(hipStreamSynchronize(s));
+    e.long_rows = unit >= 64u * uint64_t(slot - e.totals[kEntryBins - 1u]);
+    e.d_ids = ids; e.d_vals = base + ids_bytes; e.d_desc = desc; e.d_pieces = pieces;
+    e.unavailable = false;
     e.built = true;
     return HSPMM_OK;
 }
@@ -105,7 +76,7 @@ uint32_t fill_classes(const hspmm_plan *p, uint32_t lanes, int shift, uint32_t c
     const uint32_t subgroups = 256u / lanes;                 // of a workgroup
     uint32_t most = 0;
     while ((2u << most) <= subgroups) ++most;
-    const uint32_t *n = p->entries.slots;
+    const uint32_t *n = p->entries.totals;
     uint32_t group = 0, slot = 0, part = 0;
     ea->n_classes = 0;
     auto add = [&](uint32_t slots, int wanted, uint32_t units) {
@@ -207,15 +178,11 @@ static uint32_t row_blocks(const hspmm_plan *p, uint32_t row_bytes)
 bool entries_serve(const hspmm_plan *p, uint32_t N)
 {
     const Config &c = p->cfg;
-    // (the caller's own settings are settings of the gather kernels)
-    if (c.kernel_mode != 0 || c.entries == 0 || c.fused_fixup >= 0 || c.buffer_stage || c.consumer_warp_num || c.producer_warp_group_num)
-        return false;
-    if (!p->caller_cuts.empty() || p->rows >= (1u << 31)) return false;
+    if (!p->entries.counted || p->entries.unavailable) return false;
     const uint64_t row = uint64_t(N) * p->elem, all = uint64_t(p->cols) * row;
     if (row > kEntryMaxRowBytes) return false;
     if (c.entries > 0) return true;
     const double per_column = p->per_column, weight = double(row) * (per_column - 0.8);
-    if (p->G != 1 || per_column > 3.5) return false;
     const bool sparse = per_column <= 1.25;
     if (p->elem == 4u) {
         if (weight <= 100.0) return true;
@@ -227,6 +194,63 @@ bool entries_serve(const hspmm_plan *p, uint32_t N)
     // one.  Of 8, where they load 16 bytes: on a small B with very many rows, uniform 34816 x 3575, 4 per row, N = 480: 18.7 / 16.1)
     if (N % 64u != 0u) return !(N % 8u == 0u && row >= 896u && all <= (uint64_t(20) << 20) && p->rows > 16384u);
     return entries_by_xcd(p, row) || (all <= (uint64_t(64) << 20) && !(row >= 1024u && all <= (uint64_t(16) << 20)));
+}
+
+// Whether a plan whose tiles are not counted yet may want the stream.
+static bool entries_possible(const hspmm_plan *p)
+{
+    const Config &c = p->cfg;
+    // (the caller's own settings are settings of the gather kernels)
+    if (c.kernel_mode != 0 || c.entries == 0 || c.fused_fixup >= 0 || c.buffer_stage || c.consumer_warp_num || c.producer_warp_group_num)
+        return false;
+    if (!p->caller_cuts.empty() || p->rows >= (1u << 31) || !p->T || uint64_t(p->W) + p->T / hspmm::kEntryChunkTiles >= (1u << 31)) return false;
+    return c.entries > 0 || (p->G == 1 && p->per_column <= 3.5);
+}
+
+struct CountArrays { size_t most_chunks, words[6]; };
+static CountArrays count_arrays(const hspmm_plan *p)
+{
+    const size_t most = size_t(p->W) + p->T / hspmm::kEntryChunkTiles;
+    return {most, {size_t(p->W) + 1u, most, most * 8u, p->rows, p->rows, 2u * (hspmm::kEntryBins + 1u)}};
+}
+
+size_t entries_count_bytes(const hspmm_plan *p)
+{
+    size_t bytes = 0;
+    if (p->cfg.entries > 0 || p->G == 1)
+        for (size_t words : count_arrays(p).words) bytes += words * 4u + 256u;
+    return bytes;
+}
+
+// Row lengths and the sizes of all there is in the stream: enqueued by hspmm_create behind the tiles, beside its work on the
+// host, so that the first product of a plan has nothing to read back (see build_entries).  First product of a plan, counting in
+// its launch / here, us: 4096^2 at 1 %, N = 64 96 / 50; uniform 65536^2, 16 per row, N = 128 208 / 114; graph of 150001, fp32,
+// N = 100 388 / 213; of 262144, N = 16 477 / 242, N = 128 510 / 272; hspmm_create takes 0.05 ms more.
+int count_entries(hspmm_plan *p)
+{
+    using namespace hspmm;
+    hspmm_plan::Entries &e = p->entries;
+    if (!entries_possible(p)) return HSPMM_OK;
+    const CountArrays arrays = count_arrays(p);
+    uint32_t **const at[] = {&e.d_first_chunk, &e.d_chunk_window, &e.d_positions, &e.d_row_len, &e.d_row_first, &e.d_totals};
+    for (int i = 0; i < 6; ++i) {
+        void *room = nullptr;
+        if (int rc = plan_alloc(p, arrays.words[i] * 4u, &room)) return rc;
+        *at[i] = static_cast<uint32_t *>(room);
+    }
+    e.most_chunks = uint32_t(arrays.most_chunks);
+    HSPMM_HIP(launch_entry_count(int(p->elem), entry_source(p), e.most_chunks, p->rows, e.d_first_chunk, e.d_chunk_window, e.d_positions,
+                                 e.d_row_len, e.d_totals, nullptr));
+    e.counted = true;
+    return HSPMM_OK;
+}
+
+// Waits for what hspmm_create has enqueued.
+int entries_counted(hspmm_plan *p)
+{
+    if (p->entries.counted) HSPMM_HIP(hipMemcpy(p->entries.totals, p->entries.d_totals, sizeof p->entries.totals, hipMemcpyDeviceToHost));
+    else HSPMM_HIP(hipStreamSynchronize(nullptr));
+    return HSPMM_OK;
 }
 
 int run_entries(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode, bool *taken)
@@ -248,6 +272,7 @@ int run_entries(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t
             if (mode == RunMode::kLaunch && s && (hipStreamIsCapturing(s, &status) != hipSuccess || status != hipStreamCaptureStatusNone))
                 return HSPMM_OK;                // (nothing can be built under capture: the gather kernels take it)
             if (const int rc = build_entries(p, s)) return rc;
+            if (!e.built) return HSPMM_OK;
         }
         hspmm::EntryArgs &classes = e.classes[__builtin_ctz(share.lanes)];
         if (!classes.n_classes) choose_classes(p, share.lanes, true, &classes);
@@ -259,7 +284,7 @@ int run_entries(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t
         auto fits = [&]() { return size_t(ea.n_parts) * (sums_of_part + counters_of_part) <= HSPMM_STATIC_SCRATCH_BYTES; };
         if (!fits()) choose_classes(p, share.lanes, false, &ea);
         if (!fits()) return HSPMM_OK;
-        ea.n_pieces = e.n_pieces;
+        ea.n_pieces = e.totals[0];
         if (ea.n_parts) {
             const size_t sums = ea.n_parts * sums_of_part, counters = ea.n_parts * counters_of_part;
             if (const int rc = scratch_for(p, s, mode == RunMode::kStatic ? sums + counters : sums, mode, &ea.scratch)) return rc;

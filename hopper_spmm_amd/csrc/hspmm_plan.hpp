@@ -165,15 +165,19 @@ struct hspmm_plan {
         uint64_t stored = 0;
         bool from_caller = false;     // header and elements are the caller's tcBit / nnzOffset / data, uploaded as they came
     } bm;
-    // Stored entries, rows sorted by length, for narrow feature dimensions (spmm_entries.hip): made from the tiles on the
-    // device by the first launch (or hspmm_prepare) that wants it
+    // Stored entries, rows sorted by length, for narrow feature dimensions (spmm_entries.hip): counted by hspmm_create, made from
+    // the tiles on the device by the first launch (or hspmm_prepare) that wants it
     struct Entries {
+        bool counted = false;
+        bool unavailable = false;                                // no memory for it: the other kernels serve this plan
+        uint32_t most_chunks = 0;
+        uint32_t *d_first_chunk = nullptr, *d_chunk_window = nullptr, *d_positions = nullptr, *d_row_len = nullptr, *d_row_first = nullptr;
+        uint32_t *d_totals = nullptr;                            // kEntryBins + 1 counts, then as many cursors
+        uint32_t totals[hspmm::kEntryBins + 1u] = {};
         bool built = false;
         void *d_stream = nullptr;                                // one allocation for the four below
         const uint32_t *d_desc = nullptr, *d_ids = nullptr, *d_pieces = nullptr;
         const void *d_vals = nullptr;
-        uint32_t slots[hspmm::kEntryBins] = {};                  // rows per bin (bin 0: pieces)
-        uint32_t n_pieces = 0;
         bool long_rows = false;                                  // 64 units and more in a row on average
         hspmm::EntryArgs classes[6] = {};                        // by log2 lanes of a row, once a launch has asked for it
     } entries;
@@ -280,7 +284,11 @@ int build_and_upload_partition(hspmm_plan *p, int level, uint32_t group = 1, boo
 // hspmm_run.hip: memory a launch writes besides C (called with the plan's mutex held)
 int ensure_arrive(hspmm_plan *p, hipStream_t s, size_t words, RunMode mode, uint32_t **out);
 int scratch_for(hspmm_plan *p, hipStream_t s, size_t bytes, RunMode mode, float **out);
-// hspmm_entries.hip: whether the entry kernels take this launch, and the launch
+// hspmm_entries.hip: counting what the entry kernels' stream holds (enqueued; hspmm_create reads the totals once it has
+// waited) and the device memory that takes, whether they take this launch, and the launch
+size_t entries_count_bytes(const hspmm_plan *p);
+int count_entries(hspmm_plan *p);
+int entries_counted(hspmm_plan *p);
 bool entries_serve(const hspmm_plan *p, uint32_t N);
 int run_entries(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode, bool *taken);
 

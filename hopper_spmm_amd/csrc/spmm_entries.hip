@@ -333,18 +333,53 @@ __device__ __forceinline__ uint32_t tile_row_mask(const void *tiles, size_t t, u
     return mask;
 }
 
-// chunks: 4 words each {first tile, tiles, first matrix row, effective window}.  counts[chunk][8]: stored entries per row.
+// first_chunk[w]: chunks in front of window w (n_windows + 1 of them); chunk_window[chunk]: its window; totals and cursors cleared.
+// One workgroup.
+__global__ __launch_bounds__(1024) void entry_chunks_kernel(const uint32_t *__restrict__ rowOffset, uint32_t n_windows,
+                                                            uint32_t *__restrict__ first_chunk, uint32_t *__restrict__ chunk_window,
+                                                            uint32_t *__restrict__ totals)
+{
+    __shared__ uint32_t sums[1024];
+    if (threadIdx.x < 2u * (kEntryBins + 1u)) totals[threadIdx.x] = 0u;
+    const uint32_t per = (n_windows + 1023u) / 1024u, b = umin_e(threadIdx.x * per, n_windows), e = umin_e(b + per, n_windows);
+    uint32_t sum = 0;
+    for (uint32_t w = b; w < e; ++w) sum += (rowOffset[w + 1u] - rowOffset[w] + kEntryChunkTiles - 1u) / kEntryChunkTiles;
+    sums[threadIdx.x] = sum;
+    __syncthreads();
+    for (uint32_t m = 1u; m < 1024u; m <<= 1) {
+        const uint32_t x = threadIdx.x >= m ? sums[threadIdx.x - m] : 0u;
+        __syncthreads();
+        sums[threadIdx.x] += x;
+        __syncthreads();
+    }
+    uint32_t at = threadIdx.x ? sums[threadIdx.x - 1u] : 0u;
+    for (uint32_t w = b; w < e; ++w) {
+        first_chunk[w] = at;
+        for (uint32_t n = (rowOffset[w + 1u] - rowOffset[w] + kEntryChunkTiles - 1u) / kEntryChunkTiles; n; --n) chunk_window[at++] = w;
+    }
+    if (threadIdx.x == 1023u) first_chunk[n_windows] = sums[1023];
+}
+
+// Tiles t0 .. t0 + n - 1 of a chunk.
+struct ChunkTiles { uint32_t window, t0, n; };
+__device__ __forceinline__ ChunkTiles chunk_tiles(const EntrySource &src, uint32_t chunk)
+{
+    const uint32_t w = src.chunk_window[chunk], t0 = src.rowOffset[w] + (chunk - src.first_chunk[w]) * kEntryChunkTiles;
+    return {w, t0, umin_e(kEntryChunkTiles, src.rowOffset[w + 1u] - t0)};
+}
+
+// counts[chunk][8]: stored entries per row of the chunk's window.
 template <int ELEM>
-__global__ __launch_bounds__(256) void entry_count_kernel(const void *__restrict__ tiles, const uint32_t *__restrict__ chunks,
-                                                          uint32_t n_chunks, uint32_t *__restrict__ counts)
+__global__ __launch_bounds__(256) void entry_count_kernel(const EntrySource src, uint32_t *__restrict__ counts)
 {
     const uint32_t chunk = blockIdx.x * 4u + (threadIdx.x >> 6), lane = threadIdx.x & 63u;
-    if (chunk >= n_chunks) return;
-    const uint32_t t0 = chunks[size_t(chunk) * 4u], n = chunks[size_t(chunk) * 4u + 1u], r = lane & 7u;
+    if (chunk >= src.first_chunk[src.n_windows]) return;
+    const ChunkTiles c = chunk_tiles(src, chunk);
     uint32_t count = 0;
-    for (uint32_t i = lane >> 3; i < n; i += 8u) count += uint32_t(__builtin_popcount(tile_row_mask<ELEM>(tiles, size_t(t0) + i, r)));
+    for (uint32_t i = lane >> 3; i < c.n; i += 8u)
+        count += uint32_t(__builtin_popcount(tile_row_mask<ELEM>(src.tiles, size_t(c.t0) + i, lane & 7u)));
     for (uint32_t m = 8; m < 64u; m <<= 1) count += __shfl_xor(count, int(m));
-    if (lane < 8u) counts[size_t(chunk) * 8u + r] = count;
+    if (lane < 8u) counts[size_t(chunk) * 8u + lane] = count;
 }
 
 // Bin of a row of `units` units of four entries: 0 = pieces of rows above kEntryPieceUnits, then the classes from the
@@ -363,10 +398,11 @@ __device__ __forceinline__ uint32_t entry_bin(uint32_t units)
 
 // One thread per matrix row: its length (all chunks of its window; their counts become positions inside the row) and
 // the number of rows per bin.  totals: kEntryBins counts (bin 0: pieces), then the units of the rows cut into pieces.
-__global__ __launch_bounds__(256) void entry_rows_kernel(const uint32_t *__restrict__ rowIdx, const uint32_t *__restrict__ first_chunk,
-                                                         uint32_t n_windows, uint32_t rows, uint32_t *__restrict__ counts,
+__global__ __launch_bounds__(256) void entry_rows_kernel(const EntrySource src, uint32_t rows, uint32_t *__restrict__ counts,
                                                          uint32_t *__restrict__ row_len, uint32_t *__restrict__ totals)
 {
+    const uint32_t *rowIdx = src.rowIdx, *first_chunk = src.first_chunk;
+    const uint32_t n_windows = src.n_windows;
     __shared__ uint32_t bins[kEntryBins + 1u];
     if (threadIdx.x < kEntryBins + 1u) bins[threadIdx.x] = 0u;
     __syncthreads();
@@ -394,15 +430,15 @@ __global__ __launch_bounds__(256) void entry_rows_kernel(const uint32_t *__restr
     if (threadIdx.x < kEntryBins + 1u && bins[threadIdx.x]) atomicAdd(&totals[threadIdx.x], bins[threadIdx.x]);
 }
 
-// One thread per matrix row: its slot in its bin and its place in the stream.  cursors: as totals, cleared; places:
-// per bin {first slot, first unit, units of a slot's place}.
+// One thread per matrix row: its slot in its bin and its place in the stream.  cursors: as totals, cleared.
 __global__ __launch_bounds__(256) void entry_place_kernel(const uint32_t *__restrict__ row_len, uint32_t rows,
-                                                          const uint32_t *__restrict__ places, uint32_t *__restrict__ cursors,
+                                                          const EntryPlaces at, uint32_t *__restrict__ cursors,
                                                           uint32_t *__restrict__ desc, uint32_t *__restrict__ pieces,
                                                           uint32_t *__restrict__ row_first)
 {
-    __shared__ uint32_t bins[kEntryBins], base[kEntryBins];
+    __shared__ uint32_t bins[kEntryBins], base[kEntryBins], places[3u * kEntryBins];
     if (threadIdx.x < kEntryBins) bins[threadIdx.x] = 0u;
+    if (threadIdx.x < 3u * kEntryBins) places[threadIdx.x] = at.places[threadIdx.x];
     __syncthreads();
     const uint32_t row = blockIdx.x * 256u + threadIdx.x;
     const uint32_t len = row < rows ? row_len[row] : 0u, units = len / 4u + ((len & 3u) != 0u), bin = entry_bin(units);
@@ -433,17 +469,18 @@ __global__ __launch_bounds__(256) void entry_place_kernel(const uint32_t *__rest
 
 // Ids and values to their places; the last unit of a row is filled up with its last column and zeros.
 template <int ELEM>
-__global__ __launch_bounds__(256) void entry_fill_kernel(const void *__restrict__ tiles, const uint32_t *__restrict__ a2b,
-                                                         const uint32_t *__restrict__ chunks, uint32_t n_chunks,
-                                                         const uint32_t *__restrict__ positions, const uint32_t *__restrict__ row_len,
+__global__ __launch_bounds__(256) void entry_fill_kernel(const EntrySource src, const uint32_t *__restrict__ positions,
+                                                         const uint32_t *__restrict__ row_len,
                                                          const uint32_t *__restrict__ row_first, uint32_t rows,
                                                          uint32_t *__restrict__ ids, void *__restrict__ vals)
 {
     constexpr uint32_t CW = ELEM == 4 ? 8u : 16u;
     const uint32_t chunk = blockIdx.x * 4u + (threadIdx.x >> 6), lane = threadIdx.x & 63u;
-    if (chunk >= n_chunks) return;
-    const uint32_t t0 = chunks[size_t(chunk) * 4u], n = chunks[size_t(chunk) * 4u + 1u], r = lane & 7u;
-    const uint32_t row = chunks[size_t(chunk) * 4u + 2u] + r;
+    if (chunk >= src.first_chunk[src.n_windows]) return;
+    const void *tiles = src.tiles;
+    const uint32_t *a2b = src.a2b;
+    const ChunkTiles c = chunk_tiles(src, chunk);
+    const uint32_t t0 = c.t0, n = c.n, r = lane & 7u, row = src.rowIdx[c.window] + r;
     const bool inside = row < rows;
     const uint32_t len = inside ? row_len[row] : 0u;
     const size_t first = inside ? size_t(row_first[row]) * 4u : 0u;
@@ -482,34 +519,25 @@ __global__ __launch_bounds__(256) void entry_fill_kernel(const void *__restrict_
     }
 }
 
-hipError_t launch_entry_count(int elem, const void *tiles, const uint32_t *chunks, uint32_t n_chunks, uint32_t *counts, hipStream_t s)
+hipError_t launch_entry_count(int elem, const EntrySource &src, uint32_t most_chunks, uint32_t rows, uint32_t *first_chunk, uint32_t *chunk_window,
+                              uint32_t *counts, uint32_t *row_len, uint32_t *totals, hipStream_t s)
 {
-    const dim3 grid((n_chunks + 3u) / 4u);
-    if (elem == 4) entry_count_kernel<4><<<grid, 256, 0, s>>>(tiles, chunks, n_chunks, counts);
-    else entry_count_kernel<2><<<grid, 256, 0, s>>>(tiles, chunks, n_chunks, counts);
+    entry_chunks_kernel<<<dim3(1), 1024, 0, s>>>(src.rowOffset, src.n_windows, first_chunk, chunk_window, totals);
+    const dim3 grid((most_chunks + 3u) / 4u);
+    if (elem == 4) entry_count_kernel<4><<<grid, 256, 0, s>>>(src, counts);
+    else entry_count_kernel<2><<<grid, 256, 0, s>>>(src, counts);
+    entry_rows_kernel<<<dim3((rows + 255u) / 256u), 256, 0, s>>>(src, rows, counts, row_len, totals);
     return hipGetLastError();
 }
 
-hipError_t launch_entry_rows(const uint32_t *rowIdx, const uint32_t *first_chunk, uint32_t n_windows, uint32_t rows, uint32_t *counts,
-                             uint32_t *row_len, uint32_t *totals, hipStream_t s)
-{
-    entry_rows_kernel<<<dim3((rows + 255u) / 256u), 256, 0, s>>>(rowIdx, first_chunk, n_windows, rows, counts, row_len, totals);
-    return hipGetLastError();
-}
-
-hipError_t launch_entry_fill(int elem, const void *tiles, const uint32_t *a2b, const uint32_t *chunks, uint32_t n_chunks,
-                             const uint32_t *positions, const uint32_t *row_len, uint32_t rows, const uint32_t *places,
-                             uint32_t *cursors, uint32_t *desc, uint32_t *pieces, uint32_t *row_first, uint32_t *ids, void *vals,
-                             hipStream_t s)
+hipError_t launch_entry_fill(int elem, const EntrySource &src, uint32_t most_chunks, const uint32_t *positions, const uint32_t *row_len,
+                             uint32_t rows, const EntryPlaces &places, uint32_t *cursors, uint32_t *desc, uint32_t *pieces,
+                             uint32_t *row_first, uint32_t *ids, void *vals, hipStream_t s)
 {
     entry_place_kernel<<<dim3((rows + 255u) / 256u), 256, 0, s>>>(row_len, rows, places, cursors, desc, pieces, row_first);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    const dim3 grid((n_chunks + 3u) / 4u);
-    if (elem == 4)
-        entry_fill_kernel<4><<<grid, 256, 0, s>>>(tiles, a2b, chunks, n_chunks, positions, row_len, row_first, rows, ids, vals);
-    else
-        entry_fill_kernel<2><<<grid, 256, 0, s>>>(tiles, a2b, chunks, n_chunks, positions, row_len, row_first, rows, ids, vals);
+    const dim3 grid((most_chunks + 3u) / 4u);
+    if (elem == 4) entry_fill_kernel<4><<<grid, 256, 0, s>>>(src, positions, row_len, row_first, rows, ids, vals);
+    else entry_fill_kernel<2><<<grid, 256, 0, s>>>(src, positions, row_len, row_first, rows, ids, vals);
     return hipGetLastError();
 }
 

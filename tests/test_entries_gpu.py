@@ -168,3 +168,46 @@ def test_sums_that_do_not_fit_the_fixed_array_choose_another_shape(torch_cuda, h
         want = (decode(A["values"][s], 0)[:, None] * B[col_idx[s]]).sum(0)
         assert np.array_equal(got[r].astype(np.float64), want.astype(np.float16).astype(np.float64)), "row %d" % r
     plan.close()
+
+
+def test_without_memory_for_the_stream_the_other_kernels_serve(torch_cuda, hs, oracle):
+    """The stream of stored entries is a second copy of the matrix, made by the first launch that wants it: when the device
+    has no room for it, that launch and all that follow go to the kernels that need none."""
+    torch = torch_cuda
+    rng = np.random.default_rng(97)
+    rows, per_row, N = 1 << 17, 64, 16
+    col_idx = (np.arange(per_row, dtype=np.int64)[None, :] * (rows // per_row) + rng.integers(0, rows // per_row, (rows, per_row)))
+    A = dict(rows=rows, cols=rows, nnzs=rows * per_row, dtype=1, row_ptr=(np.arange(rows + 1, dtype=np.int64) * per_row).astype(np.uint32),
+             col_idx=col_idx.astype(np.uint32).reshape(-1), values=rng.integers(1, 4, rows * per_row).astype(np.float32))
+    B = rng.integers(-4, 5, (rows, N)).astype(np.float32)
+    dB = torch.from_numpy(B).cuda()
+    outs = [torch.full((rows, N), float("nan"), device="cuda") for _ in range(3)]
+    stream = torch.cuda.current_stream().cuda_stream
+    plan = hs.Plan(convert(hs, A))
+    torch.cuda.empty_cache()
+    rest = [torch.empty(torch.cuda.mem_get_info()[0] - (1 << 30), dtype=torch.uint8, device="cuda")]
+    for _ in range(512):                                # what is left, down to one block: the stream takes 67 MB
+        try:
+            rest.append(torch.empty(24 << 20, dtype=torch.uint8, device="cuda"))
+        except torch.OutOfMemoryError:
+            break
+    rest.pop()
+    torch.cuda.empty_cache()
+    try:
+        plan.run(dB.data_ptr(), outs[0].data_ptr(), N, stream)
+        assert plan.info()["last_kernel_family"] == 2 and plan.info()["last_mfma_kind"] != 0
+    finally:
+        torch.cuda.synchronize()
+        del rest
+        torch.cuda.empty_cache()
+    plan.run(dB.data_ptr(), outs[1].data_ptr(), N, stream)          # (room again: the plan's results do not change)
+    assert plan.info()["last_mfma_kind"] != 0
+    other = hs.Plan(convert(hs, A))
+    other.run(dB.data_ptr(), outs[2].data_ptr(), N, stream)
+    assert other.info()["last_mfma_kind"] == 0
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])      # (small whole numbers: every order gives the same)
+    want = oracle_spmm(oracle, A, B, N)[0]
+    assert np.array_equal(outs[0].cpu().numpy(), want)
+    plan.close()
+    other.close()
