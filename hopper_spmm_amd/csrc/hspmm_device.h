@@ -110,6 +110,8 @@ hipError_t launch_spmm_panel(int dtype, int G, bool split, bool tall, bool packe
 // rows above kEntryPieceUnits are cut into pieces of that many.
 constexpr uint32_t kEntryPieceUnits = 512u, kEntryClassesByLength = 8u, kEntryBins = 2u + 4u * kEntryClassesByLength;
 constexpr uint32_t kEntryChunkTiles = 64u, kEntryClasses = 2u + kEntryClassesByLength;
+// a launch has under 2^32 work-items: workgroups of 256 threads, and chunks of a wave each
+constexpr uint32_t kEntryMostGroups = 1u << 23, kEntryMostChunks = 1u << 25;
 struct EntryClass { uint32_t group_begin, slot_begin, slot_end, logs; };    // first workgroup; slots; log2 subgroups per row or part | log2 parts of a row << 8
 struct EntryArgs {
     const uint32_t *desc;        // per slot three words: first unit, units, matrix row (pieces: number of the piece)

@@ -196,6 +196,13 @@ bool entries_serve(const hspmm_plan *p, uint32_t N)
     return entries_by_xcd(p, row) || (all <= (uint64_t(64) << 20) && !(row >= 1024u && all <= (uint64_t(16) << 20)));
 }
 
+struct CountArrays { size_t most_chunks, words[6]; };
+static CountArrays count_arrays(const hspmm_plan *p)
+{
+    const size_t most = size_t(p->W) + p->T / hspmm::kEntryChunkTiles;
+    return {most, {size_t(p->W) + 1u, most, most * 8u, p->rows, p->rows, 2u * (hspmm::kEntryBins + 1u)}};
+}
+
 // Whether a plan whose tiles are not counted yet may want the stream.
 static bool entries_possible(const hspmm_plan *p)
 {
@@ -203,15 +210,8 @@ static bool entries_possible(const hspmm_plan *p)
     // (the caller's own settings are settings of the gather kernels)
     if (c.kernel_mode != 0 || c.entries == 0 || c.fused_fixup >= 0 || c.buffer_stage || c.consumer_warp_num || c.producer_warp_group_num)
         return false;
-    if (!p->caller_cuts.empty() || p->rows >= (1u << 31) || !p->T || uint64_t(p->W) + p->T / hspmm::kEntryChunkTiles >= (1u << 31)) return false;
+    if (!p->caller_cuts.empty() || p->rows >= (1u << 31) || !p->T || count_arrays(p).most_chunks >= hspmm::kEntryMostChunks) return false;
     return c.entries > 0 || (p->G == 1 && p->per_column <= 3.5);
-}
-
-struct CountArrays { size_t most_chunks, words[6]; };
-static CountArrays count_arrays(const hspmm_plan *p)
-{
-    const size_t most = size_t(p->W) + p->T / hspmm::kEntryChunkTiles;
-    return {most, {size_t(p->W) + 1u, most, most * 8u, p->rows, p->rows, 2u * (hspmm::kEntryBins + 1u)}};
 }
 
 size_t entries_count_bytes(const hspmm_plan *p)
@@ -283,7 +283,7 @@ int run_entries(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t
         const size_t sums_of_part = size_t(blocks) * share.lanes * share.lane_bytes / p->elem * 4u, counters_of_part = size_t(blocks) * 4u;
         auto fits = [&]() { return size_t(ea.n_parts) * (sums_of_part + counters_of_part) <= HSPMM_STATIC_SCRATCH_BYTES; };
         if (!fits()) choose_classes(p, share.lanes, false, &ea);
-        if (!fits()) return HSPMM_OK;
+        if (!fits() || uint64_t(ea.n_groups) * blocks >= hspmm::kEntryMostGroups) return HSPMM_OK;
         ea.n_pieces = e.totals[0];
         if (ea.n_parts) {
             const size_t sums = ea.n_parts * sums_of_part, counters = ea.n_parts * counters_of_part;

@@ -77,6 +77,10 @@ __global__ __launch_bounds__(256) void fill_zero_kernel(uint16_t *dst, size_t n_
     }
 }
 
+// Workgroups of 256 threads for kernels that go over a whole matrix in strides of the grid: a launch of 2^32 work-items or more,
+// which a few ten million tiles would ask for, is not a valid one.
+static dim3 strided_grid(uint64_t blocks) { return dim3(uint32_t(std::min<uint64_t>(blocks, 1u << 20))); }
+
 // Bitmap tiles -> plain 8 x 16 tiles of 16-bit elements (plans made from the reference's BTCF_MTX arrays, reference
 // src/utils/class.h:55-67): one thread per tile element; header and stored elements as the gather kernels read
 // them (hspmm_device.h: bm_header).  The kernels that take plain tiles then run on what this wrote.
@@ -84,12 +88,13 @@ __global__ __launch_bounds__(256) void expand_bitmap_kernel(const uint32_t *__re
                                                             const uint16_t *__restrict__ vals,
                                                             uint16_t *__restrict__ tiles, uint32_t n_tiles)
 {
-    const uint32_t t = blockIdx.x * 2u + (threadIdx.x >> 7), b = threadIdx.x & 127u;
-    if (t >= n_tiles) return;
-    const uint32_t *h = header + size_t(t) * 8u;
-    const uint32_t word = b >> 5, w = h[word], bit = b & 31u;
-    const uint32_t before = ((h[4] >> (8u * word)) & 0xFFu) + uint32_t(__builtin_popcount(w & ((1u << bit) - 1u)));
-    tiles[size_t(t) * 128u + b] = ((w >> bit) & 1u) ? vals[size_t(h[5]) + before] : uint16_t(0);
+    const uint32_t b = threadIdx.x & 127u;
+    for (size_t t = size_t(blockIdx.x) * 2u + (threadIdx.x >> 7); t < n_tiles; t += size_t(gridDim.x) * 2u) {
+        const uint32_t *h = header + t * 8u;
+        const uint32_t word = b >> 5, w = h[word], bit = b & 31u;
+        const uint32_t before = ((h[4] >> (8u * word)) & 0xFFu) + uint32_t(__builtin_popcount(w & ((1u << bit) - 1u)));
+        tiles[t * 128u + b] = ((w >> bit) & 1u) ? vals[size_t(h[5]) + before] : uint16_t(0);
+    }
 }
 
 // The same for 8 x 8 tiles of 32-bit elements (header words: rows 0..3, rows 4..7, position of the first stored
@@ -98,12 +103,13 @@ __global__ __launch_bounds__(256) void expand_bitmap32_kernel(const uint32_t *__
                                                               const uint32_t *__restrict__ vals,
                                                               uint32_t *__restrict__ tiles, uint32_t n_tiles)
 {
-    const uint32_t t = blockIdx.x * 4u + (threadIdx.x >> 6), b = threadIdx.x & 63u;
-    if (t >= n_tiles) return;
-    const uint32_t *h = header + size_t(t) * 4u;
-    const uint32_t upper = b >> 5, w = h[upper], bit = b & 31u;
-    const uint32_t before = (upper ? uint32_t(__builtin_popcount(h[0])) : 0u) + uint32_t(__builtin_popcount(w & ((1u << bit) - 1u)));
-    tiles[size_t(t) * 64u + b] = ((w >> bit) & 1u) ? vals[size_t(h[2]) + before] : 0u;
+    const uint32_t b = threadIdx.x & 63u;
+    for (size_t t = size_t(blockIdx.x) * 4u + (threadIdx.x >> 6); t < n_tiles; t += size_t(gridDim.x) * 4u) {
+        const uint32_t *h = header + t * 4u;
+        const uint32_t upper = b >> 5, w = h[upper], bit = b & 31u;
+        const uint32_t before = (upper ? uint32_t(__builtin_popcount(h[0])) : 0u) + uint32_t(__builtin_popcount(w & ((1u << bit) - 1u)));
+        tiles[t * 64u + b] = ((w >> bit) & 1u) ? vals[size_t(h[2]) + before] : 0u;
+    }
 }
 
 hipError_t launch_expand_bitmap(int elem_bytes, const uint32_t *header, const void *vals, void *tiles, uint32_t n_tiles,
@@ -111,10 +117,10 @@ hipError_t launch_expand_bitmap(int elem_bytes, const uint32_t *header, const vo
 {
     if (!n_tiles) return hipSuccess;
     if (elem_bytes == 2)
-        expand_bitmap_kernel<<<dim3((n_tiles + 1u) / 2u), 256, 0, s>>>(header, static_cast<const uint16_t *>(vals),
+        expand_bitmap_kernel<<<strided_grid((uint64_t(n_tiles) + 1u) / 2u), 256, 0, s>>>(header, static_cast<const uint16_t *>(vals),
                                                                       static_cast<uint16_t *>(tiles), n_tiles);
     else
-        expand_bitmap32_kernel<<<dim3((n_tiles + 3u) / 4u), 256, 0, s>>>(header, static_cast<const uint32_t *>(vals),
+        expand_bitmap32_kernel<<<strided_grid((uint64_t(n_tiles) + 3u) / 4u), 256, 0, s>>>(header, static_cast<const uint32_t *>(vals),
                                                                         static_cast<uint32_t *>(tiles), n_tiles);
     return hipGetLastError();
 }
@@ -125,16 +131,15 @@ hipError_t launch_expand_bitmap(int elem_bytes, const uint32_t *header, const vo
 __global__ __launch_bounds__(256) void lane_order32_kernel(const uint32_t *__restrict__ tiles, uint32_t *__restrict__ out,
                                                            uint32_t n_tiles)
 {
-    const uint32_t t = blockIdx.x * 4u + (threadIdx.x >> 6), o = threadIdx.x & 63u;
-    if (t >= n_tiles) return;
-    const uint32_t r = o >> 3, g = (o >> 1) & 3u, second = o & 1u;
-    out[size_t(t) * 64u + o] = tiles[size_t(t) * 64u + r * 8u + g + 4u * second];
+    const uint32_t o = threadIdx.x & 63u, r = o >> 3, g = (o >> 1) & 3u, second = o & 1u;
+    for (size_t t = size_t(blockIdx.x) * 4u + (threadIdx.x >> 6); t < n_tiles; t += size_t(gridDim.x) * 4u)
+        out[t * 64u + o] = tiles[t * 64u + r * 8u + g + 4u * second];
 }
 
 hipError_t launch_lane_order32(const void *tiles, void *out, uint32_t n_tiles, hipStream_t s)
 {
     if (!n_tiles) return hipSuccess;
-    lane_order32_kernel<<<dim3((n_tiles + 3u) / 4u), 256, 0, s>>>(static_cast<const uint32_t *>(tiles),
+    lane_order32_kernel<<<strided_grid((uint64_t(n_tiles) + 3u) / 4u), 256, 0, s>>>(static_cast<const uint32_t *>(tiles),
                                                                  static_cast<uint32_t *>(out), n_tiles);
     return hipGetLastError();
 }
@@ -145,20 +150,20 @@ hipError_t launch_lane_order32(const void *tiles, void *out, uint32_t n_tiles, h
 template <uint32_t CW>
 __global__ __launch_bounds__(256) void step_ids_kernel(const uint32_t *__restrict__ raw, uint32_t *__restrict__ out, uint32_t n_tiles)
 {
-    const uint64_t i = uint64_t(blockIdx.x) * 256u + threadIdx.x;
-    if (i >= uint64_t(n_tiles) * CW) return;
-    const uint32_t o = uint32_t(i % CW);
-    uint32_t k = CW == 8u ? (o >> 1) + 4u * (o & 1u) : o;
-    const uint32_t *tile = raw + (i - o);
-    while (k && tile[k] == kIdxMax) --k;
-    out[i] = tile[k];
+    for (uint64_t i = uint64_t(blockIdx.x) * 256u + threadIdx.x; i < uint64_t(n_tiles) * CW; i += uint64_t(gridDim.x) * 256u) {
+        const uint32_t o = uint32_t(i % CW);
+        uint32_t k = CW == 8u ? (o >> 1) + 4u * (o & 1u) : o;
+        const uint32_t *tile = raw + (i - o);
+        while (k && tile[k] == kIdxMax) --k;
+        out[i] = tile[k];
+    }
 }
 
 hipError_t launch_step_ids(int elem_bytes, const uint32_t *raw, uint32_t *out, uint32_t n_tiles, hipStream_t s)
 {
     if (!n_tiles) return hipSuccess;
     const uint32_t cw = elem_bytes == 4 ? 8u : 16u;
-    const dim3 grid(uint32_t((uint64_t(n_tiles) * cw + 255u) / 256u));
+    const dim3 grid = strided_grid((uint64_t(n_tiles) * cw + 255u) / 256u);
     if (elem_bytes == 4) step_ids_kernel<8><<<grid, 256, 0, s>>>(raw, out, n_tiles);
     else step_ids_kernel<16><<<grid, 256, 0, s>>>(raw, out, n_tiles);
     return hipGetLastError();

@@ -61,7 +61,7 @@ int build_tile_stream(hspmm_plan *p)
                             (p->elem == 4u && !(p->panel.built && p->panel.split)))) return HSPMM_OK;
     const uint32_t kk = tile_block_columns(p->dtype), n_blocks = (p->cols + kk - 1u) / kk, n_row_blocks = (p->rows + kTileBlockRows - 1u) / kTileBlockRows;
     const uint64_t cells = uint64_t(n_blocks) * n_row_blocks;
-    if (p->cols < kk || n_blocks > kTileMaxBlocks || cells >= (1u << 26)) return HSPMM_OK;
+    if (p->cols < kk || n_blocks > kTileMaxBlocks || cells >= (1u << 26) || n_row_blocks >= (1u << 23)) return HSPMM_OK;
     const TileSource src{p->d_rowOffset, p->d_rowIdx, p->d_a2b_raw, p->d_data, p->W, p->cols};
     void *room = nullptr;
     if (int rc = plan_alloc(p, (size_t(cells) + 1u) * 4u, &room)) return rc;

@@ -295,7 +295,7 @@ hipError_t launch_spmm_entries(int dtype, const EntryArgs &ea, uint32_t lane_byt
     if (ea.xcd_split && ea.n_feat_blocks != 2u && ea.n_feat_blocks != 4u && ea.n_feat_blocks != 8u) return hipErrorInvalidValue;
     // (a lane's load stays inside its block, a block inside the row, and the lanes reach over the block)
     if (ea.block_bytes < lane_bytes || ea.block_bytes > lane_bytes * lanes || ea.n_feat_blocks < 1u ||
-        uint64_t(ea.ld) * (dtype == kDtypeF32 ? 4u : 2u) < ea.block_bytes)
+        uint64_t(ea.ld) * (dtype == kDtypeF32 ? 4u : 2u) < ea.block_bytes || uint64_t(ea.n_groups) * ea.n_feat_blocks >= kEntryMostGroups)
         return hipErrorInvalidValue;
     bool cut = false;
     for (uint32_t c = 0; c < ea.n_classes; ++c) cut |= (ea.cls[c].logs >> 8) != 0u;

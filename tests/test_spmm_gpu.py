@@ -1506,6 +1506,43 @@ def test_more_than_2_to_24_tiles_and_4_gib_of_tiles_and_of_output(torch_cuda, hs
     torch.cuda.empty_cache()
 
 
+@pytest.mark.parametrize("bitmap", ["0", "1"])
+def test_more_fp32_tiles_than_one_grid_of_the_plans_kernels(torch_cuda, hs, bitmap):
+    """The kernels that write a plan's tiles and ids go over the matrix in strides of 2^20 workgroups - four fp32 tiles each -:
+    4.4 M tiles, kept in lane order and as bitmap + stored elements.  Exact sums, against the all-shapes kernel."""
+    torch = torch_cuda
+    W, N, cols = (1 << 21) + 100000, 4, 3000
+    rows = W * 8
+    rng = np.random.default_rng(2)
+    first = rng.integers(0, cols - 16 * 100, W).astype(np.uint32)
+    per_row = np.array([2, 1, 1, 1, 1, 1, 1, 1], np.int64)           # nine columns per window: two tiles
+    row_ptr = np.zeros(rows + 1, np.uint32)
+    row_ptr[1:] = np.cumsum(np.tile(per_row, W))
+    col_idx = (first[:, None] + 100 * np.array([0, 8, 1, 2, 3, 4, 5, 6, 7], np.uint32)[None, :]).astype(np.uint32).reshape(-1)
+    vals = rng.integers(1, 4, col_idx.size).astype(np.float32)
+    b = hs.csr_to_btcf(rows, cols, row_ptr, col_idx, vals, 1)
+    assert b["total_tiles"] > 1 << 22
+    dB = torch.from_numpy(rng.integers(-4, 5, (cols, N)).astype(np.float32)).cuda()
+    outs = []
+    for mode, env in ((3, {"HSPMM_GATHER_BITMAP": bitmap}), (1, {})):
+        hs.set_kernel_mode(mode)
+        os.environ.update(env)
+        try:
+            plan = hs.Plan(b)
+        finally:
+            hs.set_kernel_mode(0)
+            os.environ.pop("HSPMM_GATHER_BITMAP", None)
+        dC = torch.full((rows, N), float("nan"), device="cuda")
+        plan.run(dB.data_ptr(), dC.data_ptr(), N, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert mode == 1 or plan.info()["gather_bitmap"] == int(bitmap)
+        plan.close()
+        outs.append(dC)
+    assert torch.equal(outs[0], outs[1])
+    del outs, dC, dB
+    torch.cuda.empty_cache()
+
+
 def test_lds_panel_stream_of_more_than_4_gib(torch_cuda, hs):
     """65536 x 32768 at 10 %, fp32 storage: 3.7 M steps of 2 KB in the stream of the LDS-staging kernels (7.5 GB, past
     32-bit byte offsets), 19 M tiles from the caller.  Small integers (exact in bf16 parts and in fp32 sums): bit for
