@@ -50,20 +50,23 @@ int build_entries(hspmm_plan *p, hipStream_t s)
     const size_t units_kept = size_t(unit ? unit : 1u), ids_bytes = units_kept * 16u, vals_bytes = units_kept * 4u * p->elem;
     const size_t desc_bytes = size_t(slot) * 12u, bytes = ids_bytes + vals_bytes + desc_bytes + size_t(e.totals[0]) * 12u;
     void *stream = nullptr;
-    e.unavailable = true;                       // (what has failed once is not tried again)
-    if (slot > 0xFFFFFFFFull || unit > 0xFFFFFFFFull) return HSPMM_OK;
-    if (hipMalloc(&stream, bytes) != hipSuccess) { (void)hipGetLastError(); return HSPMM_OK; }
+    if (slot > 0xFFFFFFFFull || unit > 0xFFFFFFFFull || hipMalloc(&stream, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        e.unavailable.store(true);              // (for good: a plan's results do not change from call to call)
+        return HSPMM_OK;
+    }
     e.d_stream = stream;
     p->fixed_bytes += bytes;
     char *base = static_cast<char *>(stream);
     uint32_t *ids = reinterpret_cast<uint32_t *>(base), *desc = reinterpret_cast<uint32_t *>(base + ids_bytes + vals_bytes);
     uint32_t *pieces = reinterpret_cast<uint32_t *>(base + ids_bytes + vals_bytes + desc_bytes);
-    HSPMM_HIP(launch_entry_fill(int(p->elem), entry_source(p), e.most_chunks, e.d_positions, e.d_row_len, p->rows, at,
-                                e.d_totals + kEntryBins + 1u, desc, pieces, e.d_row_first, ids, base + ids_bytes, s));
-    HSPMM_HIP(hipStreamSynchronize(s));
+    // (a failure that uses the cursors up: not tried again either)
+    auto failed = [&](int code) { e.unavailable.store(true); return code; };
+    HSPMM_HIP_OR(launch_entry_fill(int(p->elem), entry_source(p), e.most_chunks, e.d_positions, e.d_row_len, p->rows, at,
+                                   e.d_totals + kEntryBins + 1u, desc, pieces, e.d_row_first, ids, base + ids_bytes, s), failed);
+    HSPMM_HIP_OR(hipStreamSynchronize(s), failed);
     e.long_rows = unit >= 64u * uint64_t(slot - e.totals[kEntryBins - 1u]);
     e.d_ids = ids; e.d_vals = base + ids_bytes; e.d_desc = desc; e.d_pieces = pieces;
-    e.unavailable = false;
     e.built = true;
     return HSPMM_OK;
 }
@@ -178,7 +181,7 @@ static uint32_t row_blocks(const hspmm_plan *p, uint32_t row_bytes)
 bool entries_serve(const hspmm_plan *p, uint32_t N)
 {
     const Config &c = p->cfg;
-    if (!p->entries.counted || p->entries.unavailable) return false;
+    if (!p->entries.counted || p->entries.unavailable.load()) return false;
     const uint64_t row = uint64_t(N) * p->elem, all = uint64_t(p->cols) * row;
     if (row > kEntryMaxRowBytes) return false;
     if (c.entries > 0) return true;

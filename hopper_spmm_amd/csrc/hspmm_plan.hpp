@@ -169,7 +169,7 @@ struct hspmm_plan {
     // the tiles on the device by the first launch (or hspmm_prepare) that wants it
     struct Entries {
         bool counted = false;
-        bool unavailable = false;                                // no memory for it: the other kernels serve this plan
+        std::atomic<bool> unavailable{false};                    // no memory for it: the other kernels serve this plan
         uint32_t most_chunks = 0;
         uint32_t *d_first_chunk = nullptr, *d_chunk_window = nullptr, *d_positions = nullptr, *d_row_len = nullptr, *d_row_first = nullptr;
         uint32_t *d_totals = nullptr;                            // kEntryBins + 1 counts, then as many cursors
