@@ -27,7 +27,6 @@ MFMA = {1: ("v_mfma_f32_16x16x32_f16", 2500.0), 2: ("v_mfma_f32_16x16x32_bf16", 
 # which roofline binds each configuration by its compulsory bytes and padded flops: the pruned fp32 weight and the
 # block-clustered weight at N = 512 are bound by the matrix cores, the rest by HBM
 BOUND = {(3, 256): "mfma", (4, 512): "mfma"}
-KERNELS = {1: "spmm_scalar_kernel", 2: "spmm_mfma_kernel", 3: "spmm_panel_kernel"}
 
 
 def mfma_report(info, useful_flops, kernel_ms):
@@ -75,9 +74,9 @@ def measure_config(torch, np, hs, G, index, N, steps, warmup, mode=0, matrix=Non
     flops = 2.0 * int(A["nnzs"]) * N
     bytes_alg = G.algorithmic_bytes(b, N)
     t = (main_ms + fix_ms) * 1e-3
-    out = {"workload": "configs[%d]: %s, N=%d" % (index, cfg["name"], N),
+    out = {"workload": "%s, N=%d" % (cfg["name"], N),
            "dtype": "f16 in, f32 accumulate" if A["dtype"] == hs.FP16 else "f32 (tf32 variant)",
-           "kernel": kernel_name(info),
+           "kernel": plan.last_kernel(),
            "kernel_ms": main_ms, "fixup_kernel_ms": fix_ms,
            "tflops": flops / t / 1e12, "algorithmic_bytes": bytes_alg,
            "bound": BOUND.get((index, N), "hbm"),
@@ -166,13 +165,6 @@ def kernel_sources_digest():
             with open(path, "rb") as f:
                 h.update(f.read())
     return h.hexdigest()
-
-
-def kernel_name(info):
-    """The main kernel of the last launch: the gather family without matrix instructions is the entry kernels."""
-    if info["last_kernel_family"] == 2 and info["last_mfma_kind"] == 0:
-        return "spmm_entries_kernel"
-    return KERNELS.get(info["last_kernel_family"], "none")
 
 
 def info_family(plan):
@@ -323,7 +315,7 @@ def main():
         # seeded generators of hopper_spmm_amd/generators.py: raw words of Philox 4x64-10 (numpy's bit generator, a
         # stream numpy keeps stable) through the module's own transforms (Box-Muller normals)
         "data_generator": "Philox 4x64-10 raw words, own transforms (numpy %s)" % np.__version__,
-        "config": {"workload": "configs[%d]: %s, N=%d" % (args.config, cfg["name"], N),
+        "config": {"workload": "%s, N=%d" % (cfg["name"], N),
                    "rows": A["rows"], "cols": A["cols"], "nnz": nnz, "tiles": int(b["total_tiles"]),
                    "eff_row_windows": int(b["eff_row_windows"]), "ranges": info["n_ranges"],
                    "split_windows": info["n_split_windows"]},
@@ -333,7 +325,7 @@ def main():
                      "unit": "GB/s", "frac": bytes_alg / (kernels_ms * 1e-3) / 1e9 / HBM_PEAK_GBPS,
                      # counter figures stored with the rocprofv3 summary they come from (not measured in this run)
                      "traffic": traffic,
-                     "kernel": kernel_name(info),
+                     "kernel": plan.last_kernel(),
                      "kernel_ms": main_ms, "fixup_kernel_ms": fix_ms,
                      "algorithmic_bytes": bytes_alg, "gather_bytes": bytes_gather,
                      # every gathered B row counted every time it is gathered, for comparison with the HBM peak

@@ -103,6 +103,8 @@ def load_library():
     L.hspmm_run.argtypes = [vp, vp, vp, u32, vp]
     L.hspmm_run_static.argtypes = [vp, vp, vp, u32, vp]
     L.hspmm_prepare.argtypes = [vp, u32]
+    L.hspmm_last_kernel.argtypes = [vp]
+    L.hspmm_last_kernel.restype = C.c_char_p
     L.hspmm_bench.argtypes = [vp, vp, vp, u32, i, i, vp, C.POINTER(C.c_float)]
     L.hspmm_profile.argtypes = [vp, vp, vp, u32, i, vp, C.POINTER(C.c_float), C.POINTER(C.c_float)]
     L.hspmm_measure_gather.argtypes = [vp, vp, u32, i, vp, C.POINTER(C.c_float), C.POINTER(C.c_uint64)]
@@ -495,6 +497,10 @@ class Plan:
         (no allocation; the partition for N must exist: prepare(N) or one run with N first)."""
         _check(load_library().hspmm_run_static(self._h, C.c_void_p(dB_ptr), C.c_void_p(dC_ptr), N,
                                                C.c_void_p(stream)))
+
+    def last_kernel(self):
+        """hspmm_last_kernel: the name of the last launch's main kernel ("" before the first)."""
+        return load_library().hspmm_last_kernel(self._h).decode()
 
     def prepare(self, N):
         """hspmm_prepare: builds what the first run with feature dimension N would build; launches nothing."""

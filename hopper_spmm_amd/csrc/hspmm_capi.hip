@@ -252,6 +252,8 @@ void hspmm_destroy(hspmm_plan *p)
     delete p;
 }
 
+const char *hspmm_last_kernel(const hspmm_plan *p) { return p ? p->last_kernel.load(std::memory_order_relaxed) : ""; }
+
 int hspmm_get_plan_info(const hspmm_plan *p, hspmm_plan_info *info)
 {
     if (!p || !info) return fail(HSPMM_ERR_INVALID, "null argument");

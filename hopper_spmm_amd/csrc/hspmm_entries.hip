@@ -303,7 +303,7 @@ int run_entries(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t
     if (mode == RunMode::kPrepare) return HSPMM_OK;
     ea.desc = e.d_desc; ea.ids = e.d_ids; ea.vals = e.d_vals; ea.pieces = e.d_pieces;
     ea.B = dB; ea.C = dC; ea.ld = N; ea.block_bytes = block_bytes; ea.n_feat_blocks = blocks; ea.xcd_split = by_xcd;
-    p->note_launch(2, 0, 0);
+    p->note_launch("spmm_entries_kernel", 2, 0, 0);
     HSPMM_HIP(hspmm::launch_spmm_entries(p->dtype, ea, share.lane_bytes, share.lanes, s));
     return HSPMM_OK;
 }

@@ -228,8 +228,10 @@ struct hspmm_plan {
     // matrix instructions of the last launch's main kernel: kind (hspmm_plan_info::last_mfma_kind) and count
     std::atomic<uint32_t> last_mfma_kind{0};
     std::atomic<uint64_t> last_mfma_count{0};
-    void note_launch(uint32_t family, uint32_t kind, uint64_t count)
+    std::atomic<const char *> last_kernel{""};  // its name (hspmm_last_kernel)
+    void note_launch(const char *kernel, uint32_t family, uint32_t kind, uint64_t count)
     {
+        last_kernel.store(kernel, std::memory_order_relaxed);
         last_family.store(family, std::memory_order_relaxed);
         last_mfma_kind.store(kind, std::memory_order_relaxed);
         last_mfma_count.store(count, std::memory_order_relaxed);

@@ -141,7 +141,8 @@ std::vector<hspmm_plan::StreamBuffers *> sets_for(hspmm_plan *p, hipStream_t s, 
 
 namespace hspmm_host {
 
-// Arrival counters of the in-kernel reduction (never used by hspmm_run_static).
+// Arrival counters of the in-kernel reduction.  (hspmm_run_static has none of its own: the gather and LDS-panel kernels use the
+// second launch there, the entry and full-tile kernels count behind their sums in the fixed array.)
 // Called with the plan's mutex held.
 int ensure_arrive(hspmm_plan *p, hipStream_t s, size_t words, RunMode mode, uint32_t **out)
 {
@@ -363,7 +364,7 @@ static int run_panel(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStr
         ka.uniform_chunks = sh.n_chunks;
     }
     if (mode == RunMode::kPrepare) return HSPMM_OK;
-    p->note_launch(3, sh.mfma_kind, sh.mfma_count);
+    p->note_launch("spmm_panel_kernel", 3, sh.mfma_kind, sh.mfma_count);
     HSPMM_HIP(hspmm::launch_spmm_panel(p->dtype, pl.quad ? 0 : pl.G, pl.split, pl.tall, pl.packed, pa, ka, sh.units, s, mid));
     return HSPMM_OK;
 }
@@ -415,7 +416,7 @@ static int run_impl(hspmm_plan *p, const void *dB, void *dC, uint32_t N, void *s
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (p->W == 0) {
         if (!launch) return HSPMM_OK;
-        p->note_launch(4, 0, 0);
+        p->note_launch("fill_zero_kernel", 4, 0, 0);
         HSPMM_HIP(hspmm::launch_fill_zero(dC, size_t(p->rows) * N * p->elem, s));
         return HSPMM_OK;
     }
@@ -554,7 +555,7 @@ static int run_gather(hspmm_plan *p, const void *dB, void *dC, uint32_t N, uint3
     if (c.scalar) {
         if (ld != N) return fail(HSPMM_ERR_UNSUPPORTED, "the all-shapes kernel takes whole rows");
         if (!launch) return HSPMM_OK;
-        p->note_launch(1, 0, 0);
+        p->note_launch("spmm_scalar_kernel", 1, 0, 0);
         HSPMM_HIP(hspmm::launch_spmm_scalar(p->dtype, ka, s));
         return HSPMM_OK;
     }
@@ -593,7 +594,7 @@ static int run_gather(hspmm_plan *p, const void *dB, void *dC, uint32_t N, uint3
     ka.ranges = dp.d_ranges; ka.split = dp.d_split; ka.fix_slots = dp.d_fix_slots;
     if (!launch) return HSPMM_OK;
     // (per step and feature block: G * V instructions of 16 x 16 x 32, or 2 G V of 16 x 16 x 4 for 32-bit elements)
-    p->note_launch(2, p->dtype == HSPMM_TF32 ? 3u : p->dtype == HSPMM_FP16 ? 1u : 2u,
+    p->note_launch("spmm_mfma_kernel", 2, p->dtype == HSPMM_TF32 ? 3u : p->dtype == HSPMM_FP16 ? 1u : 2u,
                    uint64_t(p->n_steps) * ka.n_feat_blocks * uint64_t(p->G) * uint64_t(c.V) * (p->dtype == HSPMM_TF32 ? 2u : 1u));
     HSPMM_HIP(hspmm::launch_spmm_mfma(p->dtype, g.layout, p->G, ka, c.V, g.prefetch, c.narrow, g.wpg, s, mid));
     return HSPMM_OK;

@@ -132,7 +132,7 @@ int run_tile(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s,
     ta.src = t.d_source;
     ta.n_row_blocks = t.n_row_blocks; ta.n_chunks = sh.n_chunks; ta.n_feat_tiles = sh.n_feat_tiles;
     const uint32_t kind = p->dtype == HSPMM_FP16 ? 1u : 2u;
-    p->note_launch(3, kind, uint64_t(sh.n_tiles) * sh.n_chunks * (sh.nt / 16u) * 8u * (p->dtype == HSPMM_TF32 ? 3u : 2u));
+    p->note_launch("spmm_tile_kernel", 3, kind, uint64_t(sh.n_tiles) * sh.n_chunks * (sh.nt / 16u) * 8u * (p->dtype == HSPMM_TF32 ? 3u : 2u));
     HSPMM_HIP(hspmm::launch_spmm_tile(p->dtype, ta, sh.nt, sh.groups, s));
     return HSPMM_OK;
 }

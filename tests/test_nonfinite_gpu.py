@@ -11,19 +11,19 @@ from util import decode, encode
 
 pytestmark = pytest.mark.gpu
 
-# kernel mode, environment, feature dimensions (16 bits / fp32 storage)
+# kernel mode, environment, feature dimensions, main kernel
 FAMILIES = {
-    "all-shapes": (1, {}, (9, 33)),
-    "gather": (3, {}, (16, 33, 64, 136)),
-    "panel": (4, {}, (128, 200)),
-    "panel, fp32 products": (5, {}, (128, 200)),
-    "entries": (0, {"HSPMM_ENTRIES": "1", "HSPMM_TILE": "0"}, (9, 16, 33, 64, 130)),
-    "tile": (0, {"HSPMM_TILE": "1"}, (9, 16, 24, 33, 64, 100, 127)),
+    "all-shapes": (1, {}, (9, 33), "spmm_scalar_kernel"),
+    "gather": (3, {}, (16, 33, 64, 136), "spmm_mfma_kernel"),
+    "panel": (4, {}, (128, 200), "spmm_panel_kernel"),
+    "panel, fp32 products": (5, {}, (128, 200), "spmm_panel_kernel"),
+    "entries": (0, {"HSPMM_ENTRIES": "1", "HSPMM_TILE": "0"}, (9, 16, 33, 64, 130), "spmm_entries_kernel"),
+    "tile": (0, {"HSPMM_TILE": "1"}, (9, 16, 24, 33, 64, 100, 127), "spmm_tile_kernel"),
 }
 
 
 def _plan(hs, A, family):
-    mode, env, _ = FAMILIES[family]
+    mode, env = FAMILIES[family][:2]
     os.environ.update(env)
     hs.set_kernel_mode(mode)
     try:
@@ -84,8 +84,6 @@ def test_infinities_and_nans_stay_with_the_rows_that_name_them(torch_cuda, hs, f
     plan = _plan(hs, _csr(D, dtype), family)
     strict = family in ("entries", "tile")
     for N in FAMILIES[family][2]:
-        if dtype == 1 and family == "gather" and N == 136:
-            continue
         Bm = rng.integers(-4, 5, (cols, N)).astype(np.float64)
         clean = _rounded(D @ Bm, dtype)
         bad, pairs = {}, {}                             # feature -> rows of B
@@ -101,6 +99,7 @@ def test_infinities_and_nans_stay_with_the_rows_that_name_them(torch_cuda, hs, f
                     if 0 <= pair < N:
                         pairs.setdefault(pair, []).extend(bad[f])
         got = decode(gpu_spmm(torch_cuda, hs, dict(dtype=dtype, rows=rows), encode(Bm.astype(np.float32), dtype), N, plan=plan), dtype)
+        assert plan.last_kernel() == FAMILIES[family][3]
         want = _rounded(_stored_sum(D, Bm), dtype)
         what = "%s, dtype %d, N=%d" % (family, dtype, N)
         fine = [f for f in range(N) if f not in bad and f not in pairs]

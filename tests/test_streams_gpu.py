@@ -30,8 +30,7 @@ def _case(hs, which, dtype):
 
 
 def _check_kernel(plan, which):
-    info = plan.info()
-    assert (info["last_kernel_family"], info["last_mfma_kind"] == 0) == ((2, True) if which == "entries" else (3, False))
+    assert plan.last_kernel() == {"entries": "spmm_entries_kernel", "tile": "spmm_tile_kernel"}[which]
 
 
 def _lane(torch, rng, A, N, dtype):
