@@ -144,24 +144,36 @@ static uint32_t entry_block_bytes(uint32_t row_bytes, uint32_t blocks)
     return blocks == 1u ? row_bytes : ((row_bytes + blocks - 1u) / blocks + 15u) & ~15u;
 }
 
-// Blocks a row of B is cut into, which are passes over the entries one after the other: as few lanes as possible (a block's
-// are a power of two) and few passes; blocks of 512 bytes are behind those of 256 where B is large, and where no row is hot a
-// pass is faster the more of its part of B an L2 holds.  Measured (1 / 2 / 4 or, where in brackets, other blocks, us):
-//   fp16, graph of 40000, N = 181: 38 / 37 (3) 33, N = 256: 28 / 28 / 31; of 73838, N = 336: (2) 126 (3) 96 (6) 121, N = 512:
-//   (2) 128 (4) 113 (8) 130;  of 262144, bf16, N = 256: 147 / 126 / 128;  uniform 61181 columns, N = 256: 141 / 121 / 102, 18432
-//   columns: 133 / 95 / 95;  fp32, uniform 17544 columns, N = 224: (2) 39 (4) 40 (7) 29
+// Lines of 128 bytes that `bytes` bytes from byte `off` of a row touch: the mean over rows that begin on multiples of `step`.
+static double lines_touched(uint32_t off, uint32_t bytes, uint32_t step)
+{
+    if (step <= 16u) return 1.0 + double((bytes - 1u) / step * step) / 128.0;         // (off, too, is a multiple of step)
+    uint32_t lines = 0;
+    for (uint32_t at = off; at < off + 128u; at += step) lines += (at + bytes - 1u) / 128u - at / 128u + 1u;
+    return double(lines) * step / 128.0;
+}
+
+// Blocks a row of B is cut into, passes over the entries one after the other: the cheapest by what an entry takes - the lines of B
+// it touches, its lanes (16 bytes each, used or not) as lines, and half a line for every pass - with a tenth more for every time
+// a block's part of B doubles beyond half an L2.  A row of 640 bytes that begins on a line is five blocks of eight lanes (5 lines
+// + 5 of lanes + 2.5) and not two of 32 (6 + 8 + 1): fp32, graph of 57344, N = 160, 48 against 72 us.  One of 300 bytes that
+// begins anywhere is one block of 32 lanes (3.3 + 4 + 0.5) and not three of eight (5.6 + 3 + 1.5): graph of 905216, N = 75, 576
+// against 861 us.  The two weights are a fit to 745 graphs and uniform matrices, all types and N, with any number of blocks: the
+// choice is 1.6 % behind the fastest on average and 12 % at the 95th percentile, and weights half or twice as large 0.3 % more.
 static uint32_t row_blocks(const hspmm_plan *p, uint32_t row_bytes)
 {
-    uint32_t best = 1;
+    const uint32_t step = row_bytes % 128u ? row_bytes & (0u - row_bytes) : 128u;
+    uint32_t best = 0;
     double least = 0.0;
-    for (uint32_t b = (row_bytes + kEntryMaxBlockBytes - 1u) / kEntryMaxBlockBytes; b <= 16u && (b == 1u || row_bytes / b >= 96u); ++b) {
+    for (uint32_t b = (row_bytes + kEntryMaxBlockBytes - 1u) / kEntryMaxBlockBytes; b == 1u || row_bytes / b >= 112u; ++b) {
         const uint32_t bytes = entry_block_bytes(row_bytes, b);
-        const RowShare share = share_row(bytes);
-        double cost = double(b * share.lanes) * (1.0 + 0.05 * double(b - 1u));
-        const double part = double(p->cols) * bytes;
-        if (bytes >= 448u && double(p->cols) * row_bytes > 16e6) cost *= 1.06;
-        if (p->even_windows && part > 3e6) cost *= 1.0 + 0.15 * std::log2(part / 3e6);
-        if (least == 0.0 || cost < least) { least = cost; best = b; }
+        if (bytes > kEntryMaxBlockBytes || (best && bytes < 128u)) continue;
+        double cost = double(b * share_row(bytes).lanes) / 8.0 + 0.5 * double(b);
+        if (step <= 16u) cost += double(b) * lines_touched(0u, bytes, step);
+        else for (uint32_t i = 0; i < b; ++i) cost += lines_touched(std::min(i * bytes, row_bytes - bytes), bytes, step);
+        const double part = double(p->cols) * bytes / double(2u << 20);
+        if (part > 1.0) cost *= 1.0 + 0.1 * std::log2(part);
+        if (!best || cost < least) { least = cost; best = b; }
     }
     return best;
 }
@@ -170,9 +182,9 @@ static uint32_t row_blocks(const hspmm_plan *p, uint32_t row_bytes)
 // on how many of its eight elements are stored nor, up to a block of 32 features (16 of fp32 storage), on N.  So the line goes by
 // the bytes of a row of B and by the stored entries per tile column (per_column: 1.0 for graphs, 1.4 for weights
 // pruned to 10 %, 1.9 to 20 %, 8 for blocks).  Measured (entry / other kernels, us):
-//   16 bits, graph 2^18 N = 1 / 16 / 64: 14.5 / 45, 26 / 41, 44 / 58;  11610 vertices N = 128 / 333 / 512 / 1000: 7.6 / 14, 17 / 36,
-//   16 / 13, 26 / 25;  40000 N = 128 / 512: 16 / 24, 50 / 60;  73838 N = 128 / 336 / 512: 31 / 45, 96 / 113, 113 / 148;  2^18, 8 per
-//   vertex, N = 128 / 200 / 256: 62 / 64, 116 / 135, 126 / 119;  2^20 N = 128: 510 / 474;  uniform 8192^2 at 2 %, N = 256: 35 / 51
+//   16 bits, graph 2^18 N = 1 / 16 / 64: 14.5 / 45, 26 / 41, 44 / 58;  11610 vertices N = 128: 7.6 / 14;  40000 N = 128: 16 / 24;
+//   73838 N = 128: 31 / 45;  16052 N = 627: 21 / 43;  117373 N = 528: 175 / 218;  uniform 16896 x 20992, 29 per row, N = 657: 90 / 132;
+//   2^20 N = 128: 510 / 474;  uniform 8192^2 at 2 %, N = 256: 35 / 51
 //   16 bits, 4096^2 pruned to 10 % N = 8 / 16: 5.8 / 10.3, 7 / 10.4; 4096 x 11008 N = 32: 24.6 / 22.5; to 30 % N = 8 / 16:
 //   10 / 15.3, 16 / 15.3;  5376 x 3328 pruned to 3 %, N = 126 / 208 / 387: 12 / 18, 18 / 21, 54 / 26 (LDS-panel kernels)
 //   fp32, graph of 150001 N = 16 / 64 / 128: 18 / 39, 43 / 68, 88 / 126;  12288 N = 128 / 256 / 500: 10 / 20, 16 / 26, 28 / 38;
@@ -193,10 +205,10 @@ bool entries_serve(const hspmm_plan *p, uint32_t N)
     }
     if (weight <= 42.0 || (sparse && row <= 128u)) return true;
     if (!sparse || panel_serves(p, N)) return false;
-    // (N a multiple of 64, where the other kernels load words: ahead on a B beyond the L2s' reach, and in eight blocks on a small
-    // one.  Of 8, where they load 16 bytes: on a small B with very many rows, uniform 34816 x 3575, 4 per row, N = 480: 18.7 / 16.1)
-    if (N % 64u != 0u) return !(N % 8u == 0u && row >= 896u && all <= (uint64_t(20) << 20) && p->rows > 16384u);
-    return entries_by_xcd(p, row) || (all <= (uint64_t(64) << 20) && !(row >= 1024u && all <= (uint64_t(16) << 20)));
+    // N a multiple of 64, hot rows and a B that fills half of the 256 MB memory-side cache: there the other kernels, which then load
+    // words and read fewer rows of B, are ahead (graph of 920569, N = 128, 236 MB: 363 / 343 us; of 434176, N = 512, 445 MB:
+    // 353 / 322; 18 such graphs: 1.02 on average, and 1.13 behind on 16 with other N a multiple of 8).
+    return p->even_windows || N % 64u != 0u || all <= (uint64_t(128) << 20);
 }
 
 struct CountArrays { size_t most_chunks, words[6]; };
