@@ -86,30 +86,21 @@ def test_infinities_and_nans_stay_with_the_rows_that_name_them(torch_cuda, hs, f
     for N in FAMILIES[family][2]:
         Bm = rng.integers(-4, 5, (cols, N)).astype(np.float64)
         clean = _rounded(D @ Bm, dtype)
-        bad, pairs = {}, {}                             # feature -> rows of B
+        bad = {}                                        # feature -> rows of B
         for f, (k, v) in enumerate([(unnamed[0], np.inf), (unnamed[1], np.nan), (named[0], np.inf), (named[1], -np.inf),
                                     (named[2], np.nan), (named[3], np.inf)]):
             Bm[k, f] = v
             bad.setdefault(f, []).append(k)
         Bm[named[0], N - 1], Bm[named[1], N - 1] = np.inf, -np.inf
         bad.setdefault(N - 1, []).extend([named[0], named[1]])
-        if family == "gather" and dtype != 1:           # (two adjacent features of a 16-bit type are one operand word)
-            for f in list(bad):
-                for pair in (f - 1, f + 1):
-                    if 0 <= pair < N:
-                        pairs.setdefault(pair, []).extend(bad[f])
         got = decode(gpu_spmm(torch_cuda, hs, dict(dtype=dtype, rows=rows), encode(Bm.astype(np.float32), dtype), N, plan=plan), dtype)
         assert plan.last_kernel() == FAMILIES[family][3]
         want = _rounded(_stored_sum(D, Bm), dtype)
         what = "%s, dtype %d, N=%d" % (family, dtype, N)
-        fine = [f for f in range(N) if f not in bad and f not in pairs]
+        fine = [f for f in range(N) if f not in bad]
         assert np.array_equal(got[:, fine], clean[:, fine]), what
-        for f in set(pairs) - set(bad):
-            reach = np.any([_near(D, k) for k in pairs[f]], axis=0)
-            assert np.array_equal(got[~reach, f], clean[~reach, f]), what + ": feature %d beside one that is not finite" % f
         for f, ks in bad.items():
-            ks = ks + pairs.get(f, [])
-            names = (D[:, bad[f]] != 0).any(1)
+            names = (D[:, ks] != 0).any(1)
             reach = names if strict else np.any([_near(D, k) for k in ks], axis=0)
             # (the features of an unnamed row have no reach at all; the row of B that is not finite counts for nothing elsewhere)
             assert np.array_equal(got[~reach, f], clean[~reach, f]), what + ": feature %d beyond the rows that name it" % f
@@ -137,4 +128,72 @@ def test_an_infinity_under_a_rows_last_entry_is_multiplied_once(torch_cuda, hs, 
         Bm[cols - 1, N - 1] = np.inf if N > 1 else -np.inf
         got = decode(gpu_spmm(torch_cuda, hs, dict(dtype=dtype, rows=rows), encode(Bm.astype(np.float32), dtype), N, plan=plan), dtype)
         assert np.array_equal(got, _rounded(_stored_sum(D, Bm), dtype), equal_nan=True), "N=%d" % N
+    plan.close()
+
+
+# environment, ranges per SIMD, paired windows
+FORMS = {
+    "whole units": ({}, 0, False),
+    "cut units, second launch": ({"HSPMM_FUSED_FIXUP": "0"}, 16, False),
+    "cut units, added where the last part ends": ({"HSPMM_FUSED_FIXUP": "1"}, 16, False),
+    "a workgroup per unit": ({"HSPMM_ALIGNED_SMALL": "4"}, 0, False),
+    "bitmap tiles": ({"HSPMM_GATHER_BITMAP": "1"}, 16, False),
+    "pairs of windows": ({}, 0, True),
+    "pairs of windows, cut": ({"HSPMM_FUSED_FIXUP": "1"}, 16, True),
+}
+
+
+@pytest.mark.parametrize("form", list(FORMS))
+@pytest.mark.parametrize("dtype", [0, 2])
+def test_adjacent_features_of_the_gather_kernels_do_not_mix(torch_cuda, hs, form, dtype):
+    """Their 16-bit operand words are two adjacent features: one that is not finite leaves the other alone."""
+    torch = torch_cuda
+    env, ranges, paired = FORMS[form]
+    rng = np.random.default_rng(70 + dtype)
+    rows, cols = 328, 6000
+    D = rng.integers(1, 4, (rows, cols)) * (rng.random((rows, cols)) < 0.02)
+    if paired:                                          # 16 rows with one list of columns
+        lists = rng.random((-(-rows // 16), cols)) < 0.05
+        lists[10] = rng.random(cols) < 0.9              # (long enough to be cut)
+        D = np.repeat(lists, 16, axis=0)[:rows] * rng.integers(1, 4, (rows, cols))
+    D[40:56] = 0
+    D[:, 77] = 0
+    D[(3, 100, 101, 250), 77] = 2
+    A = _csr(D, dtype)
+    hs.set_kernel_mode(3)
+    hs.set_window_pairing(2 if paired else 0)
+    hs.configure(producer_warp_group_num=ranges)
+    os.environ.update(env)
+    try:
+        plan = hs.Plan(convert(hs, A))
+    finally:
+        hs.set_kernel_mode(0)
+        hs.set_window_pairing(0)
+        hs.configure()
+        for name in env:
+            os.environ.pop(name, None)
+    info = plan.info()
+    assert (info["n_paired_units"] > 0) == paired and (info["n_split_windows"] > 0 or "cut" not in form)
+    assert info["gather_bitmap"] == ("HSPMM_GATHER_BITMAP" in env)
+    stream = torch.cuda.current_stream().cuda_stream
+    for N in (1, 2, 16, 31, 64, 100, 128, 136, 256):
+        Bm = rng.integers(-4, 5, (cols, N)).astype(np.float64)
+        clean = _rounded(D @ Bm, dtype)
+        bad = sorted({0, N // 2, max(0, N - 2)})
+        for f, v in zip(bad, (np.inf, np.nan, -np.inf)):
+            Bm[77, f] = v
+        dB = torch.from_numpy(encode(Bm.astype(np.float32), dtype).view(np.int16)).cuda()
+        dC = torch.empty((rows, N), dtype=torch.int16, device="cuda")
+        plan.prepare(N)
+        for launch in (plan.run, plan.run_static):
+            dC.fill_(0x7E01)
+            launch(dB.data_ptr(), dC.data_ptr(), N, stream)
+            torch.cuda.synchronize()
+            assert plan.last_kernel() == "spmm_mfma_kernel"
+            got = decode(dC.cpu().numpy().view(np.uint16), dtype)
+            fine = [f for f in range(N) if f not in bad]
+            assert np.array_equal(got[:, fine], clean[:, fine]), "N=%d" % N
+            reach = _near(D, 77)
+            assert np.array_equal(got[~reach][:, bad], clean[~reach][:, bad]), "N=%d" % N
+            assert not np.isfinite(got[(3, 100, 101, 250), :][:, bad]).any(), "N=%d" % N
     plan.close()
