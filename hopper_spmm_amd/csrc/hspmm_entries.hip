@@ -201,6 +201,11 @@ bool entries_serve(const hspmm_plan *p, uint32_t N)
     const bool sparse = per_column <= 1.25;
     if (p->elem == 4u) {
         if (weight <= 100.0) return true;
+        // Rows that are no whole 16-byte pieces, below the 64 features from which the LDS-panel kernels take any: the other fp32
+        // products come in blocks of 16 features where N is odd and of 32 where it is even (pruned 4096 x 11008 at 10 %, N = 47:
+        // 57.7 / 122; 11008 x 4096 at 20 %, N = 26 / 47: 70 / 94, 107 / 191; 1500 x 9000 at 25 %, N = 30 / 51 / 63: 56 / 41, 81 / 85,
+        // 88 / 85)
+        if (N < 64u && N % 4u != 0u) return weight <= (N % 2u ? 350.0 : 135.0);
         return sparse && !p->panel.built && (row <= 256u || all <= (uint64_t(256) << 20));
     }
     if (weight <= 42.0 || (sparse && row <= 128u)) return true;

@@ -435,7 +435,7 @@ static int run_impl(hspmm_plan *p, const void *dB, void *dC, uint32_t N, void *s
     // in front of its feature.)
     // (Cutting at the last multiple of 64 as well, so that those features run with word loads and bitmap tiles,
     // measured 1027 -> 895 us at N = 136 and 1175 -> 1259 us at N = 200: not done.)
-    // A single feature of a 16-bit type (matrix times vector): B and C widened to words - the element and a zero -
+    // A single feature of a 16-bit type (matrix times vector) that the entry kernels have not taken: B and C widened to words - the element and a zero -
     // in a buffer of the plan's, two features through the MFMA kernels, the low halves back (power-law graph 2^20:
     // 21 ms on the all-shapes kernel).  hspmm_run_static, which allocates nothing, wants the buffer made already.
     if (p->elem == 2u && N == 1u && p->cfg.kernel_mode != 1) {

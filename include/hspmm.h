@@ -70,16 +70,20 @@ int hspmm_create(hspmm_plan **plan, int dtype, uint32_t rows, uint32_t cols,
  * DEVICE pointers, row-major, aligned to the element size (the LDS-staging kernels
  * want one block of features - 256 bytes of a row - and take B and C wherever they start, the widest loads
  * of the other MFMA kernels want 16 bytes and N a multiple of 8 - of 4 for fp32 storage -; everything else
- * takes narrower loads or two launches; a single feature of a 16-bit type goes
- * through a buffer of cols + rows words that the plan allocates at the first such
- * launch or at hspmm_prepare(plan, 1)); every element of C is
+ * takes narrower loads or two launches; a single feature of a 16-bit type that the
+ * entry kernels do not take goes through a buffer of cols + rows words that the plan
+ * allocates at the first such launch or at hspmm_prepare(plan, 1)); every element of C is
  * written (rows without nonzeros become 0).  Asynchronous on `stream` (a
  * hipStream_t, NULL = default stream).
+ * An infinity or a NaN in B[k][f] reaches column f of C only, there the rows with an
+ * entry in column k and at most the other rows of their window - of the up to four
+ * windows a kernel walks as one unit - where a tile's zero multiplies it.
  * Host side: a plan is immutable after hspmm_create except for what the first
  * launch with a new N, or on a new stream, may add under the plan's own mutex -
- * a work partition for that width or, for narrow feature dimensions, the matrix
+ * a work partition for that width or, for sparse matrices, the matrix
  * once more entry by entry (made on the device, which that launch waits for; not
- * made under stream capture, where such a launch takes other kernels), and buffers for what a launch writes besides C
+ * made under stream capture, where such a launch takes other kernels; when there is
+ * no memory for it, the plan does without), and buffers for what a launch writes besides C
  * (partial sums of cut windows, their arrival counters; older buffers stay
  * allocated until hspmm_destroy, so launches recorded earlier, e.g. in a HIP
  * graph, stay valid whatever N is run afterwards).  hspmm_run may therefore be
@@ -112,10 +116,12 @@ int hspmm_prepare(hspmm_plan *plan, uint32_t N);
  * array of device memory that the library holds on every device it is loaded
  * on (HSPMM_STATIC_SCRATCH_BYTES, from library load until the process ends)
  * instead of the plan's own buffer.  It calls no hipMalloc / hipFree and builds
- * nothing: the work partition for this N (and, for a single feature of a 16-bit
- * type, the plan's buffer of cols + rows words) must exist already (hspmm_prepare, or
- * one hspmm_run with this N), else HSPMM_ERR_UNSUPPORTED; so does a launch whose
- * partial sums exceed the array (the message says how much it needs).  Results
+ * nothing: what this N needs - the work partition, the matrix entry by entry or, for
+ * a single feature of a 16-bit type, the plan's buffer of cols + rows words - must
+ * exist already (hspmm_prepare, or one hspmm_run with this N), else
+ * HSPMM_ERR_UNSUPPORTED; so does a launch of the gather or LDS-panel kernels whose
+ * partial sums exceed the array (the message says how much it needs; the entry and
+ * full-tile kernels choose shapes whose sums fit).  Results
  * are bit-identical to hspmm_run.  All calls on one device share the one array
  * whatever their plan: two calls that overlap in time on one device race. */
 #define HSPMM_STATIC_SCRATCH_BYTES (32u << 20)
@@ -174,17 +180,20 @@ void hspmm_get_config(int *buffer_stage, int *consumer_warp_num,
  * with HSPMM_ERR_INVALID / HSPMM_ERR_UNSUPPORTED. */
 int hspmm_has_experimental(void);
 
-/* Kernel selection, read by the next hspmm_create: 0 = automatic (MFMA kernels
- * whenever the feature dimension allows; the kernels that stage B through LDS
- * for matrices whose windows touch a large share of the columns), 1 = always the
+/* Kernel selection, read by the next hspmm_create: 0 = automatic (entry kernels
+ * where few of a tile's elements are stored and rows of B are short; full-tile
+ * kernels for unstructured matrices of some per cent at up to 127 features; the
+ * kernels that stage B through LDS for matrices whose windows touch a large share
+ * of the columns; MFMA gather kernels for the rest), 1 = always the
  * scalar all-shapes kernel, 2 = 16-bit MFMA kernel with wide loads only, 3 =
  * 16-bit MFMA kernel with word loads whenever N is a multiple of 32, 4 = the
  * LDS-staging kernels for every matrix (whenever N is 128 at least - 64 for fp32
  * storage, or 16 with rows of whole 16-byte pieces), 5 = the same
- * with fp32 products in the HSPMM_TF32 LDS-staging kernels (N 64 at least).  (By default those
- * kernels multiply the bf16 parts hi + lo of every fp32 factor, which keeps 16
- * mantissa bits per factor; the reference's tf32 instruction keeps 10,
- * src/ptx/wgmma.h:42-58.  The other HSPMM_TF32 kernels always multiply in fp32.) */
+ * with fp32 products in the HSPMM_TF32 LDS-staging kernels (N 64 at least).  Modes 1 to 5 have neither
+ * entry nor full-tile kernels.  (By default the LDS-staging kernels, full tiles among them, multiply the bf16
+ * parts hi + lo of every fp32 factor, which keeps 16 mantissa bits per factor; the reference's tf32 instruction
+ * keeps 10, src/ptx/wgmma.h:42-58.  They take N of 64 at least, and from 16 on in rows of whole 16-byte pieces;
+ * all other HSPMM_TF32 launches multiply in fp32.) */
 int hspmm_set_kernel_mode(int mode);
 
 /* No reference counterpart.  Two vertically adjacent windows with the same
