@@ -211,3 +211,19 @@ def test_without_memory_for_the_stream_the_other_kernels_serve(torch_cuda, hs, o
     assert np.array_equal(outs[0].cpu().numpy(), want)
     plan.close()
     other.close()
+
+
+# (rows of B of 1 to 9 blocks: whole lines in blocks of one, two and four lines, and rows that begin anywhere)
+@pytest.mark.parametrize("dtype,widths", [(0, (72, 150, 192, 320, 448, 543, 576, 640, 700, 896, 1000)), (2, (66, 171, 384, 529, 832)),
+                                          (1, (35, 75, 96, 160, 192, 224, 288, 300, 448, 500))])
+def test_every_number_of_blocks_a_row_is_cut_into(torch_cuda, hs, oracle, dtype, widths):
+    torch = torch_cuda
+    rng = np.random.default_rng(430 + dtype)
+    for cols, lengths in ((9000, list(rng.integers(0, 30, 900))), (700, [3] * 600 + [0, 257, 600])):
+        A = _rows_of_lengths(rng, lengths, cols, dtype)
+        plan = _plan(hs, A)
+        for N in widths:
+            B = make_b(rng, cols, N, dtype)
+            ref, mag = oracle_spmm(oracle, A, B, N)
+            _check_guarded(torch, plan, A, B, N, dtype, ref, mag, "cols=%d N=%d" % (cols, N))
+        plan.close()
