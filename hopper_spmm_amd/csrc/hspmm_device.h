@@ -168,6 +168,20 @@ hipError_t launch_spmm_tile(int dtype, const TileArgs &ta, uint32_t nt, uint32_t
 hipError_t launch_tile_count(int dtype, const TileSource &src, uint32_t n_row_blocks, uint32_t n_blocks, uint32_t *counts, uint32_t *blocks, hipStream_t s);
 hipError_t launch_tile_fill(int dtype, const TileSource &src, uint32_t n_row_blocks, uint32_t n_blocks, const uint32_t *counts,
                             const uint32_t *blocks, void *pos, void *vals, hipStream_t s);
+// Wide-tile kernels (spmm_wide_kernel.hip, 16-bit types): A as first operands of matrix instructions, 16 rows x 64 columns each.
+constexpr uint32_t kWideUnitBytes = 2048u;
+// A workgroup: `splits` sets of `rows` waves with `units` x 16 rows each, `blocks` x 16 features.
+struct WideShape { uint32_t units, blocks, rows, splits; };
+struct WideArgs {
+    const void     *frags;       // per unit of 16 rows and chunk of 64 columns kWideUnitBytes
+    const void     *B;
+    void           *C;
+    uint32_t rows, cols, N;
+    uint32_t n_units, n_chunks, n_feat_tiles;                    // chunks: a multiple of four
+    const TileSource *src;       // in device memory (read where B is not finite)
+};
+hipError_t launch_spmm_wide(int dtype, const WideArgs &wa, const WideShape &sh, hipStream_t s);
+hipError_t launch_wide_fill(const TileSource &src, uint32_t rows, uint32_t n_chunks, void *frags, hipStream_t s);
 hipError_t launch_fill_zero(void *dst, size_t bytes, hipStream_t s);
 // bitmap tiles -> plain tiles.  8 x 16 tiles of 16-bit elements: header as KernelArgs::bm_header; 8 x 8 tiles of 32-bit
 // elements: 4 header words per tile - rows 0..3, rows 4..7, position of the first stored element, number of stored elements

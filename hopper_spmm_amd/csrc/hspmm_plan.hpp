@@ -63,6 +63,8 @@ struct Config {
     int gather_bitmap = -1;             // gather kernels read single 16-bit windows as bitmap + stored elements (-1: by fill)
     int entries = -1;                   // entry kernels for narrow feature dimensions (-1: by width, 0 never, 1 wherever they can)
     int tile = -1;                      // full-tile kernels (-1: by density and width, 0 never, 1 wherever they can)
+    int wide = -1;                      // wide-tile kernels (-1: by density and expected time, 0 never, 1 wherever they can)
+    int wide_shape = -1;                // their workgroup's shape, an index into the table of hspmm_wide.hip (-1: by expected time)
     int xcd_split = -1;                 // gather kernels: two feature blocks dealt out by XCD half (-1: by matrix, 0 never, 1 always)
     // (set through hspmm_set_panel_stream; builds with HSPMM_EXPERIMENTAL only)
     int panel_tall = 0;                 // LDS-panel waves with two units each
@@ -79,6 +81,8 @@ struct Config {
         if (const char *e = std::getenv("HSPMM_XCD_SPLIT")) xcd_split = std::atoi(e) != 0;
         if (const char *e = std::getenv("HSPMM_ENTRIES")) entries = std::atoi(e) != 0;
         if (const char *e = std::getenv("HSPMM_TILE")) tile = std::atoi(e) != 0;
+        if (const char *e = std::getenv("HSPMM_WIDE")) wide = std::atoi(e) != 0;
+        if (const char *e = std::getenv("HSPMM_WIDE_SHAPE")) wide_shape = std::max(0, std::atoi(e));
         if (const char *e = std::getenv("HSPMM_GATHER_BITMAP")) gather_bitmap = std::atoi(e) != 0;
         if (const char *e = std::getenv("HSPMM_ALIGNED_SMALL")) { const int v = std::atoi(e); aligned_small = v == 4 || v == 8 ? v : 0; }
         if (const char *e = std::getenv("HSPMM_PANEL_UNITS_PER_GROUP")) panel_units_per_group = std::max(1, std::atoi(e));
@@ -191,6 +195,13 @@ struct hspmm_plan {
         uint32_t n_row_blocks = 0, n_blocks = 0;
         uint64_t entries = 0;                                    // stored entries, blocks rounded up to four
     } tile;
+    // The same matrices, 16-bit types, as operands of matrix instructions, for wider feature dimensions (spmm_wide_kernel.hip)
+    struct Wide {
+        bool built = false;
+        const void *d_frags = nullptr;
+        hspmm::TileSource *d_source = nullptr;
+        uint32_t n_units = 0, n_chunks = 0;
+    } wide;
     double per_column = 8.0;            // stored entries per tile column, from a sample of the tiles
     bool even_windows = false;          // no unit has over eight times the average number of steps
     // What launches write besides C, one set per stream that has launched this plan (launches on different
@@ -296,10 +307,18 @@ int run_entries(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t
 
 // hspmm_run.hip: whether the LDS-panel kernels serve feature dimension N
 bool panel_serves(const hspmm_plan *p, uint32_t N);
+// ... and the time that their launch shape is expected to take, in us beyond what every launch does (0: none to be had)
+double panel_expected(const hspmm_plan *p, uint32_t N);
 // hspmm_tile.hip: the full-tile kernels' stream, whether they take this launch, and the launch
 int build_tile_stream(hspmm_plan *p);
 bool tile_serves(const hspmm_plan *p, uint32_t N);
+double tile_expected(const hspmm_plan *p, uint32_t N);          // us
 int run_tile(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode);
+
+// hspmm_wide.hip: the wide-tile kernels' stream, whether they take this launch, and the launch
+int build_wide_stream(hspmm_plan *p);
+bool wide_serves(const hspmm_plan *p, uint32_t N);
+int run_wide(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode);
 
 // hspmm_run.hip: the address of the device's fixed scratch array (hspmm_run_static); `device` must be current
 int static_scratch_address(int device, float **out);

@@ -243,6 +243,7 @@ struct PanelShape {
     size_t acc_per_unit = 0;            // accumulator registers (of four floats per lane) a unit's chunk sums take
     uint32_t mfma_kind = 0;
     uint64_t mfma_count = 0;
+    double expected = 0.0;              // what the shape was chosen by, us
 };
 
 static int choose_panel_shape(const hspmm_plan *p, uint32_t N, PanelShape *out)
@@ -304,6 +305,7 @@ static int choose_panel_shape(const hspmm_plan *p, uint32_t N, PanelShape *out)
             if (best_cost == 0.0 || cost < best_cost) { best_cost = cost; best_units = nc; chunks = ch; }
         }
     }
+    sh.expected = best_cost;
     sh.units = units;
     sh.units_per_group = uint32_t(best_units);
     const uint64_t row_blocks = (uint64_t(wave_units) + best_units - 1) / best_units;
@@ -390,6 +392,12 @@ bool hspmm_host::panel_serves(const hspmm_plan *p, uint32_t N)
     return pays && offsets_fit && (N % block_feat == 0 || ragged_ok);
 }
 
+double hspmm_host::panel_expected(const hspmm_plan *p, uint32_t N)
+{
+    PanelShape sh;
+    return choose_panel_shape(p, N, &sh) == HSPMM_OK ? sh.expected : 0.0;
+}
+
 static int run_gather(hspmm_plan *p, const void *dB, void *dC, uint32_t N, uint32_t ld, hipStream_t s, hipEvent_t mid, RunMode mode);
 
 // One launch (or, kPrepare, everything a launch with this N and these pointer alignments would build): which
@@ -420,6 +428,7 @@ static int run_impl(hspmm_plan *p, const void *dB, void *dC, uint32_t N, void *s
         HSPMM_HIP(hspmm::launch_fill_zero(dC, size_t(p->rows) * N * p->elem, s));
         return HSPMM_OK;
     }
+    if (wide_serves(p, N)) return run_wide(p, dB, dC, N, s, mode);
     if (tile_serves(p, N)) return run_tile(p, dB, dC, N, s, mode);
     if (entries_serve(p, N)) {
         bool taken = false;

@@ -1,0 +1,86 @@
+"""The wide-tile kernels (16-bit types, A as operands of 16 rows x 64 columns) at the sizes where they can go wrong, in each of their
+shapes: rows and columns on both sides of a workgroup's and a chunk's, the last feature tile moved back, infinities and NaNs."""
+import os
+
+import numpy as np
+import pytest
+
+import test_nonfinite_gpu as nonfinite
+from test_spmm_gpu import convert, torch_cuda  # noqa: F401
+from test_tile_gpu import _matrix, _random_operand, _sampled_csr
+from util import decode, encode
+
+pytestmark = pytest.mark.gpu
+
+FEWEST = [32, 32, 64, 32, 64, 64, 64, 128, 128]         # features of a tile, by shape
+
+
+def _plan(hs, A, **env):
+    env = {"HSPMM_" + name: str(value) for name, value in env.items()}
+    os.environ.update(env)
+    try:
+        return hs.Plan(convert(hs, A))
+    finally:
+        for name in env:
+            os.environ.pop(name, None)
+
+
+@pytest.mark.parametrize("shape", range(9))
+@pytest.mark.parametrize("dtype,rows,cols", [(0, 193, 257), (2, 191, 64), (2, 417, 575), (0, 17, 65), (2, 7, 3)])
+def test_exact_sums_in_every_shape(torch_cuda, hs, shape, dtype, rows, cols):
+    torch = torch_cuda
+    rng = np.random.default_rng(100 * rows + shape)
+    D, A = _matrix(rng, rows, cols, 0.1 if cols > 3 else 0.5, dtype)
+    plan = _plan(hs, A, WIDE=1, WIDE_SHAPE=shape)
+    stream = torch.cuda.current_stream().cuda_stream
+    guard, nt = 64, FEWEST[shape]
+    for N in (nt, nt + 1, 2 * nt - 1, 2 * nt, 2 * nt + 8):
+        Bm = rng.integers(-4, 5, (cols, N))
+        want = encode((D @ Bm).astype(np.float32), dtype)
+        dB = torch.from_numpy(encode(Bm.astype(np.float32), dtype).view(np.int16)).cuda()
+        buf = torch.full((rows * N + 2 * guard,), 7, dtype=torch.int16, device="cuda")
+        dC = buf[guard:guard + rows * N]
+        for launch in (plan.run, plan.run_static):
+            dC.fill_(0x7E01)
+            launch(dB.data_ptr(), dC.data_ptr(), N, stream)
+            torch.cuda.synchronize()
+            out = buf.cpu().numpy()
+            assert (out[:guard] == 7).all() and (out[-guard:] == 7).all(), "N=%d: wrote outside C" % N
+            assert np.array_equal(out[guard:-guard].view(np.uint8), want.reshape(-1).view(np.uint8)), "N=%d" % N
+        assert plan.last_kernel() == "spmm_wide_kernel"
+    plan.close()
+
+
+@pytest.mark.parametrize("shape", [0, 6, 7])
+@pytest.mark.parametrize("dtype", [0, 2])
+@pytest.mark.parametrize("rows,cols", [(600, 700), (1100, 130)])
+def test_infinities_and_nans_stay_with_the_rows_that_name_them(torch_cuda, hs, monkeypatch, shape, dtype, rows, cols):
+    """By the rule of the kernels that multiply stored entries only, whose check this is."""
+    monkeypatch.setitem(nonfinite.FAMILIES, "tile", (0, {"HSPMM_WIDE": "1", "HSPMM_WIDE_SHAPE": str(shape)}, (128, 130, 200), "spmm_wide_kernel"))
+    nonfinite.test_infinities_and_nans_stay_with_the_rows_that_name_them(torch_cuda, hs, "tile", dtype, rows, cols)
+
+
+# Against fp64: a product of two 16-bit numbers is exact in fp32 and every addition rounds once, so the sum of n of them is off by no more
+# than n 2^-24 of the sum of their sizes, and the result's own rounding adds 2^-11 (fp16) or 2^-8 (bf16) of it.
+@pytest.mark.parametrize("dtype,rows,cols,per_row,N,kernel", [
+    (2, 5003, 3001, 600, 333, "wide"), (0, 4096, 4096, 409, 256, "wide"), (2, 3840, 1155, 340, 58, "wide"), (0, 4096, 4096, 82, 256, "panel"),
+    (0, 512, 1024, 100, 512, "wide"), (0, 512, 4096, 409, 1024, "panel"), (2, 5120, 2007, 200, 24, "tile"), (1, 4096, 4096, 409, 256, "panel")])
+def test_chosen_where_they_are_faster(torch_cuda, hs, dtype, rows, cols, per_row, N, kernel):
+    torch = torch_cuda
+    rng = np.random.default_rng(N + dtype)
+    A = _sampled_csr(rng, rows, cols, per_row, dtype, lambda n: rng.normal(size=n))
+    plan = hs.Plan(convert(hs, A))
+    B, dB = _random_operand(torch, rng, cols, N, dtype)
+    dC = torch.full((rows, N), 7, dtype=dB.dtype, device="cuda")
+    plan.run(dB.data_ptr(), dC.data_ptr(), N, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert (plan.last_kernel() == "spmm_wide_kernel") == (kernel == "wide")
+    if kernel == "wide":
+        D = np.zeros((rows, cols))
+        D[np.repeat(np.arange(rows), per_row), A["col_idx"]] = decode(A["values"], dtype)
+        Bm = decode(B, dtype).astype(np.float64)
+        bound = per_row * 2.0**-24 * (abs(D) @ abs(Bm))
+        want = D @ Bm
+        off = abs(decode(dC.cpu().numpy().view(np.uint16), dtype).astype(np.float64) - want)
+        assert (off <= bound + (2.0**-11 if dtype == 0 else 2.0**-8) * (abs(want) + bound)).all()
+    plan.close()
