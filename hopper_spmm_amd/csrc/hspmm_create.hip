@@ -762,6 +762,8 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
         }
         if ((rc = build_tile_stream(p))) return bail(rc);
         timer.mark("full-tile stream");
+        if ((rc = build_narrow_stream(p))) return bail(rc);
+        timer.mark("narrow stream");
         if ((rc = build_wide_stream(p))) return bail(rc);
         timer.mark("wide-tile stream");
         if ((rc = entries_counted(p))) return bail(rc);                 // (any stream may launch now)

@@ -182,6 +182,23 @@ struct WideArgs {
 };
 hipError_t launch_spmm_wide(int dtype, const WideArgs &wa, const WideShape &sh, hipStream_t s);
 hipError_t launch_wide_fill(const TileSource &src, uint32_t rows, uint32_t n_chunks, void *frags, hipStream_t s);
+// Narrow kernels (spmm_narrow_kernel.hip, 16-bit types): stored entries by blocks of 16 rows x kNarrowColumns columns
+constexpr uint32_t kNarrowColumns = 128u, kNarrowMostBlocks = 1024u;
+struct NarrowArgs {
+    const uint32_t *blocks;      // per unit of 16 rows and block: its first four entries (n_units x n_blocks + 1)
+    const uint32_t *entries;     // place in the block's image | value << 16
+    const void     *B;
+    void           *C;
+    uint32_t rows, cols, N;
+    uint32_t n_blocks;
+    const TileSource *src;       // in device memory (read where B is not finite)
+};
+// A workgroup of `waves` (4, 8, 16) takes 16 rows; a wave asks for `loads` (1 .. 4) x 128 entries of a block at a time.
+hipError_t launch_spmm_narrow(int dtype, const NarrowArgs &na, uint32_t waves, uint32_t loads, hipStream_t s);
+hipError_t launch_narrow_count(const TileSource &src, uint32_t n_units, uint32_t n_blocks, uint32_t *counts, uint32_t *blocks, hipStream_t s);
+hipError_t launch_narrow_fill(const TileSource &src, uint32_t n_units, uint32_t n_blocks, const uint32_t *counts, const uint32_t *blocks, uint32_t *entries, hipStream_t s);
+// blocks[i]: units of four of counts[0 .. i - 1], every count rounded up (n + 1 of them)
+hipError_t launch_tile_scan(const uint32_t *counts, uint32_t n, uint32_t *blocks, hipStream_t s);
 hipError_t launch_fill_zero(void *dst, size_t bytes, hipStream_t s);
 // bitmap tiles -> plain tiles.  8 x 16 tiles of 16-bit elements: header as KernelArgs::bm_header; 8 x 8 tiles of 32-bit
 // elements: 4 header words per tile - rows 0..3, rows 4..7, position of the first stored element, number of stored elements

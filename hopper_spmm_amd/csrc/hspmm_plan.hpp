@@ -63,6 +63,8 @@ struct Config {
     int gather_bitmap = -1;             // gather kernels read single 16-bit windows as bitmap + stored elements (-1: by fill)
     int entries = -1;                   // entry kernels for narrow feature dimensions (-1: by width, 0 never, 1 wherever they can)
     int tile = -1;                      // full-tile kernels (-1: by density and width, 0 never, 1 wherever they can)
+    int narrow = -1;                    // narrow kernels (-1: by density and expected time, 0 never, 1 wherever they can)
+    int narrow_waves = -1;              // waves of their workgroups (-1: by expected time)
     int wide = -1;                      // wide-tile kernels (-1: by density and expected time, 0 never, 1 wherever they can)
     int wide_shape = -1;                // their workgroup's shape, an index into the table of hspmm_wide.hip (-1: by expected time)
     int xcd_split = -1;                 // gather kernels: two feature blocks dealt out by XCD half (-1: by matrix, 0 never, 1 always)
@@ -81,6 +83,8 @@ struct Config {
         if (const char *e = std::getenv("HSPMM_XCD_SPLIT")) xcd_split = std::atoi(e) != 0;
         if (const char *e = std::getenv("HSPMM_ENTRIES")) entries = std::atoi(e) != 0;
         if (const char *e = std::getenv("HSPMM_TILE")) tile = std::atoi(e) != 0;
+        if (const char *e = std::getenv("HSPMM_NARROW")) narrow = std::atoi(e) != 0;
+        if (const char *e = std::getenv("HSPMM_NARROW_WAVES")) narrow_waves = std::atoi(e);
         if (const char *e = std::getenv("HSPMM_WIDE")) wide = std::atoi(e) != 0;
         if (const char *e = std::getenv("HSPMM_WIDE_SHAPE")) wide_shape = std::max(0, std::atoi(e));
         if (const char *e = std::getenv("HSPMM_GATHER_BITMAP")) gather_bitmap = std::atoi(e) != 0;
@@ -195,6 +199,14 @@ struct hspmm_plan {
         uint32_t n_row_blocks = 0, n_blocks = 0;
         uint64_t entries = 0;                                    // stored entries, blocks rounded up to four
     } tile;
+    // The same matrices, 16-bit types, their stored entries by blocks of 16 rows, for few features (spmm_narrow_kernel.hip)
+    struct Narrow {
+        bool built = false;
+        const uint32_t *d_blocks = nullptr, *d_entries = nullptr;
+        hspmm::TileSource *d_source = nullptr;
+        uint32_t n_units = 0, n_blocks = 0;
+        uint64_t entries = 0;                                    // blocks rounded up to four
+    } narrow;
     // The same matrices, 16-bit types, as operands of matrix instructions, for wider feature dimensions (spmm_wide_kernel.hip)
     struct Wide {
         bool built = false;
@@ -315,9 +327,14 @@ bool tile_serves(const hspmm_plan *p, uint32_t N);
 double tile_expected(const hspmm_plan *p, uint32_t N);          // us
 int run_tile(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode);
 
+// hspmm_narrow.hip: the narrow kernels' stream, whether they take this launch, and the launch
+int build_narrow_stream(hspmm_plan *p);
+bool narrow_serves(const hspmm_plan *p, uint32_t N);
+int run_narrow(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode);
 // hspmm_wide.hip: the wide-tile kernels' stream, whether they take this launch, and the launch
 int build_wide_stream(hspmm_plan *p);
 bool wide_serves(const hspmm_plan *p, uint32_t N);
+double wide_expected(const hspmm_plan *p, uint32_t N);          // us
 int run_wide(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode);
 
 // hspmm_run.hip: the address of the device's fixed scratch array (hspmm_run_static); `device` must be current

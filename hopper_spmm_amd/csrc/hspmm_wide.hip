@@ -80,6 +80,12 @@ int build_wide_stream(hspmm_plan *p)
     return HSPMM_OK;
 }
 
+double wide_expected(const hspmm_plan *p, uint32_t N)
+{
+    double expected = 0.0;
+    return choose_wide_shape(p, N, &expected) ? expected : 0.0;
+}
+
 // Where they are expected to be faster, by 5 % at least, than the kernels that would take the launch.  Launches of the entry kernels stay
 // theirs (at the few features they take from such matrices 1 in 20 would gain), and those of the gather kernels from 32 features on are
 // all taken (of 184, one in eight lost, 13 % at most; 1.35 times as fast on average).  Over 3078 launches the rule gives
@@ -98,7 +104,7 @@ bool wide_serves(const hspmm_plan *p, uint32_t N)
     if (c.wide > 0) return true;
     // (settings of other kernels)
     if (c.buffer_stage || c.consumer_warp_num || c.producer_warp_group_num || c.fused_fixup >= 0 || c.panel_chunks || c.panel_max_windows ||
-        c.panel_units_per_group || c.aligned_small >= 0 || c.xcd_split >= 0 || c.tile > 0 || c.entries > 0)
+        c.panel_units_per_group || c.aligned_small >= 0 || c.xcd_split >= 0 || c.gather_bitmap >= 0 || c.tile > 0 || c.entries > 0)
         return false;
     if (tile_serves(p, N)) return double(p->tile.entries) <= kMostEntries * p->rows * p->cols && expected < 0.95 * tile_expected(p, N);
     if (entries_serve(p, N)) return false;

@@ -29,6 +29,25 @@ __device__ __forceinline__ u32x4 tile_operand(const char *p)
     return b;
 }
 
+// Element types as rows are summed again by.
+template <bool BF> struct HalfStored {
+    static constexpr uint32_t kElem = 2, kPerWord = 2;
+    __device__ static __forceinline__ bool not_finite(uint32_t bits) { return (~bits & (BF ? 0x7F80u : 0x7C00u)) == 0u; }
+    __device__ static __forceinline__ float value(uint32_t bits) { return (float)__builtin_bit_cast(typename HalfOps<BF>::elem_t, uint16_t(bits)); }
+    // element i (of kPerWord) of a word of a tile
+    __device__ static __forceinline__ uint32_t bits(uint32_t word, uint32_t i) { return i ? word >> 16 : word & 0xFFFFu; }
+    __device__ static __forceinline__ uint32_t load_one(const char *p) { return *reinterpret_cast<const uint16_t *>(p); }
+    __device__ static __forceinline__ void store_one(char *p, const float v) { *reinterpret_cast<uint16_t *>(p) = uint16_t(HalfOps<BF>::pack(v, 0.f)); }
+};
+struct FloatStored {
+    static constexpr uint32_t kElem = 4, kPerWord = 1;
+    __device__ static __forceinline__ bool not_finite(uint32_t bits) { return (~bits & 0x7F800000u) == 0u; }
+    __device__ static __forceinline__ float value(uint32_t bits) { return __builtin_bit_cast(float, bits); }
+    __device__ static __forceinline__ uint32_t bits(uint32_t word, uint32_t) { return word; }
+    __device__ static __forceinline__ uint32_t load_one(const char *p) { return *reinterpret_cast<const uint32_t *>(p); }
+    __device__ static __forceinline__ void store_one(char *p, const float v) { *reinterpret_cast<float *>(p) = v; }
+};
+
 // First effective window at or behind `row`.
 __device__ __forceinline__ uint32_t first_window(const uint32_t *rowIdx, uint32_t n_windows, uint32_t row)
 {
@@ -40,11 +59,35 @@ __device__ __forceinline__ uint32_t first_window(const uint32_t *rowIdx, uint32_
     return lo;
 }
 
+// fn(row in the block, column, element number) for every stored element of row block rb; a thread takes a tile column.
+template <class E, class F>
+__device__ __forceinline__ void for_entries(const TileSource &src, uint32_t row0, uint32_t rows, F fn)
+{
+    constexpr uint32_t CW = E::kElem == 4u ? 8u : 16u;
+    const uint32_t w0 = first_window(src.rowIdx, src.n_windows, row0), w1 = first_window(src.rowIdx, src.n_windows, row0 + rows);
+    for (uint32_t w = w0; w < w1; ++w) {
+        const uint32_t m0 = src.rowIdx[w] - row0;
+        const size_t c1 = size_t(src.rowOffset[w + 1u]) * CW;
+        for (size_t c = size_t(src.rowOffset[w]) * CW + threadIdx.x; c < c1; c += blockDim.x) {
+            const uint32_t id = src.a2b[c];
+            if (id == kIdxMax) continue;
+            const size_t first = (c / CW) * (8u * CW) + c % CW;
+#pragma unroll
+            for (uint32_t r = 0; r < 8u; ++r) {
+                const size_t e = first + r * CW;
+                const bool stored = E::kElem == 4u ? static_cast<const uint32_t *>(src.tiles)[e] != 0u : static_cast<const uint16_t *>(src.tiles)[e] != 0u;
+                if (stored) fn(m0 + r, id, e);
+            }
+        }
+    }
+}
+
 // Sums 16 RF rows x WIDTH features of C again, over the stored entries of the plan's tiles alone, where C is not finite: only
 // rows that name a row of B then get what its infinities and NaNs make of them.  Features below `own` belong to another tile.
 // A wave with its lanes on features, 64 / WIDTH tiles of a window at a time, two trips to memory each: slow, and off the path of
 // finite data (bf16, 4096 x 11008 at 10 %, N = 16: 1.0 ms with an infinity in B, 17.3 us without, as before the check).
-template <class E, int RF, uint32_t WIDTH, class Args>
+// FEW: fewer registers, a trip more per row of a tile.
+template <class E, int RF, uint32_t WIDTH, bool FEW = false, class Args>
 __device__ __forceinline__ void tile_sum_again(const Args &ta, const uint32_t row0, const uint32_t f0, const uint32_t own, const uint32_t lane)
 {
     constexpr uint32_t kShares = 64u / WIDTH, CW = E::kElem == 4u ? 8u : 16u;
@@ -73,12 +116,14 @@ __device__ __forceinline__ void tile_sum_again(const Args &ta, const uint32_t ro
         for (uint32_t t = there ? src.rowOffset[w] + share : 0u; t < t1; t += kShares) {
             const u32x4 *ids = reinterpret_cast<const u32x4 *>(src.a2b + size_t(t) * CW);
             const u32x4 *tile = reinterpret_cast<const u32x4 *>(static_cast<const char *>(src.tiles) + size_t(t) * 256u);
-            u32x4 id[CW / 4u], a[16];
+            u32x4 id[CW / 4u], a[FEW ? 2 : 16];
             uint32_t b[CW];
 #pragma unroll
             for (uint32_t k = 0; k < CW / 4u; ++k) id[k] = ids[k];
+            if constexpr (!FEW) {
 #pragma unroll
-            for (uint32_t k = 0; k < 16u; ++k) a[k] = tile[k];
+                for (uint32_t k = 0; k < 16u; ++k) a[k] = tile[k];
+            }
 #pragma unroll
             for (uint32_t k = 0; k < CW; ++k) {
                 const uint32_t at = id[k / 4u][k % 4u];             // (padding: nothing is stored there)
@@ -86,9 +131,10 @@ __device__ __forceinline__ void tile_sum_again(const Args &ta, const uint32_t ro
             }
 #pragma unroll
             for (uint32_t r = 0; r < 8u; ++r) {
+                if constexpr (FEW) { a[0] = tile[2u * r]; a[1] = tile[2u * r + 1u]; }
 #pragma unroll
                 for (uint32_t k = 0; k < CW; ++k) {
-                    const uint32_t word = k / E::kPerWord, x = E::bits(a[2u * r + word / 4u][word % 4u], k % E::kPerWord);
+                    const uint32_t word = k / E::kPerWord, x = E::bits(a[(FEW ? 0u : 2u * r) + word / 4u][word % 4u], k % E::kPerWord);
                     if (x) sum[r] = __builtin_fmaf(E::value(x), E::value(b[k]), sum[r]);
                 }
                 __builtin_amdgcn_sched_barrier(0);                  // (registers: one row's elements at a time)

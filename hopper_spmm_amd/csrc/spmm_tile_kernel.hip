@@ -25,16 +25,10 @@ __device__ __forceinline__ uint32_t tile_position(uint32_t m, uint32_t k)
 
 // Element types.  A block is kK columns; kParts operands of 16 bits per element (fp32 storage: bf16 hi and lo parts, whose
 // images follow one another, see Fp32Split in spmm_panel_kernel.hpp).
-template <bool BF> struct TileHalf {
-    static constexpr uint32_t kK = 64, kParts = 1, kElem = 2;
+template <bool BF> struct TileHalf : HalfStored<BF> {
+    static constexpr uint32_t kK = 64, kParts = 1;
     typedef t_u32x2 Vals;                                   // four values
     typedef uint16_t Stored;
-    __device__ static __forceinline__ bool not_finite(uint32_t bits) { return (~bits & (BF ? 0x7F80u : 0x7C00u)) == 0u; }
-    __device__ static __forceinline__ float value(uint32_t bits) { return (float)__builtin_bit_cast(typename HalfOps<BF>::elem_t, uint16_t(bits)); }
-    // element i (of 2) of a word of a tile
-    static constexpr uint32_t kPerWord = 2;
-    __device__ static __forceinline__ uint32_t bits(uint32_t word, uint32_t i) { return i ? word >> 16 : word & 0xFFFFu; }
-    __device__ static __forceinline__ uint32_t load_one(const char *p) { return *reinterpret_cast<const uint16_t *>(p); }
     __device__ static __forceinline__ Stored stored(const void *tiles, size_t i) { return static_cast<const uint16_t *>(tiles)[i]; }
     __device__ static __forceinline__ void scatter(char *img, const uint32_t (&at)[4], const Vals v)
     {
@@ -68,15 +62,10 @@ template <bool BF> struct TileHalf {
 template <bool BF> template <int NT, uint32_t PITCH>
 __device__ __forceinline__ typename TileHalf<BF>::B TileHalf<BF>::read_b(const char *p) { return {tile_operand<PITCH>(p)}; }
 
-struct TileSplit {
-    static constexpr uint32_t kK = 32, kParts = 2, kElem = 4;
+struct TileSplit : FloatStored {
+    static constexpr uint32_t kK = 32, kParts = 2;
     typedef u32x4 Vals;                                     // four values: hi half | lo half << 16
     typedef uint32_t Stored;
-    __device__ static __forceinline__ bool not_finite(uint32_t bits) { return (~bits & 0x7F800000u) == 0u; }
-    __device__ static __forceinline__ float value(uint32_t bits) { return __builtin_bit_cast(float, bits); }
-    static constexpr uint32_t kPerWord = 1;
-    __device__ static __forceinline__ uint32_t bits(uint32_t word, uint32_t) { return word; }
-    __device__ static __forceinline__ uint32_t load_one(const char *p) { return *reinterpret_cast<const uint32_t *>(p); }
     __device__ static __forceinline__ Stored stored(const void *tiles, size_t i)
     {
         const uint32_t v = static_cast<const uint32_t *>(tiles)[i];
@@ -121,7 +110,6 @@ struct TileSplit {
         typedef f32x4 f32x4_any __attribute__((aligned(4)));
         *reinterpret_cast<f32x4_any *>(p) = v;
     }
-    __device__ static __forceinline__ void store_one(char *p, const float v) { *reinterpret_cast<float *>(p) = v; }
 };
 
 // 16 bytes from `back` (< 16) bytes further on in the 16 loaded, zeros behind them.
@@ -436,29 +424,6 @@ hipError_t launch_spmm_tile(int dtype, const TileArgs &ta, uint32_t nt, uint32_t
 // The entry stream from the plan's tiles: a workgroup per row block, whose tiles follow one another.
 // ---------------------------------------------------------------------------
 
-// fn(row in the block, column, element number) for every stored element of row block rb; a thread takes a tile column.
-template <class E, class F>
-__device__ __forceinline__ void for_entries(const TileSource &src, uint32_t rb, F fn)
-{
-    constexpr uint32_t CW = E::kElem == 4u ? 8u : 16u;
-    const uint32_t w0 = first_window(src.rowIdx, src.n_windows, rb * kTileRows), w1 = first_window(src.rowIdx, src.n_windows, (rb + 1u) * kTileRows);
-    for (uint32_t w = w0; w < w1; ++w) {
-        const uint32_t m0 = src.rowIdx[w] - rb * kTileRows;
-        const size_t c1 = size_t(src.rowOffset[w + 1u]) * CW;
-        for (size_t c = size_t(src.rowOffset[w]) * CW + threadIdx.x; c < c1; c += blockDim.x) {
-            const uint32_t id = src.a2b[c];
-            if (id == kIdxMax) continue;
-            const size_t first = (c / CW) * (8u * CW) + c % CW;
-#pragma unroll
-            for (uint32_t r = 0; r < 8u; ++r) {
-                const size_t e = first + r * CW;
-                const bool stored = E::kElem == 4u ? static_cast<const uint32_t *>(src.tiles)[e] != 0u : static_cast<const uint16_t *>(src.tiles)[e] != 0u;
-                if (stored) fn(m0 + r, id, e);
-            }
-        }
-    }
-}
-
 // counts[row block][block]: stored entries
 template <class E>
 __global__ __launch_bounds__(256) void tile_count_kernel(const TileSource src, uint32_t n_blocks, uint32_t *__restrict__ counts)
@@ -466,7 +431,7 @@ __global__ __launch_bounds__(256) void tile_count_kernel(const TileSource src, u
     __shared__ uint32_t seen[kTileMaxBlocks];
     for (uint32_t i = threadIdx.x; i < n_blocks; i += 256u) seen[i] = 0u;
     __syncthreads();
-    for_entries<E>(src, blockIdx.x, [&](uint32_t, uint32_t id, size_t) { atomicAdd(&seen[id / E::kK], 1u); });
+    for_entries<E>(src, blockIdx.x * kTileRows, kTileRows, [&](uint32_t, uint32_t id, size_t) { atomicAdd(&seen[id / E::kK], 1u); });
     __syncthreads();
     for (uint32_t i = threadIdx.x; i < n_blocks; i += 256u) counts[size_t(blockIdx.x) * n_blocks + i] = seen[i];
 }
@@ -501,7 +466,7 @@ __global__ __launch_bounds__(256) void tile_fill_kernel(const TileSource src, ui
     for (uint32_t i = threadIdx.x; i < n_blocks; i += 256u) next[i] = 0u;
     __syncthreads();
     const size_t base = size_t(blockIdx.x) * n_blocks;
-    for_entries<E>(src, blockIdx.x, [&](uint32_t m, uint32_t id, size_t e) {
+    for_entries<E>(src, blockIdx.x * kTileRows, kTileRows, [&](uint32_t m, uint32_t id, size_t e) {
         const uint32_t b = id / E::kK, p = atomicAdd(&next[b], 1u), n = counts[base + b];
         const uint16_t where = uint16_t(tile_position(m, id - tile_first_column(b, E::kK, src.cols)));
         const typename E::Stored v = E::stored(src.tiles, e);
@@ -513,13 +478,19 @@ __global__ __launch_bounds__(256) void tile_fill_kernel(const TileSource src, ui
     });
 }
 
+hipError_t launch_tile_scan(const uint32_t *counts, uint32_t n, uint32_t *blocks, hipStream_t s)
+{
+    tile_scan_kernel<<<dim3(1), 1024, 0, s>>>(counts, n, blocks);
+    return hipGetLastError();
+}
+
 hipError_t launch_tile_count(int dtype, const TileSource &src, uint32_t n_row_blocks, uint32_t n_blocks, uint32_t *counts, uint32_t *blocks, hipStream_t s)
 {
     if (n_blocks > kTileMaxBlocks || !n_row_blocks) return hipErrorInvalidValue;
     if (dtype == kDtypeF32) tile_count_kernel<TileSplit><<<dim3(n_row_blocks), 256, 0, s>>>(src, n_blocks, counts);
     else tile_count_kernel<TileHalf<false>><<<dim3(n_row_blocks), 256, 0, s>>>(src, n_blocks, counts);
-    tile_scan_kernel<<<dim3(1), 1024, 0, s>>>(counts, n_row_blocks * n_blocks, blocks);
-    return hipGetLastError();
+    if (hipError_t e = hipGetLastError()) return e;
+    return launch_tile_scan(counts, n_row_blocks * n_blocks, blocks, s);
 }
 
 hipError_t launch_tile_fill(int dtype, const TileSource &src, uint32_t n_row_blocks, uint32_t n_blocks, const uint32_t *counts,

@@ -25,13 +25,7 @@ __device__ __forceinline__ u32x8 wide_operand(const char *p)
 }
 
 // Element types.
-template <bool BF> struct WideHalf {
-    static constexpr uint32_t kElem = 2, kPerWord = 2;
-    __device__ static __forceinline__ bool not_finite(uint32_t bits) { return (~bits & (BF ? 0x7F80u : 0x7C00u)) == 0u; }
-    __device__ static __forceinline__ float value(uint32_t bits) { return (float)__builtin_bit_cast(typename HalfOps<BF>::elem_t, uint16_t(bits)); }
-    __device__ static __forceinline__ uint32_t bits(uint32_t word, uint32_t i) { return i ? word >> 16 : word & 0xFFFFu; }
-    __device__ static __forceinline__ uint32_t load_one(const char *p) { return *reinterpret_cast<const uint16_t *>(p); }
-    __device__ static __forceinline__ void store_one(char *p, const float v) { *reinterpret_cast<uint16_t *>(p) = uint16_t(HalfOps<BF>::pack(v, 0.f)); }
+template <bool BF> struct WideHalf : HalfStored<BF> {
     struct A { u32x4 f[2]; };                               // 16 rows x 64 columns
     __device__ static __forceinline__ void load_a(A &a, const char *src, uint32_t lane)
     {
