@@ -124,6 +124,7 @@ struct EntryArgs {
     void           *C;
     uint32_t ld;                 // elements from one row of B (and of C) to the next
     uint32_t block_bytes, n_feat_blocks, xcd_split;  // bytes of a row one subgroup covers; blocks side by side; != 0: on XCDs of their own
+    uint32_t odd, last_row;      // != 0: rows begin between two words, B begins on one (see spmm_entries_kernel); B's last row
     uint32_t n_groups;           // workgroups of one block
     uint32_t n_pieces, n_classes;
     EntryClass cls[kEntryClasses];   // pieces first where there are any, then from the longest rows to the empty ones

@@ -138,10 +138,13 @@ static bool entries_by_xcd(const hspmm_plan *p, uint64_t row_bytes)
            uint64_t(p->cols) * row_bytes >= (uint64_t(8) << 20);
 }
 
-// Bytes of a block: whole 16-byte pieces (the last block is moved back to end with the row).
+// Bytes of a block: whole 16-byte pieces, of an odd number of 16-bit elements pieces and 14 bytes (the last block is moved back to end
+// with the row).
 static uint32_t entry_block_bytes(uint32_t row_bytes, uint32_t blocks)
 {
-    return blocks == 1u ? row_bytes : ((row_bytes + blocks - 1u) / blocks + 15u) & ~15u;
+    if (blocks == 1u) return row_bytes;
+    const uint32_t bytes = (row_bytes + blocks - 1u) / blocks;
+    return row_bytes % 4u == 2u ? ((bytes + 1u) & ~15u) + 14u : (bytes + 15u) & ~15u;
 }
 
 // Lines of 128 bytes that `bytes` bytes from byte `off` of a row touch: the mean over rows that begin on multiples of `step`.
@@ -320,6 +323,8 @@ int run_entries(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t
     if (mode == RunMode::kPrepare) return HSPMM_OK;
     ea.desc = e.d_desc; ea.ids = e.d_ids; ea.vals = e.d_vals; ea.pieces = e.d_pieces;
     ea.B = dB; ea.C = dC; ea.ld = N; ea.block_bytes = block_bytes; ea.n_feat_blocks = blocks; ea.xcd_split = by_xcd;
+    ea.last_row = p->cols - 1u;
+    ea.odd = row_bytes % 4u == 2u && row_bytes >= 18u && ea.last_row && reinterpret_cast<uintptr_t>(dB) % 4u == 0u;
     p->note_launch("spmm_entries_kernel", 2, 0, 0);
     HSPMM_HIP(hspmm::launch_spmm_entries(p->dtype, ea, share.lane_bytes, share.lanes, s));
     return HSPMM_OK;

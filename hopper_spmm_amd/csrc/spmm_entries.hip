@@ -115,7 +115,12 @@ __device__ __forceinline__ Piece<VB> round_sums(const float (&acc)[NF])
 // (counted, us / requests under way / L2 hits: graph of 2^18, bf16, N = 16 26.4 / 79 / 82 %; of 150001, fp32, N = 100 91 / 72 /
 // 59 %; of 500000, fp16, N = 1 23.7 / 74 / 89 %; uniform 65536^2, N = 128 28.5 / 85 / 41 %, 6.3 TB/s past the L2s).  A launch as
 // short as 4096^2 at 1 %, N = 64 - 4.5 us, 22 under way - is its chain of descriptor, ids, rows and sums.
-template <class E, int VB, int L, int U, bool Cut>
+// Odd: 16-bit types with an odd number of elements in a row of B, whose every other row starts between two words, and loads that
+// are not whole words take twice their time (graph of 2^18, fp16, N = 65 / 66: 109 / 73 us).  Such a row is loaded from the word before on and
+// shifted by half a word, the word behind a lane's last one being its neighbour's first; the last lane of a block has seven features,
+// which the load holds either way.  Before / with it, us: that graph, N = 33 59.4 / 50.6, 65 109 / 75.5, 129 225 / 174; of 40001, N = 33 12.1 /
+// 10.3; uniform 16384^2, 64 per row, N = 17 13.9 / 10.7, 65 28.4 / 21.0, 129 50.1 / 31.5.
+template <class E, int VB, int L, int U, bool Cut, bool Odd>
 __global__ __launch_bounds__(256)
 void spmm_entries_kernel(const EntryArgs ea)
 {
@@ -154,13 +159,31 @@ void spmm_entries_kernel(const EntryArgs ea)
 
     // bytes of a row this block covers, and where: a last block that would reach past the row is moved back to end with it
     const uint32_t row_len = ea.block_bytes;
-    const uint32_t off = lane * VB + VB <= row_len ? lane * VB : row_len - VB;
+    static_assert(!Odd || (VB == 16 && E::kElem == 2), "16 bytes of 16-bit elements");
+    const bool last = lane * VB + VB > row_len;
+    const uint32_t off = !last ? lane * VB : row_len - (Odd ? 14u : VB);
     const size_t pitch = size_t(ea.ld) * E::kElem;
     const size_t block = umin_e(fb * row_len, uint32_t(pitch) - row_len);
     const char *B = reinterpret_cast<const char *>(ea.B) + block + off;
     const uint32_t *ids = ea.ids + size_t(first) * 4u;
     const typename E::Vals *vals = reinterpret_cast<const typename E::Vals *>(ea.vals) + first;
 
+    // A row's piece, and whether it begins half a word into what is loaded.  (The last row of B always does, so that nothing behind
+    // B is read: where that row does begin on a word, the load is the one that does not.)
+    const uint32_t flip = uint32_t(block) >> 1;
+    auto load = [&](Piece<VB> &b, uint32_t id) __attribute__((always_inline)) {
+        const uint32_t odd = Odd ? ((id + (id == ea.last_row ? 1u - (id & 1u) : 0u)) ^ flip) & 1u : 0u;
+        b.load(B + size_t(id) * pitch - odd * 2u);
+        return odd;
+    };
+    auto shift = [&](Piece<VB> &b, uint32_t odd) __attribute__((always_inline)) {
+        if constexpr (Odd) {
+            const uint32_t next = uint32_t(__builtin_amdgcn_mov_dpp(int(b.w[0]), 0x130, 0xF, 0xF, true)), by = odd * 16u;      // (the next lane's)
+#pragma unroll
+            for (int i = 0; i < 3; ++i) b.w[i] = __builtin_amdgcn_alignbit(b.w[i + 1], b.w[i], by);
+            b.w[3] = __builtin_amdgcn_alignbit(next, b.w[3], by);
+        }
+    };
     float acc[NF];
 #pragma unroll
     for (int i = 0; i < NF; ++i) acc[i] = 0.f;
@@ -181,12 +204,13 @@ void spmm_entries_kernel(const EntryArgs ea)
         for (;;) {
             Piece<VB> b[4 * U];
             typename E::Vals now[U];
+            uint32_t odds = 0;                              // a bit a row
 #pragma unroll
             for (int k = 0; k < U; ++k) {
                 now[k] = v[k];
                 if (k == 0 || u + uint32_t(k) * g < units) {
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) b[4 * k + i].load(B + size_t(id[k][i]) * pitch);
+                    for (int i = 0; i < 4; ++i) odds |= load(b[4 * k + i], id[k][i]) << (4 * k + i);
                 }
             }
             const uint32_t next = u + uint32_t(U) * g;
@@ -195,7 +219,10 @@ void spmm_entries_kernel(const EntryArgs ea)
             for (int k = 0; k < U; ++k)
                 if (k == 0 || u + uint32_t(k) * g < units) {
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) multiply_in<E, VB, NF>(acc, b[4 * k + i], E::value(now[k], i));
+                    for (int i = 0; i < 4; ++i) {
+                        shift(b[4 * k + i], odds >> (4 * k + i) & 1u);
+                        multiply_in<E, VB, NF>(acc, b[4 * k + i], E::value(now[k], i));
+                    }
                 }
             if (next >= units) break;
             u = next;
@@ -203,9 +230,12 @@ void spmm_entries_kernel(const EntryArgs ea)
         // What fills a row's last unit up (+0, which no stored value is, at the row's last column) counts for nothing, unless that
         // row of B is not finite there: then once more, the stored entries alone, in the same order.
         float met = 0.f;
+        if (Odd && last) acc[NF - 1] = 0.f;                 // (no feature)
 #pragma unroll
         for (int i = 0; i < NF; ++i) met = __builtin_fmaf(acc[i], 0.f, met);
-        if (met != 0.f) {
+        bool again = met != 0.f;
+        if constexpr (Odd) again = (__ballot(again) >> ((threadIdx.x & 63u) - lane)) & ((uint64_t(1) << L) - 1u);    // (lanes need their neighbours)
+        if (again) {
 #pragma unroll
             for (int i = 0; i < NF; ++i) acc[i] = 0.f;
             for (u = member; u < units; u += g) {
@@ -215,7 +245,8 @@ void spmm_entries_kernel(const EntryArgs ea)
                 for (int i = 0; i < 4; ++i)
                     if (E::stored(a, i)) {
                         Piece<VB> b;
-                        b.load(B + size_t(at[i]) * pitch);
+                        const uint32_t odd = load(b, at[i]);
+                        shift(b, odd);
                         multiply_in<E, VB, NF>(acc, b, E::value(a, i));
                     }
             }
@@ -275,7 +306,19 @@ void spmm_entries_kernel(const EntryArgs ea)
         if (lane == 0u) __hip_atomic_store(ea.arrive + size_t(head) * ea.n_feat_blocks + fb, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     if (lane * VB >= row_len) return;                       // (a lane behind the row's end: its neighbour's copy)
-    round_sums<E, VB, NF>(acc).store(reinterpret_cast<char *>(ea.C) + size_t(row_out) * pitch + block + off);
+    const Piece<VB> out = round_sums<E, VB, NF>(acc);
+    char *c_row = reinterpret_cast<char *>(ea.C) + size_t(row_out) * pitch + block + off;
+    if constexpr (Odd) {
+        if (last) {
+            Piece<8> front;
+            Piece<4> behind;
+            Piece<2> end;
+            front.w[0] = out.w[0]; front.w[1] = out.w[1]; behind.w[0] = out.w[2]; end.w[0] = out.w[3];
+            front.store(c_row); behind.store(c_row + 8); end.store(c_row + 12);
+            return;
+        }
+    }
+    out.store(c_row);
 }
 
 template <class E, bool Cut>
@@ -284,8 +327,11 @@ static hipError_t launch_entries_e(const EntryArgs &ea, uint32_t lane_bytes, uin
     const uint32_t sets = ea.xcd_split ? 8u / ea.n_feat_blocks : 1u;      // workgroups of one feature block in a round over the XCDs
     const uint32_t grid = ea.xcd_split ? 8u * ((ea.n_groups + sets - 1u) / sets) : ea.n_groups * ea.n_feat_blocks;
 #define HSPMM_ENTRIES(VB, L) \
-    if (lane_bytes == VB && lanes == L) { spmm_entries_kernel<E, VB, L, (E::kElem == 2 && VB * L <= 128) ? 2 : 1, Cut><<<dim3(grid), 256, 0, s>>>(ea); return hipGetLastError(); }
-    if constexpr (E::kElem == 2) { HSPMM_ENTRIES(2, 1) }
+    if (lane_bytes == VB && lanes == L) { spmm_entries_kernel<E, VB, L, (E::kElem == 2 && VB * L <= 128) ? 2 : 1, Cut, false><<<dim3(grid), 256, 0, s>>>(ea); return hipGetLastError(); }
+#define HSPMM_ENTRIES_ODD(L) \
+    if (ea.odd && lane_bytes == 16u && lanes == L) { spmm_entries_kernel<E, 16, L, L <= 8 ? 2 : 1, Cut, true><<<dim3(grid), 256, 0, s>>>(ea); return hipGetLastError(); }
+    if constexpr (E::kElem == 2) { HSPMM_ENTRIES_ODD(2) HSPMM_ENTRIES_ODD(4) HSPMM_ENTRIES_ODD(8) HSPMM_ENTRIES_ODD(16) HSPMM_ENTRIES_ODD(32) HSPMM_ENTRIES(2, 1) }
+#undef HSPMM_ENTRIES_ODD
     HSPMM_ENTRIES(4, 1) HSPMM_ENTRIES(4, 2) HSPMM_ENTRIES(8, 1) HSPMM_ENTRIES(8, 2)
     HSPMM_ENTRIES(16, 1) HSPMM_ENTRIES(16, 2) HSPMM_ENTRIES(16, 4) HSPMM_ENTRIES(16, 8) HSPMM_ENTRIES(16, 16) HSPMM_ENTRIES(16, 32)
 #undef HSPMM_ENTRIES
@@ -299,6 +345,10 @@ hipError_t launch_spmm_entries(int dtype, const EntryArgs &ea, uint32_t lane_byt
     // (a lane's load stays inside its block, a block inside the row, and the lanes reach over the block)
     if (ea.block_bytes < lane_bytes || ea.block_bytes > lane_bytes * lanes || ea.n_feat_blocks < 1u ||
         uint64_t(ea.ld) * (dtype == kDtypeF32 ? 4u : 2u) < ea.block_bytes || uint64_t(ea.n_groups) * ea.n_feat_blocks >= kEntryMostGroups)
+        return hipErrorInvalidValue;
+    // (rows of an odd number of 16-bit elements, B on a word, two of its rows at least, a block's last lane seven features)
+    if (ea.odd && (dtype == kDtypeF32 || ea.ld % 2u == 0u || ea.block_bytes % 4u != 2u || ea.block_bytes < 18u || reinterpret_cast<uintptr_t>(ea.B) % 4u || !ea.last_row ||
+                   (ea.n_feat_blocks > 1u && ea.block_bytes % 16u != 14u)))
         return hipErrorInvalidValue;
     bool cut = false;
     for (uint32_t c = 0; c < ea.n_classes; ++c) cut |= (ea.cls[c].logs >> 8) != 0u;
