@@ -174,11 +174,13 @@ constexpr uint32_t kWideUnitBytes = 2048u;
 // A workgroup: `splits` sets of `rows` waves with `units` x 16 rows each, `blocks` x 16 features.
 struct WideShape { uint32_t units, blocks, rows, splits; };
 struct WideArgs {
-    const void     *frags;       // per unit of 16 rows and chunk of 64 columns kWideUnitBytes
+    const void     *frags;       // per chunk of 64 columns and unit of 16 rows kWideUnitBytes
     const void     *B;
     void           *C;
     uint32_t rows, cols, N;
     uint32_t n_units, n_chunks, n_feat_tiles;                    // chunks: a multiple of four
+    uint32_t n_cuts;             // workgroups of a C tile, each with a part of the chunks
+    float *sums;                 // of more than one: their sums, wide_sums_bytes() of them
     const TileSource *src;       // in device memory (read where B is not finite)
 };
 hipError_t launch_spmm_wide(int dtype, const WideArgs &wa, const WideShape &sh, hipStream_t s);

@@ -38,14 +38,6 @@ uint32_t choose_waves(const hspmm_plan *p, uint32_t N, double *expected)
     return best;
 }
 
-// What the entry kernels take for pruned weights of 16 bits, us: a fit to 1993 launches (standard deviation 9 to 25 %).  Rows of up to eight
-// features that begin between two words cost them up to twice as much, longer ones a tenth more.
-double entries_expected(const hspmm_plan *p, uint32_t N)
-{
-    const double odd = N % 2u == 0u ? 1.0 : N == 1u ? 0.9 : N <= 8u ? 1.6 : 1.1;
-    return 3.9 + (N <= 8u ? 1.9 : N <= 16u ? 3.3 : 5.3) * odd * 1e-6 * double(p->narrow.entries);
-}
-
 }  // namespace
 
 namespace hspmm_host {

@@ -66,6 +66,7 @@ struct Config {
     int narrow = -1;                    // narrow kernels (-1: by density and expected time, 0 never, 1 wherever they can)
     int narrow_waves = -1;              // waves of their workgroups (-1: by expected time)
     int wide = -1;                      // wide-tile kernels (-1: by density and expected time, 0 never, 1 wherever they can)
+    int wide_cuts = -1;                 // workgroups of a C tile (-1: by expected time)
     int wide_shape = -1;                // their workgroup's shape, an index into the table of hspmm_wide.hip (-1: by expected time)
     int xcd_split = -1;                 // gather kernels: two feature blocks dealt out by XCD half (-1: by matrix, 0 never, 1 always)
     // (set through hspmm_set_panel_stream; builds with HSPMM_EXPERIMENTAL only)
@@ -87,6 +88,7 @@ struct Config {
         if (const char *e = std::getenv("HSPMM_NARROW_WAVES")) narrow_waves = std::atoi(e);
         if (const char *e = std::getenv("HSPMM_WIDE")) wide = std::atoi(e) != 0;
         if (const char *e = std::getenv("HSPMM_WIDE_SHAPE")) wide_shape = std::max(0, std::atoi(e));
+        if (const char *e = std::getenv("HSPMM_WIDE_CUTS")) wide_cuts = std::max(0, std::atoi(e));
         if (const char *e = std::getenv("HSPMM_GATHER_BITMAP")) gather_bitmap = std::atoi(e) != 0;
         if (const char *e = std::getenv("HSPMM_ALIGNED_SMALL")) { const int v = std::atoi(e); aligned_small = v == 4 || v == 8 ? v : 0; }
         if (const char *e = std::getenv("HSPMM_PANEL_UNITS_PER_GROUP")) panel_units_per_group = std::max(1, std::atoi(e));
@@ -213,6 +215,7 @@ struct hspmm_plan {
         const void *d_frags = nullptr;
         hspmm::TileSource *d_source = nullptr;
         uint32_t n_units = 0, n_chunks = 0;
+        mutable std::atomic<uint64_t> choice{0};                 // of the last N asked for (see hspmm_wide.hip)
     } wide;
     double per_column = 8.0;            // stored entries per tile column, from a sample of the tiles
     bool even_windows = false;          // no unit has over eight times the average number of steps
@@ -315,6 +318,7 @@ size_t entries_count_bytes(const hspmm_plan *p);
 int count_entries(hspmm_plan *p);
 int entries_counted(hspmm_plan *p);
 bool entries_serve(const hspmm_plan *p, uint32_t N);
+double entries_expected(const hspmm_plan *p, uint32_t N);       // us, pruned weights of 16 bits, fewer than 256 features
 int run_entries(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode, bool *taken);
 
 // hspmm_run.hip: whether the LDS-panel kernels serve feature dimension N

@@ -108,11 +108,13 @@ bool tile_serves(const hspmm_plan *p, uint32_t N)
     return N >= 8u && N < (wide ? 48u : 128u) && work >= (wide ? 75e6 : 65e6) && fill >= 0.04 && fill * N >= 1.5;
 }
 
-// 16-bit types, from 32 features on: a fit to 447 launches (standard deviation 21 %).
+// 16-bit types, from 32 features on: a fit to 1233 launches (standard deviation 10 to 18 %).  33 to 63 features, which leave a C tile of 64
+// ragged, take one and a half times as long.
 double tile_expected(const hspmm_plan *p, uint32_t N)
 {
+    const double ragged = N > 32u && N < 64u ? 1.5 : 1.0;
     const double chunks = double(p->tile.n_row_blocks) * p->tile.n_blocks / p->compute_units, tiles = double((N + 63u) / 64u);
-    return 13.3 + (N <= 32u ? 0.14 : 0.49) * chunks * tiles + 0.29e-6 * double(p->tile.entries) * tiles;
+    return ragged * (13.3 + (N <= 32u ? 0.14 : 0.49) * chunks * tiles + 0.29e-6 * double(p->tile.entries) * tiles);
 }
 
 int run_tile(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode)

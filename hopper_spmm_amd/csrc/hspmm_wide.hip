@@ -1,32 +1,36 @@
 // Host side of the wide-tile kernels (spmm_wide_kernel.hip): which plans carry their stream, which launches they take and in which
 // shape, the launch.
 #include "hspmm_plan.hpp"
+#include <cmath>
 
 using namespace hspmm_host;
 
 namespace {
 
-// A launch takes `start` us and `chunk[i]` us for every chunk of 64 columns and round of workgroups, one of them per compute unit and
-// round - a second one on a compute unit takes its time on top -; i: rows of B of whole 128-byte lines, of whole 16-byte pieces, of
-// whole words, any.  A fit to 3078 launches of 560 pruned matrices of 1024 to 16384 rows and columns at 2 to 31 %, N = 32 to 1024, every
-// shape measured: standard deviations of 3 to 7 % (the first: 12 %), and the shape it picks is 0.3 % behind the fastest on
-// average, 2.5 % at the 95th percentile.  Seven more shapes were measured and are the fastest of no launch, or by little.
-struct ShapeCost { hspmm::WideShape shape; double start, chunk[4]; };
+// A launch takes `start` us and `chunk[i]` us for every chunk of 64 columns of a workgroup and round of workgroups, one of them per
+// compute unit and round - a second one on a compute unit takes its time on top -; i: rows of B of whole 128-byte lines, of whole
+// 16-byte pieces, of whole words, any.  Where C tiles are cut, `cut` us and what is below, too.  A fit to 50153 launches of 395 matrices of
+// 64 to 16384 rows and 1024 to 16384 columns, N = 32 to 1024, every shape with one to 16 cuts: standard deviations of 5 to 9 %, and the
+// launch it picks is 1.3 % behind the fastest on average, 8 % at the 95th percentile.  Seven more shapes were measured and are
+// the fastest of no launch, or by little.
+struct ShapeCost { hspmm::WideShape shape; double start, chunk[4], cut; };
 const ShapeCost kShapes[] = {
-    {{1, 2, 2, 4}, 3.9, {0.118, 0.123, 0.135, 0.143}},       //  32 rows x  32 features
-    {{1, 2, 4, 2}, 3.9, {0.159, 0.163, 0.172, 0.178}},       //  64 x  32
-    {{1, 4, 4, 2}, 4.2, {0.191, 0.205, 0.214, 0.239}},       //  64 x  64
-    {{2, 2, 4, 2}, 3.7, {0.241, 0.244, 0.261, 0.271}},       // 128 x  32
-    {{2, 4, 4, 2}, 4.7, {0.273, 0.305, 0.315, 0.350}},       // 128 x  64
-    {{3, 4, 2, 4}, 6.6, {0.237, 0.261, 0.273, 0.298}},       //  96 x  64
-    {{3, 4, 4, 2}, 6.1, {0.355, 0.386, 0.396, 0.433}},       // 192 x  64
-    {{2, 8, 4, 2}, 7.7, {0.431, 0.434, 0.439, 0.529}},       // 128 x 128
-    {{3, 8, 4, 2}, 9.9, {0.550, 0.552, 0.555, 0.619}},       // 192 x 128
+    {{1, 2, 2, 4}, 3.5, {0.112, 0.115, 0.122, 0.135}, 2.2},       //  32 rows x  32 features
+    {{1, 2, 4, 2}, 3.7, {0.158, 0.162, 0.168, 0.178}, 1.8},       //  64 x  32
+    {{1, 4, 4, 2}, 4.2, {0.201, 0.212, 0.223, 0.247}, 1.6},       //  64 x  64
+    {{2, 2, 4, 2}, 4.2, {0.236, 0.237, 0.248, 0.257}, 1.4},       // 128 x  32
+    {{2, 4, 4, 2}, 5.0, {0.284, 0.305, 0.316, 0.343}, 1.0},       // 128 x  64
+    {{3, 4, 2, 4}, 6.7, {0.253, 0.273, 0.286, 0.308}, 0.6},       //  96 x  64
+    {{3, 4, 4, 2}, 6.1, {0.369, 0.391, 0.408, 0.432}, 0.1},       // 192 x  64
+    {{2, 8, 4, 2}, 6.6, {0.462, 0.459, 0.461, 0.518}, 0.0},       // 128 x 128
+    {{3, 8, 4, 2}, 6.9, {0.605, 0.598, 0.600, 0.638}, 0.0},       // 192 x 128
 };
-constexpr uint32_t kShapeCount = sizeof kShapes / sizeof kShapes[0], kFewestFeatures = 32u;
+constexpr double kPerCut = 0.1, kPerSumsByte = 0.34e-6;           // us
+// Streams from 75 MB on: three matrices in turn no longer share the memory-side cache of 256 MB (100 MB: 8 us more).
+constexpr double kLargeStream = 75e6;
+constexpr uint32_t kShapeCount = sizeof kShapes / sizeof kShapes[0], kFewestFeatures = 32u, kMostCuts = 16u;
 constexpr size_t kMostBytes = size_t(8) << 30;             // 64k x 64k
-constexpr double kMostEntries = 0.31, kShort = 11.0;        // us
-constexpr uint32_t kFewRows = 1024u;
+constexpr double kMostEntries = 0.31;
 
 uint64_t workgroups(const hspmm_plan *p, uint32_t N, const hspmm::WideShape &s)
 {
@@ -34,20 +38,73 @@ uint64_t workgroups(const hspmm_plan *p, uint32_t N, const hspmm::WideShape &s)
     return (p->rows + rows - 1u) / rows * ((N + features - 1u) / features);
 }
 
-// The shape of a launch, a function of the plan and N alone, and the time it is expected to take.
-const ShapeCost *choose_wide_shape(const hspmm_plan *p, uint32_t N, double *expected)
+// fp32 sums of a C tile
+uint64_t tile_sums_bytes(const hspmm::WideShape &s) { return uint64_t(s.units) * s.rows * s.blocks * 1024u; }
+
+// The shape of a launch and the workgroups of a C tile, a function of the plan and N alone, and the time it is expected to take.
+struct WideChoice { const ShapeCost *cost = nullptr; uint32_t cuts = 1; double expected = 0.0; };        // (cuts: below 256)
+WideChoice choose_wide_shape(const hspmm_plan *p, uint32_t N)
 {
     const uint64_t row_bytes = uint64_t(N) * p->elem, cu = uint64_t(p->compute_units);
     const int i = row_bytes % 128u == 0 ? 0 : row_bytes % 16u == 0 ? 1 : row_bytes % 4u == 0 ? 2 : 3;
-    const ShapeCost *best = nullptr;
+    const double stream = 2.0 * p->rows * p->cols, large = std::min(std::max((stream - kLargeStream) / 25e6, 0.0), 1.5) * 0.085e-6 * stream;
+    WideChoice best;
     for (const ShapeCost &c : kShapes) {
         if (N < c.shape.blocks * 16u || (p->cfg.wide_shape >= 0 && uint32_t(p->cfg.wide_shape) % kShapeCount != uint32_t(&c - kShapes))) continue;
-        const uint64_t groups = workgroups(p, N, c.shape);
-        const double rounds = groups <= cu ? 0.87 + 0.13 * double(groups) / double(cu) : 1.04 * double((groups + cu - 1u) / cu);
-        const double t = c.start + c.chunk[i] * p->wide.n_chunks * rounds;
-        if (!best || t < *expected) { best = &c; *expected = t; }
+        const uint64_t groups = workgroups(p, N, c.shape), sums = groups * tile_sums_bytes(c.shape);
+        const uint32_t stages = p->wide.n_chunks / c.shape.splits;
+        uint32_t tried = 0;
+        // as many cuts as there are compute units for, once and twice; two stages each at least, and sums that hspmm_run_static has room for
+        for (uint64_t round = 0; round <= 2u; ++round) {
+            const uint64_t most = std::min<uint64_t>(std::min<uint64_t>(kMostCuts, stages / 2u), HSPMM_STATIC_SCRATCH_BYTES / sums);
+            uint32_t cuts = uint32_t(std::max<uint64_t>(1u, std::min(round * cu / groups, most)));
+            if (p->cfg.wide_cuts > 0) cuts = uint32_t(std::max<uint64_t>(1u, std::min<uint64_t>(uint64_t(p->cfg.wide_cuts), most)));
+            if (cuts == tried) continue;
+            tried = cuts;
+            const double all = double(groups * cuts), rounds = all <= double(cu) ? 0.87 + 0.13 * all / double(cu) : 1.04 * std::ceil(all / double(cu));
+            double t = c.start + c.chunk[i] * double((stages + cuts - 1u) / cuts * c.shape.splits) * rounds + large;
+            if (cuts > 1u) t += c.cut + kPerCut * cuts + kPerSumsByte * double(sums) * cuts;
+            if (!best.cost || t < best.expected) { best.cost = &c; best.cuts = cuts; best.expected = t; }
+        }
     }
     return best;
+}
+
+// What the gather kernels take for matrices of 16 x 16 blocks, us: a fit to 1834 launches of 20 to 60 % (standard deviation 17 to 34 %).  Up
+// to 64 features in whole 16-byte pieces are one pass over the tiles, others one per 32.
+double blocks_gather_expected(const hspmm_plan *p, uint32_t N)
+{
+    const double tiles = 1e-3 * p->T, passes = double((N + 31u) / 32u);
+    if (N % 8u == 0u) return N <= 32u ? 4.7 + 0.077 * tiles : N <= 64u ? 5.3 + 0.112 * tiles : 12.5 + 0.162 * tiles;
+    return (N % 2u ? 10.3 + 0.25 * tiles : 6.3 + 0.18 * tiles) * (1.0 + 0.36 * (passes - 2.0));
+}
+
+bool of_blocks(const hspmm_plan *p) { return p->G == 2 && p->per_column > 4.0; }
+
+bool worth_taking(const hspmm_plan *p, uint32_t N)
+{
+    const double expected = choose_wide_shape(p, N).expected;
+    if (of_blocks(p)) {
+        if (panel_serves(p, N)) return expected < 0.9 * (6.2 + 0.9 * panel_expected(p, N));
+        return expected < 0.9 * blocks_gather_expected(p, N);
+    }
+    if (tile_serves(p, N)) return double(p->tile.entries) <= kMostEntries * p->rows * p->cols && expected < 0.95 * tile_expected(p, N);
+    if (entries_serve(p, N)) return N < 256u && expected < 0.9 * entries_expected(p, N);
+    if (panel_serves(p, N)) return expected < 0.95 * (5.56 + 1.07 * panel_expected(p, N));
+    return true;
+}
+
+// The answer for an N is the plan's alone, and is kept for the last N (a launch would otherwise take two microseconds of the host's):
+// N, index of the shape, cuts, whether the launch is taken.
+uint64_t kept_choice(const hspmm_plan *p, uint32_t N)
+{
+    uint64_t kept = p->wide.choice.load(std::memory_order_relaxed);
+    if (kept >> 32 == N) return kept;
+    const WideChoice choice = choose_wide_shape(p, N);
+    const bool taken = choice.cost && workgroups(p, N, choice.cost->shape) * choice.cuts < (1u << 22) && (p->cfg.wide > 0 || worth_taking(p, N));
+    kept = uint64_t(N) << 32 | (choice.cost ? uint32_t(choice.cost - kShapes) << 16 : 0u) | choice.cuts << 8 | (taken ? 1u : 0u);
+    p->wide.choice.store(kept, std::memory_order_relaxed);
+    return kept;
 }
 
 }  // namespace
@@ -55,15 +112,15 @@ const ShapeCost *choose_wide_shape(const hspmm_plan *p, uint32_t N, double *expe
 namespace hspmm_host {
 
 // Made where some feature dimension would take it by the stored entries as estimated from a sample: from 4 % on (at 3 to 4 % the
-// launches it would take gain 2 % of the time of all, at 4 to 6 % 12 %, above 10 % 31 %, for 2 bytes per element of the matrix).
-// Block-clustered weights (over four of a column's eight elements stored) stay with kernels that read whole tiles.
+// launches it would take gain 2 % of the time of all, at 4 to 6 % 12 %, above 10 % 31 %, for 2 bytes per element of the matrix), of weights in
+// 16 x 16 blocks (units of two windows, over four of a column's eight elements stored) from 15 % on.
 int build_wide_stream(hspmm_plan *p)
 {
     using namespace hspmm;
     hspmm_plan::Wide &w = p->wide;
     if (p->elem != 2u || p->cfg.wide == 0 || !p->canonical || p->cfg.kernel_mode != 0 || !p->T || p->W >= (1u << 23)) return HSPMM_OK;
-    const double cells = double(p->rows) * p->cols;
-    if (p->cfg.wide < 0 && (p->G != 1 || p->per_column > 4.0 || double(p->T) * p->cw * p->per_column < 0.04 * cells)) return HSPMM_OK;
+    const double fill = double(p->T) * p->cw * p->per_column / (double(p->rows) * p->cols);
+    if (p->cfg.wide < 0 && (of_blocks(p) ? fill < 0.15 : p->G != 1 || p->per_column > 4.0 || fill < 0.04)) return HSPMM_OK;
     const uint32_t n_units = (p->rows + 15u) / 16u, n_chunks = ((p->cols + 63u) / 64u + 3u) & ~3u;
     const TileSource src{p->d_rowOffset, p->d_rowIdx, p->d_a2b_raw, p->d_data, p->W, p->cols};
     // (a plan whose device memory holds no such stream is made without)
@@ -80,51 +137,44 @@ int build_wide_stream(hspmm_plan *p)
     return HSPMM_OK;
 }
 
-double wide_expected(const hspmm_plan *p, uint32_t N)
-{
-    double expected = 0.0;
-    return choose_wide_shape(p, N, &expected) ? expected : 0.0;
-}
+double wide_expected(const hspmm_plan *p, uint32_t N) { return choose_wide_shape(p, N).expected; }
 
-// Where they are expected to be faster, by 5 % at least, than the kernels that would take the launch.  Launches of the entry kernels stay
-// theirs (at the few features they take from such matrices 1 in 20 would gain), and those of the gather kernels from 32 features on are
-// all taken (of 184, one in eight lost, 13 % at most; 1.35 times as fast on average).  Over 3078 launches the rule gives
-// 1.16 times the speed of the LDS-panel kernels (1.175 if every launch took the faster one; 3 % of those taken lose, 4 % on average),
-// 1.44 of the full-tile ones (1.52; none loses), whose times are known up to kMostEntries: denser launches of theirs stay.
-// With fewer than kFewRows rows a long chain of chunks leaves compute units idle, where the other kernels cut the columns: 512 rows x
-// 11008 at 10 %, N = 64 / 128 / 512 / 1024 21 / 22 / 31 / 41 us by these kernels, 17 / 17 / 21 / 27 by the others, 512 x 4096 8 / 10 / 13 / 17
-// and 9 / 13 / 15 / 16, 512 x 1024 7.0 for each and 7.0 / 9.0 / 9.8 / 10.7: only launches expected to be short are taken.
+// Where they are expected to be faster, by 5 or 10 %, than the kernels that would take the launch; the gather kernels lose every launch
+// but one in a hundred of pruned weights.  Times by the kernels that otherwise take a launch over the time that these are expected
+// to take, with the launches taken by this rule and those left: LDS-panel 1.22 (4385 launches, 1.23 if every one took the faster kernel),
+// full-tile 1.67 (1233, whose times are known up to kMostEntries: denser launches stay), gather 1.69 (475); of blocks of 16 x 16
+// LDS-panel 1.08 (1832), gather 1.75 (1834).
+// Without cut C tiles rows x columns with few workgroups left compute units idle, us (uncut / cut / other kernels): 512 x 11008 at 10 %,
+// N = 64 20.5 / 9.9 / 17, 256 24.8 / 13.0 / 19, 4096 x 14336, N = 64 45 / 26.
 bool wide_serves(const hspmm_plan *p, uint32_t N)
 {
     const Config &c = p->cfg;
-    if (!p->wide.built || c.kernel_mode != 0 || N < kFewestFeatures || N >= (1u << 21)) return false;
-    double expected = 0.0;
-    const ShapeCost *shape = choose_wide_shape(p, N, &expected);
-    if (!shape || workgroups(p, N, shape->shape) >= (1u << 22)) return false;
-    if (c.wide > 0) return true;
+    if (!p->wide.built || c.kernel_mode != 0 || N < kFewestFeatures || N >= (1u << 20)) return false;
     // (settings of other kernels)
-    if (c.buffer_stage || c.consumer_warp_num || c.producer_warp_group_num || c.fused_fixup >= 0 || c.panel_chunks || c.panel_max_windows ||
-        c.panel_units_per_group || c.aligned_small >= 0 || c.xcd_split >= 0 || c.gather_bitmap >= 0 || c.tile > 0 || c.entries > 0)
+    if (c.wide < 0 && (c.buffer_stage || c.consumer_warp_num || c.producer_warp_group_num || c.fused_fixup >= 0 || c.panel_chunks || c.panel_max_windows ||
+                       c.panel_units_per_group || c.aligned_small >= 0 || c.xcd_split >= 0 || c.gather_bitmap >= 0 || c.tile > 0 || c.entries > 0))
         return false;
-    if (tile_serves(p, N)) return double(p->tile.entries) <= kMostEntries * p->rows * p->cols && expected < 0.95 * tile_expected(p, N);
-    if (entries_serve(p, N)) return false;
-    if (p->rows < kFewRows && expected > kShort) return false;
-    if (panel_serves(p, N)) return expected < 0.95 * (5.56 + 1.07 * panel_expected(p, N));
-    return true;
+    return kept_choice(p, N) & 1u;
 }
 
 int run_wide(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode)
 {
-    if (mode == RunMode::kPrepare) return HSPMM_OK;
     const hspmm_plan::Wide &w = p->wide;
-    double expected = 0.0;
-    const hspmm::WideShape &sh = choose_wide_shape(p, N, &expected)->shape;
+    const uint64_t choice = kept_choice(p, N);
+    const hspmm::WideShape &sh = kShapes[choice >> 16 & 0xFFu].shape;
+    const uint64_t groups = workgroups(p, N, sh);
     hspmm::WideArgs wa{};
+    wa.n_cuts = uint32_t(choice >> 8 & 0xFFu);
+    if (wa.n_cuts > 1u) {
+        std::lock_guard<std::mutex> lk(p->mu);
+        if (const int rc = scratch_for(p, s, size_t(groups * wa.n_cuts * tile_sums_bytes(sh)), mode, &wa.sums)) return rc;
+    }
+    if (mode == RunMode::kPrepare) return HSPMM_OK;
     wa.frags = w.d_frags; wa.B = dB; wa.C = dC;
     wa.rows = p->rows; wa.cols = p->cols; wa.N = N;
     wa.n_units = w.n_units; wa.n_chunks = w.n_chunks; wa.n_feat_tiles = (N + sh.blocks * 16u - 1u) / (sh.blocks * 16u);
     wa.src = w.d_source;
-    p->note_launch("spmm_wide_kernel", 3, p->dtype == HSPMM_FP16 ? 1u : 2u, workgroups(p, N, sh) * w.n_chunks * sh.units * sh.rows * sh.blocks * 2u);
+    p->note_launch("spmm_wide_kernel", 3, p->dtype == HSPMM_FP16 ? 1u : 2u, groups * w.n_chunks * sh.units * sh.rows * sh.blocks * 2u);
     HSPMM_HIP(hspmm::launch_spmm_wide(p->dtype, wa, sh, s));
     return HSPMM_OK;
 }

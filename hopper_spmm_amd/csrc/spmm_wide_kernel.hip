@@ -68,6 +68,9 @@ template <bool BF> struct WideHalf : HalfStored<BF> {
 // whatever the shape (WR, RF, CF = 4, 2, 4: 0.27 us for 24 KB; 4, 3, 8: 0.55 us for 40 KB, where the matrix instructions take 0.37).  A
 // second workgroup on a compute unit doubles the time, more loads in flight (two sets of B, four of A) change nothing, nor do sets
 // that run in step with two LDS buffers each.  Start and end are 4 us for the smallest tiles and 10 for the largest.
+// Fewer C tiles than compute units are cut: each workgroup takes a part of the chunks and leaves its sums in memory, and a second kernel adds
+// them (4096 x 14336, N = 64 45 -> 26 us, 512 x 11008, N = 256 24.8 -> 13.0).  Operands are laid out chunk by chunk, since the
+// workgroups walk the chunks side by side: unit by unit, 4096 x 14336 took 57.8 instead of 54.2 us at N = 128 and 39.3 instead of 35.8 at 32.
 // Measured, bf16 (this / the LDS-panel or full-tile kernels, us): 5003 x 3001 at 20 %, N = 64 10.5 / 15.7, 128 12.1 / 15.6, 333
 // 21.0 / 28.1; 4096^2 at 10 %, N = 256 15.7 / 20.7, 512 21.7 / 28.5; 3840 x 1155 at 29 %, N = 208 8.3 / 13.9; 14080 x 2815 at 26 %,
 // N = 101 19.8 / 42.3.  2531 launches of 508 matrices at 3 to 30 %: 1.37 times as fast on the 63 % of them where it is faster.
@@ -87,8 +90,9 @@ void spmm_wide_kernel(const WideArgs wa)
     // operands, neighbours their rows of B
     const uint32_t n_groups = gridDim.x, xcd = blockIdx.x & 7u;
     const uint32_t tile = xcd * (n_groups >> 3) + umin32(xcd, n_groups & 7u) + (blockIdx.x >> 3);
-    const uint32_t rb = tile / wa.n_feat_tiles, ft = tile - rb * wa.n_feat_tiles;
-    const uint32_t n_stages = wa.n_chunks / WK, unit0 = (rb * WR + wr) * RF, row0 = unit0 * kWideRows;
+    const uint32_t rbc = tile / wa.n_feat_tiles, ft = tile - rbc * wa.n_feat_tiles, rb = rbc / wa.n_cuts, cut = rbc - rb * wa.n_cuts;
+    const uint32_t all_stages = wa.n_chunks / WK, stage0 = cut * all_stages / wa.n_cuts, n_stages = (cut + 1u) * all_stages / wa.n_cuts - stage0;
+    const uint32_t unit0 = (rb * WR + wr) * RF, row0 = unit0 * kWideRows;
     const size_t row_bytes = size_t(wa.N) * E::kElem;
     const uint32_t own = ft * NT, f0 = umin32(own, wa.N - NT);      // the last tile is moved back to end with the row; it stores from `own` on
 
@@ -98,13 +102,13 @@ void spmm_wide_kernel(const WideArgs wa)
     for (uint32_t i = 0; i < kPer; ++i) { const uint32_t n = i * kSet + tid % kSet; piece_row[i] = n / kPieces; piece_col[i] = n % kPieces * 16u; }
     const char *src_a[RF];                                          // (units behind the last one: that unit, not stored)
 #pragma unroll
-    for (int u = 0; u < RF; ++u) src_a[u] = static_cast<const char *>(wa.frags) + (size_t(umin32(unit0 + u, wa.n_units - 1u)) * wa.n_chunks + set) * kWideUnitBytes;
+    for (int u = 0; u < RF; ++u) src_a[u] = static_cast<const char *>(wa.frags) + (size_t(set) * wa.n_units + umin32(unit0 + u, wa.n_units - 1u)) * kWideUnitBytes;
     u32x4 piece[kPer];
     typename E::A a[2][RF];
     uint32_t ask_a = 0, ask_b = 0;
     auto request_b = [&]() __attribute__((always_inline)) {
         // (rows behind the last one: that row, which the operands multiply by zero)
-        const uint32_t first = umin32((umin32(ask_b, n_stages - 1u) * WK + set) * 64u, wa.cols - 1u), last = wa.cols - 1u - first;
+        const uint32_t first = umin32(((stage0 + umin32(ask_b, n_stages - 1u)) * WK + set) * 64u, wa.cols - 1u), last = wa.cols - 1u - first;
         const char *p = src_b + size_t(first) * row_bytes;
 #pragma unroll
         for (uint32_t i = 0; i < kPer; ++i) piece[i] = *reinterpret_cast<const u32x4_any *>(p + (umin32(piece_row[i], last) * uint32_t(row_bytes) + piece_col[i]));
@@ -112,7 +116,7 @@ void spmm_wide_kernel(const WideArgs wa)
     };
     auto request_a = [&](auto set_c) __attribute__((always_inline)) {
         constexpr int S = decltype(set_c)::value;
-        const size_t off = size_t(umin32(ask_a, n_stages - 1u)) * (WK * kWideUnitBytes);
+        const size_t off = size_t(stage0 + umin32(ask_a, n_stages - 1u)) * wa.n_units * (WK * kWideUnitBytes);
 #pragma unroll
         for (int u = 0; u < RF; ++u) E::load_a(a[S][u], src_a[u] + off, lane);
         ++ask_a;
@@ -177,6 +181,12 @@ void spmm_wide_kernel(const WideArgs wa)
         }
     }
     if (set != 0u) return;
+    if (wa.n_cuts > 1u) {
+        f32x4 *out = reinterpret_cast<f32x4 *>(wa.sums) + ((size_t(cut) * (n_groups / wa.n_cuts) + rb * wa.n_feat_tiles + ft) * WR + wr) * (RF * CF * 64u) + lane;
+#pragma unroll
+        for (int i = 0; i < RF * CF; ++i) out[i * 64] = acc[i / CF][i % CF];
+        return;
+    }
     float met = 0.f;
 #pragma unroll
     for (int u = 0; u < RF; ++u) {
@@ -200,11 +210,43 @@ void spmm_wide_kernel(const WideArgs wa)
     }
 }
 
+// The sums of the cuts of a C tile, in order: a wave per 16 rows x 16 features.
+template <class E>
+__global__ __launch_bounds__(256) void wide_sum_kernel(const WideArgs wa, const WideShape sh, uint32_t n_blocks)
+{
+    const uint32_t lane = threadIdx.x & 63u, i = __builtin_amdgcn_readfirstlane(blockIdx.x * 4u + (threadIdx.x >> 6));
+    if (i >= n_blocks) return;
+    const uint32_t block = i % sh.blocks, unit_of = i / sh.blocks % (sh.units * sh.rows), tile = i / sh.blocks / (sh.units * sh.rows);
+    const uint32_t rb = tile / wa.n_feat_tiles, ft = tile - rb * wa.n_feat_tiles, nt = sh.blocks * 16u;
+    const uint32_t row0 = (rb * sh.rows * sh.units + unit_of) * kWideRows, own = ft * nt, f0 = umin32(own, wa.N - nt) + block * 16u;
+    if (row0 >= wa.rows || f0 + 16u <= own) return;
+    const f32x4 *in = reinterpret_cast<const f32x4 *>(wa.sums) + size_t(i) * 64u + lane;
+    f32x4 v = in[0];
+#pragma unroll 4
+    for (uint32_t c = 1; c < wa.n_cuts; ++c) v += in[size_t(c) * n_blocks * 64u];
+    const size_t row_bytes = size_t(wa.N) * E::kElem;
+    E::store(static_cast<char *>(wa.C) + size_t(row0) * row_bytes + size_t(f0) * E::kElem, row_bytes, wa.rows - row0, own > f0 ? own - f0 : 0u, v, lane);
+    float met = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) met = __builtin_fmaf(v[e], 0.f, met);
+    if (__ballot(met != 0.f)) tile_sum_again<E, 1, 16, true>(wa, row0, f0, own, lane);
+}
+
+template <class E>
+static hipError_t launch_wide_sums(const WideArgs &wa, const WideShape &sh, uint32_t groups, hipStream_t s)
+{
+    if (hipError_t e = hipGetLastError()) return e;
+    if (wa.n_cuts == 1u) return hipSuccess;
+    const uint32_t n_blocks = groups * sh.blocks * sh.units * sh.rows;
+    wide_sum_kernel<E><<<dim3((n_blocks + 3u) / 4u), 256, 0, s>>>(wa, sh, n_blocks);
+    return hipGetLastError();
+}
+
 template <class E>
 static hipError_t launch_wide_e(const WideArgs &wa, const WideShape &sh, uint32_t groups, hipStream_t s)
 {
 #define HSPMM_WIDE(RF, CF, WR, WK) \
-    if (sh.units == RF && sh.blocks == CF && sh.rows == WR && sh.splits == WK) { spmm_wide_kernel<E, RF, CF, WR, WK><<<dim3(groups), 64 * WR * WK, 0, s>>>(wa); return hipGetLastError(); }
+    if (sh.units == RF && sh.blocks == CF && sh.rows == WR && sh.splits == WK) { spmm_wide_kernel<E, RF, CF, WR, WK><<<dim3(groups * wa.n_cuts), 64 * WR * WK, 0, s>>>(wa); return launch_wide_sums<E>(wa, sh, groups, s); }
     HSPMM_WIDE(1, 2, 2, 4) HSPMM_WIDE(1, 2, 4, 2) HSPMM_WIDE(1, 4, 4, 2) HSPMM_WIDE(2, 2, 4, 2) HSPMM_WIDE(2, 4, 4, 2) HSPMM_WIDE(3, 4, 2, 4)
     HSPMM_WIDE(3, 4, 4, 2) HSPMM_WIDE(2, 8, 4, 2) HSPMM_WIDE(3, 8, 4, 2)
 #undef HSPMM_WIDE
@@ -219,7 +261,7 @@ hipError_t launch_spmm_wide(int dtype, const WideArgs &wa, const WideShape &sh, 
         uint64_t(wa.n_units) * kWideRows < wa.rows || wa.n_feat_tiles != (wa.N + nt - 1u) / nt)
         return hipErrorInvalidValue;
     const uint64_t groups = (wa.rows + rows - 1u) / rows * wa.n_feat_tiles;
-    if (groups >= (1u << 22)) return hipErrorInvalidValue;
+    if (!wa.n_cuts || groups * wa.n_cuts >= (1u << 22) || wa.n_cuts > wa.n_chunks / sh.splits || (wa.n_cuts > 1u && !wa.sums)) return hipErrorInvalidValue;
     if (dtype == kDtypeBf16) return launch_wide_e<WideHalf<true>>(wa, sh, uint32_t(groups), s);
     if (dtype == kDtypeF16) return launch_wide_e<WideHalf<false>>(wa, sh, uint32_t(groups), s);
     return hipErrorInvalidValue;
@@ -231,17 +273,17 @@ hipError_t launch_spmm_wide(int dtype, const WideArgs &wa, const WideShape &sh, 
 
 // Lane (g, j) of an instruction has row j and the columns 4 g .. 4 g + 3 and 16 + 4 g .. 16 + 4 g + 3 of 32: the rows of B that the
 // transposing LDS reads bring it.
-__global__ __launch_bounds__(256) void wide_fill_kernel(const TileSource src, uint32_t n_chunks, char *__restrict__ frags)
+__global__ __launch_bounds__(256) void wide_fill_kernel(const TileSource src, uint32_t n_units, char *__restrict__ frags)
 {
     const uint32_t w = blockIdx.x, row0 = src.rowIdx[w];
-    char *unit = frags + size_t(row0 / kWideRows) * n_chunks * kWideUnitBytes;
+    char *unit = frags + size_t(row0 / kWideRows) * kWideUnitBytes;
     const size_t c1 = size_t(src.rowOffset[w + 1u]) * 16u;
     for (size_t c = size_t(src.rowOffset[w]) * 16u + threadIdx.x; c < c1; c += blockDim.x) {
         const uint32_t id = src.a2b[c];
         if (id == kIdxMax) continue;
         const uint16_t *tile = static_cast<const uint16_t *>(src.tiles) + (c / 16u) * 128u + c % 16u;
         const uint32_t k = id & 31u;
-        uint16_t *to = reinterpret_cast<uint16_t *>(unit + size_t(id >> 6) * kWideUnitBytes + (id & 32u) * 32u) +
+        uint16_t *to = reinterpret_cast<uint16_t *>(unit + size_t(id >> 6) * n_units * kWideUnitBytes + (id & 32u) * 32u) +
                        (((k & 15u) >> 2) * 16u + (row0 & 15u)) * 8u + (k & 3u) + 4u * (k >> 4);
 #pragma unroll
         for (uint32_t r = 0; r < 8u; ++r) {
@@ -254,8 +296,9 @@ __global__ __launch_bounds__(256) void wide_fill_kernel(const TileSource src, ui
 hipError_t launch_wide_fill(const TileSource &src, uint32_t rows, uint32_t n_chunks, void *frags, hipStream_t s)
 {
     if (!src.n_windows || src.n_windows >= (1u << 23)) return hipErrorInvalidValue;
-    if (hipError_t e = launch_fill_zero(frags, size_t((rows + kWideRows - 1u) / kWideRows) * n_chunks * kWideUnitBytes, s)) return e;
-    wide_fill_kernel<<<dim3(src.n_windows), 256, 0, s>>>(src, n_chunks, static_cast<char *>(frags));
+    const uint32_t n_units = (rows + kWideRows - 1u) / kWideRows;
+    if (hipError_t e = launch_fill_zero(frags, size_t(n_units) * n_chunks * kWideUnitBytes, s)) return e;
+    wide_fill_kernel<<<dim3(src.n_windows), 256, 0, s>>>(src, n_units, static_cast<char *>(frags));
     return hipGetLastError();
 }
 

@@ -26,12 +26,13 @@ def _plan(hs, A, **env):
 
 
 @pytest.mark.parametrize("shape", range(9))
-@pytest.mark.parametrize("dtype,rows,cols", [(0, 193, 257), (2, 191, 64), (2, 417, 575), (0, 17, 65), (2, 7, 3)])
-def test_exact_sums_in_every_shape(torch_cuda, hs, shape, dtype, rows, cols):
+@pytest.mark.parametrize("dtype,rows,cols,cuts", [(0, 193, 257, 1), (2, 191, 64, 1), (2, 417, 575, 1), (0, 17, 65, 1), (2, 7, 3, 1), (2, 193, 575, 3), (0, 400, 2050, 5),
+                                                  (2, 33, 2100, 16)])
+def test_exact_sums_in_every_shape(torch_cuda, hs, shape, dtype, rows, cols, cuts):
     torch = torch_cuda
     rng = np.random.default_rng(100 * rows + shape)
     D, A = _matrix(rng, rows, cols, 0.1 if cols > 3 else 0.5, dtype)
-    plan = _plan(hs, A, WIDE=1, WIDE_SHAPE=shape)
+    plan = _plan(hs, A, WIDE=1, WIDE_SHAPE=shape, WIDE_CUTS=cuts)
     stream = torch.cuda.current_stream().cuda_stream
     guard, nt = 64, FEWEST[shape]
     for N in (nt, nt + 1, 2 * nt - 1, 2 * nt, 2 * nt + 8):
@@ -51,12 +52,12 @@ def test_exact_sums_in_every_shape(torch_cuda, hs, shape, dtype, rows, cols):
     plan.close()
 
 
-@pytest.mark.parametrize("shape", [0, 6, 7])
+@pytest.mark.parametrize("shape,cuts", [(0, 1), (6, 1), (7, 1), (4, 2)])
 @pytest.mark.parametrize("dtype", [0, 2])
 @pytest.mark.parametrize("rows,cols", [(600, 700), (1100, 130)])
-def test_infinities_and_nans_stay_with_the_rows_that_name_them(torch_cuda, hs, monkeypatch, shape, dtype, rows, cols):
+def test_infinities_and_nans_stay_with_the_rows_that_name_them(torch_cuda, hs, monkeypatch, shape, cuts, dtype, rows, cols):
     """By the rule of the kernels that multiply stored entries only, whose check this is."""
-    monkeypatch.setitem(nonfinite.FAMILIES, "tile", (0, {"HSPMM_WIDE": "1", "HSPMM_WIDE_SHAPE": str(shape)}, (128, 130, 200), "spmm_wide_kernel"))
+    monkeypatch.setitem(nonfinite.FAMILIES, "tile", (0, {"HSPMM_WIDE": "1", "HSPMM_WIDE_SHAPE": str(shape), "HSPMM_WIDE_CUTS": str(cuts)}, (128, 130, 200), "spmm_wide_kernel"))
     nonfinite.test_infinities_and_nans_stay_with_the_rows_that_name_them(torch_cuda, hs, "tile", dtype, rows, cols)
 
 
@@ -64,7 +65,7 @@ def test_infinities_and_nans_stay_with_the_rows_that_name_them(torch_cuda, hs, m
 # than n 2^-24 of the sum of their sizes, and the result's own rounding adds 2^-11 (fp16) or 2^-8 (bf16) of it.
 @pytest.mark.parametrize("dtype,rows,cols,per_row,N,kernel", [
     (2, 5003, 3001, 600, 333, "wide"), (0, 4096, 4096, 409, 256, "wide"), (2, 3840, 1155, 340, 58, "wide"), (0, 4096, 4096, 82, 256, "panel"),
-    (0, 512, 1024, 100, 512, "wide"), (0, 512, 4096, 409, 1024, "panel"), (2, 5120, 2007, 200, 24, "tile"), (1, 4096, 4096, 409, 256, "panel")])
+    (0, 512, 1024, 100, 512, "wide"), (0, 512, 11008, 1100, 64, "wide"), (2, 5120, 2007, 200, 24, "tile"), (1, 4096, 4096, 409, 256, "panel")])
 def test_chosen_where_they_are_faster(torch_cuda, hs, dtype, rows, cols, per_row, N, kernel):
     torch = torch_cuda
     rng = np.random.default_rng(N + dtype)
@@ -83,4 +84,23 @@ def test_chosen_where_they_are_faster(torch_cuda, hs, dtype, rows, cols, per_row
         want = D @ Bm
         off = abs(decode(dC.cpu().numpy().view(np.uint16), dtype).astype(np.float64) - want)
         assert (off <= bound + (2.0**-11 if dtype == 0 else 2.0**-8) * (abs(want) + bound)).all()
+    plan.close()
+
+
+def test_chosen_for_blocks_where_they_are_faster(torch_cuda, hs):
+    torch = torch_cuda
+    rng = np.random.default_rng(5)
+    D = np.kron(rng.random((128, 128)) < 0.4, np.ones((16, 16), int)) * rng.integers(-2, 3, (2048, 2048))
+    counts = (D != 0).sum(1)
+    A = dict(rows=2048, cols=2048, nnzs=int(counts.sum()), dtype=2, row_ptr=np.concatenate([[0], np.cumsum(counts)]).astype(np.uint32),
+             col_idx=np.nonzero(D)[1].astype(np.uint32), values=encode(D[D != 0].astype(np.float32), 2))
+    plan = hs.Plan(convert(hs, A))
+    for N, wide in ((32, False), (63, True), (95, True), (130, None)):
+        Bm = rng.integers(-2, 3, (2048, N))
+        dB = torch.from_numpy(encode(Bm.astype(np.float32), 2).view(np.int16)).cuda()
+        dC = torch.empty((2048, N), dtype=torch.int16, device="cuda")
+        plan.run(dB.data_ptr(), dC.data_ptr(), N, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert wide is None or (plan.last_kernel() == "spmm_wide_kernel") == wide, N
+        assert np.array_equal(dC.cpu().numpy().view(np.uint16), encode((D @ Bm).astype(np.float32), 2)), N
     plan.close()
