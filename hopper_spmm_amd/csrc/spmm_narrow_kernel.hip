@@ -71,15 +71,16 @@ template <bool BF, bool ODD> struct NarrowHalf : HalfStored<BF> {
         return HalfOps<BF>::mfma(a, o, acc);
     }
 };
+
 // A workgroup of W waves multiplies 16 rows of A with CF tiles of features; a wave takes every W-th block of 128 columns by itself, without
 // a barrier: it scatters the block's entries (CAP x 128 of them asked for two blocks earlier; more are loaded when their turn comes) into
 // its image in LDS, reads the image back as first operands, clears it, and multiplies it with B's rows, which come straight into
 // registers, asked for a block earlier.  The waves' sums are added in LDS at the end, always in the same order.  (LDS serves the
 // requests of a wave in order.)
-// What bounds it: requests of a compute unit - of a block, to memory 16 for B (256 bytes each, 4 cycles) and 2 CAP for entries, to LDS 8 for
-// the image and its clearing (8 cycles) and 2 CAP for entries -: 0.04 to 0.05 us a block at 10 %, of which the first wait is 3 us.  With B
-// in loads of one 16-bit feature (32 of them a block): 11.0 us instead of 9.1 for 4096 x 11008 at 10 %, N = 16, and 16.2 instead of 12.9 for
-// N = 32.
+// What bounds it: the loads of a block - 16 of B, 2 words a lane CAP times for entries -, which keep the L1's return path busy for 80 %
+// of a launch (4096 x 11008 at 10 %, N = 16), and 3 us of launch and first loads.  With B in loads of one 16-bit feature, 32 of
+// them a block, that took 11.0 us instead of 9.1, and N = 32 16.2 instead of 12.9; with B in 16-byte pieces, 4 a block, through LDS
+// and its transposing reads 11.1.
 // Measured, bf16 (this / the full-tile kernels, the entry kernels (e) or the gather kernels (g), us): 4096 x 11008 at 10 %, N = 1 9.3 / 11.7 e,
 // 8 8.9 / 15.3 e, 15 9.3 / 18.8, 16 9.1 / 17.1, 32 12.9 / 19.8;  11008 x 4096 at 30 %, N = 7 14.4 / 38.5 e, 16 14.1 / 18.6;  1500 x 9001 at 30 %,
 // N = 15 10.6 / 26.9 g, 29 13.0 / 19.1.  1994 launches of N = 1 to 32 with 2.5 to 30 %: 1.23 times the entry kernels' speed on the launches

@@ -271,8 +271,8 @@ typedef struct {
     uint32_t n_panel_paired_units;  /* of those: units of two or more windows */
     uint32_t n_panel_wide_units;    /* of those: units of three or four windows */
     uint32_t last_kernel_family;    /* what the last hspmm_run launched: 0 nothing yet, 1 all-shapes kernel, 2 gather kernels (MFMA, or entry
-                                       by entry: last_mfma_kind 0 then), 3 LDS-staging kernels (a panel of B at a time, or full tiles of A
-                                       put together in LDS), 4 clear only (matrix without entries); hspmm_last_kernel tells them apart */
+                                       by entry: last_mfma_kind 0 then), 3 LDS-staging kernels (a panel of B at a time, or full operands of A:
+                                       full-tile, narrow and wide-tile kernels), 4 clear only (matrix without entries); hspmm_last_kernel tells them apart */
     uint32_t gather_bitmap;         /* 1: the gather kernels read this plan's tiles as bitmap + stored elements (single
                                      * windows with few stored elements per tile), 0: as uncompressed tiles */
     uint32_t bitmap_from_caller;    /* 1: the plan was made from bitmap tiles (hspmm_create_bitmap / _grouped) and uploaded them as they
@@ -293,8 +293,8 @@ typedef struct {
 int hspmm_get_plan_info(const hspmm_plan *plan, hspmm_plan_info *info);
 
 /* No reference counterpart: the name of the main kernel of the last hspmm_run - spmm_entries_kernel,
- * spmm_mfma_kernel, spmm_panel_kernel, spmm_tile_kernel, spmm_scalar_kernel, or fill_zero_kernel for a matrix
- * without entries; "" before the first (hspmm_plan_info.last_kernel_family names two of them with one number). */
+ * spmm_mfma_kernel, spmm_panel_kernel, spmm_tile_kernel, spmm_narrow_kernel, spmm_wide_kernel, spmm_scalar_kernel, or
+ * fill_zero_kernel for a matrix without entries; "" before the first (hspmm_plan_info.last_kernel_family names two of them with one number). */
 const char *hspmm_last_kernel(const hspmm_plan *plan);
 
 /* No reference counterpart: copies the partition for inspection (tests).
