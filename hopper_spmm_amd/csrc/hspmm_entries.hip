@@ -203,6 +203,11 @@ bool entries_serve(const hspmm_plan *p, uint32_t N)
     const double per_column = p->per_column, weight = double(row) * (per_column - 0.8);
     const bool sparse = per_column <= 1.25;
     if (p->elem == 4u) {
+        // 33 to 63 features: the LDS-panel kernels multiply bf16 parts, which no launch that has fp32 products here may lose them to; what
+        // would be theirs or the full-tile kernels' goes by expected time, fits to 301 and 878 launches (standard deviations 10 and 7 %):
+        // 4096 x 11008 at 10 %, N = 40: 54 us here, 39 there, 67 full tiles.
+        if (N > 32u && N < 64u && p->panel.split && panel_serves(p, N) && (weight > 100.0 || tile_leaves(p, N)))
+            return 3.6 + 12.7e-6 * double(p->T) * p->cw * per_column < 5.7 + 1.2 * panel_expected(p, N);
         if (weight <= 100.0) return true;
         // Rows that are no whole 16-byte pieces, below the 64 features from which the LDS-panel kernels take any: the other fp32
         // products come in blocks of 16 features where N is odd and of 32 where it is even (pruned 4096 x 11008 at 10 %, N = 47:

@@ -328,6 +328,7 @@ double panel_expected(const hspmm_plan *p, uint32_t N);
 // hspmm_tile.hip: the full-tile kernels' stream, whether they take this launch, and the launch
 int build_tile_stream(hspmm_plan *p);
 bool tile_serves(const hspmm_plan *p, uint32_t N);
+bool tile_leaves(const hspmm_plan *p, uint32_t N);
 double tile_expected(const hspmm_plan *p, uint32_t N);          // us
 int run_tile(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode);
 

@@ -91,10 +91,11 @@ int build_tile_stream(hspmm_plan *p)
 //   bf16, 11008 x 4096 at 20 %: N = 8 15 / 18, 16 14.5 / 29, 32 16 / 34, 64 23 / 53;  4096 x 11008 at 10 %: N = 8 18 / 13,
 //   16 17 / 21, 32 19.5 / 27, 64 24 / 36;  5003 x 3001 at 20 %: N = 16 10.5 / 10.6, 32 11.7 / 15.2, 64 14.2 / 22;  4096^2 at 10 %:
 //   N = 32 12.4 / 8.8, 64 14.5 / 15.4;  fp32, 11008 x 4096 at 20 %: N = 16 24 / 42, 32 28 / 35, 64 36 / 35;
-//   4096 x 11008 at 10 %: N = 16 25.7 / 26.6, 32 29 / 34.  N = 256 and more: the LDS-panel kernels by a fifth.
+//   4096 x 11008 at 10 %: N = 16 25.7 / 26.6, 32 29 / 34 - but 36 67 / 39, 6000^2 at 15 % 49 / 35: from 33 features on, which leave a C
+//   tile ragged, not for fp32.  N = 256 and more: the LDS-panel kernels by a fifth.
 // fp32 storage is multiplied in bf16 parts here: only where the LDS-panel kernels would do the same (panel.split; N from 16 on,
 // in rows of whole 16-byte pieces).  Other N keep the fp32 products of the entry and gather kernels.
-bool tile_serves(const hspmm_plan *p, uint32_t N)
+static bool tile_takes(const hspmm_plan *p, uint32_t N)
 {
     const Config &c = p->cfg;
     if (!p->tile.built || c.kernel_mode != 0 || uint64_t(N) * p->elem < 16u) return false;
@@ -107,6 +108,12 @@ bool tile_serves(const hspmm_plan *p, uint32_t N)
     if (wide && !(p->panel.split && panel_serves(p, N))) return false;
     return N >= 8u && N < (wide ? 48u : 128u) && work >= (wide ? 75e6 : 65e6) && fill >= 0.04 && fill * N >= 1.5;
 }
+
+// 33 to 47 features of fp32 storage that they would take, by what has been said so far, and leave to the LDS-panel kernels, whose
+// arithmetic is the same (or, see entries_serve, to the entry kernels).
+bool tile_leaves(const hspmm_plan *p, uint32_t N) { return p->elem == 4u && p->cfg.tile <= 0 && N > 32u && tile_takes(p, N); }
+
+bool tile_serves(const hspmm_plan *p, uint32_t N) { return tile_takes(p, N) && !tile_leaves(p, N); }
 
 // 16-bit types, from 32 features on: a fit to 1233 launches (standard deviation 10 to 18 %).  33 to 63 features, which leave a C tile of 64
 // ragged, take one and a half times as long.
