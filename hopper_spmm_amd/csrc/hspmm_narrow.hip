@@ -74,8 +74,8 @@ int build_narrow_stream(hspmm_plan *p)
     return HSPMM_OK;
 }
 
-// Where they are expected to be faster than the kernels that would take the launch: by 10 % than the entry and the wide-tile kernels; the
-// full-tile and the gather kernels lose every launch but 2 of 249 (by 2 %).  Over 2075 launches the rule gives 1.22 times the speed
+// Where they are expected to be faster than the kernels that would take the launch: by 10 % than the wide-tile and the entry
+// kernels, and by 0.3 us more than these (whose short launches are faster than the fit says); the full-tile and the gather kernels lose every launch but 2 of 249 (by 2 %).  Over 2075 launches the rule gives 1.22 times the speed
 // of the entry kernels (1.27 if every launch took the faster one; 5 % of those taken lose, 5 % on average).  Up to 31 % of entries,
 // as far as times are known.
 bool narrow_serves(const hspmm_plan *p, uint32_t N)
@@ -92,7 +92,7 @@ bool narrow_serves(const hspmm_plan *p, uint32_t N)
     if (double(p->narrow.entries) > kMostEntries * p->rows * p->cols) return false;
     if (wide_serves(p, N)) return expected < 0.9 * wide_expected(p, N);
     if (tile_serves(p, N)) return true;
-    if (entries_serve(p, N)) return expected < 0.9 * entries_expected(p, N);
+    if (entries_serve(p, N)) return expected < 0.9 * entries_expected(p, N) - 0.3;
     return !panel_serves(p, N);
 }
 

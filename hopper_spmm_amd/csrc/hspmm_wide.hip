@@ -86,7 +86,7 @@ bool worth_taking(const hspmm_plan *p, uint32_t N)
     const double expected = choose_wide_shape(p, N).expected;
     if (of_blocks(p)) {
         if (panel_serves(p, N)) return expected < 0.9 * (6.2 + 0.9 * panel_expected(p, N));
-        return expected < 0.9 * blocks_gather_expected(p, N);
+        return expected < (N % 8u == 0u ? 0.75 : 0.9) * blocks_gather_expected(p, N);
     }
     if (tile_serves(p, N)) return double(p->tile.entries) <= kMostEntries * p->rows * p->cols && expected < 0.95 * tile_expected(p, N);
     if (entries_serve(p, N)) return N < 256u && expected < 0.9 * entries_expected(p, N);
@@ -139,8 +139,9 @@ int build_wide_stream(hspmm_plan *p)
 
 double wide_expected(const hspmm_plan *p, uint32_t N) { return choose_wide_shape(p, N).expected; }
 
-// Where they are expected to be faster, by 5 or 10 %, than the kernels that would take the launch; the gather kernels lose every launch
-// but one in a hundred of pruned weights.  Times by the kernels that otherwise take a launch over the time that these are expected
+// Where they are expected to be faster, by 5 or 10 % - or by a quarter, where the time to beat is known least: the gather kernels' in
+// whole 16-byte pieces -, than the kernels that would take the launch; the gather kernels lose every launch but one in a hundred of
+// pruned weights.  Times by the kernels that otherwise take a launch over the time that these are expected
 // to take, with the launches taken by this rule and those left: LDS-panel 1.22 (4385 launches, 1.23 if every one took the faster kernel),
 // full-tile 1.67 (1233, whose times are known up to kMostEntries: denser launches stay), gather 1.69 (475); of blocks of 16 x 16
 // LDS-panel 1.08 (1832), gather 1.75 (1834).
