@@ -9,6 +9,7 @@
 #include <stdint.h>
 #include <algorithm>
 #include "hspmm_device.h"
+#include "lane_ranges.hpp"
 
 namespace hspmm {
 
@@ -118,7 +119,8 @@ __device__ __forceinline__ Piece<VB> round_sums(const float (&acc)[NF])
 // Odd: 16-bit types with an odd number of elements in a row of B, whose every other row starts between two words, and loads that
 // are not whole words take twice their time (graph of 2^18, fp16, N = 65 / 66: 109 / 73 us).  Such a row is loaded from the word before on and
 // shifted by half a word, the word behind a lane's last one being its neighbour's first; the last lane of a block has seven features,
-// which the load holds either way.  Before / with it, us: that graph, N = 33 59.4 / 50.6, 65 109 / 75.5, 129 225 / 174; of 40001, N = 33 12.1 /
+// which the load holds either way, and is moved back, so that the last feature of the lane in front of it is another one's sum: that lane
+// stores what lies in front of the last lane's alone (entry_lane_stores).  Before / with it, us: that graph, N = 33 59.4 / 50.6, 65 109 / 75.5, 129 225 / 174; of 40001, N = 33 12.1 /
 // 10.3; uniform 16384^2, 64 per row, N = 17 13.9 / 10.7, 65 28.4 / 21.0, 129 50.1 / 31.5.
 template <class E, int VB, int L, int U, bool Cut, bool Odd>
 __global__ __launch_bounds__(256)
@@ -160,8 +162,8 @@ void spmm_entries_kernel(const EntryArgs ea)
     // bytes of a row this block covers, and where: a last block that would reach past the row is moved back to end with it
     const uint32_t row_len = ea.block_bytes;
     static_assert(!Odd || (VB == 16 && E::kElem == 2), "16 bytes of 16-bit elements");
-    const bool last = lane * VB + VB > row_len;
-    const uint32_t off = !last ? lane * VB : row_len - (Odd ? 14u : VB);
+    const bool last = entry_lane_last(lane, VB, row_len);
+    const uint32_t off = entry_lane_begin(lane, VB, row_len, Odd);
     const size_t pitch = size_t(ea.ld) * E::kElem;
     const size_t block = umin_e(fb * row_len, uint32_t(pitch) - row_len);
     const char *B = reinterpret_cast<const char *>(ea.B) + block + off;
@@ -305,16 +307,19 @@ void spmm_entries_kernel(const EntryArgs ea)
         }
         if (lane == 0u) __hip_atomic_store(ea.arrive + size_t(head) * ea.n_feat_blocks + fb, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    if (lane * VB >= row_len) return;                       // (a lane behind the row's end: its neighbour's copy)
+    const uint32_t stores = entry_lane_stores(lane, VB, row_len, Odd);
+    if (!stores) return;                                    // (a lane behind the row's end: its neighbour's copy)
     const Piece<VB> out = round_sums<E, VB, NF>(acc);
     char *c_row = reinterpret_cast<char *>(ea.C) + size_t(row_out) * pitch + block + off;
     if constexpr (Odd) {
-        if (last) {
+        if (stores < 16u) {                                 // (4, 8, 12 or 14 bytes)
             Piece<8> front;
             Piece<4> behind;
             Piece<2> end;
-            front.w[0] = out.w[0]; front.w[1] = out.w[1]; behind.w[0] = out.w[2]; end.w[0] = out.w[3];
-            front.store(c_row); behind.store(c_row + 8); end.store(c_row + 12);
+            front.w[0] = out.w[0]; front.w[1] = out.w[1]; behind.w[0] = stores & 8u ? out.w[2] : out.w[0]; end.w[0] = out.w[3];
+            if (stores & 8u) front.store(c_row);
+            if (stores & 4u) behind.store(c_row + (stores & 8u));
+            if (stores & 2u) end.store(c_row + 12);
             return;
         }
     }
