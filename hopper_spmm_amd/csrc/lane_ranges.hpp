@@ -1,5 +1,5 @@
-// Which bytes of a row of C a lane of the entry kernels stores: what must not overlap where two lanes hold different values.  Plain
-// C++, so that it can be checked without a GPU.
+// Which bytes of a row of C a lane of the entry kernels stores, and which features a wave of the narrow kernels: what must not overlap
+// where two of them may hold different values.  Plain C++, so that it can be checked without a GPU.
 #pragma once
 #include <stdint.h>
 
@@ -25,5 +25,12 @@ constexpr uint32_t entry_lane_stores(uint32_t lane, uint32_t lane_bytes, uint32_
     const uint32_t in_front = row_len - 14u - lane * 16u;
     return in_front < 16u ? in_front : 16u;
 }
+
+// Wave `tile` of a workgroup of the narrow kernels has sums of the features from narrow_tile_first on, 16 of an even N and 15 of an odd
+// one, and stores those from narrow_tile_own to narrow_tile_end (less those behind the last one).  The second tile of an odd N begins
+// with the first one's last feature, so that it, too, begins on a word.
+constexpr uint32_t narrow_tile_first(uint32_t tile, bool odd) { return tile * (odd ? 14u : 16u); }
+constexpr uint32_t narrow_tile_own(uint32_t tile, bool odd) { return tile * (odd ? 15u : 16u); }
+constexpr uint32_t narrow_tile_end(uint32_t tile, bool odd) { return narrow_tile_first(tile, odd) + (odd ? 15u : 16u); }
 
 }  // namespace hspmm

@@ -6,6 +6,7 @@
 // (spmm_tile_kernel.hip) share a C tile of 128 rows between workgroups, whose sums then go through memory, and put blocks together behind
 // barriers (13 us of every launch); the entry kernels read a row of B for every entry.
 #include "spmm_tile_common.hpp"
+#include "lane_ranges.hpp"
 
 namespace hspmm {
 
@@ -17,7 +18,7 @@ constexpr uint32_t kNarrowRows = 16, kNarrowImage = 4096;
 // are not whole words cost twice their time: 4096 x 11008 at 10 %, N = 15 14.6 us, 16 9.1), and a tile has 15 features.
 template <bool BF, bool ODD> struct NarrowHalf : HalfStored<BF> {
     static constexpr uint32_t kColumns = kNarrowColumns, kStep = 32, kLoads = 4, kLoadRows = 8;     // of an operand: columns, loads of B; rows of one
-    static constexpr uint32_t kTile = ODD ? 14 : 16;
+    static constexpr bool kOdd = ODD;
     __device__ static __forceinline__ uint32_t position(uint32_t m, uint32_t k)
     {
         return k / 32u * 1024u + ((k >> 1 & 3u) * 16u + m) * 16u + ((k >> 3 & 3u) * 2u + (k & 1u)) * 2u;
@@ -117,7 +118,7 @@ void spmm_narrow_kernel(const NarrowArgs na)
         uint32_t lane_b[CF];
 #pragma unroll
         for (int p = 0; p < CF; ++p) {
-            lane_f[p] = E::load_feature(lane, E::kTile * p, na.N);
+            lane_f[p] = E::load_feature(lane, narrow_tile_first(p, E::kOdd), na.N);
             lane_b[p] = E::load_row(lane) * row_bytes + uint32_t(lane_f[p]) * E::kElem;
         }
         auto request_b = [&](auto op_c, uint32_t i) __attribute__((always_inline)) {
@@ -190,17 +191,17 @@ void spmm_narrow_kernel(const NarrowArgs na)
     f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < W; ++w) v += *reinterpret_cast<const f32x4 *>(smem + w * kNarrowImage + wave * 1024u + lane * 16u);
-    const uint32_t f0 = wave * E::kTile, f = f0 + E::feature(lane);
+    const uint32_t f0 = narrow_tile_first(wave, E::kOdd), own = narrow_tile_own(wave, E::kOdd), f = f0 + E::feature(lane);
     char *c = static_cast<char *>(na.C) + size_t(row0 + 4u * g) * row_bytes + size_t(f) * E::kElem;
     float met = 0.f;
 #pragma unroll
     for (uint32_t e = 0; e < 4u; ++e) {
-        if (f < na.N && row0 + 4u * g + e < na.rows) {
+        if (f >= own && f < na.N && row0 + 4u * g + e < na.rows) {
             E::store_one(c + size_t(e) * row_bytes, v[e]);
             met = __builtin_fmaf(v[e], 0.f, met);
         }
     }
-    if (__ballot(met != 0.f)) tile_sum_again<E, 1, 16, true>(na, row0, f0, f0, lane);
+    if (__ballot(met != 0.f)) tile_sum_again<E, 1, 16, true>(na, row0, f0, own, narrow_tile_end(wave, E::kOdd), lane);
 }
 
 template <class E, int CF, int W>
@@ -221,10 +222,10 @@ static hipError_t launch_narrow_e(const NarrowArgs &na, uint32_t waves, uint32_t
 {
     const uint64_t groups = (uint64_t(na.rows) + kNarrowRows - 1u) / kNarrowRows;
     // (a load of B reads two elements, and a lane has the first entries of each of its wave's blocks)
-    if (!na.rows || !na.N || uint64_t(na.N) * na.cols < 2u || na.N > (E::kTile == 16u ? 32u : 29u) || groups >= (1u << 21) ||
+    if (!na.rows || !na.N || uint64_t(na.N) * na.cols < 2u || na.N > narrow_tile_end(1, E::kOdd) || groups >= (1u << 21) ||
         uint64_t(na.n_blocks) * E::kColumns < na.cols || na.n_blocks > kNarrowMostBlocks || na.n_blocks > 64u * waves)
         return hipErrorInvalidValue;
-    constexpr uint32_t kOne = E::kTile == 16u ? 16u : 15u;          // features of one tile
+    constexpr uint32_t kOne = narrow_tile_end(0, E::kOdd);          // features of one tile
     if (waves == 4u) return na.N <= kOne ? launch_narrow<E, 1, 4>(na, loads, uint32_t(groups), s) : launch_narrow<E, 2, 4>(na, loads, uint32_t(groups), s);
     if (waves == 8u) return na.N <= kOne ? launch_narrow<E, 1, 8>(na, loads, uint32_t(groups), s) : launch_narrow<E, 2, 8>(na, loads, uint32_t(groups), s);
     if (waves == 16u) return na.N <= kOne ? launch_narrow<E, 1, 16>(na, loads, uint32_t(groups), s) : launch_narrow<E, 2, 16>(na, loads, uint32_t(groups), s);

@@ -83,12 +83,13 @@ __device__ __forceinline__ void for_entries(const TileSource &src, uint32_t row0
 }
 
 // Sums 16 RF rows x WIDTH features of C again, over the stored entries of the plan's tiles alone, where C is not finite: only
-// rows that name a row of B then get what its infinities and NaNs make of them.  Features below `own` belong to another tile.
+// rows that name a row of B then get what its infinities and NaNs make of them.  Features below `own` and from `end` on belong to other
+// waves, which may still be storing them.
 // A wave with its lanes on features, 64 / WIDTH tiles of a window at a time, two trips to memory each: slow, and off the path of
 // finite data (bf16, 4096 x 11008 at 10 %, N = 16: 1.0 ms with an infinity in B, 17.3 us without, as before the check).
 // FEW: fewer registers, a trip more per row of a tile.
 template <class E, int RF, uint32_t WIDTH, bool FEW = false, class Args>
-__device__ __forceinline__ void tile_sum_again(const Args &ta, const uint32_t row0, const uint32_t f0, const uint32_t own, const uint32_t lane)
+__device__ __forceinline__ void tile_sum_again(const Args &ta, const uint32_t row0, const uint32_t f0, const uint32_t own, const uint32_t end, const uint32_t lane)
 {
     constexpr uint32_t kShares = 64u / WIDTH, CW = E::kElem == 4u ? 8u : 16u;
     const TileSource src = *ta.src;
@@ -100,7 +101,7 @@ __device__ __forceinline__ void tile_sum_again(const Args &ta, const uint32_t ro
     bool found = false;
     for (uint32_t m = share; m < RF * 16u; m += kShares)
         if (row0 + m < ta.rows) found |= E::not_finite(E::load_one(c_lane + size_t(row0 + m) * row_bytes));
-    const uint64_t lanes = __ballot(found && f >= own && f < ta.N);
+    const uint64_t lanes = __ballot(found && f >= own && f < umin32(end, ta.N));
     if (!lanes) return;
     bool again = false;
     for (uint32_t s = 0; s < kShares; ++s) again |= (lanes >> (s * WIDTH + mine)) & 1u;

@@ -387,7 +387,7 @@ void spmm_tile_kernel(const TileArgs ta)
     if (i < end) chunk(i, Set0{});
     for (uint32_t t = again_begin; t < again_end; ++t) {
         const uint32_t rb = t / ta.n_feat_tiles, ft = t - rb * ta.n_feat_tiles;
-        tile_sum_again<E, RF, CF * 16u>(ta, rb * kTileRows + wr * RF * 16u, first_feature(ft) + wc * CF * 16u, ft * NT, lane);
+        tile_sum_again<E, RF, CF * 16u>(ta, rb * kTileRows + wr * RF * 16u, first_feature(ft) + wc * CF * 16u, ft * NT, ta.N, lane);
     }
 }
 

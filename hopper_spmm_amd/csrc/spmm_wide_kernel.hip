@@ -206,7 +206,7 @@ void spmm_wide_kernel(const WideArgs wa)
     if (__ballot(met != 0.f)) {
         constexpr uint32_t kOnce = NT < 64u ? NT : 64u;
 #pragma unroll 1
-        for (uint32_t f = 0; f < NT; f += kOnce) tile_sum_again<E, RF, kOnce>(wa, row0, f0 + f, own, lane);
+        for (uint32_t f = 0; f < NT; f += kOnce) tile_sum_again<E, RF, kOnce>(wa, row0, f0 + f, own, wa.N, lane);
     }
 }
 
@@ -229,7 +229,7 @@ __global__ __launch_bounds__(256) void wide_sum_kernel(const WideArgs wa, const 
     float met = 0.f;
 #pragma unroll
     for (int e = 0; e < 4; ++e) met = __builtin_fmaf(v[e], 0.f, met);
-    if (__ballot(met != 0.f)) tile_sum_again<E, 1, 16, true>(wa, row0, f0, own, lane);
+    if (__ballot(met != 0.f)) tile_sum_again<E, 1, 16, true>(wa, row0, f0, own, wa.N, lane);
 }
 
 template <class E>

@@ -1,4 +1,4 @@
-"""Which bytes of C the lanes of a kernel store (csrc/lane_ranges.hpp, compiled here for the host): every byte once where two lanes hold
+"""Which bytes of C the lanes or waves of a kernel store (csrc/lane_ranges.hpp, compiled here for the host): every byte once where two lanes hold
 different sums, and only bytes whose sum the lane has.  No GPU needed."""
 import ctypes
 import os
@@ -12,6 +12,9 @@ SOURCE = """
 using namespace hspmm;
 extern "C" unsigned begin(unsigned lane, unsigned bytes, unsigned row_len, int odd) { return entry_lane_begin(lane, bytes, row_len, odd); }
 extern "C" unsigned stores(unsigned lane, unsigned bytes, unsigned row_len, int odd) { return entry_lane_stores(lane, bytes, row_len, odd); }
+extern "C" unsigned first(unsigned tile, int odd) { return narrow_tile_first(tile, odd); }
+extern "C" unsigned own(unsigned tile, int odd) { return narrow_tile_own(tile, odd); }
+extern "C" unsigned end(unsigned tile, int odd) { return narrow_tile_end(tile, odd); }
 """
 
 
@@ -62,3 +65,17 @@ def test_whole_rows_of_the_entry_kernels(ranges, lane_bytes, lanes, elem):
             assert b + lane_bytes <= row_len
             covered.update(range(b, b + n))
         assert covered == set(range(row_len))
+
+
+@pytest.mark.parametrize("N", range(1, 33))
+def test_a_feature_of_the_narrow_kernels_is_one_waves(ranges, N):
+    """Also where it is summed again, for which a wave reads what it has stored: not what another wave may not have."""
+    odd = N % 2
+    if N > ranges.end(1, odd):
+        pytest.skip("more than two tiles")
+    tiles = 1 if N <= ranges.end(0, odd) else 2
+    stored = [f for t in range(tiles) for f in range(ranges.own(t, odd), min(N, ranges.end(t, odd)))]
+    assert stored == list(range(N))
+    for t in range(tiles):
+        assert ranges.first(t, odd) <= ranges.own(t, odd) and ranges.end(t, odd) <= ranges.first(t, odd) + 16      # (what its lanes have)
+        assert ranges.first(t, odd) % 2 == 0

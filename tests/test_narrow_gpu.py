@@ -52,6 +52,35 @@ def test_infinities_and_nans_stay_with_the_rows_that_name_them(torch_cuda, hs, m
     nonfinite.test_infinities_and_nans_stay_with_the_rows_that_name_them(torch_cuda, hs, "tile", dtype, rows, cols)
 
 
+@pytest.mark.parametrize("dtype", [0, 2])
+def test_sums_beside_an_infinity_do_not_depend_on_what_c_held(torch_cuda, hs, dtype):
+    """Two tiles of an odd N share a feature: a wave that sums again reads its own features of C alone.  Sums of real numbers, whose bits
+    show the order of the additions; finite features are those of the product without the infinity."""
+    torch = torch_cuda
+    rng = np.random.default_rng(dtype)
+    A = _sampled_csr(rng, 1000, 1500, 200, dtype, lambda n: rng.normal(size=n))
+    plan = _plan(hs, A, NARROW=1)
+    stream = torch.cuda.current_stream().cuda_stream
+    nan = 0x7E01 if dtype == 0 else 0x7FC0
+    for N in range(17, 30, 2):
+        _, dB = _random_operand(torch, rng, 1500, N, dtype)
+        clean = torch.full((1000, N), nan, dtype=torch.int16, device="cuda")
+        plan.run(dB.data_ptr(), clean.data_ptr(), N, stream)
+        for bad in (0, 13, 14, 15, N - 1):
+            worse = dB.clone()
+            worse[700, bad] = 0x7C00 if dtype == 0 else 0x7F80
+            outs = []
+            for held in (nan, 7, nan):
+                dC = torch.full((1000, N), held, dtype=torch.int16, device="cuda")
+                plan.run(worse.data_ptr(), dC.data_ptr(), N, stream)
+                outs.append(dC)
+            assert plan.last_kernel() == "spmm_narrow_kernel"
+            assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2]), (N, bad)
+            fine = [f for f in range(N) if f != bad]
+            assert torch.equal(outs[0][:, fine], clean[:, fine]), (N, bad)
+    plan.close()
+
+
 # Against fp64, as for the wide-tile kernels: n additions of exact products, and the result's own rounding.
 @pytest.mark.parametrize("dtype,rows,cols,per_row,N,narrow", [
     (2, 4096, 11008, 1100, 16, True), (0, 4096, 4096, 1200, 15, True), (2, 1500, 9001, 2000, 29, True), (0, 4096, 11008, 1100, 1, True),
