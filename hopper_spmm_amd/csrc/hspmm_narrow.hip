@@ -55,19 +55,25 @@ int build_narrow_stream(hspmm_plan *p)
     if (n_blocks > kNarrowMostBlocks || uint64_t(n_units) * n_blocks >= (1u << 28) || n_units >= (1u << 21)) return HSPMM_OK;
     const uint32_t all = n_units * n_blocks;
     const TileSource src{p->d_rowOffset, p->d_rowIdx, p->d_a2b_raw, p->d_data, p->W, p->cols};
-    void *blocks = nullptr, *entries = nullptr;
-    if (int rc = plan_alloc(p, (size_t(all) + 1u) * 4u, &blocks)) return rc;
+    // (a plan whose device memory does not hold the stream, or what it takes to make it, is made without)
+    const size_t blocks_bytes = (size_t(all) + 1u) * 4u;
+    void *blocks = nullptr, *entries = nullptr, *source = nullptr;
     struct Temporary { void *p = nullptr; ~Temporary() { (void)hipFree(p); } } counts;
-    HSPMM_HIP(hipMalloc(&counts.p, size_t(all) * 4u));
+    auto without = [&]() {
+        (void)hipGetLastError();
+        plan_release(p, blocks, blocks_bytes);
+        plan_release(p, source, sizeof src);
+        return HSPMM_OK;
+    };
+    if (plan_alloc(p, blocks_bytes, &blocks) || plan_alloc(p, sizeof src, &source) || hipMalloc(&counts.p, size_t(all) * 4u) != hipSuccess) return without();
     HSPMM_HIP(launch_narrow_count(src, n_units, n_blocks, static_cast<uint32_t *>(counts.p), static_cast<uint32_t *>(blocks), nullptr));
     uint32_t fours = 0;
     HSPMM_HIP(hipMemcpy(&fours, static_cast<uint32_t *>(blocks) + all, 4, hipMemcpyDeviceToHost));
-    if (fours >= (1u << 30)) return HSPMM_OK;
-    if (plan_alloc(p, size_t(fours) * 16u, &entries)) { (void)hipGetLastError(); return HSPMM_OK; }        // (no memory: a plan without)
+    if (fours >= (1u << 30) || plan_alloc(p, size_t(fours) * 16u, &entries)) return without();
     HSPMM_HIP(launch_narrow_fill(src, n_units, n_blocks, static_cast<uint32_t *>(counts.p), static_cast<uint32_t *>(blocks), static_cast<uint32_t *>(entries), nullptr));
-    if (int rc = upload(p, &n.d_source, &src, 1)) return rc;
+    HSPMM_HIP(hipMemcpy(source, &src, sizeof src, hipMemcpyHostToDevice));
     HSPMM_HIP(hipStreamSynchronize(nullptr));
-    n.d_blocks = static_cast<uint32_t *>(blocks); n.d_entries = static_cast<uint32_t *>(entries);
+    n.d_blocks = static_cast<uint32_t *>(blocks); n.d_entries = static_cast<uint32_t *>(entries); n.d_source = static_cast<TileSource *>(source);
     n.entries = uint64_t(fours) * 4u;
     n.n_units = n_units; n.n_blocks = n_blocks;
     n.built = true;

@@ -123,15 +123,19 @@ int build_wide_stream(hspmm_plan *p)
     if (p->cfg.wide < 0 && (of_blocks(p) ? fill < 0.15 : p->G != 1 || p->per_column > 4.0 || fill < 0.04)) return HSPMM_OK;
     const uint32_t n_units = (p->rows + 15u) / 16u, n_chunks = ((p->cols + 63u) / 64u + 3u) & ~3u;
     const TileSource src{p->d_rowOffset, p->d_rowIdx, p->d_a2b_raw, p->d_data, p->W, p->cols};
-    // (a plan whose device memory holds no such stream is made without)
+    // (a plan whose device memory does not hold the stream is made without)
     const size_t bytes = size_t(n_units) * n_chunks * kWideUnitBytes;
-    void *frags = nullptr;
+    void *frags = nullptr, *source = nullptr;
     if (bytes > kMostBytes) return HSPMM_OK;
-    if (plan_alloc(p, bytes, &frags)) { (void)hipGetLastError(); return HSPMM_OK; }
+    if (plan_alloc(p, bytes, &frags) || plan_alloc(p, sizeof src, &source)) {
+        (void)hipGetLastError();
+        plan_release(p, frags, bytes);
+        return HSPMM_OK;
+    }
     HSPMM_HIP(launch_wide_fill(src, p->rows, n_chunks, frags, nullptr));
-    if (int rc = upload(p, &w.d_source, &src, 1)) return rc;
+    HSPMM_HIP(hipMemcpy(source, &src, sizeof src, hipMemcpyHostToDevice));
     HSPMM_HIP(hipStreamSynchronize(nullptr));
-    w.d_frags = frags;
+    w.d_frags = frags; w.d_source = static_cast<TileSource *>(source);
     w.n_units = n_units; w.n_chunks = n_chunks;
     w.built = true;
     return HSPMM_OK;

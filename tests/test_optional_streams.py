@@ -1,0 +1,94 @@
+"""Streams a plan can do without (narrow and wide-tile kernels): their host code, compiled here without its kernels and with a device
+memory that runs out at any allocation.  No GPU needed."""
+import os
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "hopper_spmm_amd", "csrc")
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
+DRIVER = r"""
+#include "hspmm_plan.hpp"
+#include <cstdarg>
+#include <set>
+
+static int left;                                    // allocations that succeed
+static std::set<void *> held;
+extern "C" {
+hipError_t hipMalloc(void **p, size_t) { if (left-- <= 0) return hipErrorOutOfMemory; held.insert(*p = std::malloc(64)); return hipSuccess; }
+hipError_t hipFree(void *p) { if (p) { held.erase(p); std::free(p); } return hipSuccess; }
+hipError_t hipMemcpy(void *to, const void *from, size_t n, hipMemcpyKind kind) { if (kind == hipMemcpyDeviceToHost) std::memset(to, 1, 1), std::memset((char *)to + 1, 0, n - 1); else std::memcpy(to, from, n); return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipGetLastError() { return hipSuccess; }
+const char *hipGetErrorString(hipError_t) { return ""; }
+}
+namespace hspmm {
+hipError_t launch_narrow_count(const TileSource &, uint32_t, uint32_t, uint32_t *, uint32_t *, hipStream_t) { return hipSuccess; }
+hipError_t launch_narrow_fill(const TileSource &, uint32_t, uint32_t, const uint32_t *, const uint32_t *, uint32_t *, hipStream_t) { return hipSuccess; }
+hipError_t launch_spmm_narrow(int, const NarrowArgs &, uint32_t, uint32_t, hipStream_t) { return hipErrorInvalidValue; }
+hipError_t launch_spmm_wide(int, const WideArgs &, const WideShape &, hipStream_t) { return hipErrorInvalidValue; }
+hipError_t launch_wide_fill(const TileSource &, uint32_t, uint32_t, void *, hipStream_t) { return hipSuccess; }
+}
+namespace hspmm_host {
+int fail(int code, const char *, ...) { return code; }
+// (as in hspmm_create.hip, without the reserved block)
+int plan_alloc(hspmm_plan *p, size_t bytes, void **out) { HSPMM_HIP(hipMalloc(out, bytes)); p->owned.push_back(*out); p->fixed_bytes += bytes; return HSPMM_OK; }
+void plan_release(hspmm_plan *p, const void *ptr, size_t bytes)
+{
+    const auto it = std::find(p->owned.begin(), p->owned.end(), ptr);
+    if (it == p->owned.end()) return;
+    (void)hipFree(*it); p->owned.erase(it); p->fixed_bytes -= bytes;
+}
+int scratch_for(hspmm_plan *, hipStream_t, size_t, RunMode, float **) { return HSPMM_ERR_DEVICE; }
+double entries_expected(const hspmm_plan *, uint32_t) { return 100.0; }
+bool entries_serve(const hspmm_plan *, uint32_t) { return false; }
+double panel_expected(const hspmm_plan *, uint32_t) { return 100.0; }
+bool panel_serves(const hspmm_plan *, uint32_t) { return true; }
+double tile_expected(const hspmm_plan *, uint32_t) { return 100.0; }
+bool tile_serves(const hspmm_plan *, uint32_t) { return false; }
+}
+
+int main()
+{
+    using namespace hspmm_host;
+    for (int which = 0; which < 2; ++which) {
+        int needs = -1;
+        for (int n = 0; n < 8; ++n) {
+            hspmm_plan p;
+            // 4096 x 4096 at 10 %, bf16: 32 columns' worth of tiles a window, a sixth of their elements stored
+            p.dtype = HSPMM_BF16; p.rows = p.cols = 4096; p.W = 512; p.T = 512 * 146; p.compute_units = 256; p.per_column = 1.4;
+            left = n;
+            const int rc = which ? build_wide_stream(&p) : build_narrow_stream(&p);
+            const bool built = which ? p.wide.built : p.narrow.built;
+            if (rc) { std::printf("%d: %d allocations: plan creation fails\n", which, n); return 1; }
+            if (built && needs < 0) needs = n;
+            if (built != (needs >= 0)) { std::printf("%d: %d allocations: built %d\n", which, n, int(built)); return 1; }
+            if (!built && (!held.empty() || !p.owned.empty() || p.fixed_bytes)) { std::printf("%d: %d allocations: %zu not given back\n", which, n, held.size()); return 1; }
+            if (built && held.size() != p.owned.size()) { std::printf("%d: %zu left behind\n", which, held.size() - p.owned.size()); return 1; }
+            for (void *x : p.owned) (void)hipFree(x);
+        }
+        if (needs < 2) { std::printf("%d: never built\n", which); return 1; }
+    }
+    std::printf("ok\n");
+    return 0;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def build(tmp_path_factory):
+    """Compiles a driver and links it with the host code of the two kernel families."""
+    at = tmp_path_factory.mktemp("streams")
+    compile_ = ["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(ROCM, "include"), "-I", CSRC, "-x", "c++"]
+
+    def make(driver):
+        (at / "driver.cpp").write_text(driver)
+        sources = [os.path.join(CSRC, "hspmm_narrow.hip"), os.path.join(CSRC, "hspmm_wide.hip"), str(at / "driver.cpp")]
+        subprocess.run(compile_ + sources + ["-o", str(at / "driver"), "-lpthread"], check=True)
+        return str(at / "driver")
+    return make
+
+
+def test_a_plan_without_memory_for_them_is_made_without(build):
+    run = subprocess.run([build(DRIVER)], stdout=subprocess.PIPE, timeout=60)
+    assert run.returncode == 0 and run.stdout == b"ok\n", run.stdout.decode()
