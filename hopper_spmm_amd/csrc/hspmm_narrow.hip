@@ -43,12 +43,13 @@ uint32_t choose_waves(const hspmm_plan *p, uint32_t N, double *expected)
 namespace hspmm_host {
 
 // Made where some feature dimension would take it by the stored entries as estimated from a sample.  Block-clustered weights (over four
-// of a column's eight elements stored) stay with kernels that read whole tiles.
+// of a column's eight elements stored) stay with kernels that read whole tiles, and plans that keep the caller's cuts of windows with
+// kernels that walk windows.
 int build_narrow_stream(hspmm_plan *p)
 {
     using namespace hspmm;
     hspmm_plan::Narrow &n = p->narrow;
-    if (p->elem != 2u || p->cfg.narrow == 0 || !p->canonical || p->cfg.kernel_mode != 0 || !p->T || p->W >= (1u << 23) || p->cols < 2u) return HSPMM_OK;
+    if (p->elem != 2u || p->cfg.narrow == 0 || !p->canonical || p->cfg.kernel_mode != 0 || !p->T || p->W >= (1u << 23) || p->cols < 2u || !p->caller_cuts.empty()) return HSPMM_OK;
     const double fill = double(p->T) * p->cw * p->per_column / (double(p->rows) * p->cols);
     if (p->cfg.narrow < 0 && (p->G != 1 || p->per_column > 4.0 || fill < kFewestEntries || fill > 1.1 * kMostEntries)) return HSPMM_OK;
     const uint32_t n_units = (p->rows + 15u) / 16u, n_blocks = (p->cols + kNarrowColumns - 1u) / kNarrowColumns;

@@ -113,12 +113,13 @@ namespace hspmm_host {
 
 // Made where some feature dimension would take it by the stored entries as estimated from a sample: from 4 % on (at 3 to 4 % the
 // launches it would take gain 2 % of the time of all, at 4 to 6 % 12 %, above 10 % 31 %, for 2 bytes per element of the matrix), of weights in
-// 16 x 16 blocks (units of two windows, over four of a column's eight elements stored) from 15 % on.
+// 16 x 16 blocks (units of two windows, over four of a column's eight elements stored) from 15 % on.  Plans that keep the caller's cuts
+// of windows stay with kernels that walk windows.
 int build_wide_stream(hspmm_plan *p)
 {
     using namespace hspmm;
     hspmm_plan::Wide &w = p->wide;
-    if (p->elem != 2u || p->cfg.wide == 0 || !p->canonical || p->cfg.kernel_mode != 0 || !p->T || p->W >= (1u << 23)) return HSPMM_OK;
+    if (p->elem != 2u || p->cfg.wide == 0 || !p->canonical || p->cfg.kernel_mode != 0 || !p->T || p->W >= (1u << 23) || !p->caller_cuts.empty()) return HSPMM_OK;
     const double fill = double(p->T) * p->cw * p->per_column / (double(p->rows) * p->cols);
     if (p->cfg.wide < 0 && (of_blocks(p) ? fill < 0.15 : p->G != 1 || p->per_column > 4.0 || fill < 0.04)) return HSPMM_OK;
     const uint32_t n_units = (p->rows + 15u) / 16u, n_chunks = ((p->cols + 63u) / 64u + 3u) & ~3u;

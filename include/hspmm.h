@@ -231,9 +231,10 @@ int hspmm_set_panel_stream(int mode);
  * groups (atomic = 1) is cut only where one of its groups ends, a window given as one group is
  * never cut; partial sums of a cut window are added in group order, not with atomics.  Kept by
  * plans whose units are the caller's single windows walked by the gather kernels
- * (hspmm_plan_info.group_cuts_kept = 1); plans that merge windows with one column list, the
- * LDS-staging kernels (they walk a re-tiled stream) and the all-shapes kernel (one wave per
- * window, nothing cut) have no use for the cuts.  The product is the same up to the order of the
+ * (hspmm_plan_info.group_cuts_kept = 1; such plans have no entry, narrow and wide-tile
+ * kernels); plans that merge windows with one column list, the LDS-panel and full-tile kernels
+ * (they walk a re-tiled stream) and the all-shapes kernel (one wave per window, nothing cut)
+ * have no use for the cuts.  The product is the same up to the order of the
  * fp32 additions of a cut window. */
 int hspmm_set_group_cuts(int mode);
 

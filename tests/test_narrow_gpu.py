@@ -52,6 +52,30 @@ def test_infinities_and_nans_stay_with_the_rows_that_name_them(torch_cuda, hs, m
     nonfinite.test_infinities_and_nans_stay_with_the_rows_that_name_them(torch_cuda, hs, "tile", dtype, rows, cols)
 
 
+def test_plans_that_keep_the_callers_cuts_leave_launches_to_the_kernels_that_honour_them(torch_cuda, hs):
+    torch = torch_cuda
+    rng = np.random.default_rng(8)
+    A = _sampled_csr(rng, 4096, 4096, 600, 2, lambda n: rng.integers(1, 3, n))
+    grouped = hs.bitmap_to_grouped(hs.csr_to_bitmap(4096, 4096, A["row_ptr"], A["col_idx"], A["values"], 2), min_len=40)
+    hs.set_group_cuts(1)
+    try:
+        kept = hs.Plan(grouped)
+    finally:
+        hs.set_group_cuts(0)
+    free = hs.Plan(grouped)
+    assert kept.info()["group_cuts_kept"] == 1 and free.info()["group_cuts_kept"] == 0
+    stream = torch.cuda.current_stream().cuda_stream
+    for N, chosen, left in ((4, "spmm_narrow_kernel", "spmm_mfma_kernel"), (16, "spmm_narrow_kernel", "spmm_mfma_kernel"), (256, "spmm_wide_kernel", "spmm_panel_kernel")):
+        dB = torch.from_numpy(encode(rng.integers(-1, 2, (4096, N)).astype(np.float32), 2).view(np.int16)).cuda()     # (exact sums)
+        outs = [torch.full((4096, N), 7, dtype=torch.int16, device="cuda") for _ in range(2)]
+        for plan, out, kernel in ((free, outs[0], chosen), (kept, outs[1], left)):
+            plan.run(dB.data_ptr(), out.data_ptr(), N, stream)
+            assert plan.last_kernel() == kernel, N
+        assert torch.equal(outs[0], outs[1])
+    kept.close()
+    free.close()
+
+
 @pytest.mark.parametrize("dtype", [0, 2])
 def test_sums_beside_an_infinity_do_not_depend_on_what_c_held(torch_cuda, hs, dtype):
     """Two tiles of an odd N share a feature: a wave that sums again reads its own features of C alone.  Sums of real numbers, whose bits

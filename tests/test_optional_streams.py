@@ -67,6 +67,13 @@ int main()
             if (built && held.size() != p.owned.size()) { std::printf("%d: %zu left behind\n", which, held.size() - p.owned.size()); return 1; }
             for (void *x : p.owned) (void)hipFree(x);
         }
+        {
+            hspmm_plan p;
+            p.dtype = HSPMM_BF16; p.rows = p.cols = 4096; p.W = 512; p.T = 512 * 146; p.compute_units = 256; p.per_column = 1.4;
+            p.caller_cuts = {0, 100, p.T};
+            left = 100;
+            if ((which ? build_wide_stream(&p) : build_narrow_stream(&p)) || p.wide.built || p.narrow.built || left != 100) { std::printf("%d: built for a plan with its own cuts\n", which); return 1; }
+        }
         if (needs < 2) { std::printf("%d: never built\n", which); return 1; }
     }
     std::printf("ok\n");
@@ -89,6 +96,6 @@ def build(tmp_path_factory):
     return make
 
 
-def test_a_plan_without_memory_for_them_is_made_without(build):
+def test_a_plan_is_made_without_them_for_want_of_memory_or_use(build):
     run = subprocess.run([build(DRIVER)], stdout=subprocess.PIPE, timeout=60)
     assert run.returncode == 0 and run.stdout == b"ok\n", run.stdout.decode()
