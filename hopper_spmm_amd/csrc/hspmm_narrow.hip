@@ -97,7 +97,7 @@ bool narrow_serves(const hspmm_plan *p, uint32_t N)
         c.panel_units_per_group || c.aligned_small >= 0 || c.xcd_split >= 0 || c.gather_bitmap >= 0 || c.tile > 0 || c.entries > 0 || c.wide > 0)
         return false;
     if (double(p->narrow.entries) > kMostEntries * p->rows * p->cols) return false;
-    if (wide_serves(p, N)) return expected < 0.9 * wide_expected(p, N);
+    if (wide_serves(p, N)) return expected < 0.9 * p->wide.expected_fewest;     // (N = 32)
     if (tile_serves(p, N)) return true;
     if (entries_serve(p, N)) return expected < 0.9 * entries_expected(p, N) - 0.3;
     return !panel_serves(p, N);

@@ -107,6 +107,20 @@ extern Config g_cfg;
 
 constexpr uint32_t kMinTilesPerRange = 24;
 
+// What a plan answers for a feature dimension, kept for the last few asked for, 32 bits each: the answers are the plan's and N's alone, so
+// threads may overwrite each other's.  (A search costs a launch 0.5 to 1 us of the host's; 16, 32, .. 1024 have a slot each.)
+class KeptAnswers {
+    std::atomic<uint64_t> slots_[16] = {};
+public:
+    template <class F> uint32_t get(uint32_t N, F find)
+    {
+        std::atomic<uint64_t> &slot = slots_[N * 0x9E3779B1u >> 28];
+        uint64_t kept = slot.load(std::memory_order_relaxed);
+        if (uint32_t(kept >> 32) != N) slot.store(kept = uint64_t(N) << 32 | find(), std::memory_order_relaxed);
+        return uint32_t(kept);
+    }
+};
+
 }  // namespace hspmm_host
 
 struct hspmm_plan {
@@ -164,6 +178,7 @@ struct hspmm_plan {
         void *d_vals = nullptr;
         uint32_t *d_step_voff = nullptr;
         double density = 0.0;                                    // steps per unit and 128 columns of the gather stream
+        mutable hspmm_host::KeptAnswers expected;                // (see panel_expected)
     } panel;
     // Bitmap stream of the gather kernels (single 16-bit windows whose tiles are mostly zeros): per tile 8 words
     // of header (the reference's tcBit words of the tile, bit counts, position of the first stored element) and
@@ -215,7 +230,8 @@ struct hspmm_plan {
         const void *d_frags = nullptr;
         hspmm::TileSource *d_source = nullptr;
         uint32_t n_units = 0, n_chunks = 0;
-        mutable std::atomic<uint64_t> choice{0};                 // of the last N asked for (see hspmm_wide.hip)
+        double expected_fewest = 0.0;                            // us, of the fewest features they take (see hspmm_wide.hip)
+        mutable hspmm_host::KeptAnswers choices;
     } wide;
     double per_column = 8.0;            // stored entries per tile column, from a sample of the tiles
     bool even_windows = false;          // no unit has over eight times the average number of steps
@@ -339,7 +355,6 @@ int run_narrow(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t 
 // hspmm_wide.hip: the wide-tile kernels' stream, whether they take this launch, and the launch
 int build_wide_stream(hspmm_plan *p);
 bool wide_serves(const hspmm_plan *p, uint32_t N);
-double wide_expected(const hspmm_plan *p, uint32_t N);          // us
 int run_wide(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode);
 
 // hspmm_run.hip: the address of the device's fixed scratch array (hspmm_run_static); `device` must be current

@@ -394,8 +394,16 @@ bool hspmm_host::panel_serves(const hspmm_plan *p, uint32_t N)
 
 double hspmm_host::panel_expected(const hspmm_plan *p, uint32_t N)
 {
-    PanelShape sh;
-    return choose_panel_shape(p, N, &sh) == HSPMM_OK ? sh.expected : 0.0;
+    const uint32_t bits = p->panel.expected.get(N, [&]() {
+        PanelShape sh;
+        const float expected = choose_panel_shape(p, N, &sh) == HSPMM_OK ? float(sh.expected) : 0.f;
+        uint32_t word;
+        std::memcpy(&word, &expected, 4);
+        return word;
+    });
+    float expected;
+    std::memcpy(&expected, &bits, 4);
+    return expected;
 }
 
 static int run_gather(hspmm_plan *p, const void *dB, void *dC, uint32_t N, uint32_t ld, hipStream_t s, hipEvent_t mid, RunMode mode);

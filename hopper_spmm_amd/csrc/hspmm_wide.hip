@@ -94,17 +94,14 @@ bool worth_taking(const hspmm_plan *p, uint32_t N)
     return true;
 }
 
-// The answer for an N is the plan's alone, and is kept for the last N (a launch would otherwise take two microseconds of the host's):
-// N, index of the shape, cuts, whether the launch is taken.
-uint64_t kept_choice(const hspmm_plan *p, uint32_t N)
+// Index of the shape, cuts, whether the launch is taken.
+uint32_t kept_choice(const hspmm_plan *p, uint32_t N)
 {
-    uint64_t kept = p->wide.choice.load(std::memory_order_relaxed);
-    if (kept >> 32 == N) return kept;
-    const WideChoice choice = choose_wide_shape(p, N);
-    const bool taken = choice.cost && workgroups(p, N, choice.cost->shape) * choice.cuts < (1u << 22) && (p->cfg.wide > 0 || worth_taking(p, N));
-    kept = uint64_t(N) << 32 | (choice.cost ? uint32_t(choice.cost - kShapes) << 16 : 0u) | choice.cuts << 8 | (taken ? 1u : 0u);
-    p->wide.choice.store(kept, std::memory_order_relaxed);
-    return kept;
+    return p->wide.choices.get(N, [&]() -> uint32_t {
+        const WideChoice choice = choose_wide_shape(p, N);
+        const bool taken = choice.cost && workgroups(p, N, choice.cost->shape) * choice.cuts < (1u << 22) && (p->cfg.wide > 0 || worth_taking(p, N));
+        return (choice.cost ? uint32_t(choice.cost - kShapes) << 16 : 0u) | choice.cuts << 8 | (taken ? 1u : 0u);
+    });
 }
 
 }  // namespace
@@ -138,11 +135,10 @@ int build_wide_stream(hspmm_plan *p)
     HSPMM_HIP(hipStreamSynchronize(nullptr));
     w.d_frags = frags; w.d_source = static_cast<TileSource *>(source);
     w.n_units = n_units; w.n_chunks = n_chunks;
+    w.expected_fewest = choose_wide_shape(p, kFewestFeatures).expected;
     w.built = true;
     return HSPMM_OK;
 }
-
-double wide_expected(const hspmm_plan *p, uint32_t N) { return choose_wide_shape(p, N).expected; }
 
 // Where they are expected to be faster, by 5 or 10 % - or by a quarter, where the time to beat is known least: the gather kernels' in
 // whole 16-byte pieces -, than the kernels that would take the launch; the gather kernels lose every launch but one in a hundred of
@@ -166,11 +162,11 @@ bool wide_serves(const hspmm_plan *p, uint32_t N)
 int run_wide(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode)
 {
     const hspmm_plan::Wide &w = p->wide;
-    const uint64_t choice = kept_choice(p, N);
+    const uint32_t choice = kept_choice(p, N);
     const hspmm::WideShape &sh = kShapes[choice >> 16 & 0xFFu].shape;
     const uint64_t groups = workgroups(p, N, sh);
     hspmm::WideArgs wa{};
-    wa.n_cuts = uint32_t(choice >> 8 & 0xFFu);
+    wa.n_cuts = choice >> 8 & 0xFFu;
     if (wa.n_cuts > 1u) {
         std::lock_guard<std::mutex> lk(p->mu);
         if (const int rc = scratch_for(p, s, size_t(groups * wa.n_cuts * tile_sums_bytes(sh)), mode, &wa.sums)) return rc;

@@ -1,5 +1,5 @@
 """Streams a plan can do without (narrow and wide-tile kernels): their host code, compiled here without its kernels and with a device
-memory that runs out at any allocation.  No GPU needed."""
+memory that runs out at any allocation; what it answers for feature dimensions in turn.  No GPU needed."""
 import os
 import subprocess
 
@@ -43,7 +43,8 @@ int scratch_for(hspmm_plan *, hipStream_t, size_t, RunMode, float **) { return H
 double entries_expected(const hspmm_plan *, uint32_t) { return 100.0; }
 bool entries_serve(const hspmm_plan *, uint32_t) { return false; }
 double panel_expected(const hspmm_plan *, uint32_t) { return 100.0; }
-bool panel_serves(const hspmm_plan *, uint32_t) { return true; }
+static int asked;                                   // searches for a feature dimension's kernel
+bool panel_serves(const hspmm_plan *, uint32_t) { ++asked; return true; }
 double tile_expected(const hspmm_plan *, uint32_t) { return 100.0; }
 bool tile_serves(const hspmm_plan *, uint32_t) { return false; }
 }
@@ -76,6 +77,18 @@ int main()
         }
         if (needs < 2) { std::printf("%d: never built\n", which); return 1; }
     }
+    hspmm_plan p;
+    p.dtype = HSPMM_BF16; p.rows = p.cols = 4096; p.W = 512; p.T = 512 * 146; p.compute_units = 256; p.per_column = 1.4;
+    left = 100;
+    if (build_wide_stream(&p)) return 1;
+    bool first[6], same = true;
+    for (int round = 0; round < 10; ++round)
+        for (int i = 0; i < 6; ++i) {
+            const bool serves = wide_serves(&p, 32u << i);
+            if (round == 0) first[i] = serves;
+            same &= serves == first[i];
+        }
+    if (asked != 6 || !same) { std::printf("%d searches for six feature dimensions in turn\n", asked); return 1; }
     std::printf("ok\n");
     return 0;
 }
@@ -96,6 +109,6 @@ def build(tmp_path_factory):
     return make
 
 
-def test_a_plan_is_made_without_them_for_want_of_memory_or_use(build):
+def test_without_memory_without_use_and_asked_in_turn(build):
     run = subprocess.run([build(DRIVER)], stdout=subprocess.PIPE, timeout=60)
     assert run.returncode == 0 and run.stdout == b"ok\n", run.stdout.decode()
