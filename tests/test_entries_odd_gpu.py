@@ -4,10 +4,11 @@ import numpy as np
 import pytest
 
 import test_nonfinite_gpu as nonfinite
+from test_entries_gpu import _rows_of_lengths
 from test_spmm_gpu import convert, torch_cuda  # noqa: F401
-from test_tile_gpu import _matrix
+from test_tile_gpu import _matrix, _random_operand
 from test_wide_gpu import _plan
-from util import encode
+from util import decode, encode
 
 pytestmark = pytest.mark.gpu
 
@@ -45,3 +46,30 @@ def test_exact_sums(torch_cuda, hs, dtype, rows, cols, density):
 def test_infinities_and_nans_stay_with_the_rows_that_name_them(torch_cuda, hs, monkeypatch, dtype, rows, cols):
     monkeypatch.setitem(nonfinite.FAMILIES, "entries", nonfinite.FAMILIES["entries"][:2] + ((15, 17, 63, 129, 301), "spmm_entries_kernel"))
     nonfinite.test_infinities_and_nans_stay_with_the_rows_that_name_them(torch_cuda, hs, "entries", dtype, rows, cols)
+
+
+# Against fp64, with real numbers, whose sums show a feature in another's place by its size and not only by a whole number: a product of
+# two 16-bit numbers is exact in fp32 and every one of the n additions rounds once (n 2^-24 of the sum of sizes), the result once more
+# (2^-11 or 2^-8 of it).  Rows cut into parts (1500 entries), rows in pieces (2600), every row with an entry in B's last row.
+@pytest.mark.parametrize("dtype,N", [(0, 9), (2, 17), (0, 33), (2, 65), (0, 77), (2, 131), (0, 257), (2, 301), (0, 511)])
+def test_rows_cut_into_parts_and_the_last_row_of_b(torch_cuda, hs, dtype, N):
+    torch = torch_cuda
+    rng = np.random.default_rng(N)
+    rows, cols = 3000, 6001
+    lengths = rng.integers(1, 12, rows)
+    lengths[[3, 700, 2100]], lengths[2900] = 1500, 2600
+    A = _rows_of_lengths(rng, [int(n) for n in lengths], cols, dtype)
+    A["col_idx"][A["row_ptr"][1:].astype(np.int64) - 1] = cols - 1
+    plan = _plan(hs, A, ENTRIES=1, TILE=0)
+    B, dB = _random_operand(torch, rng, cols, N, dtype)
+    dC = torch.full((rows, N), 0x7E01 if dtype == 0 else 0x7FC0, dtype=torch.int16, device="cuda")
+    plan.run(dB.data_ptr(), dC.data_ptr(), N, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert plan.last_kernel() == "spmm_entries_kernel"
+    D = np.zeros((rows, cols))
+    D[np.repeat(np.arange(rows), lengths), A["col_idx"]] = decode(A["values"], dtype)
+    Bm = decode(B, dtype).astype(np.float64)
+    want, bound = D @ Bm, lengths[:, None] * 2.0**-24 * (abs(D) @ abs(Bm))
+    off = abs(decode(dC.cpu().numpy().view(np.uint16), dtype).astype(np.float64) - want)
+    assert (off <= bound + (2.0**-11 if dtype == 0 else 2.0**-8) * (abs(want) + bound) + (2.0**-25 if dtype == 0 else 0.0)).all()
+    plan.close()
