@@ -183,7 +183,8 @@ struct WideArgs {
     float *sums;                 // of more than one: their sums, wide_sums_bytes() of them
     const TileSource *src;       // in device memory (read where B is not finite)
 };
-hipError_t launch_spmm_wide(int dtype, const WideArgs &wa, const WideShape &sh, hipStream_t s);
+// mid: as of launch_spmm_mfma, in front of the kernel that adds the sums of cut C tiles
+hipError_t launch_spmm_wide(int dtype, const WideArgs &wa, const WideShape &sh, hipStream_t s, hipEvent_t mid);
 hipError_t launch_wide_fill(const TileSource &src, uint32_t rows, uint32_t n_chunks, void *frags, hipStream_t s);
 // Narrow kernels (spmm_narrow_kernel.hip, 16-bit types): stored entries by blocks of 16 rows x kNarrowColumns columns
 constexpr uint32_t kNarrowColumns = 128u, kNarrowMostBlocks = 1024u;

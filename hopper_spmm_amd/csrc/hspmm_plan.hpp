@@ -355,7 +355,7 @@ int run_narrow(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t 
 // hspmm_wide.hip: the wide-tile kernels' stream, whether they take this launch, and the launch
 int build_wide_stream(hspmm_plan *p);
 bool wide_serves(const hspmm_plan *p, uint32_t N);
-int run_wide(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode);
+int run_wide(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, hipEvent_t mid, RunMode mode);
 
 // hspmm_run.hip: the address of the device's fixed scratch array (hspmm_run_static); `device` must be current
 int static_scratch_address(int device, float **out);

@@ -159,7 +159,7 @@ bool wide_serves(const hspmm_plan *p, uint32_t N)
     return kept_choice(p, N) & 1u;
 }
 
-int run_wide(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode)
+int run_wide(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, hipEvent_t mid, RunMode mode)
 {
     const hspmm_plan::Wide &w = p->wide;
     const uint32_t choice = kept_choice(p, N);
@@ -177,7 +177,7 @@ int run_wide(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s,
     wa.n_units = w.n_units; wa.n_chunks = w.n_chunks; wa.n_feat_tiles = (N + sh.blocks * 16u - 1u) / (sh.blocks * 16u);
     wa.src = w.d_source;
     p->note_launch("spmm_wide_kernel", 3, p->dtype == HSPMM_FP16 ? 1u : 2u, groups * w.n_chunks * sh.units * sh.rows * sh.blocks * 2u);
-    HSPMM_HIP(hspmm::launch_spmm_wide(p->dtype, wa, sh, s));
+    HSPMM_HIP(hspmm::launch_spmm_wide(p->dtype, wa, sh, s, mid));
     return HSPMM_OK;
 }
 

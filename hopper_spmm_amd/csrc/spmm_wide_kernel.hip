@@ -233,27 +233,28 @@ __global__ __launch_bounds__(256) void wide_sum_kernel(const WideArgs wa, const 
 }
 
 template <class E>
-static hipError_t launch_wide_sums(const WideArgs &wa, const WideShape &sh, uint32_t groups, hipStream_t s)
+static hipError_t launch_wide_sums(const WideArgs &wa, const WideShape &sh, uint32_t groups, hipStream_t s, hipEvent_t mid)
 {
     if (hipError_t e = hipGetLastError()) return e;
     if (wa.n_cuts == 1u) return hipSuccess;
+    if (mid) { if (hipError_t e = hipEventRecord(mid, s)) return e; }
     const uint32_t n_blocks = groups * sh.blocks * sh.units * sh.rows;
     wide_sum_kernel<E><<<dim3((n_blocks + 3u) / 4u), 256, 0, s>>>(wa, sh, n_blocks);
     return hipGetLastError();
 }
 
 template <class E>
-static hipError_t launch_wide_e(const WideArgs &wa, const WideShape &sh, uint32_t groups, hipStream_t s)
+static hipError_t launch_wide_e(const WideArgs &wa, const WideShape &sh, uint32_t groups, hipStream_t s, hipEvent_t mid)
 {
 #define HSPMM_WIDE(RF, CF, WR, WK) \
-    if (sh.units == RF && sh.blocks == CF && sh.rows == WR && sh.splits == WK) { spmm_wide_kernel<E, RF, CF, WR, WK><<<dim3(groups * wa.n_cuts), 64 * WR * WK, 0, s>>>(wa); return launch_wide_sums<E>(wa, sh, groups, s); }
+    if (sh.units == RF && sh.blocks == CF && sh.rows == WR && sh.splits == WK) { spmm_wide_kernel<E, RF, CF, WR, WK><<<dim3(groups * wa.n_cuts), 64 * WR * WK, 0, s>>>(wa); return launch_wide_sums<E>(wa, sh, groups, s, mid); }
     HSPMM_WIDE(1, 2, 2, 4) HSPMM_WIDE(1, 2, 4, 2) HSPMM_WIDE(1, 4, 4, 2) HSPMM_WIDE(2, 2, 4, 2) HSPMM_WIDE(2, 4, 4, 2) HSPMM_WIDE(3, 4, 2, 4)
     HSPMM_WIDE(3, 4, 4, 2) HSPMM_WIDE(2, 8, 4, 2) HSPMM_WIDE(3, 8, 4, 2)
 #undef HSPMM_WIDE
     return hipErrorInvalidValue;
 }
 
-hipError_t launch_spmm_wide(int dtype, const WideArgs &wa, const WideShape &sh, hipStream_t s)
+hipError_t launch_spmm_wide(int dtype, const WideArgs &wa, const WideShape &sh, hipStream_t s, hipEvent_t mid)
 {
     const uint64_t rows = uint64_t(sh.units) * sh.rows * kWideRows, nt = uint64_t(sh.blocks) * 16u;
     // (a row of B holds a tile, offsets inside a chunk of it fit 32 bits, and the chunks and units are all there)
@@ -262,8 +263,8 @@ hipError_t launch_spmm_wide(int dtype, const WideArgs &wa, const WideShape &sh, 
         return hipErrorInvalidValue;
     const uint64_t groups = (wa.rows + rows - 1u) / rows * wa.n_feat_tiles;
     if (!wa.n_cuts || groups * wa.n_cuts >= (1u << 22) || wa.n_cuts > wa.n_chunks / sh.splits || (wa.n_cuts > 1u && !wa.sums)) return hipErrorInvalidValue;
-    if (dtype == kDtypeBf16) return launch_wide_e<WideHalf<true>>(wa, sh, uint32_t(groups), s);
-    if (dtype == kDtypeF16) return launch_wide_e<WideHalf<false>>(wa, sh, uint32_t(groups), s);
+    if (dtype == kDtypeBf16) return launch_wide_e<WideHalf<true>>(wa, sh, uint32_t(groups), s, mid);
+    if (dtype == kDtypeF16) return launch_wide_e<WideHalf<false>>(wa, sh, uint32_t(groups), s, mid);
     return hipErrorInvalidValue;
 }
 

@@ -137,7 +137,8 @@ int hspmm_bench(hspmm_plan *plan, const void *dB, void *dC, uint32_t N,
 /* No reference counterpart (the reference times whole launches only): `runs`
  * launches with an event between the two kernels of a launch; *main_ms is the
  * total time of the main kernel, *fixup_ms of the kernel that adds the partial
- * sums of windows split across waves (0 when no window is split). */
+ * sums of windows split across waves or of C tiles cut between workgroups (0 when
+ * nothing is split). */
 int hspmm_profile(hspmm_plan *plan, const void *dB, void *dC, uint32_t N, int runs, void *stream,
                   float *main_ms, float *fixup_ms);
 

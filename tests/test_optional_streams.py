@@ -26,7 +26,7 @@ namespace hspmm {
 hipError_t launch_narrow_count(const TileSource &, uint32_t, uint32_t, uint32_t *, uint32_t *, hipStream_t) { return hipSuccess; }
 hipError_t launch_narrow_fill(const TileSource &, uint32_t, uint32_t, const uint32_t *, const uint32_t *, uint32_t *, hipStream_t) { return hipSuccess; }
 hipError_t launch_spmm_narrow(int, const NarrowArgs &, uint32_t, uint32_t, hipStream_t) { return hipErrorInvalidValue; }
-hipError_t launch_spmm_wide(int, const WideArgs &, const WideShape &, hipStream_t) { return hipErrorInvalidValue; }
+hipError_t launch_spmm_wide(int, const WideArgs &, const WideShape &, hipStream_t, hipEvent_t) { return hipErrorInvalidValue; }
 hipError_t launch_wide_fill(const TileSource &, uint32_t, uint32_t, void *, hipStream_t) { return hipSuccess; }
 }
 namespace hspmm_host {

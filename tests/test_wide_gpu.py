@@ -52,6 +52,21 @@ def test_exact_sums_in_every_shape(torch_cuda, hs, shape, dtype, rows, cols, cut
     plan.close()
 
 
+@pytest.mark.parametrize("cuts", [1, 4])
+def test_the_kernel_that_adds_cut_tiles_has_a_time_of_its_own(torch_cuda, hs, cuts):
+    """hspmm_profile: 0 ms where no C tile is cut."""
+    torch = torch_cuda
+    D, A = _matrix(np.random.default_rng(cuts), 400, 2050, 0.1, 2)
+    plan = _plan(hs, A, WIDE=1, WIDE_SHAPE=2, WIDE_CUTS=cuts)
+    dB = torch.zeros((2050, 64), dtype=torch.int16, device="cuda")
+    dC = torch.full((400, 64), 7, dtype=torch.int16, device="cuda")
+    main_ms, sum_ms = plan.profile(dB.data_ptr(), dC.data_ptr(), 64, runs=3)
+    assert plan.last_kernel() == "spmm_wide_kernel"
+    assert main_ms > 0 and (sum_ms > 0) == (cuts > 1), (main_ms, sum_ms)
+    assert not dC.any()
+    plan.close()
+
+
 @pytest.mark.parametrize("shape,cuts", [(0, 1), (6, 1), (7, 1), (4, 2)])
 @pytest.mark.parametrize("dtype", [0, 2])
 @pytest.mark.parametrize("rows,cols", [(600, 700), (1100, 130)])
