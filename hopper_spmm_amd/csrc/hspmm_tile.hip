@@ -44,24 +44,40 @@ TileShape choose_tile_shape(const hspmm_plan *p, uint32_t N)
     return sh;
 }
 
+// Stored entries, as estimated from a sample.
+double entries_estimated(const hspmm_plan *p) { return double(p->T) * p->cw * p->per_column; }
+
+// Whether a stream can be made of this matrix, and - unless they are asked for wherever they can - whether it is of the kind they are for.
+// Block-clustered weights (over four of a column's eight elements stored) stay with kernels that read whole tiles.
+bool tile_suits(const hspmm_plan *p)
+{
+    using namespace hspmm;
+    const uint32_t kk = tile_block_columns(p->dtype), n_blocks = (p->cols + kk - 1u) / kk, n_row_blocks = (p->rows + kTileBlockRows - 1u) / kTileBlockRows;
+    if (p->cfg.tile == 0 || !p->canonical || p->cfg.kernel_mode != 0) return false;
+    if (p->cols < kk || n_blocks > kTileMaxBlocks || uint64_t(n_blocks) * n_row_blocks >= (1u << 26) || n_row_blocks >= (1u << 23)) return false;
+    return p->cfg.tile > 0 || (p->G == 1 && p->per_column <= 4.0 && entries_estimated(p) >= 0.04 * double(p->rows) * p->cols &&
+                               (p->elem != 4u || (p->panel.built && p->panel.split)));
+}
+
+constexpr uint32_t kMostFloats = 32, kMostHalves = 127;       // features
+
+// Stored entries x features that a launch has at least.
+double fewest_products(const hspmm_plan *p) { return p->elem == 4u ? 75e6 : 65e6; }
+
 }  // namespace
 
 namespace hspmm_host {
 
 // Made where some feature dimension would take it (tile_serves) by the stored entries as estimated from a sample.
-// Block-clustered weights (over four of a column's eight elements stored) stay with kernels that read whole tiles.
 int build_tile_stream(hspmm_plan *p)
 {
     using namespace hspmm;
     hspmm_plan::Tile &t = p->tile;
-    const double entries = double(p->T) * p->cw * p->per_column, most_features = p->elem == 4u ? 47.0 : 127.0;
-    if (p->cfg.tile == 0 || !p->canonical || p->cfg.kernel_mode != 0) return HSPMM_OK;
-    if (p->cfg.tile < 0 && (p->G != 1 || p->per_column > 4.0 || entries * most_features < 65e6 ||
-                            entries < 0.04 * double(p->rows) * p->cols ||
-                            (p->elem == 4u && !(p->panel.built && p->panel.split)))) return HSPMM_OK;
+    // (fp32 storage: an estimate that is off by a twentieth loses no launch)
+    const double most = entries_estimated(p) * (p->elem == 4u ? kMostFloats / 0.95 : kMostHalves);
+    if (!tile_suits(p) || (p->cfg.tile < 0 && most < fewest_products(p))) return HSPMM_OK;
     const uint32_t kk = tile_block_columns(p->dtype), n_blocks = (p->cols + kk - 1u) / kk, n_row_blocks = (p->rows + kTileBlockRows - 1u) / kTileBlockRows;
     const uint64_t cells = uint64_t(n_blocks) * n_row_blocks;
-    if (p->cols < kk || n_blocks > kTileMaxBlocks || cells >= (1u << 26) || n_row_blocks >= (1u << 23)) return HSPMM_OK;
     const TileSource src{p->d_rowOffset, p->d_rowIdx, p->d_a2b_raw, p->d_data, p->W, p->cols};
     void *room = nullptr;
     if (int rc = plan_alloc(p, (size_t(cells) + 1u) * 4u, &room)) return rc;
@@ -95,25 +111,30 @@ int build_tile_stream(hspmm_plan *p)
 //   tile ragged, not for fp32.  N = 256 and more: the LDS-panel kernels by a fifth.
 // fp32 storage is multiplied in bf16 parts here: only where the LDS-panel kernels would do the same (panel.split; N from 16 on,
 // in rows of whole 16-byte pieces).  Other N keep the fp32 products of the entry and gather kernels.
-static bool tile_takes(const hspmm_plan *p, uint32_t N)
+static bool tile_pays(const hspmm_plan *p, double entries, uint32_t N, uint32_t most)
 {
-    const Config &c = p->cfg;
-    if (!p->tile.built || c.kernel_mode != 0 || uint64_t(N) * p->elem < 16u) return false;
-    if (c.buffer_stage || c.consumer_warp_num || c.producer_warp_group_num || c.fused_fixup >= 0) return false;     // (settings of other kernels)
-    const TileShape sh = choose_tile_shape(p, N);
-    if (uint64_t(sh.n_tiles) * sh.n_chunks >= (1u << 31) || uint64_t(N) * p->elem >= (1u << 24)) return false;
-    if (c.tile > 0) return true;
-    const bool wide = p->elem == 4u;
-    const double work = double(p->tile.entries) * N, fill = double(p->tile.entries) / (double(p->rows) * p->cols);
-    if (wide && !(p->panel.split && panel_serves(p, N))) return false;
-    return N >= 8u && N < (wide ? 48u : 128u) && work >= (wide ? 75e6 : 65e6) && fill >= 0.04 && fill * N >= 1.5;
+    const double fill = entries / (double(p->rows) * p->cols);
+    if (p->elem == 4u && !(p->panel.split && panel_serves(p, N))) return false;
+    return N >= 8u && N <= most && entries * N >= fewest_products(p) && fill >= 0.04 && fill * N >= 1.5;
 }
 
-// 33 to 47 features of fp32 storage that they would take, by what has been said so far, and leave to the LDS-panel kernels, whose
-// arithmetic is the same (or, see entries_serve, to the entry kernels).
-bool tile_leaves(const hspmm_plan *p, uint32_t N) { return p->elem == 4u && p->cfg.tile <= 0 && N > 32u && tile_takes(p, N); }
+static bool other_settings(const Config &c) { return c.kernel_mode != 0 || c.buffer_stage || c.consumer_warp_num || c.producer_warp_group_num || c.fused_fixup >= 0; }
 
-bool tile_serves(const hspmm_plan *p, uint32_t N) { return tile_takes(p, N) && !tile_leaves(p, N); }
+bool tile_serves(const hspmm_plan *p, uint32_t N)
+{
+    if (!p->tile.built || other_settings(p->cfg) || uint64_t(N) * p->elem < 16u) return false;
+    const TileShape sh = choose_tile_shape(p, N);
+    if (uint64_t(sh.n_tiles) * sh.n_chunks >= (1u << 31) || uint64_t(N) * p->elem >= (1u << 24)) return false;
+    return p->cfg.tile > 0 || tile_pays(p, double(p->tile.entries), N, p->elem == 4u ? kMostFloats : kMostHalves);
+}
+
+// 33 to 47 features of fp32 storage that would be theirs, by what has been said so far, and are left to the LDS-panel kernels, whose
+// arithmetic is the same (or, see entries_serve, to the entry kernels).  A plan need not have their stream for that.
+bool tile_leaves(const hspmm_plan *p, uint32_t N)
+{
+    if (p->elem != 4u || p->cfg.tile > 0 || N <= kMostFloats || other_settings(p->cfg) || !tile_suits(p)) return false;
+    return tile_pays(p, p->tile.built ? double(p->tile.entries) : entries_estimated(p), N, 47u);
+}
 
 // 16-bit types, from 32 features on: a fit to 1233 launches (standard deviation 10 to 18 %).  33 to 63 features, which leave a C tile of 64
 // ragged, take one and a half times as long.

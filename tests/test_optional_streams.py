@@ -1,4 +1,4 @@
-"""Streams a plan can do without (narrow and wide-tile kernels): their host code, compiled here without its kernels and with a device
+"""Streams a plan can do without (narrow, wide-tile and full-tile kernels): their host code, compiled here without its kernels and with a device
 memory that runs out at any allocation; what it answers for feature dimensions in turn.  No GPU needed."""
 import os
 import subprocess
@@ -7,7 +7,7 @@ import pytest
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "hopper_spmm_amd", "csrc")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
-DRIVER = r"""
+COMMON = r"""
 #include "hspmm_plan.hpp"
 #include <cstdarg>
 #include <set>
@@ -22,13 +22,6 @@ hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipGetLastError() { return hipSuccess; }
 const char *hipGetErrorString(hipError_t) { return ""; }
 }
-namespace hspmm {
-hipError_t launch_narrow_count(const TileSource &, uint32_t, uint32_t, uint32_t *, uint32_t *, hipStream_t) { return hipSuccess; }
-hipError_t launch_narrow_fill(const TileSource &, uint32_t, uint32_t, const uint32_t *, const uint32_t *, uint32_t *, hipStream_t) { return hipSuccess; }
-hipError_t launch_spmm_narrow(int, const NarrowArgs &, uint32_t, uint32_t, hipStream_t) { return hipErrorInvalidValue; }
-hipError_t launch_spmm_wide(int, const WideArgs &, const WideShape &, hipStream_t, hipEvent_t) { return hipErrorInvalidValue; }
-hipError_t launch_wide_fill(const TileSource &, uint32_t, uint32_t, void *, hipStream_t) { return hipSuccess; }
-}
 namespace hspmm_host {
 int fail(int code, const char *, ...) { return code; }
 // (as in hspmm_create.hip, without the reserved block)
@@ -40,6 +33,17 @@ void plan_release(hspmm_plan *p, const void *ptr, size_t bytes)
     (void)hipFree(*it); p->owned.erase(it); p->fixed_bytes -= bytes;
 }
 int scratch_for(hspmm_plan *, hipStream_t, size_t, RunMode, float **) { return HSPMM_ERR_DEVICE; }
+}
+"""
+DRIVER = COMMON + r"""
+namespace hspmm {
+hipError_t launch_narrow_count(const TileSource &, uint32_t, uint32_t, uint32_t *, uint32_t *, hipStream_t) { return hipSuccess; }
+hipError_t launch_narrow_fill(const TileSource &, uint32_t, uint32_t, const uint32_t *, const uint32_t *, uint32_t *, hipStream_t) { return hipSuccess; }
+hipError_t launch_spmm_narrow(int, const NarrowArgs &, uint32_t, uint32_t, hipStream_t) { return hipErrorInvalidValue; }
+hipError_t launch_spmm_wide(int, const WideArgs &, const WideShape &, hipStream_t, hipEvent_t) { return hipErrorInvalidValue; }
+hipError_t launch_wide_fill(const TileSource &, uint32_t, uint32_t, void *, hipStream_t) { return hipSuccess; }
+}
+namespace hspmm_host {
 double entries_expected(const hspmm_plan *, uint32_t) { return 100.0; }
 bool entries_serve(const hspmm_plan *, uint32_t) { return false; }
 double panel_expected(const hspmm_plan *, uint32_t) { return 100.0; }
@@ -93,22 +97,64 @@ int main()
     return 0;
 }
 """
+TILE_DRIVER = COMMON + r"""
+namespace hspmm {
+uint32_t tile_block_columns(int) { return 64; }
+hipError_t launch_tile_count(int, const TileSource &, uint32_t, uint32_t, uint32_t *, uint32_t *, hipStream_t) { return hipSuccess; }
+hipError_t launch_tile_fill(int, const TileSource &, uint32_t, uint32_t, const uint32_t *, const uint32_t *, void *, void *, hipStream_t) { return hipSuccess; }
+hipError_t launch_spmm_tile(int, const TileArgs &, uint32_t, uint32_t, hipStream_t) { return hipErrorInvalidValue; }
+hipError_t launch_fill_zero(void *, size_t, hipStream_t) { return hipErrorInvalidValue; }
+}
+namespace hspmm_host {
+int ensure_arrive(hspmm_plan *, hipStream_t, size_t, RunMode, uint32_t **) { return HSPMM_ERR_DEVICE; }
+bool panel_serves(const hspmm_plan *, uint32_t N) { return N >= 16u && N % 4u == 0u; }
+}
+
+int main()
+{
+    using namespace hspmm_host;
+    for (uint32_t rows = 1024; rows <= 8192; rows += 256) {
+        // fp32, 4096 columns at 12 %, tiles 8 wide, the LDS-panel kernels multiply bf16 parts
+        hspmm_plan p;
+        p.dtype = HSPMM_TF32; p.elem = 4; p.cw = 8; p.rows = rows; p.cols = 4096; p.W = rows / 8; p.compute_units = 256; p.per_column = 1.5;
+        p.panel.built = p.panel.split = true;
+        p.T = uint32_t(0.12 * rows * 4096.0 / (8.0 * 1.5));
+        const double entries = double(p.T) * 8.0 * 1.5;
+        left = 100;
+        if (build_tile_stream(&p)) return 1;
+        if (entries * 32.0 >= 75e6 && !p.tile.built) { std::printf("%u rows: no stream\n", rows); return 1; }
+        if (entries * 32.0 < 0.94 * 75e6 && (p.tile.built || left != 100)) { std::printf("%u rows: a stream that no launch reads\n", rows); return 1; }
+        if (p.tile.built) p.tile.entries = uint64_t(entries);
+        for (uint32_t N = 4; N <= 64; N += 4) {
+            if (tile_serves(&p, N) != (N >= 16 && N <= 32 && entries * N >= 75e6)) { std::printf("%u rows, N = %u: taken %d\n", rows, N, int(tile_serves(&p, N))); return 1; }
+            if (tile_leaves(&p, N) != (N > 32 && N < 48 && entries * N >= 75e6)) { std::printf("%u rows, N = %u: left %d\n", rows, N, int(tile_leaves(&p, N))); return 1; }
+        }
+    }
+    std::printf("ok\n");
+    return 0;
+}
+"""
 
 
 @pytest.fixture(scope="module")
 def build(tmp_path_factory):
-    """Compiles a driver and links it with the host code of the two kernel families."""
+    """Compiles a driver and links it with the host code of kernel families."""
     at = tmp_path_factory.mktemp("streams")
     compile_ = ["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(ROCM, "include"), "-I", CSRC, "-x", "c++"]
 
-    def make(driver):
+    def make(driver, *families):
         (at / "driver.cpp").write_text(driver)
-        sources = [os.path.join(CSRC, "hspmm_narrow.hip"), os.path.join(CSRC, "hspmm_wide.hip"), str(at / "driver.cpp")]
+        sources = [os.path.join(CSRC, "hspmm_%s.hip" % f) for f in families] + [str(at / "driver.cpp")]
         subprocess.run(compile_ + sources + ["-o", str(at / "driver"), "-lpthread"], check=True)
         return str(at / "driver")
     return make
 
 
 def test_without_memory_without_use_and_asked_in_turn(build):
-    run = subprocess.run([build(DRIVER)], stdout=subprocess.PIPE, timeout=60)
+    run = subprocess.run([build(DRIVER, "narrow", "wide")], stdout=subprocess.PIPE, timeout=60)
+    assert run.returncode == 0 and run.stdout == b"ok\n", run.stdout.decode()
+
+
+def test_full_tile_streams_of_fp32_plans_only_where_a_launch_reads_them(build):
+    run = subprocess.run([build(TILE_DRIVER, "tile")], stdout=subprocess.PIPE, timeout=60)
     assert run.returncode == 0 and run.stdout == b"ok\n", run.stdout.decode()
