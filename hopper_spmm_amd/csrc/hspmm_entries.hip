@@ -138,13 +138,13 @@ static bool entries_by_xcd(const hspmm_plan *p, uint64_t row_bytes)
            uint64_t(p->cols) * row_bytes >= (uint64_t(8) << 20);
 }
 
-// Bytes of a block: whole 16-byte pieces, of an odd number of 16-bit elements pieces and 14 bytes (the last block is moved back to end
-// with the row).
-static uint32_t entry_block_bytes(uint32_t row_bytes, uint32_t blocks)
+// Bytes of a block: whole 16-byte pieces, or, where rows are loaded from the word before on (EntryArgs::odd), pieces and 14 bytes (the
+// last block is moved back to end with the row).
+static uint32_t entry_block_bytes(uint32_t row_bytes, uint32_t blocks, bool odd)
 {
     if (blocks == 1u) return row_bytes;
     const uint32_t bytes = (row_bytes + blocks - 1u) / blocks;
-    return row_bytes % 4u == 2u ? ((bytes + 1u) & ~15u) + 14u : (bytes + 15u) & ~15u;
+    return odd ? ((bytes + 1u) & ~15u) + 14u : (bytes + 15u) & ~15u;
 }
 
 // Lines of 128 bytes that `bytes` bytes from byte `off` of a row touch: the mean over rows that begin on multiples of `step`.
@@ -163,13 +163,13 @@ static double lines_touched(uint32_t off, uint32_t bytes, uint32_t step)
 // begins anywhere is one block of 32 lanes (3.3 + 4 + 0.5) and not three of eight (5.6 + 3 + 1.5): graph of 905216, N = 75, 576
 // against 861 us.  The two weights are a fit to 745 graphs and uniform matrices, all types and N, with any number of blocks: the
 // choice is 1.6 % behind the fastest on average and 12 % at the 95th percentile, and weights half or twice as large 0.3 % more.
-static uint32_t row_blocks(const hspmm_plan *p, uint32_t row_bytes)
+static uint32_t row_blocks(const hspmm_plan *p, uint32_t row_bytes, bool odd)
 {
     const uint32_t step = row_bytes % 128u ? row_bytes & (0u - row_bytes) : 128u;
     uint32_t best = 0;
     double least = 0.0;
     for (uint32_t b = (row_bytes + kEntryMaxBlockBytes - 1u) / kEntryMaxBlockBytes; b == 1u || row_bytes / b >= 112u; ++b) {
-        const uint32_t bytes = entry_block_bytes(row_bytes, b);
+        const uint32_t bytes = entry_block_bytes(row_bytes, b, odd);
         if (bytes > kEntryMaxBlockBytes || (best && bytes < 128u)) continue;
         double cost = double(b * share_row(bytes).lanes) / 8.0 + 0.5 * double(b);
         if (step <= 16u) cost += double(b) * lines_touched(0u, bytes, step);
@@ -179,6 +179,21 @@ static uint32_t row_blocks(const hspmm_plan *p, uint32_t row_bytes)
         if (!best || cost < least) { least = cost; best = b; }
     }
     return best;
+}
+
+// The blocks of a row, and whether rows are loaded from the word before on: 16-bit types, an odd number of them, B on a word and two of
+// its rows at least.  Not where the blocks fill all of their lanes (N = 383, 511, 767, 1023): there is no place for a last lane of seven
+// features then, and more blocks, or lanes twice as many, cost what the whole words gain (uniform 26880 x 120320, 25 per row, N = 511
+// 116 / 148 us, graph of 65536, N = 383 58 / 73, 6779 launches at odd N: 195 of the 258 that lost by more than 3 %, up to 27 %).
+struct RowShape { uint32_t blocks, block_bytes; bool odd; };
+static RowShape choose_row_shape(const hspmm_plan *p, uint32_t row_bytes, bool on_word)
+{
+    if (entries_by_xcd(p, row_bytes)) return {2u, entry_block_bytes(row_bytes, 2u, false), false};
+    const uint32_t blocks = row_blocks(p, row_bytes, false), bytes = entry_block_bytes(row_bytes, blocks, false);
+    if (p->elem != 2u || row_bytes % 4u != 2u || row_bytes < 18u || p->cols < 2u || !on_word || entry_block_bytes(row_bytes, blocks, true) > 16u * share_row(bytes).lanes)
+        return {blocks, bytes, false};
+    const uint32_t odd_blocks = row_blocks(p, row_bytes, true);
+    return {odd_blocks, entry_block_bytes(row_bytes, odd_blocks, true), true};
 }
 
 // What an entry costs here is the lines of its row of B, what a tile column costs in the MFMA kernels does not depend
@@ -293,8 +308,8 @@ int entries_counted(hspmm_plan *p)
 int run_entries(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode, bool *taken)
 {
     const uint32_t row_bytes = N * p->elem;
-    const bool by_xcd = entries_by_xcd(p, row_bytes);
-    const uint32_t blocks = by_xcd ? 2u : row_blocks(p, row_bytes), block_bytes = entry_block_bytes(row_bytes, blocks);
+    const RowShape row = choose_row_shape(p, row_bytes, reinterpret_cast<uintptr_t>(dB) % 4u == 0u);
+    const uint32_t blocks = row.blocks, block_bytes = row.block_bytes;
     const RowShare share = share_row(block_bytes);
     hspmm::EntryArgs ea{};
     hspmm_plan::Entries &e = p->entries;
@@ -336,9 +351,9 @@ int run_entries(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t
     *taken = true;
     if (mode == RunMode::kPrepare) return HSPMM_OK;
     ea.desc = e.d_desc; ea.ids = e.d_ids; ea.vals = e.d_vals; ea.pieces = e.d_pieces;
-    ea.B = dB; ea.C = dC; ea.ld = N; ea.block_bytes = block_bytes; ea.n_feat_blocks = blocks; ea.xcd_split = by_xcd;
+    ea.B = dB; ea.C = dC; ea.ld = N; ea.block_bytes = block_bytes; ea.n_feat_blocks = blocks; ea.xcd_split = entries_by_xcd(p, row_bytes);
     ea.last_row = p->cols - 1u;
-    ea.odd = row_bytes % 4u == 2u && row_bytes >= 18u && ea.last_row && reinterpret_cast<uintptr_t>(dB) % 4u == 0u;
+    ea.odd = row.odd;
     p->note_launch("spmm_entries_kernel", 2, 0, 0);
     HSPMM_HIP(hspmm::launch_spmm_entries(p->dtype, ea, share.lane_bytes, share.lanes, s));
     return HSPMM_OK;

@@ -1,5 +1,6 @@
-"""Streams a plan can do without (narrow, wide-tile and full-tile kernels): their host code, compiled here without its kernels and with a device
-memory that runs out at any allocation; what it answers for feature dimensions in turn.  No GPU needed."""
+"""Host code of the kernel families, compiled here without its kernels and with a device memory that runs out at any allocation: streams a
+plan can do without (narrow, wide-tile and full-tile kernels), what it answers for feature dimensions in turn, the shape of a row of B in the
+entry kernels.  No GPU needed."""
 import os
 import subprocess
 
@@ -134,6 +135,58 @@ int main()
     return 0;
 }
 """
+ENTRY_DRIVER = COMMON + r"""
+namespace hspmm {
+hipError_t launch_entry_count(int, const EntrySource &, uint32_t, uint32_t, uint32_t *, uint32_t *, uint32_t *, uint32_t *, uint32_t *, hipStream_t) { return hipSuccess; }
+hipError_t launch_fill_zero(void *, size_t, hipStream_t) { return hipErrorInvalidValue; }
+static EntryArgs got;
+static uint32_t lane_bytes, lanes;
+hipError_t launch_spmm_entries(int, const EntryArgs &ea, uint32_t bytes, uint32_t of, hipStream_t) { got = ea; lane_bytes = bytes; lanes = of; return hipSuccess; }
+hipError_t launch_entry_fill(int, const EntrySource &, uint32_t, const uint32_t *, const uint32_t *, uint32_t, const EntryPlaces &, uint32_t *, uint32_t *, uint32_t *,
+                             uint32_t *, uint32_t *, void *, hipStream_t) { return hipSuccess; }
+}
+extern "C" hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *) { return hipErrorInvalidValue; }
+namespace hspmm_host {
+int ensure_arrive(hspmm_plan *, hipStream_t, size_t, RunMode, uint32_t **) { return HSPMM_ERR_DEVICE; }
+bool panel_serves(const hspmm_plan *, uint32_t) { return false; }
+double panel_expected(const hspmm_plan *, uint32_t) { return 0.0; }
+bool tile_leaves(const hspmm_plan *, uint32_t) { return false; }
+}
+
+int main()
+{
+    using namespace hspmm_host;
+    using hspmm::got;
+    for (uint32_t cols : {2u, 2048u, 65536u, 1u << 20}) {
+        hspmm_plan p;
+        p.dtype = HSPMM_BF16; p.rows = 100; p.cols = cols; p.compute_units = 256;
+        p.entries.built = p.entries.counted = true;
+        for (auto &c : p.entries.classes) { c.n_classes = 1; c.n_groups = 1; }
+        for (uint32_t N = 1; N <= 1024; ++N) {
+            hspmm::EntryArgs at[2];
+            uint32_t loaded[2];
+            for (int off : {0, 2}) {
+                bool taken = false;
+                if (run_entries(&p, reinterpret_cast<const void *>(uintptr_t(4096 + off)), nullptr, N, nullptr, RunMode::kLaunch, &taken) || !taken) { std::printf("N = %u: not run\n", N); return 1; }
+                at[off / 2] = got; loaded[off / 2] = got.n_feat_blocks * hspmm::lanes;
+                const uint32_t row = 2u * N, bytes = got.block_bytes, blocks = got.n_feat_blocks;
+                if (bytes > row || bytes < hspmm::lane_bytes || bytes > hspmm::lane_bytes * hspmm::lanes || bytes * blocks < row) { std::printf("N = %u: %u blocks of %u bytes\n", N, blocks, bytes); return 1; }
+                if (blocks > 1u && bytes % 16u != (got.odd ? 14u : 0u)) { std::printf("N = %u, off %d: blocks of %u bytes\n", N, off, bytes); return 1; }
+            }
+            const bool may = N % 2u && N >= 9u;
+            if (at[1].odd || (at[0].odd && !may)) { std::printf("N = %u: whole words %u %u\n", N, at[0].odd, at[1].odd); return 1; }
+            // whole words but where a lane of seven features would cost lanes
+            const uint32_t bytes = at[1].block_bytes, blocks = at[1].n_feat_blocks, each = (2u * N + blocks - 1u) / blocks;
+            const bool full = blocks > 1u && ((each + 1u) & ~15u) + 14u > 16u * (loaded[1] / blocks);
+            if (may && (at[0].odd != 0u) != !full) { std::printf("N = %u: whole words %u of %u blocks of %u bytes\n", N, at[0].odd, blocks, bytes); return 1; }
+            if (!at[0].odd && (at[0].block_bytes != bytes || at[0].n_feat_blocks != blocks)) { std::printf("N = %u: another shape by the place of B\n", N); return 1; }
+            if (cols > 2u && (N == 511u || N == 767u) && at[0].odd) { std::printf("N = %u: %u lanes instead of %u\n", N, loaded[0], loaded[1]); return 1; }
+        }
+    }
+    std::printf("ok\n");
+    return 0;
+}
+"""
 
 
 @pytest.fixture(scope="module")
@@ -157,4 +210,9 @@ def test_without_memory_without_use_and_asked_in_turn(build):
 
 def test_full_tile_streams_of_fp32_plans_only_where_a_launch_reads_them(build):
     run = subprocess.run([build(TILE_DRIVER, "tile")], stdout=subprocess.PIPE, timeout=60)
+    assert run.returncode == 0 and run.stdout == b"ok\n", run.stdout.decode()
+
+
+def test_rows_of_the_entry_kernels_by_their_size_and_place(build):
+    run = subprocess.run([build(ENTRY_DRIVER, "entries")], stdout=subprocess.PIPE, timeout=60)
     assert run.returncode == 0 and run.stdout == b"ok\n", run.stdout.decode()
