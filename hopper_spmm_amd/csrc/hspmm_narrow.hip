@@ -85,7 +85,10 @@ int build_narrow_stream(hspmm_plan *p)
 // kernels, and by 0.3 us more than these (whose short launches are faster than the fit says); the full-tile and the gather kernels lose every launch but 2 of 249 (by 2 %).  Over 2075 launches the rule gives 1.22 times the speed
 // of the entry kernels (1.27 if every launch took the faster one; 5 % of those taken lose, 5 % on average).  Up to 31 % of entries,
 // as far as times are known.
-bool narrow_serves(const hspmm_plan *p, uint32_t N)
+// B that begins between two words makes these kernels half as slow again, and with two tiles of features 1.7 times; the full-tile and wide-tile
+// kernels take as long as ever, the entry kernels 1.5 times, but not at up to eight features (8704 x 5120 at 5 %, N = 32 34 us, full tiles
+// 17.9; 12800 x 1963 at 9 %, N = 2 12.5, entries 6.8, N = 16 12.6, entries 16.8).
+bool narrow_serves(const hspmm_plan *p, uint32_t N, bool on_word)
 {
     const Config &c = p->cfg;
     if (!p->narrow.built || c.kernel_mode != 0 || !N || N > most_features(N)) return false;
@@ -97,6 +100,7 @@ bool narrow_serves(const hspmm_plan *p, uint32_t N)
         c.panel_units_per_group || c.aligned_small >= 0 || c.xcd_split >= 0 || c.gather_bitmap >= 0 || c.tile > 0 || c.entries > 0 || c.wide > 0)
         return false;
     if (double(p->narrow.entries) > kMostEntries * p->rows * p->cols) return false;
+    if (!on_word && (wide_serves(p, N) || tile_serves(p, N) || (N <= 8u && entries_serve(p, N)))) return false;
     if (wide_serves(p, N)) return expected < 0.9 * p->wide.expected_fewest;     // (N = 32)
     if (tile_serves(p, N)) return true;
     if (entries_serve(p, N)) return expected < 0.9 * entries_expected(p, N) - 0.3;

@@ -350,7 +350,7 @@ int run_tile(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s,
 
 // hspmm_narrow.hip: the narrow kernels' stream, whether they take this launch, and the launch
 int build_narrow_stream(hspmm_plan *p);
-bool narrow_serves(const hspmm_plan *p, uint32_t N);
+bool narrow_serves(const hspmm_plan *p, uint32_t N, bool on_word);        // on_word: B begins on a word
 int run_narrow(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode);
 // hspmm_wide.hip: the wide-tile kernels' stream, whether they take this launch, and the launch
 int build_wide_stream(hspmm_plan *p);

@@ -46,12 +46,13 @@ hipError_t launch_wide_fill(const TileSource &, uint32_t, uint32_t, void *, hipS
 }
 namespace hspmm_host {
 double entries_expected(const hspmm_plan *, uint32_t) { return 100.0; }
-bool entries_serve(const hspmm_plan *, uint32_t) { return false; }
+static bool by_entries, by_tile;                    // kernels that would take a launch
+bool entries_serve(const hspmm_plan *, uint32_t) { return by_entries; }
 double panel_expected(const hspmm_plan *, uint32_t) { return 100.0; }
 static int asked;                                   // searches for a feature dimension's kernel
 bool panel_serves(const hspmm_plan *, uint32_t) { ++asked; return true; }
 double tile_expected(const hspmm_plan *, uint32_t) { return 100.0; }
-bool tile_serves(const hspmm_plan *, uint32_t) { return false; }
+bool tile_serves(const hspmm_plan *, uint32_t) { return by_tile; }
 }
 
 int main()
@@ -94,6 +95,17 @@ int main()
             same &= serves == first[i];
         }
     if (asked != 6 || !same) { std::printf("%d searches for six feature dimensions in turn\n", asked); return 1; }
+    // B between two words: launches of the entry kernels are taken from nine features on, those of the full-tile kernels are not
+    hspmm_plan q;
+    q.dtype = HSPMM_BF16; q.rows = q.cols = 4096; q.W = 512; q.T = 512 * 146; q.compute_units = 256; q.per_column = 1.4;
+    left = 100;
+    if (build_narrow_stream(&q)) return 1;
+    q.narrow.entries = 1677721;
+    for (int which = 0; which < 2; ++which) {
+        by_entries = which == 0; by_tile = which == 1;
+        for (uint32_t N : {1u, 2u, 7u, 8u, 9u, 15u, 16u, 29u, 32u})
+            if (!narrow_serves(&q, N, true) || narrow_serves(&q, N, false) != (by_entries && N > 8u)) { std::printf("N = %u: taken %d %d\n", N, int(narrow_serves(&q, N, true)), int(narrow_serves(&q, N, false))); return 1; }
+    }
     std::printf("ok\n");
     return 0;
 }
