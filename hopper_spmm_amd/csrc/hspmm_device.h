@@ -180,7 +180,7 @@ struct WideArgs {
     uint32_t rows, cols, N;
     uint32_t n_units, n_chunks, n_feat_tiles;                    // chunks: a multiple of four
     uint32_t n_cuts;             // workgroups of a C tile, each with a part of the chunks
-    float *sums;                 // of more than one: their sums, wide_sums_bytes() of them
+    float *sums;                 // of more than one: their sums, a C tile of fp32 each
     const TileSource *src;       // in device memory (read where B is not finite)
 };
 // mid: as of launch_spmm_mfma, in front of the kernel that adds the sums of cut C tiles

@@ -82,9 +82,11 @@ int build_narrow_stream(hspmm_plan *p)
 }
 
 // Where they are expected to be faster than the kernels that would take the launch: by 10 % than the wide-tile and the entry
-// kernels, and by 0.3 us more than these (whose short launches are faster than the fit says); the full-tile and the gather kernels lose every launch but 2 of 249 (by 2 %).  Over 2075 launches the rule gives 1.22 times the speed
-// of the entry kernels (1.27 if every launch took the faster one; 5 % of those taken lose, 5 % on average).  Up to 31 % of entries,
-// as far as times are known.
+// kernels, and by 0.3 us more than these (whose short launches are faster than the fit says); the full-tile and the gather kernels lose every
+// launch but 2 of 249 (by 2 %).  Over 2075 launches the rule gives 1.22 times the speed of the entry kernels (1.27 if every launch took the
+// faster one; 5 % of those taken lose, 5 % on average).  Up to 31 % of entries, as far as times are known.
+// 480 launches taken, six to 48 matrices of 800 MB together in turn, whose streams come from memory / one matrix over and over, old time
+// over new: entry kernels 1.65 / 1.48, full-tile 1.21 / 1.34, gather 2.2 / 2.0; 7 / 23 lose more than 3 %, up to 20 %, most of them of less than 10 us.
 // B that begins between two words makes these kernels half as slow again, and with two tiles of features 1.7 times; the full-tile and wide-tile
 // kernels take as long as ever, the entry kernels 1.5 times, but not at up to eight features (8704 x 5120 at 5 %, N = 32 34 us, full tiles
 // 17.9; 12800 x 1963 at 9 %, N = 2 12.5, entries 6.8, N = 16 12.6, entries 16.8).

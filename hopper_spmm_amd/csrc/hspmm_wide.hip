@@ -26,7 +26,8 @@ const ShapeCost kShapes[] = {
     {{3, 8, 4, 2}, 6.9, {0.605, 0.598, 0.600, 0.638}, 0.0},       // 192 x 128
 };
 constexpr double kPerCut = 0.1, kPerSumsByte = 0.34e-6;           // us
-// Streams from 75 MB on: three matrices in turn no longer share the memory-side cache of 256 MB (100 MB: 8 us more).
+// Times are of three matrices in turn, whose streams share the memory-side cache of 256 MB; from 75 MB on they no longer do, which is what
+// this adds (100 MB: 8 us more).  See wide_serves for streams of any size that come from memory.
 constexpr double kLargeStream = 75e6;
 constexpr uint32_t kShapeCount = sizeof kShapes / sizeof kShapes[0], kFewestFeatures = 32u, kMostCuts = 16u;
 constexpr size_t kMostBytes = size_t(8) << 30;             // 64k x 64k
@@ -148,6 +149,11 @@ int build_wide_stream(hspmm_plan *p)
 // LDS-panel 1.08 (1832), gather 1.75 (1834).
 // Without cut C tiles rows x columns with few workgroups left compute units idle, us (uncut / cut / other kernels): 512 x 11008 at 10 %,
 // N = 64 20.5 / 9.9 / 17, 256 24.8 / 13.0 / 19, 4096 x 14336, N = 64 45 / 26.
+// In a model of many layers every stream comes from memory, and this one is the largest: 678 launches taken by the rule, six to 48 matrices
+// of 800 MB together in turn / one matrix over and over, old time over new: LDS-panel 1.14 / 1.27, full-tile 1.54 / 2.0, gather 1.9 / 2.2;
+// of blocks LDS-panel 1.11 / 1.29, gather 2.3 / 2.5.  35 / 4 of them lose more than 3 %, 25 of the former by less than 6 % or below 6 % of entries.
+// The launches from the LDS-panel kernels take 0.9 / 0.1 % longer than if each took the faster one.  Of 177 launches beyond 75 MB the rule
+// leaves the LDS-panel kernels 126, which would be 7 / 10 % faster if each took the faster one.
 bool wide_serves(const hspmm_plan *p, uint32_t N)
 {
     const Config &c = p->cfg;

@@ -112,8 +112,8 @@ __device__ __forceinline__ Piece<VB> round_sums(const float (&acc)[NF])
 // so that the subgroups of a wave run alike; the classes of EntryArgs say how many subgroups a row gets.
 // What bounds it: the rows of B.  A wave keeps four of them per subgroup in flight and has no other loads to wait for than the next
 // unit's, and with up to eight waves per SIMD (64 registers) a compute unit has 72 to 85 requests to its L2 under way all the time
-// and its L1's return path busy for 88 to 94 % of it; what a request takes - 250 to 580 cycles - goes by how many hit the L2
-// (counted, us / requests under way / L2 hits: graph of 2^18, bf16, N = 16 26.4 / 79 / 82 %; of 150001, fp32, N = 100 91 / 72 /
+// and its L1's return path busy for 25 to 62 % of it and waiting for the L2 for most of the rest; what a request takes - 250 to 580
+// cycles - goes by how many hit the L2 (counted, us / requests under way / L2 hits: graph of 2^18, bf16, N = 16 26.4 / 79 / 82 %; of 150001, fp32, N = 100 91 / 72 /
 // 59 %; of 500000, fp16, N = 1 23.7 / 74 / 89 %; uniform 65536^2, N = 128 28.5 / 85 / 41 %, 6.3 TB/s past the L2s).  A launch as
 // short as 4096^2 at 1 %, N = 64 - 4.5 us, 22 under way - is its chain of descriptor, ids, rows and sums.
 // Odd: 16-bit types with an odd number of elements in a row of B, whose every other row starts between two words, and loads that

@@ -78,7 +78,7 @@ template <bool BF, bool ODD> struct NarrowHalf : HalfStored<BF> {
 // its image in LDS, reads the image back as first operands, clears it, and multiplies it with B's rows, which come straight into
 // registers, asked for a block earlier.  The waves' sums are added in LDS at the end, always in the same order.  (LDS serves the
 // requests of a wave in order.)
-// What bounds it: the loads of a block - 16 of B, 2 words a lane CAP times for entries -, which keep the L1's return path busy for 80 %
+// What bounds it: the loads of a block - 16 of B, 2 words a lane CAP times for entries -, which keep the L1's return path busy for 54 %
 // of a launch (4096 x 11008 at 10 %, N = 16), and 3 us of launch and first loads.  With B in loads of one 16-bit feature, 32 of
 // them a block, that took 11.0 us instead of 9.1, and N = 32 16.2 instead of 12.9; with B in 16-byte pieces, 4 a block, through LDS
 // and its transposing reads 11.1.

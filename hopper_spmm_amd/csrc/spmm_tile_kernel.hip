@@ -136,7 +136,7 @@ __device__ __forceinline__ u32x4 shift_down(u32x4 v, uint32_t back)
 // SIMD cover in part (0.55 us per 128 x 64 x 64 chunk and compute unit, 0.35 with 16 features; matrix instructions 0.1), and
 // 6 to 8 us of launch, first loads and sums of parts: pruned to 20 %, 11008 x 4096, bf16, N = 32: 16.4 us where the gather
 // kernels took 34.5.  Counted, 4096 x 11008 at 10 %, bf16, N = 16, 17.1 us: matrix instructions busy for 4 % of the time, the L1s'
-// return path for 58 %, 14 requests under way per compute unit.  Tiles of 128 features and fp32 storage from N = 48 on measured slower than the LDS-panel kernels.
+// return path for 28 %, 14 requests under way per compute unit.  Tiles of 128 features and fp32 storage from N = 48 on measured slower than the LDS-panel kernels.
 template <class E, int NT, int WR, int OCC, bool RAGGED>
 __global__ __launch_bounds__(256, OCC)
 void spmm_tile_kernel(const TileArgs ta)

@@ -5,7 +5,7 @@
 // At 10 % density and more a 16-row unit touches 81 % of all columns and more: the LDS-panel kernels (spmm_panel_kernel.hpp), which
 // condense columns, read a second operand from LDS for every matrix instruction and stream tiles that are mostly zeros all the same.
 // Here A is kept as first operands, 16 rows x 64 columns each, no columns condensed: a wave loads an operand straight into the
-// registers of its matrix instructions, and a second operand serves the one to four units of a wave.
+// registers of its matrix instructions, and a second operand serves the one to three units of a wave.
 #include "spmm_tile_common.hpp"
 
 namespace hspmm {
