@@ -16,6 +16,7 @@ const Cost kCosts[2][3] = {
     {{4, 2.75, 0.0, 0.441, 0.050}, {8, 2.2, 0.77, 0.241, 0.063}, {16, 1.5, 1.22, 0.0, 0.077}},
 };
 constexpr double kFewestEntries = 0.028, kMostEntries = 0.31;         // of all
+constexpr uint32_t kMostRowsTwoTiles = 16384;                         // see narrow_serves
 
 uint32_t one_tile(uint32_t N) { return N % 2u ? 15u : 16u; }
 uint32_t most_features(uint32_t N) { return N % 2u ? 29u : 32u; }
@@ -87,6 +88,9 @@ int build_narrow_stream(hspmm_plan *p)
 // faster one; 5 % of those taken lose, 5 % on average).  Up to 31 % of entries, as far as times are known.
 // 480 launches taken, six to 48 matrices of 800 MB together in turn, whose streams come from memory / one matrix over and over, old time
 // over new: entry kernels 1.65 / 1.48, full-tile 1.21 / 1.34, gather 2.2 / 2.0; 7 / 23 lose more than 3 %, up to 20 %, most of them of less than 10 us.
+// Matrices of more rows than those of the fit take many rounds of workgroups, and with more than one tile of features the full-tile kernels, which
+// put a block of A together once for 128 rows, are ahead (39040 x 5440 at 15 %, N = 32 52.1 / 41.6 us, 21888 x 5952 at 11 % 34.4 / 29.4,
+// but N = 16 25.0 / 26.1).
 // B that begins between two words makes these kernels half as slow again, and with two tiles of features 1.7 times; the full-tile and wide-tile
 // kernels take as long as ever, the entry kernels 1.5 times, but not at up to eight features (8704 x 5120 at 5 %, N = 32 34 us, full tiles
 // 17.9; 12800 x 1963 at 9 %, N = 2 12.5, entries 6.8, N = 16 12.6, entries 16.8).
@@ -104,7 +108,7 @@ bool narrow_serves(const hspmm_plan *p, uint32_t N, bool on_word)
     if (double(p->narrow.entries) > kMostEntries * p->rows * p->cols) return false;
     if (!on_word && (wide_serves(p, N) || tile_serves(p, N) || (N <= 8u && entries_serve(p, N)))) return false;
     if (wide_serves(p, N)) return expected < 0.9 * p->wide.expected_fewest;     // (N = 32)
-    if (tile_serves(p, N)) return true;
+    if (tile_serves(p, N)) return N <= one_tile(N) || p->rows <= kMostRowsTwoTiles;
     if (entries_serve(p, N)) return expected < 0.9 * entries_expected(p, N) - 0.3;
     return !panel_serves(p, N);
 }

@@ -106,6 +106,17 @@ int main()
         for (uint32_t N : {1u, 2u, 7u, 8u, 9u, 15u, 16u, 29u, 32u})
             if (!narrow_serves(&q, N, true) || narrow_serves(&q, N, false) != (by_entries && N > 8u)) { std::printf("N = %u: taken %d %d\n", N, int(narrow_serves(&q, N, true)), int(narrow_serves(&q, N, false))); return 1; }
     }
+    // many rows and more than a tile of features are the full-tile kernels'
+    for (uint32_t rows : {16384u, 20480u}) {
+        hspmm_plan m;
+        m.dtype = HSPMM_BF16; m.rows = rows; m.cols = 4096; m.W = rows / 8; m.T = rows / 8 * 146; m.compute_units = 256; m.per_column = 1.4;
+        left = 100;
+        if (build_narrow_stream(&m)) return 1;
+        m.narrow.entries = uint64_t(rows) * 410u;
+        by_entries = false; by_tile = true;
+        for (uint32_t N : {8u, 15u, 16u, 17u, 32u})
+            if (narrow_serves(&m, N, true) != (N <= 16u || rows <= 16384u)) { std::printf("%u rows, N = %u: taken %d\n", rows, N, int(narrow_serves(&m, N, true))); return 1; }
+    }
     std::printf("ok\n");
     return 0;
 }
