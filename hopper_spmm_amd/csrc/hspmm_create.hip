@@ -766,6 +766,8 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
         timer.mark("narrow stream");
         if ((rc = build_wide_stream(p))) return bail(rc);
         timer.mark("wide-tile stream");
+        if ((rc = build_block_units(p, st, rowOffset, tcA2B))) return bail(rc);
+        timer.mark("block units");
         if ((rc = entries_counted(p))) return bail(rc);                 // (any stream may launch now)
     } catch (const std::bad_alloc &) {
         return bail(fail(HSPMM_ERR_ALLOC, "out of host memory"));

@@ -66,6 +66,7 @@ struct Config {
     int narrow = -1;                    // narrow kernels (-1: by density and expected time, 0 never, 1 wherever they can)
     int narrow_waves = -1;              // waves of their workgroups (-1: by expected time)
     int wide = -1;                      // wide-tile kernels (-1: by density and expected time, 0 never, 1 wherever they can)
+    int block = -1;                     // block kernels (-1: by expected time, 0 never, 1 wherever they can)
     int wide_cuts = -1;                 // workgroups of a C tile (-1: by expected time)
     int wide_shape = -1;                // their workgroup's shape, an index into the table of hspmm_wide.hip (-1: by expected time)
     int xcd_split = -1;                 // gather kernels: two feature blocks dealt out by XCD half (-1: by matrix, 0 never, 1 always)
@@ -86,6 +87,7 @@ struct Config {
         if (const char *e = std::getenv("HSPMM_TILE")) tile = std::atoi(e) != 0;
         if (const char *e = std::getenv("HSPMM_NARROW")) narrow = std::atoi(e) != 0;
         if (const char *e = std::getenv("HSPMM_NARROW_WAVES")) narrow_waves = std::atoi(e);
+        if (const char *e = std::getenv("HSPMM_BLOCK")) block = std::atoi(e) != 0;
         if (const char *e = std::getenv("HSPMM_WIDE")) wide = std::atoi(e) != 0;
         if (const char *e = std::getenv("HSPMM_WIDE_SHAPE")) wide_shape = std::max(0, std::atoi(e));
         if (const char *e = std::getenv("HSPMM_WIDE_CUTS")) wide_cuts = std::max(0, std::atoi(e));
@@ -233,6 +235,15 @@ struct hspmm_plan {
         double expected_fewest = 0.0;                            // us, of the fewest features they take (see hspmm_wide.hip)
         mutable hspmm_host::KeptAnswers choices;
     } wide;
+    // Weights in 16 x 16 blocks, 16-bit types, for few features: units of windows whose steps are neighbouring columns (spmm_block_kernel.hip)
+    struct Block {
+        bool built = false;
+        const hspmm::BlockUnit *d_units = nullptr;
+        const uint32_t *d_columns = nullptr;
+        const hspmm::TileSource *d_source = nullptr;
+        uint32_t n_units = 0;
+        mutable hspmm_host::KeptAnswers taken;
+    } block_units;
     double per_column = 8.0;            // stored entries per tile column, from a sample of the tiles
     bool even_windows = false;          // no unit has over eight times the average number of steps
     // What launches write besides C, one set per stream that has launched this plan (launches on different
@@ -352,9 +363,14 @@ int run_tile(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s,
 int build_narrow_stream(hspmm_plan *p);
 bool narrow_serves(const hspmm_plan *p, uint32_t N, bool on_word);        // on_word: B begins on a word
 int run_narrow(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode);
+// hspmm_block.hip: what the block kernels need to know of the units, whether they take this launch, and the launch
+int build_block_units(hspmm_plan *p, const StepStream &st, const uint32_t *rowOffset, const uint32_t *tcA2B);
+bool block_serves(const hspmm_plan *p, uint32_t N);
+int run_block(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode);
 // hspmm_wide.hip: the wide-tile kernels' stream, whether they take this launch, and the launch
 int build_wide_stream(hspmm_plan *p);
 bool wide_serves(const hspmm_plan *p, uint32_t N);
+double blocks_expected(const hspmm_plan *p, uint32_t N);        // us, weights in 16 x 16 blocks, by these or the gather kernels
 int run_wide(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, hipEvent_t mid, RunMode mode);
 
 // hspmm_run.hip: the address of the device's fixed scratch array (hspmm_run_static); `device` must be current

@@ -165,6 +165,8 @@ bool wide_serves(const hspmm_plan *p, uint32_t N)
     return kept_choice(p, N) & 1u;
 }
 
+double blocks_expected(const hspmm_plan *p, uint32_t N) { return wide_serves(p, N) ? choose_wide_shape(p, N).expected : blocks_gather_expected(p, N); }
+
 int run_wide(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, hipEvent_t mid, RunMode mode)
 {
     const hspmm_plan::Wide &w = p->wide;

@@ -232,7 +232,7 @@ int hspmm_set_panel_stream(int mode);
  * groups (atomic = 1) is cut only where one of its groups ends, a window given as one group is
  * never cut; partial sums of a cut window are added in group order, not with atomics.  Kept by
  * plans whose units are the caller's single windows walked by the gather kernels
- * (hspmm_plan_info.group_cuts_kept = 1; such plans have no entry, narrow and wide-tile
+ * (hspmm_plan_info.group_cuts_kept = 1; such plans have no entry, block, narrow and wide-tile
  * kernels); plans that merge windows with one column list, the LDS-panel and full-tile kernels
  * (they walk a re-tiled stream) and the all-shapes kernel (one wave per window, nothing cut)
  * have no use for the cuts.  The product is the same up to the order of the
@@ -272,8 +272,8 @@ typedef struct {
     uint32_t n_panel_units;     /* units of that stream: groups of up to four adjacent windows that share, or were given, one column list */
     uint32_t n_panel_paired_units;  /* of those: units of two or more windows */
     uint32_t n_panel_wide_units;    /* of those: units of three or four windows */
-    uint32_t last_kernel_family;    /* what the last hspmm_run launched: 0 nothing yet, 1 all-shapes kernel, 2 gather kernels (MFMA, or entry
-                                       by entry: last_mfma_kind 0 then), 3 LDS-staging kernels (a panel of B at a time, or full operands of A:
+    uint32_t last_kernel_family;    /* what the last hspmm_run launched: 0 nothing yet, 1 all-shapes kernel, 2 gather kernels (MFMA, whole
+                                       16 x 16 blocks among them, or entry by entry: last_mfma_kind 0 then), 3 LDS-staging kernels (a panel of B at a time, or full operands of A:
                                        full-tile, narrow and wide-tile kernels), 4 clear only (matrix without entries); hspmm_last_kernel tells them apart */
     uint32_t gather_bitmap;         /* 1: the gather kernels read this plan's tiles as bitmap + stored elements (single
                                      * windows with few stored elements per tile), 0: as uncompressed tiles */
@@ -295,7 +295,7 @@ typedef struct {
 int hspmm_get_plan_info(const hspmm_plan *plan, hspmm_plan_info *info);
 
 /* No reference counterpart: the name of the main kernel of the last hspmm_run - spmm_entries_kernel,
- * spmm_mfma_kernel, spmm_panel_kernel, spmm_tile_kernel, spmm_narrow_kernel, spmm_wide_kernel, spmm_scalar_kernel, or
+ * spmm_mfma_kernel, spmm_panel_kernel, spmm_tile_kernel, spmm_narrow_kernel, spmm_wide_kernel, spmm_block_kernel, spmm_scalar_kernel, or
  * fill_zero_kernel for a matrix without entries; "" before the first (hspmm_plan_info.last_kernel_family names two of them with one number). */
 const char *hspmm_last_kernel(const hspmm_plan *plan);
 
