@@ -186,8 +186,8 @@ struct WideArgs {
 // mid: as of launch_spmm_mfma, in front of the kernel that adds the sums of cut C tiles
 hipError_t launch_spmm_wide(int dtype, const WideArgs &wa, const WideShape &sh, hipStream_t s, hipEvent_t mid);
 hipError_t launch_wide_fill(const TileSource &src, uint32_t rows, uint32_t n_chunks, void *frags, hipStream_t s);
-// Block kernels (spmm_block_kernel.hip, 16-bit types): units of two windows with one column list (lower: kIdxMax where a window is alone),
-// in steps of 16 neighbouring columns
+// Block kernels (spmm_block_kernel.hip): units of two windows with one column list (lower: kIdxMax where a window is alone),
+// in steps of 16 (fp32 storage: 8) neighbouring columns
 struct BlockUnit { uint32_t upper, lower, steps, row, next_row, pair_begin, spare[2]; };     // first tiles; steps; first row, that of the unit behind; first pair of steps
 struct BlockArgs {
     const BlockUnit *units;

@@ -235,7 +235,7 @@ struct hspmm_plan {
         double expected_fewest = 0.0;                            // us, of the fewest features they take (see hspmm_wide.hip)
         mutable hspmm_host::KeptAnswers choices;
     } wide;
-    // Weights in 16 x 16 blocks, 16-bit types, for few features: units of windows whose steps are neighbouring columns (spmm_block_kernel.hip)
+    // Weights in 16 x 16 blocks, for few features: units of windows whose steps are neighbouring columns (spmm_block_kernel.hip)
     struct Block {
         bool built = false;
         const hspmm::BlockUnit *d_units = nullptr;

@@ -1,4 +1,4 @@
-// Kernels for few features of weights kept in 16 x 16 blocks, 16-bit types: C = A * B by whole blocks, read where a plan's tiles lie (the
+// Kernels for few features of weights kept in 16 x 16 blocks: C = A * B by whole blocks, read where a plan's tiles lie (the
 // reference's 8-row windows, src/utils/class.h:74-85): two windows with one column list are the halves of a row of blocks.
 //
 // The gather kernels (spmm_mfma_kernel.hpp), which take any column list, load a row of B at a time, in words: with 16 features a
@@ -183,9 +183,111 @@ odds[S] = 0u;
     }
 }
 
+// The same of fp32 storage, in fp32 products: a unit's steps are eight columns, two of them four matrix instructions per 16 features.  Their
+// second operands are a feature of four rows of B, which lanes load as they lie: lane (g, j) the features V j .. V j + V - 1.
+// What bounds it: the tiles' way from memory, and for 64 features the matrix instructions (32 cycles each).  us, three matrices in turn, by the
+// gather or LDS-panel kernels / here: 4096 x 14336 at 50 %, N = 8 36.0 / 33.7, 15 47.1 / 33.6, 33 79.7 / 54.3; 4096^2 at 50 %, N = 16 15.1 / 10.2,
+// 32 14.9 / 11.6, 47 39.0 / 17.9; 16000 x 1111 at 25 %, N = 16 12.2 / 8.7.
+template <int V, int W>
+__global__ __launch_bounds__(64 * W, 2) void spmm_block_f32_kernel(const BlockArgs ba)
+{
+    constexpr int kAhead = 3;
+    typedef float floats __attribute__((ext_vector_type(4)));
+    __shared__ float smem[W * V * 256];
+    __shared__ uint32_t not_finite;
+
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, j = lane & 15u;
+    const BlockUnit unit = ba.units[blockIdx.x];
+    const uint32_t rows_here = unit.lower != kIdxMax ? 16u : 8u;
+    const size_t row_bytes = size_t(ba.N) * 4u;
+    if (tid == 0u) not_finite = 0u;
+
+    const uint32_t features = umin32(uint32_t(V) * j, ba.N - V) * 4u;       // (lanes behind the last feature are moved back to end with the row)
+    const bool upper = j < 8u, a_there = upper || rows_here == 16u;
+    const char *const a_lane = static_cast<const char *>(ba.tiles) + size_t(upper || rows_here == 8u ? unit.upper : unit.lower) * 256u + (j & 7u) * 32u + (g & 1u) * 16u;
+    const char *const B = static_cast<const char *>(ba.B) + features;
+
+    f32x4 acc[V];
+#pragma unroll
+    for (int c = 0; c < V; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const uint32_t pairs = (unit.steps + 1u) >> 1;
+    for (uint32_t q0 = wave; q0 < pairs; q0 += 64u * W) {
+        const uint32_t n = umin32((pairs - q0 + W - 1u) / W, 64u);
+        const u32x2 mine = reinterpret_cast<const u32x2 *>(ba.columns)[unit.pair_begin + umin32(q0 + lane * W, pairs - 1u)];
+        floats a[kAhead];
+        float b[kAhead][4][V];
+        auto request = [&](auto slot, uint32_t i) __attribute__((always_inline)) {
+            constexpr int S = decltype(slot)::value;
+            const uint32_t at = umin32(i, n - 1u), step = 2u * (q0 + at * W) + (g >> 1);
+            a[S] = *reinterpret_cast<const floats *>(a_lane + size_t(umin32(step, unit.steps - 1u)) * 256u);
+            if (!a_there || step >= unit.steps) a[S] = floats{0.f, 0.f, 0.f, 0.f};
+            const uint32_t first = __builtin_amdgcn_readlane(mine[0], int(at)), second = __builtin_amdgcn_readlane(mine[1], int(at));
+            const uint32_t column = (g < 2u ? first : second) + (g & 1u) * 4u;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const char *from = B + umin32(column + k, ba.cols - 1u) * uint32_t(row_bytes);      // (behind the last column: zeros multiply it)
+                if constexpr (V == 1) {
+                    b[S][k][0] = *reinterpret_cast<const float *>(from);
+                } else {
+                    typedef float some __attribute__((ext_vector_type(V), aligned(4)));
+                    const some x = *reinterpret_cast<const some *>(from);
+#pragma unroll
+                    for (int c = 0; c < V; ++c) b[S][k][c] = x[c];
+                }
+            }
+        };
+        auto multiply = [&](auto slot, uint32_t i) __attribute__((always_inline)) {
+            constexpr int S = decltype(slot)::value;
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+#pragma unroll
+                for (int c = 0; c < V; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[S][k], b[S][k][c], acc[c], 0, 0, 0);
+            request(slot, i + kAhead);
+        };
+        typedef std::integral_constant<int, 0> S0;
+        typedef std::integral_constant<int, 1> S1;
+        typedef std::integral_constant<int, 2> S2;
+        request(S0{}, 0); request(S1{}, 1); request(S2{}, 2);
+        uint32_t i = 0;
+        for (; i + 3u <= n; i += 3u) { multiply(S0{}, i); multiply(S1{}, i + 1u); multiply(S2{}, i + 2u); }
+        if (i < n) multiply(S0{}, i);
+        if (i + 1u < n) multiply(S1{}, i + 1u);
+    }
+
+    // lane (g, j) has rows 4 g .. 4 g + 3 of its features
+#pragma unroll
+    for (int c = 0; c < V; ++c)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) smem[(wave * V + c) * 256 + e * 64 + lane] = acc[c][e];
+    __syncthreads();
+    float *const C = static_cast<float *>(ba.C);
+    for (uint32_t t = tid; t < 256u * V; t += 64u * W) {
+        const uint32_t r = t / (16u * V), of = t % (16u * V) / V, c = t % V, feature = umin32(V * of, ba.N - V) + c, row = unit.row + r;
+        float x = 0.f;
+#pragma unroll
+        for (int w = 0; w < W; ++w) x += smem[(w * V + c) * 256 + (r & 3u) * 64 + (r >> 2) * 16 + of];
+        if (r < rows_here && row < ba.rows && V * of < ba.N && feature >= V * of) {
+            C[size_t(row) * ba.N + feature] = x;
+            if (!(x * 0.f == 0.f)) not_finite = 1u;
+        }
+    }
+    for (uint32_t range = blockIdx.x ? 1u : 0u; range < 2u; ++range) {
+        const uint32_t from = range ? unit.row + rows_here : 0u, to = umin32(range ? unit.next_row : unit.row, ba.rows);
+        if (from < to)
+            for (size_t at = size_t(from) * ba.N + tid; at < size_t(to) * ba.N; at += 64u * W) C[at] = 0.f;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (not_finite) {
+        BlockArgs again = ba;
+        again.rows = umin32(ba.rows, unit.row + rows_here);
+        for (uint32_t f = wave * 16u; f < ba.N; f += W * 16u) tile_sum_again<FloatStored, 1, 16, true>(again, unit.row, f, f, umin32(ba.N, f + 16u), lane);
+    }
+}
+
 hipError_t launch_spmm_block(int dtype, const BlockArgs &ba, uint32_t n_units, hipStream_t s)
 {
-    if (!n_units || n_units >= (1u << 22) || !ba.N || ba.N > 64u || !ba.cols || uint64_t(ba.cols) * ba.N * 2u > (1ull << 32)) return hipErrorInvalidValue;
+    if (!n_units || n_units >= (1u << 22) || !ba.N || ba.N > 64u || !ba.cols || uint64_t(ba.cols) * ba.N * (dtype == kDtypeF32 ? 4u : 2u) > (1ull << 32)) return hipErrorInvalidValue;
     const uint32_t blocks = (ba.N + 15u) / 16u;
     const bool odd = ba.N % 2u && ba.N > 8u && reinterpret_cast<uintptr_t>(ba.B) % 4u == 0u;
 #define HSPMM_BLOCK(CF, BF, ODD, NARROW) { spmm_block_kernel<BF, CF, 8, ODD, NARROW><<<dim3(n_units), 512, 0, s>>>(ba); return hipGetLastError(); }
@@ -195,6 +297,12 @@ hipError_t launch_spmm_block(int dtype, const BlockArgs &ba, uint32_t n_units, h
 #define HSPMM_BLOCKS_ODD(CF) \
     if (odd && blocks == CF && dtype == kDtypeF16) HSPMM_BLOCK(CF, false, true, false) \
     if (odd && blocks == CF && dtype == kDtypeBf16) HSPMM_BLOCK(CF, true, true, false)
+    if (dtype == kDtypeF32) {
+        if (ba.N <= 16u) spmm_block_f32_kernel<1, 8><<<dim3(n_units), 512, 0, s>>>(ba);
+        else if (ba.N <= 32u) spmm_block_f32_kernel<2, 8><<<dim3(n_units), 512, 0, s>>>(ba);
+        else spmm_block_f32_kernel<4, 8><<<dim3(n_units), 512, 0, s>>>(ba);
+        return hipGetLastError();
+    }
     if (ba.N < 8u && dtype == kDtypeF16) HSPMM_BLOCK(1, false, false, true)
     if (ba.N < 8u && dtype == kDtypeBf16) HSPMM_BLOCK(1, true, false, true)
     HSPMM_BLOCKS_ODD(1) HSPMM_BLOCKS_ODD(2) HSPMM_BLOCKS(1) HSPMM_BLOCKS(2) HSPMM_BLOCKS(3) HSPMM_BLOCKS(4)
