@@ -9,13 +9,10 @@ using namespace hspmm_host;
 
 namespace hspmm_host {
 
-// canonical (optional): whether every window's real column ids ascend strictly with padding only behind
-// the window's last column, as the reference's converter writes them (src/utils/convert.h:166-181).
-int validate_format(uint32_t rows, uint32_t cols, uint32_t W, uint32_t T, uint32_t cw,
-                    const uint32_t *rowOffset, const uint32_t *tcA2B, const void *data, const uint32_t *rowIdx,
-                    bool *canonical, uint32_t *header, uint32_t *window_stored)
+// The windows: what says how long the arrays of the tiles are.
+static int validate_windows(uint32_t rows, uint32_t cols, uint32_t W, uint32_t T, const uint32_t *rowOffset, const uint32_t *tcA2B,
+                            const void *data, const uint32_t *rowIdx)
 {
-    if (canonical) *canonical = true;
     if (W == 0) {
         if (T != 0) return fail(HSPMM_ERR_INVALID, "total_tiles = %u with no effective row window", T);
         return HSPMM_OK;
@@ -35,6 +32,16 @@ int validate_format(uint32_t rows, uint32_t cols, uint32_t W, uint32_t T, uint32
     }
     if (rowOffset[W] != T)
         return fail(HSPMM_ERR_INVALID, "rowOffset[%u] = %u differs from total_tiles = %u", W, rowOffset[W], T);
+    return HSPMM_OK;
+}
+
+// The tiles of windows found good.  canonical (optional): whether every window's real column ids ascend strictly with padding only behind
+// the window's last column, as the reference's converter writes them (src/utils/convert.h:166-181).
+static int validate_tiles(uint32_t cols, uint32_t W, uint32_t T, uint32_t cw, const uint32_t *rowOffset, const uint32_t *tcA2B, const void *data,
+                          bool *canonical, uint32_t *header, uint32_t *window_stored)
+{
+    if (canonical) *canonical = true;
+    if (W == 0) return HSPMM_OK;
     // every tile's ids: real columns below `cols`, padding only behind them.  Checked on all cores; the message
     // names the first tile that fails.
     auto tile_error = [&](uint32_t t, bool report) -> bool {
@@ -75,6 +82,13 @@ int validate_format(uint32_t rows, uint32_t cols, uint32_t W, uint32_t T, uint32
     if (first_bad.load() < T) { tile_error(first_bad.load(), true); return HSPMM_ERR_INVALID; }
     if (canonical) *canonical = ordered.load();
     return HSPMM_OK;
+}
+
+int validate_format(uint32_t rows, uint32_t cols, uint32_t W, uint32_t T, uint32_t cw,
+                    const uint32_t *rowOffset, const uint32_t *tcA2B, const void *data, const uint32_t *rowIdx, bool *canonical)
+{
+    if (int rc = validate_windows(rows, cols, W, T, rowOffset, tcA2B, data, rowIdx)) return rc;
+    return validate_tiles(cols, W, T, cw, rowOffset, tcA2B, data, canonical, nullptr, nullptr);
 }
 
 int plan_reserve(hspmm_plan *p, size_t bytes)
@@ -519,8 +533,10 @@ double entries_per_column(uint32_t T, uint32_t cw, uint32_t elem, const uint32_t
 // 32 + 2 e bytes against 256 per tile with e stored elements (16 + 4 e for fp32) - worth it below about a third full, and
 // where the tile stream is large enough to be traffic at all (a matrix whose tiles sit in the L2s only pays the longer
 // dependent chain: 4096 x 4096 at 1 %, 2.7 MB of tiles: 6.8 -> 7.5 us).  From 64 groups of 64 tiles spread over the matrix.
-bool tiles_look_sparse(const Config &cfg, uint32_t T, uint32_t elem, const void *data)
+// share: the part of their elements that the sample stores (0: not looked at).
+bool tiles_look_sparse(const Config &cfg, uint32_t T, uint32_t elem, const void *data, double *share)
 {
+    *share = 0.0;
     if (cfg.gather_bitmap >= 0) return cfg.gather_bitmap > 0;
     if (size_t(T) * 256u < (size_t(8) << 20)) return false;
     std::vector<uint32_t> header(64u * 8u);
@@ -530,7 +546,56 @@ bool tiles_look_sparse(const Config &cfg, uint32_t T, uint32_t elem, const void 
         stored += hspmm_host::tile_masks(static_cast<const char *>(data) + t0 * 256u, n, elem, header.data());
         seen += n * (256u / elem);
     }
+    *share = double(stored) / double(seen);
     return stored * 3u < seen;
+}
+
+// What a step of a plan's creation that may run on another thread came to: its code, and its message, which belongs to that thread.
+struct Outcome {
+    int rc = HSPMM_OK;
+    std::string text;
+    static Outcome of(int rc) { return {rc, rc ? hspmm_last_error() : ""}; }
+};
+
+// The device the plan is for.
+int find_device(hspmm_plan *p)
+{
+    hipError_t e = hipGetDevice(&p->device);
+    if (e != hipSuccess) return fail(HSPMM_ERR_DEVICE, "hipGetDevice failed: %s", hipGetErrorString(e));
+    hipDeviceProp_t prop;
+    e = hipGetDeviceProperties(&prop, p->device);
+    if (e != hipSuccess) return fail(HSPMM_ERR_DEVICE, "hipGetDeviceProperties failed: %s", hipGetErrorString(e));
+    if (strncmp(prop.gcnArchName, "gfx950", 6) != 0)
+        return fail(HSPMM_ERR_UNSUPPORTED, "device %d is %s; this library is built for gfx950 only", p->device, prop.gcnArchName);
+    p->compute_units = p->cfg.sm_num > 0 ? p->cfg.sm_num : prop.multiProcessorCount;
+    // the address of this device's fixed scratch array, for hspmm_run_static (which then looks nothing up)
+    float *unused = nullptr;
+    return static_scratch_address(p->device, &unused);
+}
+
+// (worker threads start on the first device)
+int copy_up(const hspmm_plan *p, void *to, const void *from, size_t bytes)
+{
+    HSPMM_HIP(hipSetDevice(p->device));
+    HSPMM_HIP(hipMemcpy(to, from, bytes, hipMemcpyHostToDevice));
+    return HSPMM_OK;
+}
+
+// One block of device memory for everything whose size is known early, and the arrays that are checked already or lie inside checked bounds.
+int upload_windows(hspmm_plan *p, const uint32_t *rowOffset, const uint32_t *rowIdx, const uint32_t *tcA2B, size_t block)
+{
+    HSPMM_HIP(hipSetDevice(p->device));
+    if (int rc = plan_reserve(p, block)) return rc;
+    if (int rc = upload(p, &p->d_rowOffset, rowOffset, size_t(p->W) + 1)) return rc;
+    if (int rc = upload(p, &p->d_rowIdx, rowIdx, size_t(p->W))) return rc;
+    return upload(p, &p->d_a2b_raw, tcA2B, size_t(p->T) * p->cw);
+}
+
+int upload_units(hspmm_plan *p, const StepStream &st)
+{
+    HSPMM_HIP(hipSetDevice(p->device));
+    if (int rc = upload(p, &p->d_unitOffset, st.unitOffset.data(), st.unitOffset.size())) return rc;
+    return upload(p, &p->d_unitRow, st.unitRow.data(), st.unitRow.size());
 }
 
 // hspmm_create; with `bitmap` (data == nullptr) the tiles come as the caller's bitmap arrays,
@@ -556,83 +621,113 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
     // read that stream, and a graph of 2^18 vertices is 24 MB to send instead of 77.
     hspmm_host::ZeroedBuffer<uint32_t> header;
     std::vector<uint32_t> window_stored;
-    bool sparse_tiles = !bitmap && data && eff_row_windows && total_tiles && tiles_look_sparse(cfg, total_tiles, elem, data);
+    double likely_stored = 0.0;
+    bool sparse_tiles = !bitmap && data && eff_row_windows && total_tiles && tiles_look_sparse(cfg, total_tiles, elem, data, &likely_stored);
     try {
         if (sparse_tiles) {
             header = hspmm_host::ZeroedBuffer<uint32_t>(size_t(total_tiles) * (elem == 2u ? 8u : 4u));
             window_stored.assign(size_t(eff_row_windows) + 1u, 0u);
         }
     } catch (const std::bad_alloc &) { return fail(HSPMM_ERR_ALLOC, "out of host memory"); }
-    int rc = validate_format(rows, cols, eff_row_windows, total_tiles, cw, rowOffset, tcA2B, bitmap ? bitmap->data : data, rowIdx,
-                             &canonical, sparse_tiles ? header.data() : nullptr, window_stored.data());
+    const void *tile_values = bitmap ? bitmap->data : data;
+    int rc = validate_windows(rows, cols, eff_row_windows, total_tiles, rowOffset, tcA2B, tile_values, rowIdx);
     if (rc) return rc;
-    timer.mark("validate");
 
     hspmm_plan *p = new (std::nothrow) hspmm_plan;
     if (!p) return fail(HSPMM_ERR_ALLOC, "out of host memory");
     p->dtype = dtype; p->rows = rows; p->cols = cols; p->W = eff_row_windows; p->T = total_tiles;
-    p->cw = cw; p->elem = elem; p->canonical = canonical;
+    p->cw = cw; p->elem = elem;
     p->cfg = cfg;
 
     auto bail = [&](int code) { hspmm_destroy(p); return code; };
-    hipError_t e = hipGetDevice(&p->device);
-    if (e != hipSuccess) return bail(fail(HSPMM_ERR_DEVICE, "hipGetDevice failed: %s", hipGetErrorString(e)));
-    hipDeviceProp_t prop;
-    e = hipGetDeviceProperties(&prop, p->device);
-    if (e != hipSuccess) return bail(fail(HSPMM_ERR_DEVICE, "hipGetDeviceProperties failed: %s", hipGetErrorString(e)));
-    if (strncmp(prop.gcnArchName, "gfx950", 6) != 0)
-        return bail(fail(HSPMM_ERR_UNSUPPORTED, "device %d is %s; this library is built for gfx950 only", p->device,
-                         prop.gcnArchName));
-    p->compute_units = p->cfg.sm_num > 0 ? p->cfg.sm_num : prop.multiProcessorCount;
-    {
-        // the address of this device's fixed scratch array, for hspmm_run_static (which then looks nothing up)
-        float *unused = nullptr;
-        if ((rc = static_scratch_address(p->device, &unused))) return bail(rc);
-    }
+    // (arrays that are not good are told of before a device that is not there)
+    Outcome device = Outcome::of(find_device(p));
+    StepStream st;
+    const size_t n_ids = size_t(total_tiles) * cw, tile_bytes = size_t(total_tiles) * 256u;
+    const size_t spare = 8u / elem;                                     // a lane may read 8 bytes from the last element on
+    try {
+        // Side by side: the tiles' checks and masks on all cores, the units, device memory and the arrays whose sizes are known.
+        Outcome tiles, arrays;
+        std::atomic<int> next{0};
+        parallel_workers(p->W ? 3u : 1u, [&](unsigned) {
+            for (int task = next++; task < 3; task = next++) {
+                if (task == 0) {
+                    tiles = Outcome::of(validate_tiles(cols, eff_row_windows, total_tiles, cw, rowOffset, tcA2B, tile_values, &canonical,
+                                                       sparse_tiles ? header.data() : nullptr, window_stored.data()));
+                } else if (task == 1 && !device.rc && p->W) {
+                    arrays = Outcome::of(upload_windows(p, rowOffset, rowIdx, tcA2B,
+                                                        entries_count_bytes(p) + (size_t(p->W) * 4u + 2u) * 4u + n_ids * 8u + tile_bytes + header.size() * 4u +
+                                                            size_t(likely_stored * 1.1 * double(tile_bytes)) + (size_t(1) << 20)));
+                } else if (task == 2 && p->W) {
+                    st = build_units(p->W, cw, rowOffset, rowIdx, tcA2B, p->cfg.pairing);
+                }
+            }
+        });
+        for (const Outcome *o : {&tiles, &device, &arrays})
+            if (o->rc) return bail(fail(o->rc, "%s", o->text.c_str()));
+    } catch (const std::bad_alloc &) { return bail(fail(HSPMM_ERR_ALLOC, "out of host memory")); }
+    p->canonical = canonical;
+    timer.mark("checks, masks, units, ids");
 
     // (a host allocation that fails anywhere below ends the call with HSPMM_ERR_ALLOC)
     if (p->W) try {
-        const size_t n_ids = size_t(total_tiles) * cw, tile_bytes = size_t(total_tiles) * 256u;
-        const StepStream st = build_units(p->W, cw, rowOffset, rowIdx, tcA2B, p->cfg.pairing);
         if (bitmap && st.G != 1) return bail(kNeedsPlainTiles);         // paired windows: their tiles are re-laid out on the host
         p->G = st.G;
         p->n_units = uint32_t(st.unitRow.size());
         p->n_paired = st.n_paired;
         p->n_steps = st.n_steps;
-        timer.mark("units");
-        const size_t spare = 8u / elem;                                 // a lane may read 8 bytes from the last element on
+        p->h_unitOffset = st.unitOffset;
+        p->h_unitRow = st.unitRow;
+        // single windows walked tile by tile: the caller's tile numbers are the stream's, its cuts can be kept
+        if (cuts && p->cfg.group_cuts && st.G == 1) p->caller_cuts.assign(cuts->offsets, cuts->offsets + size_t(cuts->n_groups) + 1u);
         uint64_t stored = 0;
         for (uint32_t w = 0; sparse_tiles && w < p->W; ++w) stored += window_stored[w];
         sparse_tiles = sparse_tiles && st.G == 1 && stored + spare < (uint64_t(1) << 31) &&
                        (p->cfg.gather_bitmap > 0 || stored * 3u < uint64_t(total_tiles) * 8u * cw);
-        // one block for everything whose size is known here, and a megabyte for the partitions
-        if ((rc = plan_reserve(p, entries_count_bytes(p) + (size_t(p->W) * 4u + 2u) * 4u + n_ids * 8u + tile_bytes + header.size() * 4u +
-                                      (sparse_tiles ? (size_t(stored) + spare) * elem : 0u) + (size_t(1) << 20))))
-            return bail(rc);
-        timer.mark("device memory");
-        if ((rc = upload(p, &p->d_rowOffset, rowOffset, size_t(p->W) + 1))) return bail(rc);
-        if ((rc = upload(p, &p->d_rowIdx, rowIdx, size_t(p->W)))) return bail(rc);
-        if ((rc = upload(p, &p->d_a2b_raw, tcA2B, n_ids))) return bail(rc);
-        timer.mark("upload ids");
         void *room = nullptr;
         if (sparse_tiles) {
-            hspmm_host::ZeroedBuffer<uint8_t> vals((size_t(stored) + spare) * elem);
-            uint64_t at = 0;
+            // Side by side: the stored elements one after the other, and what else the launches need of the host.
             std::vector<uint64_t> first(p->W);
-            for (uint32_t w = 0; w < p->W; ++w) { first[w] = at; at += window_stored[w]; }
-            hspmm_host::parallel_weighted(p->W, size_t(1) << 13, [=](size_t w) { return rowOffset[w]; }, [&](size_t wb, size_t we) {
-                const uint32_t t0 = rowOffset[wb];
-                hspmm_host::pack_tiles(static_cast<const char *>(data) + size_t(t0) * 256u, rowOffset[we] - t0, elem,
-                                       header.data() + size_t(t0) * (elem == 2u ? 8u : 4u), first[wb], vals.data());
-            });
-            timer.mark("bitmap tiles");
-            uint8_t *dv = nullptr;
-            if ((rc = upload(p, &p->bm.d_header, header.data(), header.size()))) return bail(rc);
-            if ((rc = upload(p, &dv, vals.data(), vals.size()))) return bail(rc);
-            p->bm.d_vals = dv; p->bm.stored = stored; p->bm.built = true;
+            for (uint64_t w = 0, at = 0; w < p->W; ++w) { first[w] = at; at += window_stored[w]; }
+            const size_t vals_bytes = (size_t(stored) + spare) * elem, header_bytes = header.size() * 4u;
+            hspmm_host::ZeroedBuffer<uint8_t> vals(vals_bytes);
+            if ((rc = plan_alloc(p, header_bytes, &room))) return bail(rc);
+            p->bm.d_header = static_cast<uint32_t *>(room);
+            if ((rc = plan_alloc(p, vals_bytes, &room))) return bail(rc);
+            p->bm.d_vals = room;
             if ((rc = plan_alloc(p, tile_bytes, &room))) return bail(rc);
             p->d_data = room;
-            HSPMM_HIP_OR(hspmm::launch_expand_bitmap(int(elem), p->bm.d_header, dv, room, total_tiles, nullptr), bail);
+            const uint32_t header_words = elem == 2u ? 8u : 4u;
+            auto by_windows = [&](auto fn) {
+                hspmm_host::parallel_weighted(p->W, size_t(1) << 13, [=](size_t w) { return rowOffset[w]; }, fn);
+            };
+            Outcome elements, rest;
+            std::atomic<int> next{0};
+            parallel_workers(2u, [&](unsigned) {
+                for (int task = next++; task < 2; task = next++) {
+                    if (task == 0) {
+                        by_windows([&](size_t wb, size_t we) {
+                            const uint32_t t0 = rowOffset[wb];
+                            hspmm_host::pack_tiles(static_cast<const char *>(data) + size_t(t0) * 256u, rowOffset[we] - t0, elem,
+                                                   header.data() + size_t(t0) * header_words, first[wb], vals.data());
+                        });
+                        elements = Outcome::of(copy_up(p, const_cast<void *>(p->bm.d_vals), vals.data(), vals_bytes));
+                    } else {
+                        rest = Outcome::of(upload_units(p, st));
+                        if (!rest.rc) rest = Outcome::of(build_and_upload_partition(p, 0));
+                        by_windows([&](size_t wb, size_t we) {
+                            const uint32_t t0 = rowOffset[wb];
+                            hspmm_host::place_tiles(header.data() + size_t(t0) * header_words, rowOffset[we] - t0, elem, first[wb]);
+                        });
+                        if (!rest.rc) rest = Outcome::of(copy_up(p, p->bm.d_header, header.data(), header_bytes));
+                    }
+                }
+            });
+            for (const Outcome *o : {&elements, &rest})
+                if (o->rc) return bail(fail(o->rc, "%s", o->text.c_str()));
+            p->bm.stored = stored; p->bm.built = true;
+            HSPMM_HIP_OR(hspmm::launch_expand_bitmap(int(elem), p->bm.d_header, p->bm.d_vals, p->d_data, total_tiles, nullptr), bail);
+            timer.mark("bitmap tiles, partition");
         } else if (!bitmap) {
             uint8_t *dd = nullptr;
             if ((rc = upload(p, &dd, static_cast<const uint8_t *>(data), tile_bytes))) return bail(rc);
@@ -659,8 +754,7 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
             p->bm.from_caller = true;
         }
         timer.mark("upload format arrays");
-        if ((rc = upload(p, &p->d_unitOffset, st.unitOffset.data(), st.unitOffset.size()))) return bail(rc);
-        if ((rc = upload(p, &p->d_unitRow, st.unitRow.data(), st.unitRow.size()))) return bail(rc);
+        if (!sparse_tiles && (rc = upload_units(p, st))) return bail(rc);
         // padding ids -> the real id in front of them (the tile column is all zero; no tile starts with padding)
         if (st.G == 1) {
             // single windows: the steps are the caller's tiles in the caller's order
@@ -710,15 +804,11 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
             HSPMM_HIP_OR(hspmm::launch_lane_order32(p->d_data, room, total_tiles, nullptr), bail);
         }
         p->per_column = entries_per_column(total_tiles, cw, elem, tcA2B, data, bitmap, sparse_tiles ? header.data() : nullptr);
-        // single windows walked tile by tile: the caller's tile numbers are the stream's, its cuts can be kept
-        if (cuts && p->cfg.group_cuts && st.G == 1) p->caller_cuts.assign(cuts->offsets, cuts->offsets + size_t(cuts->n_groups) + 1u);
         {
             uint32_t longest = 0;
             for (size_t u = 0; u + 1 < st.unitOffset.size(); ++u) longest = std::max(longest, st.unitOffset[u + 1] - st.unitOffset[u]);
             p->even_windows = uint64_t(longest) * p->n_units <= uint64_t(p->n_steps) * 8u;
         }
-        p->h_unitOffset = st.unitOffset;
-        p->h_unitRow = st.unitRow;
         if (st.G != 1) {
             p->h_winOffset.assign(rowOffset, rowOffset + size_t(p->W) + 1u);
             p->h_winRow.assign(rowIdx, rowIdx + size_t(p->W));

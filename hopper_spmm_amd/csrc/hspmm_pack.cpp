@@ -80,22 +80,33 @@ uint64_t tile_masks(const void *tiles, size_t n, uint32_t elem, uint32_t *header
     return stored;
 }
 
-void pack_tiles(const void *tiles, size_t n, uint32_t elem, uint32_t *header, uint64_t first, void *stored)
+void place_tiles(uint32_t *header, size_t n, uint32_t elem, uint64_t first)
+{
+    uint32_t at = uint32_t(first);
+    for (size_t t = 0; t < n; ++t) {
+        if (elem == 2u) {
+            header[5] = at;
+            at += (header[4] >> 24) + uint32_t(__builtin_popcount(header[3]));     // (in front of the last word, in it)
+            header += 8;
+        } else {
+            header[2] = at;
+            at += header[3];
+            header += 4;
+        }
+    }
+}
+
+void pack_tiles(const void *tiles, size_t n, uint32_t elem, const uint32_t *header, uint64_t first, void *stored)
 {
     if (elem == 2u) {
         const uint16_t *v = static_cast<const uint16_t *>(tiles);
-        uint16_t *base = static_cast<uint16_t *>(stored), *to = base + first;
-        for (size_t t = 0; t < n; ++t, v += 128, header += 8) {
-            header[5] = uint32_t(to - base);
+        uint16_t *to = static_cast<uint16_t *>(stored) + first;
+        for (size_t t = 0; t < n; ++t, v += 128, header += 8)
             for (uint32_t q = 0; q < 4; ++q) to = take(to, v + 32 * q, header[q]);
-        }
     } else {
         const uint32_t *v = static_cast<const uint32_t *>(tiles);
-        uint32_t *base = static_cast<uint32_t *>(stored), *to = base + first;
-        for (size_t t = 0; t < n; ++t, v += 64, header += 4) {
-            header[2] = uint32_t(to - base);
-            to = take(take(to, v, header[0]), v + 32, header[1]);
-        }
+        uint32_t *to = static_cast<uint32_t *>(stored) + first;
+        for (size_t t = 0; t < n; ++t, v += 64, header += 4) to = take(take(to, v, header[0]), v + 32, header[1]);
     }
 }
 

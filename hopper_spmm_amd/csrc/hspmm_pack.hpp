@@ -9,7 +9,9 @@ namespace hspmm_host {
 
 // The masks and counts of n tiles; returns their number of stored elements (those whose bit pattern is not +0).
 uint64_t tile_masks(const void *tiles, size_t n, uint32_t elem, uint32_t *header);
-// The stored elements of n tiles to stored[first ..] and their positions to the header.
-void pack_tiles(const void *tiles, size_t n, uint32_t elem, uint32_t *header, uint64_t first, void *stored);
+// The positions of n tiles' stored elements, which begin at `first`, to the header.
+void place_tiles(uint32_t *header, size_t n, uint32_t elem, uint64_t first);
+// The stored elements of n tiles to stored[first ..].
+void pack_tiles(const void *tiles, size_t n, uint32_t elem, const uint32_t *header, uint64_t first, void *stored);
 
 }  // namespace hspmm_host

@@ -332,7 +332,7 @@ enum class RunMode { kLaunch, kPrepare, kStatic };
 // hspmm_create.hip
 int validate_format(uint32_t rows, uint32_t cols, uint32_t W, uint32_t T, uint32_t cw,
                     const uint32_t *rowOffset, const uint32_t *tcA2B, const void *data, const uint32_t *rowIdx,
-                    bool *canonical = nullptr, uint32_t *header = nullptr, uint32_t *window_stored = nullptr);
+                    bool *canonical = nullptr);
 int choose_ranges(const hspmm_plan *p);
 int build_and_upload_partition(hspmm_plan *p, int level, uint32_t group = 1, bool aligned = false);
 
