@@ -598,6 +598,96 @@ int upload_units(hspmm_plan *p, const StepStream &st)
     return upload(p, &p->d_unitRow, st.unitRow.data(), st.unitRow.size());
 }
 
+// What the kernels walk of a schedule, in host memory.
+struct ScheduleTables {
+    enum { kOffset, kInfo, kItems, kRanges, kSplit, kFix, kCount };
+    std::vector<uint32_t> words;
+    size_t at[kCount] = {};
+    uint32_t n_units = 0, n_ranges = 0, n_split = 0, n_slots = 0;
+    bool wanted() const { return n_units != 0; }
+};
+
+// (from the caller's windows: what they say is checked already, their tiles may not be)
+ScheduleTables schedule_tables(const hspmm_plan *p, const uint32_t *rowOffset, const uint32_t *rowIdx)
+{
+    ScheduleTables out;
+    const uint32_t T = p->T, W = p->W;
+    if (p->cfg.schedule == 0 || p->elem != 2u || (p->cfg.kernel_mode != 0 && p->cfg.kernel_mode != 3) || p->cfg.gather_bitmap == 0 || p->cfg.consumer_warp_num ||
+        p->cfg.producer_warp_group_num || p->cfg.buffer_stage)
+        return out;
+    if (p->cfg.schedule < 0 && p->cols < kScheduledColumns) return out;
+    uint32_t longest = 0, shortest = HSPMM_IDX_MAX;
+    for (uint32_t w = 0; w < W; ++w) {
+        longest = std::max(longest, rowOffset[w + 1] - rowOffset[w]);
+        shortest = std::min(shortest, rowOffset[w + 1] - rowOffset[w]);
+    }
+    if (!shortest || (p->cfg.schedule < 0 && windows_are_even(longest, W, T))) return out;
+    const uint32_t most = (T + kMinTilesPerRange - 1u) / kMinTilesPerRange;
+    const uint32_t n_waves = std::max(1u, std::min(p->cfg.schedule > 1 ? uint32_t(p->cfg.schedule) : uint32_t(p->compute_units) * 8u, most));
+    const hspmm::Schedule s = hspmm::build_schedule(W, rowOffset, n_waves);
+    const uint32_t n = uint32_t(s.items.size()), n_ranges = std::min(n_waves, n);   // (the first waves are the ones that have items)
+    // cut windows: their parts have neighbouring slots
+    std::vector<uint32_t> entry_of(W, HSPMM_IDX_MAX), split;
+    uint32_t n_slots = 0;
+    for (uint32_t i = 0; i < n; ++i) {
+        const hspmm::ScheduleItem &it = s.items[i];
+        if (it.parts == 1u || entry_of[it.window] != HSPMM_IDX_MAX) continue;
+        entry_of[it.window] = uint32_t(split.size() / hspmm::kFixWords);
+        split.insert(split.end(), {i, n_slots, it.parts, 0u});
+        n_slots += it.parts;
+    }
+    const size_t sizes[ScheduleTables::kCount] = {size_t(n) + 1u, size_t(n) * 4u, size_t(n) * 4u, size_t(n_ranges) * hspmm::kRangeWords, split.size(),
+                                                  size_t(n_slots) * 2u};
+    size_t total = 0;
+    for (size_t k = 0; k < ScheduleTables::kCount; ++k) { out.at[k] = total; total += (sizes[k] + 63u) & ~size_t(63); }
+    out.words.assign(total, 0u);
+    auto table = [&](int k) { return out.words.data() + out.at[k]; };
+    uint32_t *offset = table(ScheduleTables::kOffset), *info = table(ScheduleTables::kInfo), *items = table(ScheduleTables::kItems),
+             *ranges = table(ScheduleTables::kRanges), *fix = table(ScheduleTables::kFix);
+    for (uint32_t i = 0; i < n; ++i, info += 4, items += 4) {
+        const hspmm::ScheduleItem &it = s.items[i];
+        const bool cut = it.parts > 1u, last = it.part + 1u == it.parts;
+        const uint32_t slot = cut ? split[size_t(entry_of[it.window]) * hspmm::kFixWords + 1u] + it.part : HSPMM_IDX_MAX;
+        offset[i + 1u] = offset[i] + it.steps;
+        info[0] = (rowIdx[it.window] & ~7u) | (it.window == 0u && it.part == 0u ? 1u : 0u);
+        info[1] = !last ? 0u : it.window + 1u < W ? rowIdx[it.window + 1u] & ~7u : p->rows;
+        info[2] = slot;
+        info[3] = entry_of[it.window];
+        if (cut) { fix[slot] = slot; fix[size_t(n_slots) + slot] = i; }
+        items[0] = it.first; items[1] = it.stride; items[2] = offset[i]; items[3] = it.steps;
+    }
+    for (uint32_t w = 0; w < n_ranges; ++w, ranges += hspmm::kRangeWords) {
+        std::fill(ranges, ranges + hspmm::kRangeWords, HSPMM_IDX_MAX);
+        ranges[0] = offset[s.waves[w]]; ranges[1] = offset[s.waves[w + 1u]]; ranges[2] = s.waves[w]; ranges[7] = 0u;
+    }
+    for (size_t k = 0; k < split.size(); k += hspmm::kFixWords) split[k + 3u] = n_slots + split[k + 1u];
+    std::copy(split.begin(), split.end(), table(ScheduleTables::kSplit));
+    out.n_units = n; out.n_ranges = n_ranges; out.n_split = uint32_t(split.size() / hspmm::kFixWords); out.n_slots = n_slots;
+    return out;
+}
+
+// Device memory of the schedule: ids, headers and tables in one piece; null where there is none for it (the plan is made without).
+uint32_t *schedule_room(hspmm_plan *p, const ScheduleTables &t)
+{
+    void *room = nullptr;
+    if (plan_alloc(p, (size_t(p->T) * 24u + t.words.size()) * 4u, &room)) { (void)hipGetLastError(); return nullptr; }
+    return static_cast<uint32_t *>(room);
+}
+
+// Behind its tables (copied) and the plan's ids and headers.
+int fill_schedule(hspmm_plan *p, const ScheduleTables &t, uint32_t *room)
+{
+    hspmm_plan::Scheduled &sc = p->scheduled;
+    uint32_t *ids = room, *header = room + size_t(p->T) * 16u, *tables = header + size_t(p->T) * 8u;
+    HSPMM_HIP(hspmm::launch_schedule_fill(tables + t.at[ScheduleTables::kItems], t.n_units, p->d_ids, p->bm.d_header, ids, header, nullptr));
+    sc.d_ids = ids; sc.d_header = header;
+    sc.d_unitOffset = tables + t.at[ScheduleTables::kOffset]; sc.d_info = tables + t.at[ScheduleTables::kInfo];
+    sc.d_ranges = tables + t.at[ScheduleTables::kRanges]; sc.d_split = tables + t.at[ScheduleTables::kSplit]; sc.d_fix_slots = tables + t.at[ScheduleTables::kFix];
+    sc.n_units = t.n_units; sc.n_ranges = t.n_ranges; sc.n_split = t.n_split; sc.n_slots = t.n_slots;
+    sc.built = true;
+    return HSPMM_OK;
+}
+
 // hspmm_create; with `bitmap` (data == nullptr) the tiles come as the caller's bitmap arrays,
 // which are uploaded as they are, kept as the gather kernels' bitmap stream and expanded on the device for the
 // kernels that read plain tiles.  Returns kNeedsPlainTiles when the plan would need the tiles on the host
@@ -643,14 +733,15 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
     // (arrays that are not good are told of before a device that is not there)
     Outcome device = Outcome::of(find_device(p));
     StepStream st;
+    ScheduleTables schedule;
     const size_t n_ids = size_t(total_tiles) * cw, tile_bytes = size_t(total_tiles) * 256u;
     const size_t spare = 8u / elem;                                     // a lane may read 8 bytes from the last element on
     try {
         // Side by side: the tiles' checks and masks on all cores, the units, device memory and the arrays whose sizes are known.
         Outcome tiles, arrays;
         std::atomic<int> next{0};
-        parallel_workers(p->W ? 3u : 1u, [&](unsigned) {
-            for (int task = next++; task < 3; task = next++) {
+        parallel_workers(p->W ? 4u : 1u, [&](unsigned) {
+            for (int task = next++; task < 4; task = next++) {
                 if (task == 0) {
                     tiles = Outcome::of(validate_tiles(cols, eff_row_windows, total_tiles, cw, rowOffset, tcA2B, tile_values, &canonical,
                                                        sparse_tiles ? header.data() : nullptr, window_stored.data()));
@@ -660,6 +751,8 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
                                                             size_t(likely_stored * 1.1 * double(tile_bytes)) + (size_t(1) << 20)));
                 } else if (task == 2 && p->W) {
                     st = build_units(p->W, cw, rowOffset, rowIdx, tcA2B, p->cfg.pairing);
+                } else if (task == 3 && !device.rc && p->W) {
+                    schedule = schedule_tables(p, rowOffset, rowIdx);
                 }
             }
         });
@@ -685,6 +778,8 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
         sparse_tiles = sparse_tiles && st.G == 1 && stored + spare < (uint64_t(1) << 31) &&
                        (p->cfg.gather_bitmap > 0 || stored * 3u < uint64_t(total_tiles) * 8u * cw);
         void *room = nullptr;
+        uint32_t *schedule_at = nullptr;
+        auto copy_schedule = [&] { return copy_up(p, schedule_at + size_t(total_tiles) * 24u, schedule.words.data(), schedule.words.size() * 4u); };
         if (sparse_tiles) {
             // Side by side: the stored elements one after the other, and what else the launches need of the host.
             std::vector<uint64_t> first(p->W);
@@ -697,14 +792,15 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
             p->bm.d_vals = room;
             if ((rc = plan_alloc(p, tile_bytes, &room))) return bail(rc);
             p->d_data = room;
+            if (schedule.wanted() && p->canonical && p->caller_cuts.empty()) schedule_at = schedule_room(p, schedule);
             const uint32_t header_words = elem == 2u ? 8u : 4u;
             auto by_windows = [&](auto fn) {
                 hspmm_host::parallel_weighted(p->W, size_t(1) << 13, [=](size_t w) { return rowOffset[w]; }, fn);
             };
-            Outcome elements, rest;
+            Outcome elements, rest, walk;
             std::atomic<int> next{0};
-            parallel_workers(2u, [&](unsigned) {
-                for (int task = next++; task < 2; task = next++) {
+            parallel_workers(schedule_at ? 3u : 2u, [&](unsigned) {
+                for (int task = next++; task < 3; task = next++) {
                     if (task == 0) {
                         by_windows([&](size_t wb, size_t we) {
                             const uint32_t t0 = rowOffset[wb];
@@ -712,6 +808,8 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
                                                    header.data() + size_t(t0) * header_words, first[wb], vals.data());
                         });
                         elements = Outcome::of(copy_up(p, const_cast<void *>(p->bm.d_vals), vals.data(), vals_bytes));
+                    } else if (task == 2) {
+                        if (schedule_at) walk = Outcome::of(copy_schedule());
                     } else {
                         rest = Outcome::of(upload_units(p, st));
                         if (!rest.rc) rest = Outcome::of(build_and_upload_partition(p, 0));
@@ -723,7 +821,7 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
                     }
                 }
             });
-            for (const Outcome *o : {&elements, &rest})
+            for (const Outcome *o : {&elements, &rest, &walk})
                 if (o->rc) return bail(fail(o->rc, "%s", o->text.c_str()));
             p->bm.stored = stored; p->bm.built = true;
             HSPMM_HIP_OR(hspmm::launch_expand_bitmap(int(elem), p->bm.d_header, p->bm.d_vals, p->d_data, total_tiles, nullptr), bail);
@@ -807,7 +905,7 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
         {
             uint32_t longest = 0;
             for (size_t u = 0; u + 1 < st.unitOffset.size(); ++u) longest = std::max(longest, st.unitOffset[u + 1] - st.unitOffset[u]);
-            p->even_windows = uint64_t(longest) * p->n_units <= uint64_t(p->n_steps) * 8u;
+            p->even_windows = windows_are_even(longest, p->n_units, p->n_steps);
         }
         if (st.G != 1) {
             p->h_winOffset.assign(rowOffset, rowOffset + size_t(p->W) + 1u);
@@ -816,6 +914,11 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
         if ((rc = build_and_upload_partition(p, 0))) return bail(rc);
         if ((rc = count_entries(p))) return bail(rc);                   // (behind the last of the small uploads, which would wait for it)
         timer.mark("partition");
+        if (!schedule_at && schedule.wanted() && p->G == 1 && p->bm.built && p->canonical && p->caller_cuts.empty() && (schedule_at = schedule_room(p, schedule)) &&
+            (rc = copy_schedule()))
+            return bail(rc);
+        if (schedule_at && (rc = fill_schedule(p, schedule, schedule_at))) return bail(rc);
+        timer.mark("schedule");
         {
             // all units long, and so long that the balanced partition cuts each of them several ways:
             // eight ranges per unit where it would cut eight ways or more, four from `four_from` ways on

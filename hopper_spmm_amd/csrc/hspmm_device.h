@@ -25,6 +25,8 @@ struct KernelArgs {
     // the step stream the MFMA kernels walk
     const uint32_t *unitOffset;  // n_units + 1: first step of every unit
     const uint32_t *unitRow;     // n_units: first matrix row of the unit | its windows less one (1: a pair)
+                                 // of a schedule four words: first row (| 1: the first window, rows in front of it are to be cleared), end of the
+                                 // rows to be cleared behind it (0: none), its slot (kIdxMax: a whole window), its entry in split
     const uint32_t *ids;         // per step, lane order, padding ids renamed
     const void     *tiles;       // per step, lane order; bitmap stream: the stored elements, tile after tile
     const uint32_t *bm_header;   // bitmap stream (kLayoutDWB): per step 8 words - the tile's four bitmap words, the bit
@@ -32,7 +34,7 @@ struct KernelArgs {
     // partition
     const uint32_t *ranges;      // n_ranges x kRangeWords
     const uint32_t *split;       // n_split x kFixWords {unit, slot_begin, slot_count, 0}
-    const uint32_t *fix_slots;
+    const uint32_t *fix_slots;   // (of a schedule, behind the slots: the units of a window's parts, from the split entry's fourth word on)
     float          *scratch;     // partial sums: [slot][feature block][acc reg][lane] x 4 floats
     uint32_t       *arrive;      // [split unit][feature block] arrival counters (all zero between launches);
                                  // null: the partial sums are added by a second kernel
@@ -66,6 +68,12 @@ constexpr int default_prefetch(int elem_bytes, int G, int V)
 hipError_t launch_spmm_mfma(int dtype, int layout, int G, const KernelArgs &ka, int V, int prefetch, bool narrow,
                             int waves_per_group, hipStream_t s, hipEvent_t mid);
 hipError_t launch_spmm_scalar(int dtype, const KernelArgs &ka, hipStream_t s);
+
+// 16-bit bitmap tiles in the order of a schedule, words at 64 features a block, 32-bit gather offsets; ids and headers of that order by
+// launch_schedule_fill (items: first tile, stride, first step, steps).
+hipError_t launch_spmm_scheduled(int dtype, const KernelArgs &ka, int waves_per_group, hipStream_t s, hipEvent_t mid);
+hipError_t launch_schedule_fill(const uint32_t *items, uint32_t n_items, const uint32_t *ids, const uint32_t *header, uint32_t *to_ids, uint32_t *to_header,
+                                hipStream_t s);
 
 // LDS-panel kernels (spmm_panel_kernel.hpp).
 constexpr uint32_t kPanelRowBytes = 256;       // bytes of a B row one workgroup covers (128 halves / 64 floats)

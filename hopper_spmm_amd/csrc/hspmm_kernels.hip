@@ -209,6 +209,42 @@ hipError_t launch_mfma_bf16_bm(const KernelArgs &ka, int V, int prefetch, bool n
 hipError_t launch_mfma_f32_bm(const KernelArgs &ka, int V, int prefetch, bool narrow, int waves_per_group, hipStream_t s,
                               hipEvent_t mid);
 
+hipError_t launch_mfma_f16_scheduled(const KernelArgs &ka, int waves_per_group, hipStream_t s, hipEvent_t mid);
+hipError_t launch_mfma_bf16_scheduled(const KernelArgs &ka, int waves_per_group, hipStream_t s, hipEvent_t mid);
+hipError_t launch_spmm_scheduled(int dtype, const KernelArgs &ka, int waves_per_group, hipStream_t s, hipEvent_t mid)
+{
+    if (dtype == kDtypeF16) return launch_mfma_f16_scheduled(ka, waves_per_group, s, mid);
+    if (dtype == kDtypeBf16) return launch_mfma_bf16_scheduled(ka, waves_per_group, s, mid);
+    return hipErrorInvalidValue;
+}
+
+// Ids (16 words) and headers (8) of the tiles of a schedule's items, a wave an item.
+__global__ __launch_bounds__(256) void schedule_fill_kernel(const uint32_t *__restrict__ items, uint32_t n_items, const uint32_t *__restrict__ ids,
+                                                            const uint32_t *__restrict__ header, uint32_t *__restrict__ to_ids, uint32_t *__restrict__ to_header)
+{
+    const uint32_t i = blockIdx.x * 4u + (threadIdx.x >> 6), lane = threadIdx.x & 63u;
+    if (i >= n_items) return;
+    const uint32_t first = items[4u * i], stride = items[4u * i + 1u], step = items[4u * i + 2u], n = items[4u * i + 3u];
+    // two tiles at a time: lanes 0 .. 31 their ids, 32 .. 47 their headers
+    for (uint32_t k = 0; k < n; k += 2u) {
+        if (lane < 32u) {
+            const uint32_t at = k + (lane >> 4);
+            if (at < n) to_ids[size_t(step + at) * 16u + (lane & 15u)] = ids[(size_t(first) + size_t(at) * stride) * 16u + (lane & 15u)];
+        } else if (lane < 48u) {
+            const uint32_t at = k + ((lane >> 3) & 1u);
+            if (at < n) to_header[size_t(step + at) * 8u + (lane & 7u)] = header[(size_t(first) + size_t(at) * stride) * 8u + (lane & 7u)];
+        }
+    }
+}
+
+hipError_t launch_schedule_fill(const uint32_t *items, uint32_t n_items, const uint32_t *ids, const uint32_t *header, uint32_t *to_ids, uint32_t *to_header,
+                                hipStream_t s)
+{
+    if (!n_items) return hipSuccess;
+    schedule_fill_kernel<<<dim3((n_items + 3u) / 4u), 256, 0, s>>>(items, n_items, ids, header, to_ids, to_header);
+    return hipGetLastError();
+}
+
 hipError_t launch_spmm_mfma(int dtype, int layout, int G, const KernelArgs &ka, int V, int prefetch, bool narrow,
                             int waves_per_group, hipStream_t s, hipEvent_t mid)
 {

@@ -18,6 +18,7 @@
 #include "../../include/hspmm.h"
 #include "hspmm_device.h"
 #include "partition.hpp"
+#include "schedule.hpp"
 #include "host_parallel.hpp"
 #include "step_stream.hpp"
 
@@ -69,6 +70,7 @@ struct Config {
     int block = -1;                     // block kernels (-1: by expected time, 0 never, 1 wherever they can)
     int wide_cuts = -1;                 // workgroups of a C tile (-1: by expected time)
     int wide_shape = -1;                // their workgroup's shape, an index into the table of hspmm_wide.hip (-1: by expected time)
+    int schedule = -1;                  // gather kernels: waves that sweep the columns together (-1: by matrix, 0 never, 1 wherever they can)
     int xcd_split = -1;                 // gather kernels: two feature blocks dealt out by XCD half (-1: by matrix, 0 never, 1 always)
     // (set through hspmm_set_panel_stream; builds with HSPMM_EXPERIMENTAL only)
     int panel_tall = 0;                 // LDS-panel waves with two units each
@@ -83,6 +85,7 @@ struct Config {
         if (const char *e = std::getenv("HSPMM_PANEL_CHUNKS")) panel_chunks = std::max(1, std::atoi(e));
         if (const char *e = std::getenv("HSPMM_PANEL_MAX_WINDOWS")) panel_max_windows = std::atoi(e) >= 4 ? 4 : 2;
         if (const char *e = std::getenv("HSPMM_XCD_SPLIT")) xcd_split = std::atoi(e) != 0;
+        if (const char *e = std::getenv("HSPMM_SCHEDULE")) schedule = std::atoi(e);
         if (const char *e = std::getenv("HSPMM_ENTRIES")) entries = std::atoi(e) != 0;
         if (const char *e = std::getenv("HSPMM_TILE")) tile = std::atoi(e) != 0;
         if (const char *e = std::getenv("HSPMM_NARROW")) narrow = std::atoi(e) != 0;
@@ -108,6 +111,18 @@ extern std::mutex g_cfg_mutex;          // guards g_cfg (hspmm_capi.hip)
 extern Config g_cfg;
 
 constexpr uint32_t kMinTilesPerRange = 24;
+// Plans that carry a schedule (power-law graphs, 16-bit bitmap tiles): from 2^18 columns on; built beside the packing of the tiles it adds nothing
+// that shows to hspmm_create (10.6 / 10.3 ms at 2^20 vertices, 2.4 / 2.5 at 2^18, 3.7 / 4.0 at 600000) and 24 words a tile to its device memory
+// (431 -> 527 MB at 2^20).  Against the partition it was ahead on all of 62 launches (12 graphs of 2^18 to 2^20 vertices, 4 to 32 edges each,
+// N = 64 to 512) by 2 to 33 %; graphs of 131072 and 150001, with 8 to 18 MB of B for each 64 features, are the entry kernels' (N = 128:
+// 60 / 63 and 43 / 48 us).
+constexpr uint32_t kScheduledColumns = 1u << 18;
+// Bytes of B in a block of 64 features from which a single block, or an odd number of them, goes by the schedule rather than to the entry kernels
+// (N = 64: 2^20 vertices 260 / 207 us, 800000 112 / 107, 600000 73 / 77, 350000 55 / 63, 2^18 42 / 50).  Two, four or eight blocks, each with XCDs of
+// its own, from the first such plan on (N = 128: 2^19 240 / 177, 350000 116 / 108, 2^18 94 / 80; N = 256 at 2^18: 193 / 170).
+constexpr uint64_t kScheduledSlice = uint64_t(96) << 20;
+// No unit has over eight times the average number of steps.
+inline bool windows_are_even(uint32_t longest, uint32_t units, uint32_t steps) { return uint64_t(longest) * units <= uint64_t(steps) * 8u; }
 
 // What a plan answers for a feature dimension, kept for the last few asked for, 32 bits each: the answers are the plan's and N's alone, so
 // threads may overwrite each other's.  (A search costs a launch 0.5 to 1 us of the host's; 16, 32, .. 1024 have a slot each.)
@@ -192,6 +207,13 @@ struct hspmm_plan {
         uint64_t stored = 0;
         bool from_caller = false;     // header and elements are the caller's tcBit / nnzOffset / data, uploaded as they came
     } bm;
+    // The same tiles in the order of a schedule (schedule.hpp), for a B far larger than the L2s: ids and headers are copies, elements are not
+    struct Scheduled {
+        bool built = false;
+        const uint32_t *d_ids = nullptr, *d_header = nullptr, *d_unitOffset = nullptr, *d_info = nullptr, *d_ranges = nullptr,
+                       *d_split = nullptr, *d_fix_slots = nullptr;
+        uint32_t n_units = 0, n_ranges = 0, n_split = 0, n_slots = 0;
+    } scheduled;
     // Stored entries, rows sorted by length, for narrow feature dimensions (spmm_entries.hip): counted by hspmm_create, made from
     // the tiles on the device by the first launch (or hspmm_prepare) that wants it
     struct Entries {
@@ -345,6 +367,21 @@ size_t entries_count_bytes(const hspmm_plan *p);
 int count_entries(hspmm_plan *p);
 int entries_counted(hspmm_plan *p);
 bool entries_serve(const hspmm_plan *p, uint32_t N);
+
+// Whether a launch of the gather kernels walks the plan's schedule, given words of B and C (a launch in blocks of 64 features, which N fills).
+inline bool scheduled_serves(const hspmm_plan *p, uint32_t N)
+{
+    const hspmm_plan::Scheduled &sc = p->scheduled;
+    if (!sc.built || (N % 128u != 64u && N != 128u && N != 256u && N != 512u)) return false;
+    return size_t(sc.n_slots) * (N / 64u) * 2048u <= HSPMM_STATIC_SCRATCH_BYTES;     // (however it is launched)
+}
+
+// Where the entry kernels would serve as well.
+inline bool scheduled_before_entries(const hspmm_plan *p, uint32_t N, uintptr_t align)
+{
+    return p->cfg.entries < 0 && align % 4u == 0u && scheduled_serves(p, N) && (N % 128u == 0u || uint64_t(p->cols) * 128u >= kScheduledSlice);
+}
+
 double entries_expected(const hspmm_plan *p, uint32_t N);       // us, pruned weights of 16 bits, fewer than 256 features
 int run_entries(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode, bool *taken);
 

@@ -440,7 +440,7 @@ static int run_impl(hspmm_plan *p, const void *dB, void *dC, uint32_t N, void *s
     if (block_serves(p, N)) return run_block(p, dB, dC, N, s, mode);
     if (wide_serves(p, N)) return run_wide(p, dB, dC, N, s, mid, mode);
     if (tile_serves(p, N)) return run_tile(p, dB, dC, N, s, mode);
-    if (entries_serve(p, N)) {
+    if (entries_serve(p, N) && !scheduled_before_entries(p, N, reinterpret_cast<uintptr_t>(dB) | reinterpret_cast<uintptr_t>(dC))) {
         bool taken = false;
         const int rc = run_entries(p, dB, dC, N, s, mode, &taken);
         if (rc || taken) return rc;
@@ -511,6 +511,7 @@ struct GatherShape {
     int level = 0;                      // which partition: fewer, longer ranges for more feature blocks
     int wpg = 0;                        // waves per workgroup
     bool combine = false;               // the waves of a workgroup add the sums of one unit among themselves
+    bool scheduled = false;             // the plan's schedule in place of a partition
     bool aligned = false;               // every unit is cut into the ranges of one workgroup, which stores it
     int prefetch = 0;
     int partition_index() const { return aligned ? 4 : combine ? 3 : level; }
@@ -553,6 +554,8 @@ static GatherShape choose_gather_shape(const hspmm_plan *p, const void *dB, cons
                 (p->cfg.buffer_stage == 0 || p->aligned_group == hspmm::kMaxWavesPerGroup) &&
                 p->cfg.producer_warp_group_num == 0;
     if (g.aligned) g.wpg = p->aligned_group;
+    g.scheduled = g.layout == hspmm::kLayoutDWB && c.V == 2 && c.narrow && scheduled_serves(p, N);
+    if (g.scheduled) { g.combine = g.aligned = false; g.level = 0; g.wpg = hspmm::kMaxWavesPerGroup; }
     const int default_depth = hspmm::default_prefetch(int(p->elem), p->G, c.V);
     g.prefetch = p->cfg.buffer_stage > 0 ? p->cfg.buffer_stage : default_depth;
 #ifndef HSPMM_EXPERIMENTAL
@@ -585,9 +588,10 @@ static int run_gather(hspmm_plan *p, const void *dB, void *dC, uint32_t N, uint3
     ka.xcd_split = g.xcd_split;
     // acquire: the partition this shape walks, the partial sums of its cut units, their arrival counters
     hspmm_plan::DevPartition &dp = p->parts[g.partition_index()];
+    const hspmm_plan::Scheduled &sc = p->scheduled;
     {
         std::lock_guard<std::mutex> lk(p->mu);
-        if (!dp.built) {
+        if (!g.scheduled && !dp.built) {
             if (mode == RunMode::kStatic)
                 return fail(HSPMM_ERR_UNSUPPORTED,
                             "hspmm_run_static: the work partition for N = %u is not built yet; call hspmm_prepare(plan, N) "
@@ -595,8 +599,8 @@ static int run_gather(hspmm_plan *p, const void *dB, void *dC, uint32_t N, uint3
             const int rc = build_and_upload_partition(p, g.level, g.combine ? uint32_t(g.wpg) : 1u, g.aligned);
             if (rc) return rc;
         }
-        ka.n_ranges = uint32_t(dp.part.ranges.size());
-        ka.n_split = uint32_t(dp.part.split.size());
+        ka.n_ranges = g.scheduled ? sc.n_ranges : uint32_t(dp.part.ranges.size());
+        ka.n_split = g.scheduled ? sc.n_split : uint32_t(dp.part.split.size());
         // The wave that brings a cut unit's last partial sum adds them itself (in range order, as the second
         // kernel would): worth it where few units are cut and the second launch is most of what they cost
         // (power-law graph, 382 of 110 746 units: 540.6 + 9.4 -> 541.1 us); where every unit is cut the
@@ -605,17 +609,23 @@ static int run_gather(hspmm_plan *p, const void *dB, void *dC, uint32_t N, uint3
                            (p->cfg.fused_fixup > 0 || (p->cfg.fused_fixup < 0 && ka.n_split && uint64_t(ka.n_split) * 32u <= p->n_units));
         if (uint64_t(ka.n_ranges) * ka.n_feat_blocks > 0x7FFFFFFFull)
             return fail(HSPMM_ERR_UNSUPPORTED, "feature dimension %u needs too many work items", N);
-        const size_t need = size_t(dp.part.n_slots) * ka.n_feat_blocks * size_t(c.V) * size_t(p->G) * 64u * 16u;
+        const size_t need = size_t(g.scheduled ? sc.n_slots : dp.part.n_slots) * ka.n_feat_blocks * size_t(c.V) * size_t(p->G) * 64u * 16u;
         int rc = scratch_for(p, s, need, mode, &ka.scratch);
         if (rc) return rc;
         if (fused && ka.n_split && (rc = ensure_arrive(p, s, size_t(ka.n_split) * ka.n_feat_blocks, mode, &ka.arrive))) return rc;
     }
     ka.ranges = dp.d_ranges; ka.split = dp.d_split; ka.fix_slots = dp.d_fix_slots;
+    if (g.scheduled) {
+        ka.unitOffset = sc.d_unitOffset; ka.unitRow = sc.d_info; ka.ids = sc.d_ids; ka.bm_header = sc.d_header;
+        ka.ranges = sc.d_ranges; ka.split = sc.d_split; ka.fix_slots = sc.d_fix_slots;
+        ka.n_units = sc.n_units;
+    }
     if (!launch) return HSPMM_OK;
     // (per step and feature block: G * V instructions of 16 x 16 x 32, or 2 G V of 16 x 16 x 4 for 32-bit elements)
     p->note_launch("spmm_mfma_kernel", 2, p->dtype == HSPMM_TF32 ? 3u : p->dtype == HSPMM_FP16 ? 1u : 2u,
                    uint64_t(p->n_steps) * ka.n_feat_blocks * uint64_t(p->G) * uint64_t(c.V) * (p->dtype == HSPMM_TF32 ? 2u : 1u));
-    HSPMM_HIP(hspmm::launch_spmm_mfma(p->dtype, g.layout, p->G, ka, c.V, g.prefetch, c.narrow, g.wpg, s, mid));
+    if (g.scheduled) HSPMM_HIP(hspmm::launch_spmm_scheduled(p->dtype, ka, g.wpg, s, mid));
+    else HSPMM_HIP(hspmm::launch_spmm_mfma(p->dtype, g.layout, p->G, ka, c.V, g.prefetch, c.narrow, g.wpg, s, mid));
     return HSPMM_OK;
 }
 

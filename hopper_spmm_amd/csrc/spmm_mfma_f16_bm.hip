@@ -12,4 +12,9 @@ hipError_t launch_mfma_f16_bm(const KernelArgs &ka, int V, int prefetch, bool na
     return hipErrorInvalidValue;
 }
 
+hipError_t launch_mfma_f16_scheduled(const KernelArgs &ka, int waves_per_group, hipStream_t s, hipEvent_t mid)
+{
+    return launch_default<Scheduled<Fp16TileDWB<2, false>>>(ka, waves_per_group, s, mid);
+}
+
 }  // namespace hspmm

@@ -475,8 +475,12 @@ struct Fp16TileDWB : Fp16TileDW<V_, 1, BF> {
         if constexpr (V > 3) acc[3] = HalfOps<BF>::mfma(av, b3, acc[3]);
     }
 };
-template <class TT> struct TileTraits { static constexpr bool kBitmap = false; };
-template <int V, bool BF> struct TileTraits<Fp16TileDWB<V, BF>> { static constexpr bool kBitmap = true; };
+template <class TT> struct TileTraits { static constexpr bool kBitmap = false, kScheduled = false; };
+template <int V, bool BF> struct TileTraits<Fp16TileDWB<V, BF>> { static constexpr bool kBitmap = true, kScheduled = false; };
+// The same tiles in the order of a schedule (schedule.hpp): units are windows, or parts of them, with a record of four words each
+// (KernelArgs::unitRow).
+template <class TT> struct Scheduled : TT {};
+template <class TT> struct TileTraits<Scheduled<TT>> { static constexpr bool kBitmap = TileTraits<TT>::kBitmap, kScheduled = true; };
 
 // fp32 storage ("tf32" build of the reference): 8x8 tiles, v_mfma_f32_16x16x4_f32.
 // MFMA rows 0..7 are the window rows, rows 8..15 zero; lane (g, j) supplies k = g
@@ -641,7 +645,7 @@ struct Fp32TileB : Fp32Tile<V_, 1> {
         Base::template mma_one<0, 2>(a1, b1, acc); Base::template mma_one<0, 3>(a1, b1, acc);
     }
 };
-template <int V> struct TileTraits<Fp32TileB<V>> { static constexpr bool kBitmap = true; };
+template <int V> struct TileTraits<Fp32TileB<V>> { static constexpr bool kBitmap = true, kScheduled = false; };
 
 // ---------------------------------------------------------------------------
 // Main kernel: one wave per (step range, feature block).
@@ -654,7 +658,13 @@ struct UnitWalk {
     uint32_t row;          // its first matrix row | paired bit
     uint32_t next_row;     // first row of the next unit (or rows)
     uint32_t seg_start, seg_end;   // part of the span inside this wave's range
+    uint32_t slot, split;          // (of a schedule) where a part's sums go, its entry among the cut units
 };
+// Unit u of a schedule.
+__device__ __forceinline__ void scheduled_unit(UnitWalk &ww, const const_u32_ptr info, uint32_t u)
+{
+    ww.row = info[4u * u]; ww.next_row = info[4u * u + 1u]; ww.slot = info[4u * u + 2u]; ww.split = info[4u * u + 3u];
+}
 
 // Windows of a unit: the low bits of its row word hold the count less one (1: a pair; the
 // LDS-panel kernels also have units of three and four windows).
@@ -738,8 +748,9 @@ __device__ __forceinline__ const KernelArgs &late_arguments()
     asm volatile("" : "+s"(p));
     return *reinterpret_cast<const KernelArgs *>(p);
 }
+// parts (of a schedule): the units that the window is cut into, n_parts of them.
 template <class TT>
-__device__ __forceinline__ void unit_sum_again(const uint32_t unit, const uint32_t fb)
+__device__ __forceinline__ void unit_sum_again(const uint32_t unit, const uint32_t fb, const uint32_t *parts = nullptr, const uint32_t n_parts = 1u)
 {
     if constexpr (FeaturePairs<TT>::value) {
         constexpr int NACC = TT::G * TT::V;
@@ -755,13 +766,15 @@ __device__ __forceinline__ void unit_sum_again(const uint32_t unit, const uint32
         gat.base = reinterpret_cast<const char *>(ka.B);
         gat.row_bytes = uint32_t(row_bytes);
         gat.lane_off = (active ? feat * TT::kElem : 0u) - mark_half_lane<TT>(L, ka.N, feat);
-        const uint32_t row = ka.unitRow[unit], end = ka.unitOffset[unit + 1u];
+        const uint32_t row = TileTraits<TT>::kScheduled ? ka.unitRow[4u * unit] & ~7u : ka.unitRow[unit];
         // (the lane that has the last feature of an odd N alone has it in its upper half)
         const uint32_t first = L.half_shift ? 0xFFFF0000u : 0xFFFFu;
         f32x4 acc[NACC], second[NACC];
 #pragma unroll
         for (int p = 0; p < NACC; ++p) acc[p] = second[p] = f32x4{0.f, 0.f, 0.f, 0.f};
-        for (uint32_t step = ka.unitOffset[unit]; step < end; ++step) {
+        for (uint32_t part = 0; part < n_parts; ++part) {
+        const uint32_t u = TileTraits<TT>::kScheduled && parts ? parts[part] : unit, end = ka.unitOffset[u + 1u];
+        for (uint32_t step = ka.unitOffset[u]; step < end; ++step) {
             typename TT::BVec b0, b1, b2, b3;
             typename TT::AVec a;
             const typename TT::Idx idx = TT::load_idx(L, step);
@@ -770,6 +783,7 @@ __device__ __forceinline__ void unit_sum_again(const uint32_t unit, const uint32
             if constexpr (TT::V < 4 && sizeof(b1) == 16) b2 = b3 = b0;
             TT::mma(L, b0 & first, b1 & first, b2 & first, b3 & first, a, acc);
             TT::mma(L, b0 & ~first, b1 & ~first, b2 & ~first, b3 & ~first, a, second);
+        }
         }
 #pragma unroll
         for (int p = 0; p < NACC; ++p) { acc[p][1] = second[p][1]; acc[p][3] = second[p][3]; }
@@ -859,15 +873,21 @@ void spmm_mfma_kernel(const KernelArgs ka)
     ww.u = rd[2];
     ww.ustart = unitOffset[ww.u];
     ww.uend = unitOffset[ww.u + 1u];
-    ww.row = unitRow[ww.u];
-    ww.next_row = (ww.u + 1u < U) ? (unitRow[ww.u + 1u] & ~7u) : rows;
+    constexpr bool kScheduled = TileTraits<TT>::kScheduled;
+    if constexpr (kScheduled) {
+        scheduled_unit(ww, unitRow, ww.u);
+    } else {
+        ww.row = unitRow[ww.u];
+        ww.next_row = (ww.u + 1u < U) ? (unitRow[ww.u + 1u] & ~7u) : rows;
+    }
     ww.seg_start = t0;
     ww.seg_end = umin32(ww.uend, t1);
-    const uint32_t first_row = unitRow[0] & ~7u;
+    const uint32_t first_row = kScheduled ? 0u : unitRow[0] & ~7u;
     __builtin_amdgcn_sched_barrier(0);
     HSPMM_FOR_STAGES(HSPMM_PRO_TILE)
     // Rows before the first effective window belong to the wave that starts at step 0.
-    if (t0 == 0u) TT::zero_rows(L, c_lane, row_bytes, 0u, first_row, active);
+    if (!kScheduled && t0 == 0u) TT::zero_rows(L, c_lane, row_bytes, 0u, first_row, active);
+    const uint32_t first_unit = ww.u;
 
     uint32_t again = 0;                                 // 1: a sum that is not finite was stored here; 2, 4: the first, the last cut unit
     // MFMAs of `step` from its registers, then the unit bookkeeping.
@@ -877,7 +897,7 @@ void spmm_mfma_kernel(const KernelArgs ka)
         if (step + 1u == ww.seg_end) {
             const uint32_t row0 = ww.row & ~7u;
             const bool paired = (G > 1) && (ww.row & 1u);
-            const bool complete = (ww.seg_start == ww.ustart) && (ww.seg_end == ww.uend);
+            const bool complete = kScheduled ? ww.slot == kIdxMax : (ww.seg_start == ww.ustart) && (ww.seg_end == ww.uend);
             if (complete) {
                 again |= not_finite<TT>(acc);
                 TT::template store_window<0>(L, acc, c_lane, row_bytes, row0, rows, active);
@@ -886,7 +906,7 @@ void spmm_mfma_kernel(const KernelArgs ka)
                 }
             } else {
                 const bool head = ww.seg_start == t0;
-                const uint32_t slot = head ? head_slot : tail_slot;
+                const uint32_t slot = kScheduled ? ww.slot : head ? head_slot : tail_slot;
                 if (slot != kIdxMax && !combine) {
                     f32x4 *slot_sums = reinterpret_cast<f32x4 *>(ka.scratch) + (size_t(slot) * ka.n_feat_blocks + fb) * (NACC * 64u);
                     if (!ka.arrive) {
@@ -904,7 +924,7 @@ void spmm_mfma_kernel(const KernelArgs ka)
 #pragma unroll
                         for (int p = 0; p < NACC; ++p) store_device_scope(out, lane * 16u + uint32_t(p) * 1024u, acc[p]);
                         wait_stores_acknowledged();
-                        const uint32_t entry = head ? head_split : tail_split;
+                        const uint32_t entry = kScheduled ? ww.split : head ? head_split : tail_split;
                         const uint32_t *fx = ka.split + size_t(entry) * kFixWords;
                         uint32_t *ctr = ka.arrive + size_t(entry) * ka.n_feat_blocks + fb;
                         uint32_t old = 0;
@@ -923,7 +943,8 @@ void spmm_mfma_kernel(const KernelArgs ka)
 #pragma unroll
                                 for (int p = 0; p < NACC; ++p) acc[p] += load_device_scope(in, lane * 16u + uint32_t(p) * 1024u);
                             }
-                            again |= not_finite<TT>(acc) | (head ? 2u : 4u);
+                            // (a schedule's parts are among the first, longest units of a wave)
+                            again |= not_finite<TT>(acc) | (kScheduled ? 2u << umin32(ww.u - first_unit, 30u) : head ? 2u : 4u);
                             TT::template store_window<0>(L, acc, c_lane, row_bytes, row0, rows, active);
                             if constexpr (G > 1) {
                                 if (paired) TT::template store_window<G - 1>(L, acc, c_lane, row_bytes, row0 + kRowWindow, rows, active);
@@ -938,6 +959,7 @@ void spmm_mfma_kernel(const KernelArgs ka)
                 // windows that follow (rows up to the next effective window)
                 const uint32_t gap_begin = row0 + (paired ? 2u * kRowWindow : kRowWindow);
                 if (gap_begin < ww.next_row) TT::zero_rows(L, c_lane, row_bytes, gap_begin, ww.next_row, active);
+                if (kScheduled && (ww.row & 1u)) TT::zero_rows(L, c_lane, row_bytes, 0u, row0, active);     // (in front of the first window)
             }
             if (!combine) {                     // (a combining wave ends here and still needs its sums)
 #pragma unroll
@@ -947,8 +969,12 @@ void spmm_mfma_kernel(const KernelArgs ka)
             ++ww.u;
             ww.ustart = ww.uend;
             ww.uend = unitOffset[umin32(ww.u + 1u, U)];
-            ww.row = unitRow[umin32(ww.u, U - 1u)];
-            ww.next_row = (ww.u + 1u < U) ? (unitRow[ww.u + 1u] & ~7u) : rows;
+            if constexpr (kScheduled) {
+                scheduled_unit(ww, unitRow, umin32(ww.u, U - 1u));
+            } else {
+                ww.row = unitRow[umin32(ww.u, U - 1u)];
+                ww.next_row = (ww.u + 1u < U) ? (unitRow[ww.u + 1u] & ~7u) : rows;
+            }
             ww.seg_start = ww.seg_end;
             ww.seg_end = umin32(ww.uend, t1);
         }
@@ -1006,7 +1032,15 @@ void spmm_mfma_kernel(const KernelArgs ka)
         for (uint32_t u = bounds[2]; u < late.n_units; ++u) {
             const uint32_t start = late.unitOffset[u], end = late.unitOffset[u + 1u];
             if (start >= bounds[1]) break;
-            if ((start >= bounds[0] && end <= bounds[1]) || (again & (start <= bounds[0] ? 2u : 4u)))
+            if constexpr (kScheduled) {
+                const uint32_t entry = late.unitRow[4u * u + 3u];
+                if (late.unitRow[4u * u + 2u] == kIdxMax) {
+                    unit_sum_again<TT>(u, fb);
+                } else if (again & (2u << umin32(u - bounds[2], 30u))) {
+                    const uint32_t *fx = late.split + size_t(entry) * kFixWords;
+                    unit_sum_again<TT>(u, fb, late.fix_slots + fx[3], fx[2]);
+                }
+            } else if ((start >= bounds[0] && end <= bounds[1]) || (again & (start <= bounds[0] ? 2u : 4u)))
                 unit_sum_again<TT>(u, fb);
         }
     }
@@ -1063,9 +1097,12 @@ void spmm_fixup_kernel(const KernelArgs ka)
 #pragma unroll
         for (int p = 0; p < NACC; ++p) acc[p] += src[p * 64];
     }
-    const uint32_t row = ka.unitRow[u];
+    const uint32_t row = TileTraits<TT>::kScheduled ? ka.unitRow[4u * u] & ~7u : ka.unitRow[u];
     store_unit<TT>(L, acc, c_lane, row_bytes, row & ~7u, unit_windows<TT>(row), ka.rows, active);
-    if (not_finite<TT>(acc)) unit_sum_again<TT>(u, fb);
+    if (not_finite<TT>(acc)) {
+        if (TileTraits<TT>::kScheduled) unit_sum_again<TT>(u, fb, ka.fix_slots + fx[3], sc);
+        else unit_sum_again<TT>(u, fb);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1107,25 +1144,46 @@ static hipError_t launch_main_p(const KernelArgs &ka, int prefetch, dim3 grid, d
     return hipGetLastError();
 }
 
+// The kernel that adds the sums of cut units, where the main one does not.
 template <class TT>
-static hipError_t launch_tt(const KernelArgs &ka, int prefetch, bool narrow, int waves_per_group, hipStream_t s,
-                            hipEvent_t mid)
+static hipError_t launch_sums(const KernelArgs &ka, int waves_per_group, hipStream_t s, hipEvent_t mid)
 {
-    const uint32_t items = ka.n_ranges * ka.n_feat_blocks;
-    const dim3 block(64u * waves_per_group);
-    // (feature blocks dealt out by XCD: sets of eight workgroups, 8 / feature blocks of them per block)
-    const uint32_t per_set = (8u / (ka.xcd_split ? ka.n_feat_blocks : 1u)) * uint32_t(waves_per_group);
-    const dim3 grid(ka.xcd_split ? 8u * ((ka.n_ranges + per_set - 1u) / per_set)
-                                  : (items + waves_per_group - 1) / waves_per_group);
-    hipError_t e = narrow ? launch_main_p<TT, true>(ka, prefetch, grid, block, s)
-                          : launch_main_p<TT, false>(ka, prefetch, grid, block, s);
-    if (e != hipSuccess || ka.n_split == 0 || ka.arrive) return e;
+    hipError_t e = hipSuccess;
+    if (ka.n_split == 0 || ka.arrive) return e;
     if (mid && (e = hipEventRecord(mid, s)) != hipSuccess) return e;
     const uint32_t fitems = ka.n_split * ka.n_feat_blocks;
     const uint32_t fwaves = uint32_t(std::min(waves_per_group, kMaxWavesPerGroup));
     const dim3 fgrid((fitems + fwaves - 1) / fwaves);
     spmm_fixup_kernel<TT><<<fgrid, dim3(64u * fwaves), 0, s>>>(ka);
     return hipGetLastError();
+}
+
+static dim3 gather_grid(const KernelArgs &ka, int waves_per_group)
+{
+    const uint32_t items = ka.n_ranges * ka.n_feat_blocks;
+    // (feature blocks dealt out by XCD: sets of eight workgroups, 8 / feature blocks of them per block)
+    const uint32_t per_set = (8u / (ka.xcd_split ? ka.n_feat_blocks : 1u)) * uint32_t(waves_per_group);
+    return dim3(ka.xcd_split ? 8u * ((ka.n_ranges + per_set - 1u) / per_set) : (items + waves_per_group - 1) / waves_per_group);
+}
+
+template <class TT>
+static hipError_t launch_tt(const KernelArgs &ka, int prefetch, bool narrow, int waves_per_group, hipStream_t s,
+                            hipEvent_t mid)
+{
+    const dim3 block(64u * waves_per_group), grid = gather_grid(ka, waves_per_group);
+    hipError_t e = narrow ? launch_main_p<TT, true>(ka, prefetch, grid, block, s)
+                          : launch_main_p<TT, false>(ka, prefetch, grid, block, s);
+    return e != hipSuccess ? e : launch_sums<TT>(ka, waves_per_group, s, mid);
+}
+
+// The default depth, 32-bit gather offsets and workgroups of up to kMaxWavesPerGroup waves alone.
+template <class TT>
+static hipError_t launch_default(const KernelArgs &ka, int waves_per_group, hipStream_t s, hipEvent_t mid)
+{
+    if (waves_per_group < 1 || waves_per_group > kMaxWavesPerGroup) return hipErrorInvalidValue;
+    spmm_mfma_kernel<TT, default_prefetch(TT::kElem, TT::G, TT::V), true><<<gather_grid(ka, waves_per_group), dim3(64u * waves_per_group), 0, s>>>(ka);
+    const hipError_t e = hipGetLastError();
+    return e != hipSuccess ? e : launch_sums<TT>(ka, waves_per_group, s, mid);
 }
 
 template <template <int, int> class TTV, int G>

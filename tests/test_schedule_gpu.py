@@ -1,0 +1,128 @@
+"""The gather kernels on windows dealt out by a schedule where they can go wrong: windows cut into many parts and a window alone, rows without
+entries in front, between and behind, both feature splits, the sums of parts in one kernel and in two, infinities and NaNs."""
+import os
+
+import numpy as np
+import pytest
+
+from test_block_gpu import _csr, _device, _host
+from test_spmm_gpu import convert, torch_cuda  # noqa: F401
+from util import decode, encode
+
+pytestmark = pytest.mark.gpu
+
+
+def _plan(hs, A, **env):
+    env = dict(HSPMM_SCHEDULE="16", HSPMM_GATHER_BITMAP="1", HSPMM_XCD_SPLIT="1", **env)
+    os.environ.update(env)
+    hs.set_kernel_mode(3)
+    try:
+        return hs.Plan(convert(hs, A))
+    finally:
+        hs.set_kernel_mode(0)
+        for name in env:
+            os.environ.pop(name)
+
+
+def _mask(rng, rows, cols, heavy, empty):
+    """Rows of 0 to 30 entries, every tenth window's first row `heavy` of the columns; windows whose number `empty` says are without."""
+    counts = rng.integers(0, 31, rows)
+    counts[::80] = int(heavy * cols)
+    mask = np.argsort(rng.random((rows, cols)), 1) < counts[:, None]
+    for w in empty:
+        mask[8 * w:8 * w + 8] = False
+    return mask
+
+
+@pytest.mark.parametrize("dtype", [0, 2])
+@pytest.mark.parametrize("fused", ["0", "1"])
+@pytest.mark.parametrize("rows,cols,heavy,empty", [(8, 9000, 0.9, ()), (8, 1, 1.0, ()), (163, 7000, 0.8, (0, 1, 7, 8, 20)), (3001, 2500, 0.7, (0, 2, 374, 375)),
+                                                   (700, 400, 0.0, (87,))])
+def test_exact_sums(torch_cuda, hs, dtype, fused, rows, cols, heavy, empty):
+    torch = torch_cuda
+    rng = np.random.default_rng(rows)
+    mask = _mask(rng, rows, cols, heavy, empty)
+    values = rng.choice([-2, -1, 1, 2], int(mask.sum()))
+    D = np.zeros((rows, cols), np.float32)              # (whole numbers below 2^24: exact in any order)
+    D[mask] = values
+    plan = _plan(hs, _csr(mask, values, dtype), HSPMM_FUSED_FIXUP=fused)
+    stream = torch.cuda.current_stream().cuda_stream
+    for N in (64, 128, 192, 256):
+        Bm = rng.integers(-1, 2, (cols, N)).astype(np.float32)
+        want = _device(torch, D @ Bm, dtype)
+        dB = _device(torch, Bm, dtype)
+        plan.prepare(N)
+        for launch in (plan.run, plan.run_static, plan.run):
+            dC = torch.full_like(want, 0x7E01)
+            launch(dB.data_ptr(), dC.data_ptr(), N, stream)
+            torch.cuda.synchronize()
+            assert torch.equal(dC, want), "N=%d" % N
+        assert plan.last_kernel() == "spmm_mfma_kernel"
+    plan.close()
+
+
+def test_infinities_and_nans_stay_with_the_rows_that_name_them(torch_cuda, hs):
+    torch = torch_cuda
+    rng = np.random.default_rng(11)
+    rows, cols = 330, 3000
+    mask = _mask(rng, rows, cols, 0.6, (3,))
+    A = _csr(mask, rng.normal(size=int(mask.sum())), 0)
+    D = np.zeros(mask.shape)
+    D[mask] = decode(A["values"], 0)
+    windows = np.kron(np.logical_or.reduceat(mask, np.arange(0, rows, 8)), np.ones((8, 1), bool))[:rows]
+    for fused in ("0", "1"):
+        plan = _plan(hs, A, HSPMM_FUSED_FIXUP=fused)
+        for N in (64, 128):
+            B = decode(encode(rng.normal(size=(cols, N)).astype(np.float32), 0), 0)
+            finite = D @ B
+            B[17, 5], B[2900, 6] = np.inf, np.nan
+            dB = _device(torch, B, 0)
+            dC = torch.empty((rows, N), dtype=dB.dtype, device="cuda")
+            plan.run(dB.data_ptr(), dC.data_ptr(), N, torch.cuda.current_stream().cuda_stream)
+            torch.cuda.synchronize()
+            got = decode(_host(dC, 0), 0)
+            hit, near = np.zeros(got.shape, bool), np.zeros(got.shape, bool)
+            hit[mask[:, 17], 5] = hit[mask[:, 2900], 6] = True
+            near[windows[:, 17], 5] = near[windows[:, 2900], 6] = True
+            assert not np.isfinite(got[hit]).any() and np.isfinite(got[~near]).all()
+            # (sums of up to 1800 products, each within 2^-24 of its size, and one rounding to fp16)
+            assert (abs(got - finite)[~near] <= 1801 * 2.0**-24 * (abs(D) @ abs(np.where(np.isfinite(B), B, 0)))[~near] + 2.0**-11 * abs(finite)[~near] + 1e-7).all()
+        plan.close()
+
+
+def test_graphs_of_many_columns_have_one(torch_cuda, hs):
+    """Words of B and C at 128 features are walked by it, also where nothing may be built; between two words the launch is another kernel's."""
+    torch = torch_cuda
+    rng = np.random.default_rng(5)
+    rows, cols, N = 4096, 1 << 18, 128
+    counts = np.minimum(rng.zipf(1.6, rows), 20000)
+    columns = [np.sort(rng.choice(cols, n, replace=False)) for n in counts]
+    values = rng.choice([-2.0, -1.0, 1.0, 2.0], int(counts.sum()))
+    A = dict(rows=rows, cols=cols, nnzs=int(counts.sum()), dtype=0, row_ptr=np.concatenate([[0], np.cumsum(counts)]).astype(np.uint32),
+             col_idx=np.concatenate(columns).astype(np.uint32), values=encode(values.astype(np.float32), 0))
+    Bm = rng.integers(-1, 2, (cols, N)).astype(np.float32)
+    ends = np.cumsum(counts)
+    want = _device(torch, np.stack([values[e - n:e] @ Bm[c] for n, e, c in zip(counts, ends, columns)]), 0)
+    os.environ["HSPMM_GATHER_BITMAP"] = "1"             # (tiles of 8 MB and more have them by themselves)
+    try:
+        plan = hs.Plan(convert(hs, A))
+        os.environ["HSPMM_SCHEDULE"] = "0"
+        without = hs.Plan(convert(hs, A))
+    finally:
+        os.environ.pop("HSPMM_GATHER_BITMAP")
+        os.environ.pop("HSPMM_SCHEDULE", None)
+    assert plan.info()["device_bytes"] > without.info()["device_bytes"]
+    stream = torch.cuda.current_stream().cuda_stream
+    flat = _device(torch, Bm.reshape(-1), 0)
+    for shift in (0, 1, 0):
+        b = torch.cat([flat[:shift], flat])
+        plan.prepare(N)
+        for launch in (plan.run_static, plan.run, plan.run_static):
+            dC = torch.full_like(want, 0x7E01)
+            launch(b.data_ptr() + 2 * shift, dC.data_ptr(), N, stream)
+            torch.cuda.synchronize()
+            assert torch.equal(dC, want)
+            if not shift:
+                assert plan.last_kernel() == "spmm_mfma_kernel"
+    plan.close()
+    without.close()
