@@ -126,7 +126,7 @@ void choose_classes(const hspmm_plan *p, uint32_t lanes, bool may_cut, hspmm::En
 
 namespace hspmm_host {
 
-constexpr uint32_t kEntryMaxBlockBytes = 512, kEntryMaxRowBytes = 2048;        // 32 lanes of 16 bytes; four blocks
+constexpr uint32_t kEntryMaxBlockBytes = 512, kEntryMaxRowBytes = 4096;        // 32 lanes of 16 bytes; 1024 features of fp32 storage
 
 // Feature blocks of 128 bytes resp. half a row on XCDs of their own (see spmm_mfma_kernel.hpp), here for rows of 256 bytes
 // (fp32 storage: also 512): pays where B is far larger than an L2 and no row of it is hot (uniform 65536^2, 16 per row:
@@ -216,7 +216,10 @@ bool entries_serve(const hspmm_plan *p, uint32_t N)
     if (row > kEntryMaxRowBytes) return false;
     if (c.entries > 0) return true;
     const double per_column = p->per_column, weight = double(row) * (per_column - 0.8);
-    const bool sparse = per_column <= 1.25;
+    // Power-law graphs that are dense in their hot columns count as sparse up to 1.4 (8192 to 16000 vertices, 18 to 32 edges each, 1.26 to 1.35;
+    // entry / gather kernels, us: 16 bits N = 45 8.0 / 24.3, 64 7.0 / 11.2, 133 12.3 / 27.5, 200 11.0 / 14.0, 512 17.8 / 19.4; fp32 N = 64 8.6 / 15.6,
+    // 94 12.9 / 32.2, 512 29.8 / 44.5; even rows of that density are weights, for which the other kernels have their own streams).
+    const bool sparse = per_column <= 1.25 || (!p->even_windows && per_column <= 1.4);
     if (p->elem == 4u) {
         // 33 to 63 features: the LDS-panel kernels multiply bf16 parts, which no launch that has fp32 products here may lose them to; what
         // would be theirs or the full-tile kernels' goes by expected time, fits to 301 and 878 launches (standard deviations 10 and 7 %):
@@ -229,10 +232,17 @@ bool entries_serve(const hspmm_plan *p, uint32_t N)
         // 57.7 / 122; 11008 x 4096 at 20 %, N = 26 / 47: 70 / 94, 107 / 191; 1500 x 9000 at 25 %, N = 30 / 51 / 63: 56 / 41, 81 / 85,
         // 88 / 85)
         if (N < 64u && N % 4u != 0u) return weight <= (N % 2u ? 350.0 : 135.0);
-        return sparse && !p->panel.built && (row <= 256u || all <= (uint64_t(256) << 20));
+        // Rows of B of more than 512 features: 12544 x 20250, 24 per row, N = 640 / 933 66 / 108, 149 / 198; 60000 x 8000, 9 per row, 91 / 173,
+        // 180 / 334; graph of 16000, 32 edges each, 65 / 104, 107 / 175.  Where columns are hot and B is larger than 156 MB the other kernels read
+        // less of it (graph of 81984, 5 edges each, N = 640 / 768 / 1024: 148 / 135, 193 / 162, 274 / 200; of 40000, N = 1024, 156 MB: 140 / 163);
+        // uniform ones were ahead at all sizes up to 460 MB (27793 x 118016, N = 768 103 / 112, 1024 140 / 142; 2048 x 100000, N = 1024 108 / 140).
+        const uint64_t most = p->even_windows ? uint64_t(512) << 20 : row <= 2048u ? uint64_t(256) << 20 : uint64_t(160) << 20;
+        return sparse && !p->panel.built && (row <= 256u || all <= most);
     }
     if (weight <= 42.0 || (sparse && row <= 128u)) return true;
     if (!sparse || panel_serves(p, N)) return false;
+    // (those dense graphs, wide loads in blocks of 128 features: N = 800 31.0 / 27.6 us at 8192 vertices, 46.8 / 35.9 at 12288; N = 640 20.3 / 22.1)
+    if (per_column > 1.25 && N > 640u && N % 8u == 0u && N % 64u != 0u) return false;
     // N a multiple of 64, hot rows and a B that fills half of the 256 MB memory-side cache: there the other kernels, which then load
     // words and read fewer rows of B, are ahead (graph of 920569, N = 128, 236 MB: 363 / 343 us; of 434176, N = 512, 445 MB:
     // 353 / 322; 18 such graphs: 1.02 on average, and 1.13 behind on 16 with other N a multiple of 8).
