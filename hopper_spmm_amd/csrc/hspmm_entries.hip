@@ -65,6 +65,7 @@ int build_entries(hspmm_plan *p, hipStream_t s)
     HSPMM_HIP_OR(launch_entry_fill(int(p->elem), entry_source(p), e.most_chunks, e.d_positions, e.d_row_len, p->rows, at,
                                    e.d_totals + kEntryBins + 1u, desc, pieces, e.d_row_first, ids, base + ids_bytes, s), failed);
     HSPMM_HIP_OR(hipStreamSynchronize(s), failed);
+    e.units = unit;
     e.long_rows = unit >= 64u * uint64_t(slot - e.totals[kEntryBins - 1u]);
     e.d_ids = ids; e.d_vals = base + ids_bytes; e.d_desc = desc; e.d_pieces = pieces;
     e.built = true;
@@ -107,7 +108,10 @@ uint32_t fill_classes(const hspmm_plan *p, uint32_t lanes, int shift, uint32_t c
 }
 
 // Units per subgroup: long chains need few waves and add few sums (all rows long: 4096 x 11008 at 10 %, N = 8: 17.4 -> 13.0 us
-// from 4 to 16), but where rows are short a launch takes as long as its longest chain (graph of 2^18, N = 16: 30 us at 8, 26
+// from 4 to 16), but a matrix of few rows then has no workgroups for all compute units: up to 2.5 for each at 4 units it takes these, up to two (one
+// and two lanes) or three at 8 units these (bf16, 4 / 8 / 16 units, us: 1274 x 7041 at 4 %, N = 1 3.9 / 5.0 / 7.2, N = 8 4.6 / 6.0 / 9.1, N = 64 6.4 / 7.1 / 8.4;
+// 4096^2 at 10 %, N = 8 5.9 / 6.3 / 8.9, N = 16 8.7 / 6.9 / 8.2, N = 32 11.4 / 10.6 / 8.9; fp32, 1551 x 1412 at 19 %, N = 16 4.5 / 5.1 / 6.4).  Not
+// rows of over 1024 entries, whose sums are many at 4 units (1100 x 16000 at 10 %, fp32, N = 4 9.0 / 8.3 / 7.3).  And where rows are short a launch takes as long as its longest chain (graph of 2^18, N = 16: 30 us at 8, 26
 // at 4) unless it has waves for several rounds.
 // A launch of few rounds also cuts rows that a workgroup's subgroups cannot bring down to 8 units each into parts (24894 vertices,
 // fp16, N = 88: 20.9 us uncut, 15.2 / 14.5 / 16.7 at 16 / 8 / 4 units; 12288, fp32, N = 128: 20.2 -> 10.2; rows all long, 4096 x
@@ -117,7 +121,13 @@ void choose_classes(const hspmm_plan *p, uint32_t lanes, bool may_cut, hspmm::En
 {
     const uint32_t round = uint32_t(p->compute_units) * 8u;
     int shift = 2;
-    if (!p->entries.long_rows) shift = fill_classes(p, lanes, 1, 0, ea) < 2u * round ? 0 : 1;
+    if (!p->entries.long_rows) {
+        shift = fill_classes(p, lanes, 1, 0, ea) < 2u * round ? 0 : 1;
+    } else if (p->entries.units <= 256u * uint64_t(p->rows)) {
+        const uint32_t cu = uint32_t(p->compute_units);
+        if (fill_classes(p, lanes, 0, 0, ea) * 2u <= 5u * cu) shift = 0;
+        else if (fill_classes(p, lanes, 1, 0, ea) <= (lanes <= 2u ? 2u : 3u) * cu) shift = 1;
+    }
     ea->n_groups = fill_classes(p, lanes, shift, 0, ea);
     if (may_cut && !p->entries.long_rows && ea->n_groups < 4u * round) ea->n_groups = fill_classes(p, lanes, shift, 8, ea);
 }

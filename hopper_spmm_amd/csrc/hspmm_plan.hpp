@@ -227,6 +227,7 @@ struct hspmm_plan {
         void *d_stream = nullptr;                                // one allocation for the four below
         const uint32_t *d_desc = nullptr, *d_ids = nullptr, *d_pieces = nullptr;
         const void *d_vals = nullptr;
+        uint64_t units = 0;
         bool long_rows = false;                                  // 64 units and more in a row on average
         hspmm::EntryArgs classes[6] = {};                        // by log2 lanes of a row, once a launch has asked for it
     } entries;

@@ -54,3 +54,27 @@ def test_graphs_with_dense_columns(torch_cuda, hs, dtype, N, taken):
         assert torch.equal(dC, want) if dtype != 1 else torch.equal(dC.view(torch.float32), want.view(torch.float32))
     assert (plan.last_kernel() == "spmm_entries_kernel") == taken
     plan.close()
+
+
+# few rows, all long: 4, 8 and 16 units of four entries to a subgroup
+@pytest.mark.parametrize("dtype", [0, 1, 2])
+@pytest.mark.parametrize("rows,cols,keep", [(33, 1100, 0.9), (1274, 2000, 0.15), (3000, 1024, 0.3), (1000, 2100, 0.55)])
+def test_rows_all_long(torch_cuda, hs, dtype, rows, cols, keep):
+    torch = torch_cuda
+    rng = np.random.default_rng(rows)
+    mask = rng.random((rows, cols)) < keep
+    values = rng.choice([-2, -1, 1, 2], int(mask.sum()))
+    D = np.zeros(mask.shape, np.float32)                # (whole numbers below 2^24: exact in any order)
+    D[mask] = values
+    plan = _plan(hs, _csr(mask, values, dtype))
+    for N in (1, 2, 5, 8, 16, 33, 64):
+        Bm = rng.integers(-1, 2, (cols, N)).astype(np.float32)
+        want, dB = _device(torch, D @ Bm, dtype), _device(torch, Bm, dtype)
+        plan.prepare(N)
+        for launch in (plan.run, plan.run_static):
+            dC = torch.full_like(want, 0x7E01)
+            launch(dB.data_ptr(), dC.data_ptr(), N, torch.cuda.current_stream().cuda_stream)
+            torch.cuda.synchronize()
+            assert torch.equal(dC, want) if dtype != 1 else torch.equal(dC.view(torch.float32), want.view(torch.float32)), "N=%d" % N
+        assert plan.last_kernel() == "spmm_entries_kernel"
+    plan.close()
