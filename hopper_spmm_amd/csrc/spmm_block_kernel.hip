@@ -77,7 +77,7 @@ __global__ __launch_bounds__(64 * W, CF <= 2 ? 6 : 2) void spmm_block_kernel(con
             constexpr int S = decltype(slot)::value;
             const int at = int(umin32(i, n - 1u));
             const uint32_t first = __builtin_amdgcn_readlane(mine[0], at), second = __builtin_amdgcn_readlane(mine[1], at);
-odds[S] = 0u;
+            odds[S] = 0u;
 #pragma unroll
             for (int k = 0; k < kPieces; ++k) {
                 // (a block that ends behind the last column: that row of B, which zeros multiply)
