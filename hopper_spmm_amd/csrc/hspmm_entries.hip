@@ -136,7 +136,7 @@ void choose_classes(const hspmm_plan *p, uint32_t lanes, bool may_cut, hspmm::En
 
 namespace hspmm_host {
 
-constexpr uint32_t kEntryMaxBlockBytes = 512, kEntryMaxRowBytes = 4096;        // 32 lanes of 16 bytes; 1024 features of fp32 storage
+constexpr uint32_t kEntryMaxBlockBytes = 512, kEntryMostFeatures = 1024;       // 32 lanes of 16 bytes; rows of 2 KB, fp32 storage of 4 KB
 
 // Feature blocks of 128 bytes resp. half a row on XCDs of their own (see spmm_mfma_kernel.hpp), here for rows of 256 bytes
 // (fp32 storage: also 512): pays where B is far larger than an L2 and no row of it is hot (uniform 65536^2, 16 per row:
@@ -223,7 +223,7 @@ bool entries_serve(const hspmm_plan *p, uint32_t N)
     const Config &c = p->cfg;
     if (!p->entries.counted || p->entries.unavailable.load()) return false;
     const uint64_t row = uint64_t(N) * p->elem, all = uint64_t(p->cols) * row;
-    if (row > kEntryMaxRowBytes) return false;
+    if (N > kEntryMostFeatures) return false;       // (16-bit rows of more than 2 KB have not been measured here)
     if (c.entries > 0) return true;
     const double per_column = p->per_column, weight = double(row) * (per_column - 0.8);
     // Power-law graphs that are dense in their hot columns count as sparse up to 1.4 (8192 to 16000 vertices, 18 to 32 edges each, 1.26 to 1.35;

@@ -1,0 +1,43 @@
+"""Which launches a kernel family takes, and in what shape: the host code's rules at their lines, compiled here without kernels and device.  No
+GPU needed."""
+import subprocess
+
+import pytest
+
+from test_optional_streams import COMMON, ENTRY_DRIVER, build  # noqa: F401
+
+ENTRY_STUBS = ENTRY_DRIVER[:ENTRY_DRIVER.index("int main()")]
+
+
+def _run(build, driver, *families):
+    run = subprocess.run([build(driver, *families)], stdout=subprocess.PIPE, timeout=60)
+    assert run.returncode == 0 and run.stdout == b"ok\n", run.stdout.decode()
+
+
+def _driver(stubs, body):
+    return stubs + """
+#define EXPECT(x) do { if (!(x)) { std::printf("line %d: %s\\n", __LINE__, #x); return 1; } } while (0)
+int main()
+{
+    using namespace hspmm_host;
+#line 1 "body"
+""" + body + """
+    std::printf("ok\\n");
+    return 0;
+}
+"""
+
+
+def test_entry_kernels_take_rows_of_up_to_1024_features(build):  # noqa: F811
+    _run(build, _driver(ENTRY_STUBS, """
+    for (int dtype : {HSPMM_FP16, HSPMM_TF32, HSPMM_BF16})
+        for (int forced : {-1, 1})
+            for (bool even : {false, true}) {
+                hspmm_plan p;
+                p.dtype = dtype; p.elem = dtype == HSPMM_TF32 ? 4 : 2; p.cw = dtype == HSPMM_TF32 ? 8 : 16;
+                p.rows = p.cols = 10000; p.W = 1250; p.T = 10000; p.compute_units = 256; p.per_column = 1.0; p.even_windows = even;
+                p.entries.counted = true; p.cfg.entries = forced;
+                for (uint32_t N : {1u, 512u, 1000u, 1023u, 1024u}) EXPECT(entries_serve(&p, N));
+                for (uint32_t N : {1025u, 1030u, 1088u, 1536u, 2047u, 2048u, 4096u}) EXPECT(!entries_serve(&p, N));
+            }
+"""), "entries")
