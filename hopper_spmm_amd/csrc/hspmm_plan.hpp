@@ -369,11 +369,22 @@ int count_entries(hspmm_plan *p);
 int entries_counted(hspmm_plan *p);
 bool entries_serve(const hspmm_plan *p, uint32_t N);
 
-// Whether a launch of the gather kernels walks the plan's schedule, given words of B and C (a launch in blocks of 64 features, which N fills).
+// Feature blocks of one 128-byte line, with XCDs of their own where there are two, four or eight (see spmm_mfma_kernel): pays when B is far
+// larger than an XCD's 4 MB L2, so that what an L2 can keep of it decides the hit rate of the gathers (power-law graph 2^20, N = 128: 575 -> 535 us;
+// uniform 65536^2: 39.7 -> 35.5 us), and costs a second pass over the tile stream.  Requests below a 128-byte line lose (N = 64 as two blocks of
+// 32: 280 -> 510 us).
+inline bool splits_features(const hspmm_plan *p, uint32_t N)
+{
+    return p->cfg.xcd_split > 0 || (p->cfg.xcd_split < 0 && uint64_t(p->cols) * N * p->elem >= (uint64_t(8) << 20));
+}
+
+// Whether a launch of the gather kernels walks the plan's schedule, given words of B and C (a launch in blocks of 64 features, which N fills, with
+// 32-bit offsets into B).
 inline bool scheduled_serves(const hspmm_plan *p, uint32_t N)
 {
     const hspmm_plan::Scheduled &sc = p->scheduled;
-    if (!sc.built || (N % 128u != 64u && N != 128u && N != 256u && N != 512u)) return false;
+    if (!sc.built || !(N % 128u == 64u || (splits_features(p, N) && (N == 128u || N == 256u || N == 512u)))) return false;
+    if (p->cols >= (1u << 24) || uint64_t(p->cols) * N * p->elem > (uint64_t(1) << 32)) return false;
     return size_t(sc.n_slots) * (N / 64u) * 2048u <= HSPMM_STATIC_SCRATCH_BYTES;     // (however it is launched)
 }
 

@@ -520,12 +520,7 @@ struct GatherShape {
 static GatherShape choose_gather_shape(const hspmm_plan *p, const void *dB, const void *dC, uint32_t N, uint32_t ld)
 {
     GatherShape g;
-    // Feature blocks with XCDs of their own (see spmm_mfma_kernel): pays when B is far larger than an
-    // XCD's 4 MB L2, so that what an L2 can keep of it decides the hit rate of the gathers (power-law
-    // graph 2^20, N = 128: 575 -> 535 us; uniform 65536^2: 39.7 -> 35.5 us), and costs a second pass over
-    // the tile stream.  Requests below a 128-byte line lose (N = 64 as two blocks of 32: 280 -> 510 us).
-    const bool want_split = p->cfg.xcd_split > 0 ||
-                             (p->cfg.xcd_split < 0 && uint64_t(p->cols) * N * p->elem >= (uint64_t(8) << 20));
+    const bool want_split = splits_features(p, N);
     g.c = choose_kernel(p, dB, dC, N, ld, want_split);
     if (g.c.scalar) return g;
     const Choice &c = g.c;

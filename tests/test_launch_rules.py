@@ -41,3 +41,23 @@ def test_entry_kernels_take_rows_of_up_to_1024_features(build):  # noqa: F811
                 for (uint32_t N : {1025u, 1030u, 1088u, 1536u, 2047u, 2048u, 4096u}) EXPECT(!entries_serve(&p, N));
             }
 """), "entries")
+
+
+def test_schedules_serve_where_the_gather_kernels_could_walk_them(build):  # noqa: F811
+    """Blocks of 64 features, 32-bit offsets into B: launches of other shapes are not kept from the entry kernels."""
+    _run(build, _driver(ENTRY_STUBS, """
+    hspmm_plan p;
+    p.dtype = HSPMM_FP16; p.rows = 1 << 20; p.per_column = 1.05;
+    p.scheduled.built = true; p.scheduled.n_slots = 350;
+    for (uint32_t cols : {1u << 18, 1u << 20, 1u << 22, (1u << 23) + 8u, (1u << 24) - 1u, 1u << 24, (1u << 24) + 1000u, 1u << 26})
+        for (uint32_t N : {32u, 64u, 96u, 128u, 192u, 256u, 320u, 384u, 512u, 1024u}) {
+            const bool blocks = N % 128u == 64u || N == 128u || N == 256u || N == 512u;
+            const bool reached = cols < (1u << 24) && uint64_t(cols) * N * 2u <= (uint64_t(1) << 32);
+            p.cols = cols; p.cfg.xcd_split = -1;
+            EXPECT(scheduled_serves(&p, N) == (blocks && reached));
+            EXPECT(!scheduled_before_entries(&p, N, 0u) || scheduled_serves(&p, N));
+            EXPECT(!scheduled_before_entries(&p, N, 2u));
+            p.cfg.xcd_split = 0;                            // (two, four and eight blocks in one wave then)
+            EXPECT(scheduled_serves(&p, N) == (blocks && reached && N % 128u == 64u));
+        }
+"""), "entries")
