@@ -388,10 +388,13 @@ inline bool scheduled_serves(const hspmm_plan *p, uint32_t N)
     return size_t(sc.n_slots) * (N / 64u) * 2048u <= HSPMM_STATIC_SCRATCH_BYTES;     // (however it is launched)
 }
 
-// Where the entry kernels would serve as well.
+// Where the entry kernels would serve as well: graphs whose columns are hot, so that windows share them.  Uneven rows over uniform columns (one
+// entry per tile column; graphs of 2^18 to 2^21 vertices with 2 to 30 edges each have 1.02 to 1.14) gain nothing from the order: N = 128, us, by
+// schedule / entry kernels: 2^19 columns 207 / 191, 300000 59.7 / 55.2, 2^18 58.6 / 53.7; N = 64, 2^20 columns 101 / 94, 240 / 218, 66 / 58.
 inline bool scheduled_before_entries(const hspmm_plan *p, uint32_t N, uintptr_t align)
 {
-    return p->cfg.entries < 0 && align % 4u == 0u && scheduled_serves(p, N) && (N % 128u == 0u || uint64_t(p->cols) * 128u >= kScheduledSlice);
+    return p->cfg.entries < 0 && p->per_column > 1.01 && align % 4u == 0u && scheduled_serves(p, N) &&
+           (N % 128u == 0u || uint64_t(p->cols) * 128u >= kScheduledSlice);
 }
 
 double entries_expected(const hspmm_plan *p, uint32_t N);       // us, pruned weights of 16 bits, fewer than 256 features

@@ -61,3 +61,16 @@ def test_schedules_serve_where_the_gather_kernels_could_walk_them(build):  # noq
             EXPECT(scheduled_serves(&p, N) == (blocks && reached && N % 128u == 64u));
         }
 """), "entries")
+
+
+def test_schedules_come_before_the_entry_kernels_where_columns_are_hot(build):  # noqa: F811
+    """Uneven rows over uniform columns have one stored entry per tile column: no order of the windows brings rows of B back sooner."""
+    _run(build, _driver(ENTRY_STUBS, """
+    hspmm_plan p;
+    p.dtype = HSPMM_FP16; p.rows = p.cols = 1 << 20;
+    p.scheduled.built = true; p.scheduled.n_slots = 350;
+    for (double per_column : {1.0, 1.0003, 1.004, 1.018, 1.03, 1.1}) {
+        p.per_column = per_column;
+        for (uint32_t N : {64u, 128u, 256u, 512u, 576u}) EXPECT(scheduled_serves(&p, N) && scheduled_before_entries(&p, N, 0u) == (per_column > 1.01));
+    }
+"""), "entries")
