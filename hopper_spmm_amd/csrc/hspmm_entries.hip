@@ -337,7 +337,6 @@ int run_entries(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t
     {
         std::lock_guard<std::mutex> lk(p->mu);
         if (!e.built) {
-            if (mode == RunMode::kStatic && scheduled_before_entries(p, N, 0u)) return HSPMM_OK;    // (B or C between two words: hspmm_prepare has looked at those on one)
             if (mode == RunMode::kStatic)
                 return fail(HSPMM_ERR_UNSUPPORTED, "hspmm_run_static: the entry stream of narrow feature dimensions is not built yet; "
                             "call hspmm_prepare(plan, N) or hspmm_run once with this N first");

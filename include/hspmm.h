@@ -87,8 +87,8 @@ int hspmm_create(hspmm_plan **plan, int dtype, uint32_t rows, uint32_t cols,
  * (partial sums of cut windows, their arrival counters; older buffers stay
  * allocated until hspmm_destroy, so launches recorded earlier, e.g. in a HIP
  * graph, stay valid whatever N is run afterwards).  hspmm_run may therefore be
- * called from several threads; after one earlier call with that N on that
- * stream it only launches kernels (no allocation, memset or copy) and can be
+ * called from several threads; after one earlier call with that N, and with B and C
+ * on that alignment, on that stream it only launches kernels (no allocation, memset or copy) and can be
  * captured in a HIP graph.
  * Device side: every stream that launches a plan gets buffers of its own at its
  * first launch, so launches of one plan on different streams may overlap in time
@@ -118,7 +118,8 @@ int hspmm_prepare(hspmm_plan *plan, uint32_t N);
  * instead of the plan's own buffer.  It calls no hipMalloc / hipFree and builds
  * nothing: what this N needs - the work partition, the matrix entry by entry or, for
  * a single feature of a 16-bit type, the plan's buffer of cols + rows words - must
- * exist already (hspmm_prepare, or one hspmm_run with this N), else
+ * exist already (hspmm_prepare, or one hspmm_run with this N and with B and C on the
+ * same alignment, which may decide the kernel), else
  * HSPMM_ERR_UNSUPPORTED; so does a launch of the gather or LDS-panel kernels whose
  * partial sums exceed the array (the message says how much it needs; the entry and
  * full-tile kernels choose shapes whose sums fit).  Results

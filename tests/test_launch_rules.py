@@ -74,3 +74,16 @@ def test_schedules_come_before_the_entry_kernels_where_columns_are_hot(build):  
         for (uint32_t N : {64u, 128u, 256u, 512u, 576u}) EXPECT(scheduled_serves(&p, N) && scheduled_before_entries(&p, N, 0u) == (per_column > 1.01));
     }
 """), "entries")
+
+
+def test_static_launches_do_not_change_kernels_with_what_ran_before(build):  # noqa: F811
+    """B between two words on a plan with a schedule: the entry kernels' launch, so refused while their stream is not built."""
+    _run(build, _driver(ENTRY_STUBS, """
+    hspmm_plan p;
+    p.dtype = HSPMM_FP16; p.rows = p.cols = 1 << 20; p.W = 1 << 17; p.T = 1 << 20; p.compute_units = 256; p.per_column = 1.05;
+    p.scheduled.built = true; p.scheduled.n_slots = 350; p.entries.counted = true;
+    const void *B = reinterpret_cast<const void *>(uintptr_t(4098));
+    EXPECT(entries_serve(&p, 64u) && scheduled_before_entries(&p, 64u, 0u) && !scheduled_before_entries(&p, 64u, 4098u));
+    bool taken = true;
+    EXPECT(run_entries(&p, B, nullptr, 64u, nullptr, RunMode::kStatic, &taken) == HSPMM_ERR_UNSUPPORTED && !taken);
+"""), "entries")
