@@ -123,7 +123,7 @@ void choose_classes(const hspmm_plan *p, uint32_t lanes, bool may_cut, hspmm::En
     int shift = 2;
     if (!p->entries.long_rows) {
         shift = fill_classes(p, lanes, 1, 0, ea) < 2u * round ? 0 : 1;
-    } else if (p->entries.units <= 256u * uint64_t(p->rows)) {
+    } else if (p->entries.units <= 256u * uint64_t(p->rows - p->entries.totals[hspmm::kEntryBins - 1u])) {      // (of the rows that have entries)
         const uint32_t cu = uint32_t(p->compute_units);
         if (fill_classes(p, lanes, 0, 0, ea) * 2u <= 5u * cu) shift = 0;
         else if (fill_classes(p, lanes, 1, 0, ea) <= (lanes <= 2u ? 2u : 3u) * cu) shift = 1;

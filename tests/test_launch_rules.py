@@ -87,3 +87,25 @@ def test_static_launches_do_not_change_kernels_with_what_ran_before(build):  # n
     bool taken = true;
     EXPECT(run_entries(&p, B, nullptr, 64u, nullptr, RunMode::kStatic, &taken) == HSPMM_ERR_UNSUPPORTED && !taken);
 """), "entries")
+
+
+def test_rows_without_entries_do_not_change_the_shape_of_long_ones(build):  # noqa: F811
+    """300 rows of 1500 entries (places of 384 units of four), or of 500 (128), alone and among ten thousand without entries."""
+    _run(build, _driver(ENTRY_STUBS, """
+    uint32_t of[2][2];
+    for (int len : {0, 1})
+        for (int empty : {0, 1}) {
+            hspmm_plan p;
+            p.dtype = HSPMM_TF32; p.elem = 4; p.cw = 8; p.cols = 4096; p.compute_units = 256; p.per_column = 1.0;
+            p.rows = 300u + empty * 10000u; p.W = (p.rows + 7u) / 8u; p.T = 100000;
+            p.entries.counted = true;
+            p.entries.totals[len ? 3 : 9] = 300; p.entries.totals[hspmm::kEntryBins - 1u] = empty * 10000u;
+            left = 100;
+            bool taken = false;
+            EXPECT(!run_entries(&p, reinterpret_cast<const void *>(uintptr_t(4096)), nullptr, 4u, nullptr, RunMode::kLaunch, &taken) && taken && p.entries.long_rows);
+            EXPECT(hspmm::got.cls[0].slot_begin == 0u && hspmm::got.cls[0].slot_end == 300u);
+            of[len][empty] = hspmm::got.cls[0].logs;
+        }
+    EXPECT(of[0][0] == of[0][1]);
+    EXPECT(of[1][0] == of[1][1]);
+"""), "entries")
