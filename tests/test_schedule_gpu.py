@@ -95,8 +95,9 @@ def test_graphs_of_many_columns_have_one(torch_cuda, hs):
     torch = torch_cuda
     rng = np.random.default_rng(5)
     rows, cols, N = 4096, 1 << 18, 128
-    counts = np.minimum(rng.zipf(1.6, rows), 20000)
-    columns = [np.sort(rng.choice(cols, n, replace=False)) for n in counts]
+    # (hot columns: over uniform ones the entry kernels come first)
+    columns = [np.unique((cols * rng.random(n) ** 6).astype(np.uint32)) for n in np.minimum(rng.zipf(1.6, rows), 20000)]
+    counts = np.array([len(c) for c in columns])
     values = rng.choice([-2.0, -1.0, 1.0, 2.0], int(counts.sum()))
     A = dict(rows=rows, cols=cols, nnzs=int(counts.sum()), dtype=0, row_ptr=np.concatenate([[0], np.cumsum(counts)]).astype(np.uint32),
              col_idx=np.concatenate(columns).astype(np.uint32), values=encode(values.astype(np.float32), 0))
@@ -105,7 +106,9 @@ def test_graphs_of_many_columns_have_one(torch_cuda, hs):
     want = _device(torch, np.stack([values[e - n:e] @ Bm[c] for n, e, c in zip(counts, ends, columns)]), 0)
     os.environ["HSPMM_GATHER_BITMAP"] = "1"             # (tiles of 8 MB and more have them by themselves)
     try:
-        plan = hs.Plan(convert(hs, A))
+        tiles = convert(hs, A)
+        assert A["nnzs"] > 1.01 * (tiles["tcA2B"] != 0xFFFFFFFF).sum()
+        plan = hs.Plan(tiles)
         os.environ["HSPMM_SCHEDULE"] = "0"
         without = hs.Plan(convert(hs, A))
     finally:
