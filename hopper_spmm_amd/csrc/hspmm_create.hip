@@ -98,6 +98,7 @@ int plan_reserve(hspmm_plan *p, size_t bytes)
     p->owned.push_back(fresh);
     p->block = static_cast<char *>(fresh);
     p->block_left = bytes;
+    p->fixed_bytes += bytes;
     return HSPMM_OK;
 }
 
@@ -111,8 +112,8 @@ int plan_alloc(hspmm_plan *p, size_t bytes, void **out)
     } else {
         HSPMM_HIP(hipMalloc(out, bytes));
         p->owned.push_back(*out);
+        p->fixed_bytes += bytes;
     }
-    p->fixed_bytes += bytes;
     return HSPMM_OK;
 }
 
@@ -533,7 +534,7 @@ double entries_per_column(uint32_t T, uint32_t cw, uint32_t elem, const uint32_t
 // 32 + 2 e bytes against 256 per tile with e stored elements (16 + 4 e for fp32) - worth it below about a third full, and
 // where the tile stream is large enough to be traffic at all (a matrix whose tiles sit in the L2s only pays the longer
 // dependent chain: 4096 x 4096 at 1 %, 2.7 MB of tiles: 6.8 -> 7.5 us).  From 64 groups of 64 tiles spread over the matrix.
-// share: the part of their elements that the sample stores (0: not looked at).
+// share: the part of their elements that the sample stores (0: not looked at), whatever the answer.
 bool tiles_look_sparse(const Config &cfg, uint32_t T, uint32_t elem, const void *data, double *share)
 {
     *share = 0.0;
@@ -581,11 +582,14 @@ int copy_up(const hspmm_plan *p, void *to, const void *from, size_t bytes)
     return HSPMM_OK;
 }
 
-// One block of device memory for everything whose size is known early, and the arrays that are checked already or lie inside checked bounds.
-int upload_windows(hspmm_plan *p, const uint32_t *rowOffset, const uint32_t *rowIdx, const uint32_t *tcA2B, size_t block)
+// One block of device memory for everything whose size is known early and, where there is as much, for `likely` bytes that a sample speaks of, and
+// the arrays that are checked already or lie inside checked bounds.
+int upload_windows(hspmm_plan *p, const uint32_t *rowOffset, const uint32_t *rowIdx, const uint32_t *tcA2B, size_t block, size_t likely)
 {
     HSPMM_HIP(hipSetDevice(p->device));
-    if (int rc = plan_reserve(p, block)) return rc;
+    int rc = plan_reserve(p, block + likely);
+    if (rc && likely) { (void)hipGetLastError(); rc = plan_reserve(p, block); }
+    if (rc) return rc;
     if (int rc = upload(p, &p->d_rowOffset, rowOffset, size_t(p->W) + 1)) return rc;
     if (int rc = upload(p, &p->d_rowIdx, rowIdx, size_t(p->W))) return rc;
     return upload(p, &p->d_a2b_raw, tcA2B, size_t(p->T) * p->cw);
@@ -747,8 +751,8 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
                                                        sparse_tiles ? header.data() : nullptr, window_stored.data()));
                 } else if (task == 1 && !device.rc && p->W) {
                     arrays = Outcome::of(upload_windows(p, rowOffset, rowIdx, tcA2B,
-                                                        entries_count_bytes(p) + (size_t(p->W) * 4u + 2u) * 4u + n_ids * 8u + tile_bytes + header.size() * 4u +
-                                                            size_t(likely_stored * 1.1 * double(tile_bytes)) + (size_t(1) << 20)));
+                                                        entries_count_bytes(p) + (size_t(p->W) * 4u + 2u) * 4u + n_ids * 8u + tile_bytes + header.size() * 4u + (size_t(1) << 20),
+                                                        sparse_tiles ? size_t(likely_stored * 1.1 * double(tile_bytes)) : 0u));
                 } else if (task == 2 && p->W) {
                     st = build_units(p->W, cw, rowOffset, rowIdx, tcA2B, p->cfg.pairing);
                 } else if (task == 3 && !device.rc && p->W) {
