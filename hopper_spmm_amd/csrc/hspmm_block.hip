@@ -8,17 +8,41 @@ namespace {
 constexpr uint32_t kMostFeatures = 64u, kAlwaysFeatures = 32u;
 
 // us, from 33 features on, an even number: a fit to 140 launches of 160 matrices of 1024 to 16384 rows, 20 to 60 % of blocks kept, three matrices
-// in turn (standard deviation 11 to 14 %).
+// in turn (standard deviation 11 to 14 %), or the longest unit's walk (50 units of 200 steps, one of 401: N = 44 9.7, 62 11.2; one of 1024 30.5).
 double expected(const hspmm_plan *p, uint32_t N)
 {
     const double steps = double(p->n_steps);
-    return 3.5 + (N <= 48u ? 0.13e-3 : 0.15e-3) * steps + 0.008 * steps / double(p->n_units);
+    return 3.5 + std::max((N <= 48u ? 0.13e-3 : 0.15e-3) * steps + 0.008 * steps / double(p->n_units), (N <= 48u ? 0.0165 : 0.025) * double(p->block_units.longest));
 }
 
-// us, fp32 storage up to 32 features: the tiles' way from memory, or the walk of a wave over its share of a unit's blocks.
-double expected_f32(const hspmm_plan *p)
+// us, fp32 storage up to 32 features: the tiles' way from memory, or the walk of a wave over its share of the longest unit's blocks (one unit of 2048
+// steps: N = 16 46.7, 32 58.3).
+double expected_f32(const hspmm_plan *p, uint32_t N)
 {
-    return 3.5 + std::max(256.0 * p->T / 4.0e6, 0.02 * double(p->n_steps) / double(p->n_units));
+    return 3.5 + std::max(256.0 * p->T / 4.0e6, (N <= 16u ? 0.02 : 0.025) * double(p->block_units.longest));
+}
+
+// A workgroup has a unit: a launch takes as long as the longest unit, and every unit costs a workgroup however short it is.  us, by the kernels that
+// take them otherwise / here.  Many short units, N = 16 / 64, 16 bits: 2048 of 6 blocks 8.4 / 5.5, 10.0 / 10.6; 3072 of 6 9.1 / 7.9, 10.2 / 15.1; 4096
+// of 10 10.4 / 11.6, 12.3 / 20.8; 8192 of 6 10.9 / 18.7, 12.9 / 34.6; fp32 2048 of 6 10.4 / 7.9, 29.6 / 15.7, 8192 of 6 18.4 / 23.6: up to eight a
+// compute unit (from 33 features on, 16 bits, four: block_serves).
+// Uneven ones: where the gather kernels give every unit a workgroup's waves, too (aligned_group), units of up to six times the mean were ahead on all
+// launches (64 to 1024 units of 6 to 200 blocks, one of 1.5 to 6 times as many).  Where their waves have even shares they do not wait for the longest
+// unit (1024 units of 55 blocks, one of 1024, N = 16 / 64: 17.4 / 34.3, 21.9 / 55.9; 256 of 20 blocks, eight of 1024, fp32, N = 32: 21.3 / 59.1;
+// lengths drawn between 1 and 400, 64 units, fp32, N = 8: 14.1 / 19.2): twice the mean and 16 blocks, 256 blocks or 160 of fp32 storage.
+// Workgroups go to the eight XCDs in turn: units of which every other one is short leave half of them with little (1600 units of 1 and 44 blocks in
+// turn, N = 23: 11.4 / 12.7, 808 of 1 and 64, N = 52: 10.5 / 12.6).
+// 900 matrices of 16 to 6000 units, even ones and uneven, five N each: of 3300 launches taken 14 slower by more than 3 % (21 % at most), twice as fast
+// on the mean.
+bool units_suit(const hspmm_plan *p, const StepStream &st, uint32_t longest)
+{
+    const uint64_t units = p->n_units, steps = p->n_steps, all = uint64_t(longest) * units, block = 16u / p->cw;
+    if (units > uint64_t(p->compute_units) * 8u) return false;
+    uint64_t of_xcd[8] = {};
+    for (size_t u = 0; u < units; ++u) of_xcd[u % 8u] += st.unitOffset[u + 1] - st.unitOffset[u];
+    if (units > uint32_t(p->compute_units) && *std::max_element(of_xcd, of_xcd + 8) * 32u > steps * 5u) return false;
+    if (p->aligned_group) return all <= 6u * steps;
+    return all <= 2u * steps + 16u * block * units && longest <= (p->elem == 4u ? 160u : 256u) * block;
 }
 
 }  // namespace
@@ -31,8 +55,10 @@ int build_block_units(hspmm_plan *p, const StepStream &st, const uint32_t *rowOf
 {
     using namespace hspmm;
     if (p->cfg.block == 0 || !p->canonical || p->cfg.kernel_mode != 0 || p->G != 2 || !p->caller_cuts.empty() || p->n_units >= (1u << 22)) return HSPMM_OK;
-    if (p->cfg.block < 0 && p->per_column <= 4.0) return HSPMM_OK;
     const size_t n = st.unitRow.size(), cw = p->cw;
+    uint32_t longest = 0;
+    for (size_t u = 0; u < n; ++u) longest = std::max(longest, st.unitOffset[u + 1] - st.unitOffset[u]);
+    if (p->cfg.block < 0 && (p->per_column <= 4.0 || !units_suit(p, st, longest))) return HSPMM_OK;
     std::vector<uint32_t> pairs(n + 1);
     for (size_t u = 0; u < n; ++u) pairs[u + 1] = pairs[u] + (st.unitOffset[u + 1] - st.unitOffset[u] + 1u) / 2u;
     // one upload: where the tiles are, the units, the first columns
@@ -71,6 +97,7 @@ int build_block_units(hspmm_plan *p, const StepStream &st, const uint32_t *rowOf
     b.d_units = reinterpret_cast<const BlockUnit *>(device + 64u);
     b.d_columns = reinterpret_cast<const uint32_t *>(device + columns_at);
     b.n_units = uint32_t(n);
+    b.longest = longest;
     b.built = true;
     return HSPMM_OK;
 }
@@ -90,11 +117,12 @@ bool block_serves(const hspmm_plan *p, uint32_t N)
         return false;
     if (p->elem == 4u) {
         if (c.block > 0 || N < 16u || N % 4u || !panel_serves(p, N)) return true;
-        return N <= kAlwaysFeatures && p->block_units.taken.get(N, [&]() -> uint32_t { return expected_f32(p) < 0.95 * (6.2 + 0.9 * panel_expected(p, N)); });
+        return N <= kAlwaysFeatures && p->block_units.taken.get(N, [&]() -> uint32_t { return expected_f32(p, N) < 0.95 * (6.2 + 0.9 * panel_expected(p, N)); });
     }
     if (N <= kAlwaysFeatures) return true;
     if (N % 2u) return false;
     if (c.block > 0) return true;
+    if (p->n_units > uint32_t(p->compute_units) * 4u) return false;
     return p->block_units.taken.get(N, [&]() -> uint32_t { return expected(p, N) < blocks_expected(p, N); });
 }
 

@@ -264,7 +264,7 @@ struct hspmm_plan {
         const hspmm::BlockUnit *d_units = nullptr;
         const uint32_t *d_columns = nullptr;
         const hspmm::TileSource *d_source = nullptr;
-        uint32_t n_units = 0;
+        uint32_t n_units = 0, longest = 0;                       // (steps of the longest unit)
         mutable hspmm_host::KeptAnswers taken;
     } block_units;
     double per_column = 8.0;            // stored entries per tile column, from a sample of the tiles

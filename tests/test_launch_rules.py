@@ -109,3 +109,82 @@ def test_rows_without_entries_do_not_change_the_shape_of_long_ones(build):  # no
     EXPECT(of[0][0] == of[0][1]);
     EXPECT(of[1][0] == of[1][1]);
 """), "entries")
+
+
+# (device memory as large as it is asked for)
+BLOCK_STUBS = COMMON.replace("hipMalloc(void **p, size_t) {", "hipMalloc(void **p, size_t n) {").replace("std::malloc(64)", "std::malloc(n)") + """
+namespace hspmm { hipError_t launch_spmm_block(int, const BlockArgs &, uint32_t, hipStream_t) { return hipErrorInvalidValue; } }
+namespace hspmm_host {
+static double panel = 0.0;                          // us the LDS-panel kernels would take (0: not theirs)
+bool panel_serves(const hspmm_plan *, uint32_t) { return panel > 0.0; }
+double panel_expected(const hspmm_plan *, uint32_t) { return panel; }
+double blocks_expected(const hspmm_plan *, uint32_t) { return 1e9; }
+// A plan of rows of blocks with so many blocks each, every block behind the one in front of it; aligned: the gather kernels cut every unit.
+static bool built(hspmm_plan *p, int dtype, const std::vector<uint32_t> &blocks, bool aligned)
+{
+    StepStream st;
+    const uint32_t each = dtype == HSPMM_TF32 ? 2u : 1u;
+    p->dtype = dtype; p->elem = 2u * each; p->cw = 16u / each; p->G = 2; p->compute_units = 256; p->aligned_group = aligned ? 4 : 0;
+    p->rows = uint32_t(blocks.size()) * 16u;
+    std::vector<uint32_t> rowOffset(1, 0u), ids;
+    st.unitOffset.push_back(0);
+    for (size_t u = 0; u < blocks.size(); ++u) {
+        st.unitWindow.push_back(uint32_t(2 * u)); st.unitRow.push_back(uint32_t(u) * 16u | 1u);
+        st.unitOffset.push_back(st.unitOffset.back() + blocks[u] * each);
+        for (int w = 0; w < 2; ++w) {
+            rowOffset.push_back(rowOffset.back() + blocks[u] * each);
+            for (uint32_t c = 0; c < blocks[u] * 16u; ++c) ids.push_back(c);
+        }
+        p->cols = std::max(p->cols, blocks[u] * 16u);
+    }
+    p->W = uint32_t(2 * blocks.size()); p->T = rowOffset.back();
+    p->n_units = uint32_t(blocks.size()); p->n_steps = st.unitOffset.back();
+    left = 100;
+    return build_block_units(p, st, rowOffset.data(), ids.data()) == HSPMM_OK && p->block_units.built;
+}
+static std::vector<uint32_t> one_long(size_t units, uint32_t mean, uint32_t longest) { std::vector<uint32_t> b(units, mean); b[units / 2] = longest; return b; }
+}
+"""
+
+
+def test_block_kernels_take_even_rows_of_blocks(build):  # noqa: F811
+    """A workgroup has a row of blocks: not where one is much longer than the others, nor where there are many thousands of short ones."""
+    _run(build, _driver(BLOCK_STUBS, """
+    for (int dtype : {HSPMM_FP16, HSPMM_BF16, HSPMM_TF32}) {
+        const uint32_t most = dtype == HSPMM_TF32 ? 160u : 256u;
+        struct { std::vector<uint32_t> blocks; bool aligned, taken; } at[] = {
+            {one_long(256, 448, 480), true, true}, {one_long(64, 13, 30), false, true}, {one_long(1024, 40, 64), false, true},
+            {one_long(64, 200, 1024), true, true}, {one_long(256, 40, 260), true, false}, {one_long(1024, 55, 1024), false, false},
+            {one_long(256, 10, 36), false, true}, {one_long(256, 10, 38), false, false}, {one_long(64, most, most), false, true},
+            {one_long(64, most, most + 1u), false, false}, {one_long(1, 4096, 4096), true, true}, {one_long(2048, 5, 12), false, true},
+            {one_long(2049, 5, 12), false, false}, {one_long(8192, 10, 20), false, false},
+        };
+        for (auto &a : at) {
+            hspmm_plan p;
+            const bool b = built(&p, dtype, a.blocks, a.aligned);
+            if (b != a.taken) { std::printf("dtype %d, %zu units, first of %u, longest of %u: %d\\n", dtype, a.blocks.size(), a.blocks[0], a.blocks[a.blocks.size() / 2], int(b)); return 1; }
+            EXPECT(block_serves(&p, 16u) == a.taken && block_serves(&p, 31u) == a.taken);
+            hspmm_plan forced;
+            forced.cfg.block = 1;
+            EXPECT(built(&forced, dtype, a.blocks, a.aligned));         // (as the tests of the kernels ask for)
+        }
+        // every other, or every eighth, row of blocks is short or long: the XCDs, which take them in turn, have uneven shares
+        for (uint32_t units : {256u, 264u, 1600u})
+            for (uint32_t nth : {2u, 8u, 7u}) {
+                std::vector<uint32_t> blocks(units, 10);
+                for (uint32_t u = 0; u < units; u += nth) blocks[u] = 20;
+                hspmm_plan p;
+                EXPECT(built(&p, dtype, blocks, true) == (units <= 256u || nth == 7u));
+            }
+        for (uint32_t units : {512u, 1024u, 1025u, 2048u}) {
+            hspmm_plan p;
+            EXPECT(built(&p, dtype, one_long(units, 5, 5), false) && block_serves(&p, 32u) && block_serves(&p, 64u) == (dtype == HSPMM_TF32 || units <= 1024u));
+        }
+    }
+    // fp32 where the LDS-panel kernels would serve: by the longest row of blocks
+    panel = 13.5;
+    for (uint32_t longest : {80u, 320u, 480u}) {
+        hspmm_plan p;
+        EXPECT(built(&p, HSPMM_TF32, one_long(64, 80, longest), true) && block_serves(&p, 16u) == (longest < 480u) && block_serves(&p, 24u) == (longest < 320u) && !block_serves(&p, 48u));
+    }
+"""), "block")
