@@ -735,12 +735,13 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
 
     auto bail = [&](int code) { hspmm_destroy(p); return code; };
     // (arrays that are not good are told of before a device that is not there)
-    Outcome device = Outcome::of(find_device(p));
+    Outcome device;
     StepStream st;
     ScheduleTables schedule;
     const size_t n_ids = size_t(total_tiles) * cw, tile_bytes = size_t(total_tiles) * 256u;
     const size_t spare = 8u / elem;                                     // a lane may read 8 bytes from the last element on
     try {
+        device = Outcome::of(find_device(p));
         // Side by side: the tiles' checks and masks on all cores, the units, device memory and the arrays whose sizes are known.
         Outcome tiles, arrays;
         std::atomic<int> next{0};
