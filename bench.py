@@ -293,6 +293,9 @@ def main():
     bytes_alg = G.algorithmic_bytes(b, N)
     bytes_gather = G.gather_bytes(b, N)
     info = plan.info()
+    walk = plan.last_walk()             # (kernels other than the gather kernels': the plan's partition)
+    if not walk["ranges"]:
+        walk = {"ranges": info["n_ranges"], "split_windows": info["n_split_windows"]}
     traffic = None
     tfile = os.path.join(ROOT, "profiles", "traffic.json")
     if os.path.exists(tfile):
@@ -317,8 +320,8 @@ def main():
         "data_generator": "Philox 4x64-10 raw words, own transforms (numpy %s)" % np.__version__,
         "config": {"workload": "%s, N=%d" % (cfg["name"], N),
                    "rows": A["rows"], "cols": A["cols"], "nnz": nnz, "tiles": int(b["total_tiles"]),
-                   "eff_row_windows": int(b["eff_row_windows"]), "ranges": info["n_ranges"],
-                   "split_windows": info["n_split_windows"]},
+                   "eff_row_windows": int(b["eff_row_windows"]), "ranges": walk["ranges"],
+                   "split_windows": walk["split_windows"]},
         "effective_gbps": bytes_alg / (ms_per_step * 1e-3) / 1e9,
         # achieved: algorithmic bytes of one launch / (main kernel + partial-sum kernel), device events
         "roofline": {"bound": BOUND.get((args.config, N), "hbm"), "achieved": bytes_alg / (kernels_ms * 1e-3) / 1e9, "peak": HBM_PEAK_GBPS,

@@ -105,6 +105,7 @@ def load_library():
     L.hspmm_prepare.argtypes = [vp, u32]
     L.hspmm_last_kernel.argtypes = [vp]
     L.hspmm_last_kernel.restype = C.c_char_p
+    L.hspmm_last_walk.argtypes = [vp, C.POINTER(u32), C.POINTER(u32), C.POINTER(u32)]
     L.hspmm_bench.argtypes = [vp, vp, vp, u32, i, i, vp, C.POINTER(C.c_float)]
     L.hspmm_profile.argtypes = [vp, vp, vp, u32, i, vp, C.POINTER(C.c_float), C.POINTER(C.c_float)]
     L.hspmm_measure_gather.argtypes = [vp, vp, u32, i, vp, C.POINTER(C.c_float), C.POINTER(C.c_uint64)]
@@ -501,6 +502,12 @@ class Plan:
     def last_kernel(self):
         """hspmm_last_kernel: the name of the last launch's main kernel ("" before the first)."""
         return load_library().hspmm_last_kernel(self._h).decode()
+
+    def last_walk(self):
+        """hspmm_last_walk: what the waves of the last launch walked, where it was one of the MFMA gather kernels."""
+        scheduled, ranges, split = C.c_uint32(), C.c_uint32(), C.c_uint32()
+        _check(load_library().hspmm_last_walk(self._h, C.byref(scheduled), C.byref(ranges), C.byref(split)))
+        return dict(scheduled=bool(scheduled.value), ranges=ranges.value, split_windows=split.value)
 
     def prepare(self, N):
         """hspmm_prepare: builds what the first run with feature dimension N would build; launches nothing."""

@@ -254,6 +254,15 @@ void hspmm_destroy(hspmm_plan *p)
 
 const char *hspmm_last_kernel(const hspmm_plan *p) { return p ? p->last_kernel.load(std::memory_order_relaxed) : ""; }
 
+int hspmm_last_walk(const hspmm_plan *p, uint32_t *scheduled, uint32_t *n_ranges, uint32_t *n_split_windows)
+{
+    if (!p) return fail(HSPMM_ERR_INVALID, "null plan");
+    if (scheduled) *scheduled = p->last_scheduled.load(std::memory_order_relaxed);
+    if (n_ranges) *n_ranges = p->last_ranges.load(std::memory_order_relaxed);
+    if (n_split_windows) *n_split_windows = p->last_split.load(std::memory_order_relaxed);
+    return HSPMM_OK;
+}
+
 int hspmm_get_plan_info(const hspmm_plan *p, hspmm_plan_info *info)
 {
     if (!p || !info) return fail(HSPMM_ERR_INVALID, "null argument");

@@ -305,8 +305,13 @@ struct hspmm_plan {
     std::atomic<uint32_t> last_mfma_kind{0};
     std::atomic<uint64_t> last_mfma_count{0};
     std::atomic<const char *> last_kernel{""};  // its name (hspmm_last_kernel)
-    void note_launch(const char *kernel, uint32_t family, uint32_t kind, uint64_t count)
+    // what the waves of the gather kernels walked in it (hspmm_last_walk)
+    std::atomic<uint32_t> last_scheduled{0}, last_ranges{0}, last_split{0};
+    void note_launch(const char *kernel, uint32_t family, uint32_t kind, uint64_t count, uint32_t scheduled = 0, uint32_t ranges = 0, uint32_t split = 0)
     {
+        last_scheduled.store(scheduled, std::memory_order_relaxed);
+        last_ranges.store(ranges, std::memory_order_relaxed);
+        last_split.store(split, std::memory_order_relaxed);
         last_kernel.store(kernel, std::memory_order_relaxed);
         last_family.store(family, std::memory_order_relaxed);
         last_mfma_kind.store(kind, std::memory_order_relaxed);

@@ -618,7 +618,8 @@ static int run_gather(hspmm_plan *p, const void *dB, void *dC, uint32_t N, uint3
     if (!launch) return HSPMM_OK;
     // (per step and feature block: G * V instructions of 16 x 16 x 32, or 2 G V of 16 x 16 x 4 for 32-bit elements)
     p->note_launch("spmm_mfma_kernel", 2, p->dtype == HSPMM_TF32 ? 3u : p->dtype == HSPMM_FP16 ? 1u : 2u,
-                   uint64_t(p->n_steps) * ka.n_feat_blocks * uint64_t(p->G) * uint64_t(c.V) * (p->dtype == HSPMM_TF32 ? 2u : 1u));
+                   uint64_t(p->n_steps) * ka.n_feat_blocks * uint64_t(p->G) * uint64_t(c.V) * (p->dtype == HSPMM_TF32 ? 2u : 1u),
+                   g.scheduled, ka.n_ranges, ka.n_split);
     if (g.scheduled) HSPMM_HIP(hspmm::launch_spmm_scheduled(p->dtype, ka, g.wpg, s, mid));
     else HSPMM_HIP(hspmm::launch_spmm_mfma(p->dtype, g.layout, p->G, ka, c.V, g.prefetch, c.narrow, g.wpg, s, mid));
     return HSPMM_OK;

@@ -261,9 +261,9 @@ int hspmm_panel_units_preview(int dtype, uint32_t rows, uint32_t cols, uint32_t 
 typedef struct {
     uint32_t rows, cols, eff_row_windows, total_tiles;
     int32_t  dtype;
-    uint32_t n_ranges;          /* tile ranges (one wave each per feature block) */
-    uint32_t n_split_windows;   /* windows whose tiles span more than one range */
-    uint32_t n_partial_slots;   /* fp32 partial accumulators the split windows use */
+    uint32_t n_ranges;          /* tile ranges of the plan's balanced partition (one wave each per feature block); a launch may walk another, or a schedule: hspmm_last_walk */
+    uint32_t n_split_windows;   /* windows whose tiles span more than one of these ranges */
+    uint32_t n_partial_slots;   /* fp32 partial accumulators those windows use */
     uint32_t compute_units;
     uint32_t n_units;           /* units of the step stream: single windows and pairs */
     uint32_t n_paired_units;    /* units made of two adjacent windows with one column list */
@@ -299,6 +299,12 @@ int hspmm_get_plan_info(const hspmm_plan *plan, hspmm_plan_info *info);
  * spmm_mfma_kernel, spmm_panel_kernel, spmm_tile_kernel, spmm_narrow_kernel, spmm_wide_kernel, spmm_block_kernel, spmm_scalar_kernel, or
  * fill_zero_kernel for a matrix without entries; "" before the first (hspmm_plan_info.last_kernel_family names two of them with one number). */
 const char *hspmm_last_kernel(const hspmm_plan *plan);
+
+/* No reference counterpart: what the waves of the last hspmm_run walked, where it was one of the MFMA gather kernels
+ * (spmm_mfma_kernel; all 0 after any other).  *scheduled: 1 a schedule - windows dealt out by length, which plans of graphs of
+ * many columns carry -, 0 the steps in the order of the rows; *n_ranges: waves of a feature block; *n_split_windows: windows cut
+ * between them.  Any output may be NULL. */
+int hspmm_last_walk(const hspmm_plan *plan, uint32_t *scheduled, uint32_t *n_ranges, uint32_t *n_split_windows);
 
 /* No reference counterpart: copies the partition for inspection (tests).
  * ranges: n_ranges x 5 words {tile_begin, tile_end, first_window, head_slot,

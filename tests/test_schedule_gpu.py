@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 
 def _plan(hs, A, **env):
-    env = dict(HSPMM_SCHEDULE="16", HSPMM_GATHER_BITMAP="1", HSPMM_XCD_SPLIT="1", **env)
+    env = {**dict(HSPMM_SCHEDULE="16", HSPMM_GATHER_BITMAP="1", HSPMM_XCD_SPLIT="1"), **env}
     os.environ.update(env)
     hs.set_kernel_mode(3)
     try:
@@ -45,9 +45,11 @@ def test_exact_sums(torch_cuda, hs, dtype, fused, rows, cols, heavy, empty):
     values = rng.choice([-2, -1, 1, 2], int(mask.sum()))
     D = np.zeros((rows, cols), np.float32)              # (whole numbers below 2^24: exact in any order)
     D[mask] = values
-    plan = _plan(hs, _csr(mask, values, dtype), HSPMM_FUSED_FIXUP=fused)
+    A = _csr(mask, values, dtype)
+    tiles = convert(hs, A)
+    plan = _plan(hs, A, HSPMM_FUSED_FIXUP=fused)
     stream = torch.cuda.current_stream().cuda_stream
-    for N in (64, 128, 192, 256):
+    for N in (64, 128, 192, 256, 320, 512):
         Bm = rng.integers(-1, 2, (cols, N)).astype(np.float32)
         want = _device(torch, D @ Bm, dtype)
         dB = _device(torch, Bm, dtype)
@@ -57,11 +59,64 @@ def test_exact_sums(torch_cuda, hs, dtype, fused, rows, cols, heavy, empty):
             launch(dB.data_ptr(), dC.data_ptr(), N, stream)
             torch.cuda.synchronize()
             assert torch.equal(dC, want), "N=%d" % N
-        assert plan.last_kernel() == "spmm_mfma_kernel"
+            assert plan.last_kernel() == "spmm_mfma_kernel" and plan.last_walk()["scheduled"]
+        # (16 waves of 24 tiles and more; cut are the windows that are longer than a wave's share)
+        waves = min(16, -(-tiles["total_tiles"] // 24))
+        cut = int((np.diff(tiles["rowOffset"].astype(np.int64)) > -(-tiles["total_tiles"] // waves)).sum())
+        assert plan.last_walk()["split_windows"] == cut and plan.last_walk()["ranges"] <= waves
     plan.close()
 
 
-def test_infinities_and_nans_stay_with_the_rows_that_name_them(torch_cuda, hs):
+@pytest.mark.parametrize("fused", ["0", "1"])
+def test_features_behind_the_last_block_take_a_launch_of_their_own(torch_cuda, hs, fused):
+    """128 features of rows of 130: the sums are those of rows of 128, bit for bit, and not those in the order of the rows."""
+    torch = torch_cuda
+    rng = np.random.default_rng(9)
+    rows, cols = 1003, 2500
+    mask = _mask(rng, rows, cols, 0.7, (0, 2, 60))
+    A = _csr(mask, rng.normal(size=int(mask.sum())), 0)
+    stream = torch.cuda.current_stream().cuda_stream
+    wide = _device(torch, rng.normal(size=(cols, 130)), 0)
+    got = {}
+    for schedule in ("16", "0"):
+        plan = _plan(hs, A, HSPMM_FUSED_FIXUP=fused, HSPMM_SCHEDULE=schedule)
+        for N in (130, 128):
+            B = wide[:, :N].contiguous()
+            C = torch.full((rows, N), 0x7E01, dtype=torch.int16, device="cuda")
+            plan.run(B.data_ptr(), C.data_ptr(), N, stream)
+            torch.cuda.synchronize()
+            got[schedule, N] = C[:, :128]
+        assert plan.last_walk()["scheduled"] == (schedule == "16")
+        plan.close()
+    assert torch.equal(got["16", 130], got["16", 128]) and torch.equal(got["0", 130], got["0", 128])
+    assert not torch.equal(got["16", 130], got["0", 130])
+
+
+@pytest.mark.parametrize("fused", ["0", "1"])
+def test_two_streams_on_one_plan(torch_cuda, hs, fused):
+    torch = torch_cuda
+    rng = np.random.default_rng(10)
+    rows, cols, N = 163, 7000, 128
+    mask = _mask(rng, rows, cols, 0.8, (0, 7))
+    values = rng.choice([-2, -1, 1, 2], int(mask.sum()))
+    D = np.zeros((rows, cols), np.float32)
+    D[mask] = values
+    plan = _plan(hs, _csr(mask, values, 0), HSPMM_FUSED_FIXUP=fused)
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    Bs = [rng.integers(-1, 2, (cols, N)).astype(np.float32) for _ in streams]
+    want, dB = [_device(torch, D @ B, 0) for B in Bs], [_device(torch, B, 0) for B in Bs]
+    dC = [[torch.full_like(w, 0x7E01) for _ in range(20)] for w in want]
+    torch.cuda.synchronize()
+    for i in range(20):
+        for s, b, c in zip(streams, dB, dC):
+            plan.run(b.data_ptr(), c[i].data_ptr(), N, s.cuda_stream)
+    torch.cuda.synchronize()
+    assert plan.last_walk()["scheduled"] and plan.last_walk()["split_windows"] > 0
+    assert all(torch.equal(x, w) for c, w in zip(dC, want) for x in c)
+    plan.close()
+
+
+def test_infinities_and_nans_stay_with_the_windows_that_name_them(torch_cuda, hs):
     torch = torch_cuda
     rng = np.random.default_rng(11)
     rows, cols = 330, 3000
@@ -80,6 +135,7 @@ def test_infinities_and_nans_stay_with_the_rows_that_name_them(torch_cuda, hs):
             dC = torch.empty((rows, N), dtype=dB.dtype, device="cuda")
             plan.run(dB.data_ptr(), dC.data_ptr(), N, torch.cuda.current_stream().cuda_stream)
             torch.cuda.synchronize()
+            assert plan.last_walk()["scheduled"]
             got = decode(_host(dC, 0), 0)
             hit, near = np.zeros(got.shape, bool), np.zeros(got.shape, bool)
             hit[mask[:, 17], 5] = hit[mask[:, 2900], 6] = True
@@ -125,7 +181,60 @@ def test_graphs_of_many_columns_have_one(torch_cuda, hs):
             launch(b.data_ptr() + 2 * shift, dC.data_ptr(), N, stream)
             torch.cuda.synchronize()
             assert torch.equal(dC, want)
-            if not shift:
-                assert plan.last_kernel() == "spmm_mfma_kernel"
+            if shift:
+                assert not plan.last_walk()["scheduled"]
+            else:
+                assert plan.last_kernel() == "spmm_mfma_kernel" and plan.last_walk()["scheduled"]
+            without.run(b.data_ptr() + 2 * shift, dC.data_ptr(), N, stream)
+            torch.cuda.synchronize()
+            assert torch.equal(dC, want) and not without.last_walk()["scheduled"]
+    plan.close()
+    # the static entry point does not change kernels with what ran before: B between two words is the entry kernels' launch
+    os.environ["HSPMM_GATHER_BITMAP"] = "1"
+    try:
+        plan = hs.Plan(tiles)
+    finally:
+        os.environ.pop("HSPMM_GATHER_BITMAP")
+    between = torch.cat([flat[:1], flat])
+    for _ in range(2):
+        plan.run(flat.data_ptr(), dC.data_ptr(), N, stream)
+    with pytest.raises(hs.HspmmError, match="hspmm_prepare"):
+        plan.run_static(between.data_ptr() + 2, dC.data_ptr(), N, stream)
+    plan.run(between.data_ptr() + 2, dC.data_ptr(), N, stream)
+    torch.cuda.synchronize()
+    assert torch.equal(dC, want) and plan.last_kernel() == "spmm_entries_kernel"
+    plan.run_static(between.data_ptr() + 2, dC.data_ptr(), N, stream)
+    torch.cuda.synchronize()
+    assert torch.equal(dC, want) and plan.last_kernel() == "spmm_entries_kernel"
     plan.close()
     without.close()
+
+
+def test_more_columns_than_a_schedule_reaches(torch_cuda, hs):
+    """2^24 columns: offsets into B do not fit 32 bits and the launch is the entry kernels'."""
+    torch = torch_cuda
+    rng = np.random.default_rng(6)
+    rows, cols, N = 2048, (1 << 24) + 40, 64
+    columns = [np.unique((cols * rng.random(n) ** 8).astype(np.uint32)) for n in np.minimum(rng.zipf(1.6, rows), 9000)]
+    columns[3] = np.unique(np.append(columns[3], cols - 1)).astype(np.uint32)
+    counts = np.array([len(c) for c in columns])
+    values = rng.choice([-2.0, -1.0, 1.0, 2.0], int(counts.sum())).astype(np.float32)
+    ids = np.concatenate(columns).astype(np.uint32)
+    A = dict(rows=rows, cols=cols, nnzs=int(counts.sum()), dtype=0, row_ptr=np.concatenate([[0], np.cumsum(counts)]).astype(np.uint32),
+             col_idx=ids, values=encode(values, 0))
+    tiles = convert(hs, A)
+    assert A["nnzs"] > 1.01 * (tiles["tcA2B"] != 0xFFFFFFFF).sum()
+    os.environ["HSPMM_GATHER_BITMAP"] = "1"
+    try:
+        plan = hs.Plan(tiles)
+    finally:
+        os.environ.pop("HSPMM_GATHER_BITMAP")
+    B = torch.randint(-1, 2, (cols, N), dtype=torch.int8, device="cuda").half()
+    C = torch.full((rows, N), float("nan"), dtype=torch.float16, device="cuda")
+    plan.run(B.data_ptr(), C.data_ptr(), N, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert plan.last_kernel() == "spmm_entries_kernel" and not plan.last_walk()["scheduled"]
+    entries = B[torch.from_numpy(ids.astype(np.int64)).cuda()].float().cpu().numpy() * values[:, None]
+    want = np.add.reduceat(entries, A["row_ptr"][:-1].astype(np.int64), axis=0)     # (no row is empty; whole numbers, exact in any order)
+    assert (C.float().cpu().numpy() == want).all()
+    plan.close()
