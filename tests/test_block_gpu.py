@@ -5,7 +5,6 @@ import os
 import numpy as np
 import pytest
 
-import test_nonfinite_gpu as nonfinite
 from test_spmm_gpu import convert, torch_cuda  # noqa: F401
 from util import decode, encode
 
@@ -48,7 +47,8 @@ def _plan(hs, A, block):
 
 @pytest.mark.parametrize("dtype", [0, 1, 2])
 @pytest.mark.parametrize("rows,cols,keep,without,half", [(16, 16, 1.0, 0, False), (40, 24, 1.0, 0.3, False), (250, 333, 0.5, 0.2, True), (9, 100, 1.0, 0, False),
-                                                         (1000, 2000, 0.3, 0.05, True), (130, 16500, 0.9, 0, False)])
+                                                         (1000, 2000, 0.3, 0.05, True), (130, 16500, 0.9, 0, False),
+                                                         (34, 17400, 1.0, 0, False)])           # (over 1024 steps: a wave's second 64 pairs)
 def test_exact_sums_at_every_edge(torch_cuda, hs, dtype, rows, cols, keep, without, half):
     torch = torch_cuda
     rng = np.random.default_rng(rows + cols)
@@ -78,19 +78,23 @@ def test_exact_sums_at_every_edge(torch_cuda, hs, dtype, rows, cols, keep, witho
 
 
 @pytest.mark.parametrize("dtype", [0, 1, 2])
-def test_infinities_and_nans_stay_with_the_rows_that_name_them(torch_cuda, hs, monkeypatch, dtype):
-    """A column of the matrix loses half of its entries first, so that blocks hold zeros beside them."""
+def test_infinities_and_nans_stay_with_the_rows_that_name_them(torch_cuda, hs, dtype):
+    """A column of the matrix loses half of its entries first, so that blocks hold zeros beside them; rows of blocks without any, windows alone.
+    Every other sum, those of the same features among them, is what it is without (bound: see below)."""
     torch = torch_cuda
     rng = np.random.default_rng(3 + dtype)
-    mask = _blocks(rng, 300, 400, 0.5)
+    mask = _blocks(rng, 300, 400, 0.5, 0.1, True)
     mask[::3, ::5] = False
+    mask[24:32] = False
+    mask[8:16] = False
     A = _csr(mask, rng.normal(size=int(mask.sum())), dtype)
     D = np.zeros(mask.shape)
     D[mask] = decode(A["values"], dtype)
     plan = _plan(hs, A, 1)
+    assert plan.info()["n_units"] > plan.info()["n_paired_units"] > 0
     for N in (5, 16, 31, 64):
         B = decode(encode(rng.normal(size=(400, N)).astype(np.float32), dtype), dtype)
-        finite = D @ B
+        finite, sizes = D @ B, abs(D) @ abs(B)
         bad = B.copy()
         bad[17, N - 1], bad[240, 0] = np.inf, np.nan
         dB = _device(torch, bad, dtype)
@@ -103,6 +107,8 @@ def test_infinities_and_nans_stay_with_the_rows_that_name_them(torch_cuda, hs, m
         hit[mask[:, 240], 0] = True
         assert not np.isfinite(got[hit]).any() and np.isfinite(got[~hit]).all()
         assert (np.isinf(got[:, N - 1]) == mask[:, 17])[~mask[:, 240] | (N > 1)].all()
+        off = abs(got - finite)
+        assert (off <= (mask.sum(1).max() + 1) * 2.0**-24 * sizes + 2.0**{0: -11, 1: -24, 2: -8}[dtype] * abs(finite) + 1e-7)[~hit].all()
     assert plan.last_kernel() == "spmm_block_kernel"
     plan.close()
 
