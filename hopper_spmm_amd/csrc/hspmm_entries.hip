@@ -251,8 +251,10 @@ bool entries_serve(const hspmm_plan *p, uint32_t N)
     }
     if (weight <= 42.0 || (sparse && row <= 128u)) return true;
     if (!sparse || panel_serves(p, N)) return false;
-    // (those dense graphs, wide loads in blocks of 128 features: N = 800 31.0 / 27.6 us at 8192 vertices, 46.8 / 35.9 at 12288; N = 640 20.3 / 22.1)
-    if (per_column > 1.25 && N > 640u && N % 8u == 0u && N % 64u != 0u) return false;
+    // Those dense graphs by wide loads or words above 640 features: graph of 12288, 24 edges each, N = 704 / 800 / 832 / 1024 29.6 / 27.7, 39.8 / 34.7,
+    // 34.0 / 31.8, 37.2 / 31.9; of 16000, 40 edges, 1024 64.3 / 58.0; 512, 576 and 640 0.96 to 1.18 times as fast here on eight graphs of 8192 to 16000
+    // (768 and 896 0.96 to 1.11: left), other N there 0.98 to 1.9 (700 33.5 / 44.1, 1023 54.1 / 58.1).
+    if (per_column > 1.25 && N > 640u && N % 8u == 0u) return false;
     // N a multiple of 64, hot rows and a B that fills half of the 256 MB memory-side cache: there the other kernels, which then load
     // words and read fewer rows of B, are ahead (graph of 920569, N = 128, 236 MB: 363 / 343 us; of 434176, N = 512, 445 MB:
     // 353 / 322; 18 such graphs: 1.02 on average, and 1.13 behind on 16 with other N a multiple of 8).
