@@ -628,6 +628,7 @@ ScheduleTables schedule_tables(const hspmm_plan *p, const uint32_t *rowOffset, c
     if (!shortest || (p->cfg.schedule < 0 && windows_are_even(longest, W, T))) return out;
     const uint32_t most = (T + kMinTilesPerRange - 1u) / kMinTilesPerRange;
     const uint32_t n_waves = std::max(1u, std::min(p->cfg.schedule > 1 ? uint32_t(p->cfg.schedule) : uint32_t(p->compute_units) * 8u, most));
+    if (p->cfg.schedule < 0 && uint64_t(longest) * n_waves > uint64_t(T) * kScheduledLongest) return out;
     const hspmm::Schedule s = hspmm::build_schedule(W, rowOffset, n_waves);
     const uint32_t n = uint32_t(s.items.size()), n_ranges = std::min(n_waves, n);   // (the first waves are the ones that have items)
     // cut windows: their parts have neighbouring slots
@@ -782,6 +783,8 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
         for (uint32_t w = 0; sparse_tiles && w < p->W; ++w) stored += window_stored[w];
         sparse_tiles = sparse_tiles && st.G == 1 && stored + spare < (uint64_t(1) << 31) &&
                        (p->cfg.gather_bitmap > 0 || stored * 3u < uint64_t(total_tiles) * 8u * cw);
+        p->per_column = entries_per_column(total_tiles, cw, elem, tcA2B, data, bitmap, sparse_tiles ? header.data() : nullptr);
+        const bool scheduled = schedule.wanted() && p->canonical && p->caller_cuts.empty() && (p->cfg.schedule > 0 || p->per_column > kScheduledColumnsShared);
         void *room = nullptr;
         uint32_t *schedule_at = nullptr;
         auto copy_schedule = [&] { return copy_up(p, schedule_at + size_t(total_tiles) * 24u, schedule.words.data(), schedule.words.size() * 4u); };
@@ -797,7 +800,7 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
             p->bm.d_vals = room;
             if ((rc = plan_alloc(p, tile_bytes, &room))) return bail(rc);
             p->d_data = room;
-            if (schedule.wanted() && p->canonical && p->caller_cuts.empty()) schedule_at = schedule_room(p, schedule);
+            if (scheduled) schedule_at = schedule_room(p, schedule);
             const uint32_t header_words = elem == 2u ? 8u : 4u;
             auto by_windows = [&](auto fn) {
                 hspmm_host::parallel_weighted(p->W, size_t(1) << 13, [=](size_t w) { return rowOffset[w]; }, fn);
@@ -906,7 +909,6 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
             p->d_tiles = room;
             HSPMM_HIP_OR(hspmm::launch_lane_order32(p->d_data, room, total_tiles, nullptr), bail);
         }
-        p->per_column = entries_per_column(total_tiles, cw, elem, tcA2B, data, bitmap, sparse_tiles ? header.data() : nullptr);
         {
             uint32_t longest = 0;
             for (size_t u = 0; u + 1 < st.unitOffset.size(); ++u) longest = std::max(longest, st.unitOffset[u + 1] - st.unitOffset[u]);
@@ -919,9 +921,7 @@ int create_plan(hspmm_plan **out, int dtype, uint32_t rows, uint32_t cols, uint3
         if ((rc = build_and_upload_partition(p, 0))) return bail(rc);
         if ((rc = count_entries(p))) return bail(rc);                   // (behind the last of the small uploads, which would wait for it)
         timer.mark("partition");
-        if (!schedule_at && schedule.wanted() && p->G == 1 && p->bm.built && p->canonical && p->caller_cuts.empty() && (schedule_at = schedule_room(p, schedule)) &&
-            (rc = copy_schedule()))
-            return bail(rc);
+        if (!schedule_at && scheduled && p->G == 1 && p->bm.built && (schedule_at = schedule_room(p, schedule)) && (rc = copy_schedule())) return bail(rc);
         if (schedule_at && (rc = fill_schedule(p, schedule, schedule_at))) return bail(rc);
         timer.mark("schedule");
         {

@@ -121,6 +121,14 @@ constexpr uint32_t kScheduledColumns = 1u << 18;
 // (N = 64: 2^20 vertices 260 / 207 us, 800000 112 / 107, 600000 73 / 77, 350000 55 / 63, 2^18 42 / 50).  Two, four or eight blocks, each with XCDs of
 // its own, from the first such plan on (N = 128: 2^19 240 / 177, 350000 116 / 108, 2^18 94 / 80; N = 256 at 2^18: 193 / 170).
 constexpr uint64_t kScheduledSlice = uint64_t(96) << 20;
+// What keeps a launch from the order's gain, of 804 launches of matrices of 4000 to 800000 rows and 2^18 to 1.2 million columns (R-MAT, and rows and
+// columns drawn by powers), at all these N: windows so long that the sums of many parts are added one after the other (the longest over 32 of a
+// wave's shares: 0.94 times as fast on the mean, 0.27 at least); columns that no windows share (1.01 entries per tile column and less: 1.0, 0.88 at
+// least, and slower than the entry kernels); launches too short for it, in which few rows name many columns (C below 64 MB: 0.98, 0.51).  195 launches
+// are left, 1.12 times as fast on the mean, 5 slower by more than 3 % (8 % at most).  Graphs as tall as they are wide are all among them.
+constexpr uint32_t kScheduledLongest = 32;
+constexpr double kScheduledColumnsShared = 1.01;
+constexpr uint64_t kScheduledProduct = uint64_t(64) << 20;
 // No unit has over eight times the average number of steps.
 inline bool windows_are_even(uint32_t longest, uint32_t units, uint32_t steps) { return uint64_t(longest) * units <= uint64_t(steps) * 8u; }
 
@@ -390,6 +398,7 @@ inline bool scheduled_serves(const hspmm_plan *p, uint32_t N)
     const hspmm_plan::Scheduled &sc = p->scheduled;
     if (!sc.built || !(N % 128u == 64u || (splits_features(p, N) && (N == 128u || N == 256u || N == 512u)))) return false;
     if (p->cols >= (1u << 24) || uint64_t(p->cols) * N * p->elem > (uint64_t(1) << 32)) return false;
+    if (p->cfg.schedule < 0 && uint64_t(p->rows) * N * p->elem < kScheduledProduct) return false;
     return size_t(sc.n_slots) * (N / 64u) * 2048u <= HSPMM_STATIC_SCRATCH_BYTES;     // (however it is launched)
 }
 
@@ -398,7 +407,7 @@ inline bool scheduled_serves(const hspmm_plan *p, uint32_t N)
 // schedule / entry kernels: 2^19 columns 207 / 191, 300000 59.7 / 55.2, 2^18 58.6 / 53.7; N = 64, 2^20 columns 101 / 94, 240 / 218, 66 / 58.
 inline bool scheduled_before_entries(const hspmm_plan *p, uint32_t N, uintptr_t align)
 {
-    return p->cfg.entries < 0 && p->per_column > 1.01 && align % 4u == 0u && scheduled_serves(p, N) &&
+    return p->cfg.entries < 0 && p->per_column > kScheduledColumnsShared && align % 4u == 0u && scheduled_serves(p, N) &&
            (N % 128u == 0u || uint64_t(p->cols) * 128u >= kScheduledSlice);
 }
 

@@ -47,7 +47,7 @@ def test_schedules_serve_where_the_gather_kernels_could_walk_them(build):  # noq
     """Blocks of 64 features, 32-bit offsets into B: launches of other shapes are not kept from the entry kernels."""
     _run(build, _driver(ENTRY_STUBS, """
     hspmm_plan p;
-    p.dtype = HSPMM_FP16; p.rows = 1 << 20; p.per_column = 1.05;
+    p.dtype = HSPMM_FP16; p.rows = 1 << 21; p.per_column = 1.05;
     p.scheduled.built = true; p.scheduled.n_slots = 350;
     for (uint32_t cols : {1u << 18, 1u << 20, 1u << 22, (1u << 23) + 8u, (1u << 24) - 1u, 1u << 24, (1u << 24) + 1000u, 1u << 26})
         for (uint32_t N : {32u, 64u, 96u, 128u, 192u, 256u, 320u, 384u, 512u, 1024u}) {
@@ -201,4 +201,19 @@ def test_graphs_dense_in_their_hot_columns_by_their_loads(build):  # noqa: F811
     for (uint32_t N = 1; N <= 1024; ++N) EXPECT(entries_serve(&p, N));
     p.per_column = 1.3; p.even_windows = true;
     EXPECT(!entries_serve(&p, 512u) && !entries_serve(&p, 45u));
+"""), "entries")
+
+
+def test_schedules_of_launches_that_gain_from_the_order(build):  # noqa: F811
+    _run(build, _driver(ENTRY_STUBS, """
+    hspmm_plan p;
+    p.dtype = HSPMM_BF16; p.cols = 1 << 18; p.per_column = 1.1;
+    p.scheduled.built = true; p.scheduled.n_slots = 350;
+    for (uint32_t rows : {1000u, (1u << 17) - 1u, 1u << 17, 1u << 18, 1u << 20})
+        for (uint32_t N : {64u, 128u, 256u, 576u}) {
+            p.rows = rows; p.cfg.schedule = -1;
+            EXPECT(scheduled_serves(&p, N) == (uint64_t(rows) * N * 2u >= (64u << 20)));
+            p.cfg.schedule = 1;
+            EXPECT(scheduled_serves(&p, N));
+        }
 """), "entries")

@@ -146,95 +146,87 @@ def test_infinities_and_nans_stay_with_the_windows_that_name_them(torch_cuda, hs
         plan.close()
 
 
+def _hot(rng, rows, cols, power):
+    """A graph of uneven rows over hot columns: CSR of whole numbers, the row of every entry."""
+    counts = np.minimum(rng.zipf(2.0, rows), 2000)
+    keys = np.unique(np.repeat(np.arange(rows), counts) * cols + (cols * rng.random(int(counts.sum())) ** power).astype(np.int64))
+    r, c = keys // cols, keys % cols
+    values = rng.choice([-2.0, -1.0, 1.0, 2.0], len(keys)).astype(np.float32)
+    A = dict(rows=rows, cols=cols, nnzs=len(keys), dtype=0, row_ptr=np.concatenate([[0], np.cumsum(np.bincount(r, minlength=rows))]).astype(np.uint32),
+             col_idx=c.astype(np.uint32), values=encode(values, 0))
+    return A, r, values
+
+
+def _sums(torch, A, r, values, B):
+    """(whole numbers below 2^24: exact in any order, and rounded once)"""
+    out = torch.zeros((A["rows"], B.shape[1]), dtype=torch.float32, device="cuda")
+    r, c, v = (torch.from_numpy(np.ascontiguousarray(x)).cuda() for x in (r, A["col_idx"].astype(np.int64), values))
+    for at in range(0, len(values), 1 << 18):
+        out.index_add_(0, r[at:at + (1 << 18)], B[c[at:at + (1 << 18)]].float() * v[at:at + (1 << 18), None])
+    return out.half()
+
+
+def _graph_plans(hs, A, *schedules):
+    tiles = convert(hs, A)
+    assert A["nnzs"] > 1.01 * (tiles["tcA2B"] != 0xFFFFFFFF).sum()
+    os.environ["HSPMM_GATHER_BITMAP"] = "1"             # (tiles of 8 MB and more have them by themselves)
+    plans = []
+    try:
+        for schedule in schedules:
+            os.environ["HSPMM_SCHEDULE"] = schedule
+            plans.append(hs.Plan(tiles))
+    finally:
+        os.environ.pop("HSPMM_GATHER_BITMAP")
+        os.environ.pop("HSPMM_SCHEDULE", None)
+    return plans
+
+
 def test_graphs_of_many_columns_have_one(torch_cuda, hs):
     """Words of B and C at 128 features are walked by it, also where nothing may be built; between two words the launch is another kernel's."""
     torch = torch_cuda
     rng = np.random.default_rng(5)
-    rows, cols, N = 4096, 1 << 18, 128
-    # (hot columns: over uniform ones the entry kernels come first)
-    columns = [np.unique((cols * rng.random(n) ** 6).astype(np.uint32)) for n in np.minimum(rng.zipf(1.6, rows), 20000)]
-    counts = np.array([len(c) for c in columns])
-    values = rng.choice([-2.0, -1.0, 1.0, 2.0], int(counts.sum()))
-    A = dict(rows=rows, cols=cols, nnzs=int(counts.sum()), dtype=0, row_ptr=np.concatenate([[0], np.cumsum(counts)]).astype(np.uint32),
-             col_idx=np.concatenate(columns).astype(np.uint32), values=encode(values.astype(np.float32), 0))
-    Bm = rng.integers(-1, 2, (cols, N)).astype(np.float32)
-    ends = np.cumsum(counts)
-    want = _device(torch, np.stack([values[e - n:e] @ Bm[c] for n, e, c in zip(counts, ends, columns)]), 0)
-    os.environ["HSPMM_GATHER_BITMAP"] = "1"             # (tiles of 8 MB and more have them by themselves)
-    try:
-        tiles = convert(hs, A)
-        assert A["nnzs"] > 1.01 * (tiles["tcA2B"] != 0xFFFFFFFF).sum()
-        plan = hs.Plan(tiles)
-        os.environ["HSPMM_SCHEDULE"] = "0"
-        without = hs.Plan(convert(hs, A))
-    finally:
-        os.environ.pop("HSPMM_GATHER_BITMAP")
-        os.environ.pop("HSPMM_SCHEDULE", None)
+    rows, cols, N = 1 << 18, 1 << 18, 128
+    A, r, values = _hot(rng, rows, cols, 6)
+    plan, without = _graph_plans(hs, A, "-1", "0")
     assert plan.info()["device_bytes"] > without.info()["device_bytes"]
+    B = torch.randint(-1, 2, (cols, N), dtype=torch.int8, device="cuda").half()
+    want = _sums(torch, A, r, values, B)
     stream = torch.cuda.current_stream().cuda_stream
-    flat = _device(torch, Bm.reshape(-1), 0)
-    for shift in (0, 1, 0):
-        b = torch.cat([flat[:shift], flat])
-        plan.prepare(N)
-        for launch in (plan.run_static, plan.run, plan.run_static):
-            dC = torch.full_like(want, 0x7E01)
-            launch(b.data_ptr() + 2 * shift, dC.data_ptr(), N, stream)
-            torch.cuda.synchronize()
-            assert torch.equal(dC, want)
-            if shift:
-                assert not plan.last_walk()["scheduled"]
-            else:
-                assert plan.last_kernel() == "spmm_mfma_kernel" and plan.last_walk()["scheduled"]
-            without.run(b.data_ptr() + 2 * shift, dC.data_ptr(), N, stream)
-            torch.cuda.synchronize()
-            assert torch.equal(dC, want) and not without.last_walk()["scheduled"]
-    plan.close()
+    between = torch.cat([B.reshape(-1)[:1], B.reshape(-1)])
     # the static entry point does not change kernels with what ran before: B between two words is the entry kernels' launch
-    os.environ["HSPMM_GATHER_BITMAP"] = "1"
-    try:
-        plan = hs.Plan(tiles)
-    finally:
-        os.environ.pop("HSPMM_GATHER_BITMAP")
-    between = torch.cat([flat[:1], flat])
+    dC = torch.full_like(want, float("nan"))
     for _ in range(2):
-        plan.run(flat.data_ptr(), dC.data_ptr(), N, stream)
+        plan.run(B.data_ptr(), dC.data_ptr(), N, stream)
     with pytest.raises(hs.HspmmError, match="hspmm_prepare"):
         plan.run_static(between.data_ptr() + 2, dC.data_ptr(), N, stream)
-    plan.run(between.data_ptr() + 2, dC.data_ptr(), N, stream)
-    torch.cuda.synchronize()
-    assert torch.equal(dC, want) and plan.last_kernel() == "spmm_entries_kernel"
-    plan.run_static(between.data_ptr() + 2, dC.data_ptr(), N, stream)
-    torch.cuda.synchronize()
-    assert torch.equal(dC, want) and plan.last_kernel() == "spmm_entries_kernel"
-    plan.close()
-    without.close()
+    for p, walked in ((plan, True), (without, False)):
+        p.prepare(N)
+        for at in (B.data_ptr(), between.data_ptr() + 2, B.data_ptr()):
+            for launch in (p.run_static, p.run, p.run_static):
+                dC.fill_(float("nan"))
+                launch(at, dC.data_ptr(), N, stream)
+                torch.cuda.synchronize()
+                assert torch.equal(dC, want)
+                scheduled = walked and at == B.data_ptr()
+                assert p.last_walk()["scheduled"] == scheduled and p.last_kernel() == ("spmm_mfma_kernel" if scheduled else "spmm_entries_kernel")
+        # (C of 32 MB: too short a launch)
+        p.run(B.data_ptr(), dC.data_ptr(), 64, stream)
+        torch.cuda.synchronize()
+        assert not p.last_walk()["scheduled"]
+        p.close()
 
 
 def test_more_columns_than_a_schedule_reaches(torch_cuda, hs):
     """2^24 columns: offsets into B do not fit 32 bits and the launch is the entry kernels'."""
     torch = torch_cuda
     rng = np.random.default_rng(6)
-    rows, cols, N = 2048, (1 << 24) + 40, 64
-    columns = [np.unique((cols * rng.random(n) ** 8).astype(np.uint32)) for n in np.minimum(rng.zipf(1.6, rows), 9000)]
-    columns[3] = np.unique(np.append(columns[3], cols - 1)).astype(np.uint32)
-    counts = np.array([len(c) for c in columns])
-    values = rng.choice([-2.0, -1.0, 1.0, 2.0], int(counts.sum())).astype(np.float32)
-    ids = np.concatenate(columns).astype(np.uint32)
-    A = dict(rows=rows, cols=cols, nnzs=int(counts.sum()), dtype=0, row_ptr=np.concatenate([[0], np.cumsum(counts)]).astype(np.uint32),
-             col_idx=ids, values=encode(values, 0))
-    tiles = convert(hs, A)
-    assert A["nnzs"] > 1.01 * (tiles["tcA2B"] != 0xFFFFFFFF).sum()
-    os.environ["HSPMM_GATHER_BITMAP"] = "1"
-    try:
-        plan = hs.Plan(tiles)
-    finally:
-        os.environ.pop("HSPMM_GATHER_BITMAP")
+    rows, cols, N = 1 << 19, (1 << 24) + 40, 64
+    A, r, values = _hot(rng, rows, cols, 8)
+    (plan,) = _graph_plans(hs, A, "-1")
     B = torch.randint(-1, 2, (cols, N), dtype=torch.int8, device="cuda").half()
     C = torch.full((rows, N), float("nan"), dtype=torch.float16, device="cuda")
     plan.run(B.data_ptr(), C.data_ptr(), N, torch.cuda.current_stream().cuda_stream)
     torch.cuda.synchronize()
     assert plan.last_kernel() == "spmm_entries_kernel" and not plan.last_walk()["scheduled"]
-    entries = B[torch.from_numpy(ids.astype(np.int64)).cuda()].float().cpu().numpy() * values[:, None]
-    want = np.add.reduceat(entries, A["row_ptr"][:-1].astype(np.int64), axis=0)     # (no row is empty; whole numbers, exact in any order)
-    assert (C.float().cpu().numpy() == want).all()
+    assert torch.equal(C, _sums(torch, A, r, values, B))
     plan.close()
