@@ -222,7 +222,7 @@ bool entries_serve(const hspmm_plan *p, uint32_t N)
 {
     const Config &c = p->cfg;
     if (!p->entries.counted || p->entries.unavailable.load()) return false;
-    const uint64_t row = uint64_t(N) * p->elem, all = uint64_t(p->cols) * row;
+    const uint64_t row = uint64_t(N) * p->elem, all = uint64_t(p->cols) * row, product = uint64_t(p->rows) * row;
     if (N > kEntryMostFeatures) return false;       // (16-bit rows of more than 2 KB have not been measured here)
     if (c.entries > 0) return true;
     const double per_column = p->per_column, weight = double(row) * (per_column - 0.8);
@@ -254,7 +254,13 @@ bool entries_serve(const hspmm_plan *p, uint32_t N)
     // Those dense graphs by wide loads or words above 640 features: graph of 12288, 24 edges each, N = 704 / 800 / 832 / 1024 29.6 / 27.7, 39.8 / 34.7,
     // 34.0 / 31.8, 37.2 / 31.9; of 16000, 40 edges, 1024 64.3 / 58.0; 512, 576 and 640 0.96 to 1.18 times as fast here on eight graphs of 8192 to 16000
     // (768 and 896 0.96 to 1.11: left), other N there 0.98 to 1.9 (700 33.5 / 44.1, 1023 54.1 / 58.1).
-    if (per_column > 1.25 && N > 640u && N % 8u == 0u) return false;
+    // Above 96 features the wide loads keep N a multiple of 8 but not of 64 (0.7 to 1.5 on 126 launches, a third of them behind), and with them a C of
+    // more than 16 MB, with others one of more than 32 MB, is the gather kernels' (333 launches left to them: 1.08 on the mean here, 113 behind, by up to 33 %;
+    // 752 taken: 1.73 times as fast, 14 behind by more than 3 %, 18 % at most).
+    if (per_column > 1.25) {
+        if (N % 8u == 0u && (N > 640u || (N > 96u && N % 64u != 0u))) return false;
+        if (product > (uint64_t(N % 8u == 0u ? 16u : 32u) << 20)) return false;
+    }
     // N a multiple of 64, hot rows and a B that fills half of the 256 MB memory-side cache: there the other kernels, which then load
     // words and read fewer rows of B, are ahead (graph of 920569, N = 128, 236 MB: 363 / 343 us; of 434176, N = 512, 445 MB:
     // 353 / 322; 18 such graphs: 1.02 on average, and 1.13 behind on 16 with other N a multiple of 8).

@@ -191,16 +191,19 @@ def test_block_kernels_take_even_rows_of_blocks(build):  # noqa: F811
 
 
 def test_graphs_dense_in_their_hot_columns_by_their_loads(build):  # noqa: F811
-    """1.25 to 1.4 entries per tile column: above 640 features the gather kernels' wide loads come first, where N is a multiple of 8."""
+    """1.25 to 1.4 entries per tile column: the gather kernels' wide loads come first where N is a multiple of 8, and where C is large."""
     _run(build, _driver(ENTRY_STUBS, """
     hspmm_plan p;
-    p.dtype = HSPMM_FP16; p.rows = p.cols = 12288; p.W = 1536; p.T = 14000; p.compute_units = 256; p.per_column = 1.3;
+    p.dtype = HSPMM_FP16; p.rows = p.cols = 8000; p.W = 1000; p.T = 14000; p.compute_units = 256; p.per_column = 1.3;
     p.entries.counted = true;
-    for (uint32_t N = 1; N <= 1024; ++N) EXPECT(entries_serve(&p, N) == (N <= 640u || N % 8u != 0u));
+    for (uint32_t N = 1; N <= 1024; ++N) EXPECT(entries_serve(&p, N) == (N <= 96u || N % 8u != 0u || (N <= 640u && N % 64u == 0u)));
+    p.rows = 40000;
+    for (uint32_t N = 65; N <= 1024; ++N) EXPECT(entries_serve(&p, N) == (N % 8u ? N * 80000u <= (32u << 20) : (N <= 96u || N % 64u == 0u) && N * 80000u <= (16u << 20)));
+    for (uint32_t N = 1; N <= 64; ++N) EXPECT(entries_serve(&p, N));
     p.per_column = 1.1;
     for (uint32_t N = 1; N <= 1024; ++N) EXPECT(entries_serve(&p, N));
     p.per_column = 1.3; p.even_windows = true;
-    EXPECT(!entries_serve(&p, 512u) && !entries_serve(&p, 45u));
+    EXPECT(!entries_serve(&p, 512u) && !entries_serve(&p, 97u));
 """), "entries")
 
 
