@@ -246,6 +246,11 @@ bool entries_serve(const hspmm_plan *p, uint32_t N)
         // 180 / 334; graph of 16000, 32 edges each, 65 / 104, 107 / 175.  Where columns are hot and B is larger than 156 MB the other kernels read
         // less of it (graph of 81984, 5 edges each, N = 640 / 768 / 1024: 148 / 135, 193 / 162, 274 / 200; of 40000, N = 1024, 156 MB: 140 / 163);
         // uniform ones were ahead at all sizes up to 460 MB (27793 x 118016, N = 768 103 / 112, 1024 140 / 142; 2048 x 100000, N = 1024 108 / 140).
+        // (Not where rows of a few entries make a large C, which the other kernels write faster: 341404 x 2685, 1.8 per row, N = 1024 362 / 573; 407281 x
+        // 5276, 1 per row, 316 / 449; 465282 x 221802, 1 per row, N = 320 197 / 259; graph of 1.3 entries per tile column, 4 per row, N = 400 0.70.  Up to
+        // 64 MB of C all of 682 launches with fewer than 6 entries a row but three were ahead, from 6 entries on all of 899 but four, by up to 8 %.)
+        const bool extended = row > 2048u || all > (uint64_t(256) << 20) || per_column > 1.25;
+        if (extended && product > (uint64_t(64) << 20) && double(p->T) * p->cw * per_column < 6.0 * p->rows) return false;
         const uint64_t most = p->even_windows ? uint64_t(512) << 20 : row <= 2048u ? uint64_t(256) << 20 : uint64_t(160) << 20;
         return sparse && !p->panel.built && (row <= 256u || all <= most);
     }

@@ -207,6 +207,26 @@ def test_graphs_dense_in_their_hot_columns_by_their_loads(build):  # noqa: F811
 """), "entries")
 
 
+def test_large_products_of_short_rows_in_fp32(build):  # noqa: F811
+    """Rows of B of over 2 KB, or a B of over 256 MB, or dense graphs: not where a few entries a row make a C of over 64 MB."""
+    _run(build, _driver(ENTRY_STUBS, """
+    for (double per_row : {1.0, 5.0, 7.0, 20.0})
+        for (uint32_t rows : {10000u, 16384u, 20000u, 400000u})
+            for (bool even : {false, true}) {
+                hspmm_plan p;
+                p.dtype = HSPMM_TF32; p.elem = 4; p.cw = 8; p.rows = rows; p.cols = 5000; p.W = rows / 8; p.compute_units = 256; p.per_column = 1.0;
+                p.T = uint32_t(per_row * rows / 8.0); p.entries.counted = true; p.even_windows = even;
+                for (uint32_t N : {513u, 640u, 1024u}) EXPECT(entries_serve(&p, N) == (per_row >= 6.0 || uint64_t(rows) * N * 4u <= (64u << 20)));
+                for (uint32_t N : {65u, 128u, 512u}) EXPECT(entries_serve(&p, N));
+                p.cols = 200000;
+                EXPECT(entries_serve(&p, 320u));                                        // 256 MB
+                EXPECT(entries_serve(&p, 512u) == (even && (per_row >= 6.0 || rows <= 20000u)));
+                p.cols = 5000; p.per_column = 1.3; p.T = uint32_t(p.T / 1.3);
+                if (!even) EXPECT(entries_serve(&p, 256u) == (per_row >= 6.0 || rows <= 20000u));
+            }
+"""), "entries")
+
+
 def test_schedules_of_launches_that_gain_from_the_order(build):  # noqa: F811
     _run(build, _driver(ENTRY_STUBS, """
     hspmm_plan p;
