@@ -107,7 +107,11 @@ int build_block_units(hspmm_plan *p, const StepStream &st, const uint32_t *rowOf
 // most), 1.45 times as fast on the mean.  Odd ones stay with the wide-tile kernels (0.9 to 1.2 there), and from 65 on all (0.7 to 1.2).  fp32 storage: every launch
 // of the gather kernels (207 of 60 matrices: 1.07 to 3.5 times as fast); those of the LDS-panel kernels, which are faster from 33 features on
 // and for the largest matrices, by expected time (134 taken: 1.49 on the mean, 0.88 at least; 26 up to 32 features left).
-bool block_serves(const hspmm_plan *p, uint32_t N)
+// Not at N = 32 on more than 65 % of all blocks, where the wide-tile kernels take it (11 of 12 launches were 2 to 20 % slower here, of 22 below none), and
+// not above 32 features on rows of over 512 blocks of fp32 storage (nine with B off its alignment: 0.9).  A B that begins between two words has loads of
+// twice the time: the wide-tile kernels keep theirs (224 launches: 0.87 times as fast here), and above 32 features units of over 128 blocks stay (91:
+// 1.1, 26 behind, by up to 34 %); the others were 1.28 (up to 32 features) and 1.46 times as fast.
+bool block_serves(const hspmm_plan *p, uint32_t N, bool on_word)
 {
     const Config &c = p->cfg;
     if (!p->block_units.built || N > kMostFeatures || uint64_t(p->cols) * N * p->elem > (uint64_t(1) << 32)) return false;
@@ -116,12 +120,15 @@ bool block_serves(const hspmm_plan *p, uint32_t N)
                         c.panel_units_per_group || c.aligned_small >= 0 || c.xcd_split >= 0 || c.gather_bitmap >= 0 || c.tile > 0 || c.entries > 0 || c.wide > 0))
         return false;
     if (p->elem == 4u) {
+        if (c.block <= 0 && N > kAlwaysFeatures && p->block_units.longest > 1024u) return false;
         if (c.block > 0 || N < 16u || N % 4u || !panel_serves(p, N)) return true;
         return N <= kAlwaysFeatures && p->block_units.taken.get(N, [&]() -> uint32_t { return expected_f32(p, N) < 0.95 * (6.2 + 0.9 * panel_expected(p, N)); });
     }
-    if (N <= kAlwaysFeatures) return true;
+    if (c.block > 0) return N <= kAlwaysFeatures || N % 2u == 0u;
+    if (!on_word && (wide_serves(p, N) || (N > kAlwaysFeatures && p->block_units.longest > 128u))) return false;
+    if (N < kAlwaysFeatures) return true;
+    if (N == kAlwaysFeatures) return uint64_t(p->n_steps) * 320u <= uint64_t(p->n_units) * p->cols * 13u || !wide_serves(p, N);
     if (N % 2u) return false;
-    if (c.block > 0) return true;
     if (p->n_units > uint32_t(p->compute_units) * 4u) return false;
     return p->block_units.taken.get(N, [&]() -> uint32_t { return expected(p, N) < blocks_expected(p, N); });
 }

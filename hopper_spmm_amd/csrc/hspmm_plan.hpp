@@ -431,7 +431,7 @@ bool narrow_serves(const hspmm_plan *p, uint32_t N, bool on_word);        // on_
 int run_narrow(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode);
 // hspmm_block.hip: what the block kernels need to know of the units, whether they take this launch, and the launch
 int build_block_units(hspmm_plan *p, const StepStream &st, const uint32_t *rowOffset, const uint32_t *tcA2B);
-bool block_serves(const hspmm_plan *p, uint32_t N);
+bool block_serves(const hspmm_plan *p, uint32_t N, bool on_word);        // on_word: B begins on a word
 int run_block(hspmm_plan *p, const void *dB, void *dC, uint32_t N, hipStream_t s, RunMode mode);
 // hspmm_wide.hip: the wide-tile kernels' stream, whether they take this launch, and the launch
 int build_wide_stream(hspmm_plan *p);

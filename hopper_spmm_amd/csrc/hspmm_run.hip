@@ -436,8 +436,9 @@ static int run_impl(hspmm_plan *p, const void *dB, void *dC, uint32_t N, void *s
         HSPMM_HIP(hspmm::launch_fill_zero(dC, size_t(p->rows) * N * p->elem, s));
         return HSPMM_OK;
     }
-    if (narrow_serves(p, N, reinterpret_cast<uintptr_t>(dB) % 4u == 0u)) return run_narrow(p, dB, dC, N, s, mode);
-    if (block_serves(p, N)) return run_block(p, dB, dC, N, s, mode);
+    const bool on_word = reinterpret_cast<uintptr_t>(dB) % 4u == 0u;
+    if (narrow_serves(p, N, on_word)) return run_narrow(p, dB, dC, N, s, mode);
+    if (block_serves(p, N, on_word)) return run_block(p, dB, dC, N, s, mode);
     if (wide_serves(p, N)) return run_wide(p, dB, dC, N, s, mid, mode);
     if (tile_serves(p, N)) return run_tile(p, dB, dC, N, s, mode);
     if (entries_serve(p, N) && !scheduled_before_entries(p, N, reinterpret_cast<uintptr_t>(dB) | reinterpret_cast<uintptr_t>(dC))) {

@@ -119,6 +119,8 @@ static double panel = 0.0;                          // us the LDS-panel kernels 
 bool panel_serves(const hspmm_plan *, uint32_t) { return panel > 0.0; }
 double panel_expected(const hspmm_plan *, uint32_t) { return panel; }
 double blocks_expected(const hspmm_plan *, uint32_t) { return 1e9; }
+static bool wide = false;                           // whether the wide-tile kernels take it
+bool wide_serves(const hspmm_plan *, uint32_t N) { return wide && N >= 32u; }
 // A plan of rows of blocks with so many blocks each, every block behind the one in front of it; aligned: the gather kernels cut every unit.
 static bool built(hspmm_plan *p, int dtype, const std::vector<uint32_t> &blocks, bool aligned)
 {
@@ -163,7 +165,7 @@ def test_block_kernels_take_even_rows_of_blocks(build):  # noqa: F811
             hspmm_plan p;
             const bool b = built(&p, dtype, a.blocks, a.aligned);
             if (b != a.taken) { std::printf("dtype %d, %zu units, first of %u, longest of %u: %d\\n", dtype, a.blocks.size(), a.blocks[0], a.blocks[a.blocks.size() / 2], int(b)); return 1; }
-            EXPECT(block_serves(&p, 16u) == a.taken && block_serves(&p, 31u) == a.taken);
+            EXPECT(block_serves(&p, 16u, true) == a.taken && block_serves(&p, 31u, true) == a.taken);
             hspmm_plan forced;
             forced.cfg.block = 1;
             EXPECT(built(&forced, dtype, a.blocks, a.aligned));         // (as the tests of the kernels ask for)
@@ -178,14 +180,14 @@ def test_block_kernels_take_even_rows_of_blocks(build):  # noqa: F811
             }
         for (uint32_t units : {512u, 1024u, 1025u, 2048u}) {
             hspmm_plan p;
-            EXPECT(built(&p, dtype, one_long(units, 5, 5), false) && block_serves(&p, 32u) && block_serves(&p, 64u) == (dtype == HSPMM_TF32 || units <= 1024u));
+            EXPECT(built(&p, dtype, one_long(units, 5, 5), false) && block_serves(&p, 32u, true) && block_serves(&p, 64u, true) == (dtype == HSPMM_TF32 || units <= 1024u));
         }
     }
     // fp32 where the LDS-panel kernels would serve: by the longest row of blocks
     panel = 13.5;
     for (uint32_t longest : {80u, 320u, 480u}) {
         hspmm_plan p;
-        EXPECT(built(&p, HSPMM_TF32, one_long(64, 80, longest), true) && block_serves(&p, 16u) == (longest < 480u) && block_serves(&p, 24u) == (longest < 320u) && !block_serves(&p, 48u));
+        EXPECT(built(&p, HSPMM_TF32, one_long(64, 80, longest), true) && block_serves(&p, 16u, true) == (longest < 480u) && block_serves(&p, 24u, true) == (longest < 320u) && !block_serves(&p, 48u, true));
     }
 """), "block")
 
@@ -240,3 +242,26 @@ def test_schedules_of_launches_that_gain_from_the_order(build):  # noqa: F811
             EXPECT(scheduled_serves(&p, N));
         }
 """), "entries")
+
+
+def test_block_kernels_where_the_wide_tile_kernels_are_or_b_lies_between_two_words(build):  # noqa: F811
+    _run(build, _driver(BLOCK_STUBS, """
+    for (int dtype : {HSPMM_FP16, HSPMM_BF16})
+        for (uint32_t blocks : {60u, 66u, 100u, 129u})
+            for (bool wide_too : {false, true}) {
+                hspmm_plan p;
+                EXPECT(built(&p, dtype, one_long(64, blocks, blocks), true));
+                p.cols = 1600;                                              // (60 to 100 of 100 blocks)
+                wide = wide_too;
+                for (uint32_t N : {1u, 7u, 16u, 31u}) EXPECT(block_serves(&p, N, true) && block_serves(&p, N, false));
+                EXPECT(block_serves(&p, 32u, true) == (!wide_too || blocks == 60u) && block_serves(&p, 32u, false) == !wide_too);
+                EXPECT(block_serves(&p, 34u, true) && block_serves(&p, 64u, true) && !block_serves(&p, 33u, true));
+                EXPECT(block_serves(&p, 34u, false) == (!wide_too && blocks <= 128u) && block_serves(&p, 64u, false) == (!wide_too && blocks <= 128u));
+                p.cfg.block = 1;
+                for (uint32_t N : {1u, 32u, 34u, 64u}) EXPECT(block_serves(&p, N, false));
+            }
+    for (uint32_t longest : {512u, 513u}) {
+        hspmm_plan p;
+        EXPECT(built(&p, HSPMM_TF32, one_long(64, 400, longest), true) && block_serves(&p, 32u, false) && block_serves(&p, 64u, true) == (longest == 512u));
+    }
+"""), "block")
