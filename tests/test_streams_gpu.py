@@ -1,12 +1,14 @@
 """One plan launched on several streams, first launched by several threads, and recorded in a graph, where its kernels leave sums of parts
-in memory and are chosen automatically - cut rows of the entry kernels, cut C tiles of the full-tile and the wide-tile kernels -, and
-the narrow kernels, which leave none."""
+in memory and are chosen automatically - cut rows of the entry kernels, cut C tiles of the full-tile and the wide-tile kernels, cut windows
+of the gather kernels' schedule -, and the narrow and the block kernels, which leave none."""
 import threading
 
 import numpy as np
 import pytest
 
+from test_block_gpu import _blocks, _csr
 from test_entries_gpu import _rows_of_lengths
+from test_schedule_gpu import _hot
 from test_spmm_gpu import convert, torch_cuda  # noqa: F401
 from test_tile_gpu import _random_operand, _sampled_csr
 
@@ -23,13 +25,19 @@ def _entry_rows(rng, dtype):
 
 # (entries, N = 65 and 301: rows of an odd number of elements, one block and several)
 CASES = [("entries", 0, 88), ("entries", 1, 24), ("entries", 2, 65), ("entries", 0, 301), ("tile", 2, 64), ("tile", 0, 24), ("tile", 1, 16),
-         ("wide", 2, 64), ("wide", 0, 333), ("narrow", 0, 16), ("narrow", 2, 29)]
+         ("wide", 2, 64), ("wide", 0, 333), ("narrow", 0, 16), ("narrow", 2, 29),
+         ("block", 0, 16), ("block", 2, 31), ("block", 1, 47), ("mfma", 0, 128)]
 
 
 def _case(hs, which, dtype):
     rng = np.random.default_rng(60 + dtype)
     if which == "entries":
         A = _entry_rows(rng, dtype)
+    elif which == "block":
+        mask = _blocks(rng, 1024, 2000, 0.4)
+        A = _csr(mask, rng.normal(size=int(mask.sum())), dtype)
+    elif which == "mfma":
+        A = _hot(rng, 1 << 18, 1 << 18, 6)[0]
     else:
         rows, cols, per_row = {"tile": (4096, 4096, 1300), "wide": (512, 11008, 1100), "narrow": (4096, 4096, 600)}[which]
         A = _sampled_csr(rng, rows, cols, per_row, dtype, lambda n: rng.normal(size=n))
@@ -38,6 +46,7 @@ def _case(hs, which, dtype):
 
 def _check_kernel(plan, which):
     assert plan.last_kernel() == "spmm_%s_kernel" % which
+    assert plan.last_walk()["scheduled"] == (which == "mfma") and (which != "mfma" or plan.last_walk()["split_windows"])
 
 
 def _lane(torch, rng, A, N, dtype):
@@ -63,7 +72,7 @@ def test_launches_on_three_streams_leave_each_others_sums_alone(torch_cuda, hs, 
         for dB, dC, stream in lanes:
             plan.run(dB.data_ptr(), dC.data_ptr(), N, stream.cuda_stream)
     torch.cuda.synchronize()
-    assert (plan.info()["device_bytes"] > one_stream) == (which != "narrow")      # (a set of sums and counters each)
+    assert (plan.info()["device_bytes"] > one_stream) == (which not in ("narrow", "block"))      # (a set of sums and counters each)
     for (_, dC, _), want in zip(lanes, alone):
         assert torch.equal(dC.view(torch.uint8), want.view(torch.uint8))
     plan.close()
