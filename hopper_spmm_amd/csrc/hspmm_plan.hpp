@@ -114,12 +114,14 @@ constexpr uint32_t kMinTilesPerRange = 24;
 // Plans that carry a schedule (power-law graphs, 16-bit bitmap tiles): from 2^18 columns on; built beside the packing of the tiles it adds nothing
 // that shows to hspmm_create (10.6 / 10.3 ms at 2^20 vertices, 2.4 / 2.5 at 2^18, 3.7 / 4.0 at 600000) and 24 words a tile to its device memory
 // (431 -> 527 MB at 2^20).  Against the partition it was ahead on all of 62 launches (12 graphs of 2^18 to 2^20 vertices, 4 to 32 edges each,
-// N = 64 to 512) by 2 to 33 %; graphs of 131072 and 150001, with 8 to 18 MB of B for each 64 features, are the entry kernels' (N = 128:
-// 60 / 63 and 43 / 48 us).
+// N = 64 to 512) by 2 to 33 %, and at N = 192, 320, .. 1984 on all of 42 (six graphs) by 5 to 23 %; graphs of fewer vertices, with 8 to 32 MB of B for each
+// 64 features, are the entry kernels' (entry kernels / schedule, N = 128: 131072 vertices 60 / 63 us, 150001 43 / 47, 200000 58 / 61, 230000 51 / 50,
+// 250000 74 / 76; N = 512, where the partition is the other choice, 4 to 7 % ahead on all of these: not worth the memory).
 constexpr uint32_t kScheduledColumns = 1u << 18;
 // Bytes of B in a block of 64 features from which a single block, or an odd number of them, goes by the schedule rather than to the entry kernels
-// (N = 64: 2^20 vertices 260 / 207 us, 800000 112 / 107, 600000 73 / 77, 350000 55 / 63, 2^18 42 / 50).  Two, four or eight blocks, each with XCDs of
-// its own, from the first such plan on (N = 128: 2^19 240 / 177, 350000 116 / 108, 2^18 94 / 80; N = 256 at 2^18: 193 / 170).
+// (entry kernels / schedule, us, N = 64: 2^20 vertices, 16 edges each, 262 / 203, 900000, 12 edges, 130 / 123, 800000, 8 edges, 87 / 82, 600000 73 / 77,
+// 350000 55 / 63, 2^18 42 / 50).  Two, four or eight blocks, each with XCDs of its own, from the first such plan on (N = 128: 2^19, 16 edges, 239 / 175,
+// 350000, 10 edges, 84 / 76, 2^18, 16 edges, 94 / 80; N = 256 at 2^18: 195 / 168).
 constexpr uint64_t kScheduledSlice = uint64_t(96) << 20;
 // What keeps a launch from the order's gain, of 804 launches of matrices of 4000 to 800000 rows and 2^18 to 1.2 million columns (R-MAT, and rows and
 // columns drawn by powers), at all these N: windows so long that the sums of many parts are added one after the other (the longest over 32 of a

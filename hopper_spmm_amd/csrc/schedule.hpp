@@ -2,9 +2,10 @@
 // a row of B that one of them brings into an L2 is still there when others ask for it.  A power-law graph's gathers are bound by the L2s' misses:
 // walked in the order of the rows a wave is anywhere in the columns at any time, and an L2 keeps what its latest few thousand gathers asked for
 // (2^20 vertices, N = 128: 44 % of the reads hit, 0.47 in a model of the L2 alone and 0.69 there with windows of like length side by side).  Tiles of
-// a window ascend in their columns and so do its items here.  2^20 vertices, 16 edges each, fp16, N = 128: 472 -> 400 us; N = 64: 252 -> 206,
-// 256: 940 -> 877, 512: 2215 -> 2099; 2^18, bf16, N = 128: 87 -> 80.
-// Eight waves a compute unit: 4 / 8 / 12 / 16 measured 430 / 400 / 400 / 397 us at 2^20, N = 128, 281 / 206 / 204 / 204 at N = 64, 82 / 80 / 88 / 85 at 2^18,
+// a window ascend in their columns and so do its items here.  Gather kernels in the order of the rows / of a schedule, us, one plan over and over: 2^20
+// vertices, 16 edges each, fp16, N = 64 252 / 203, 128 480 / 395, 256 949 / 871, 512 2173 / 2078; 2^18, bf16, N = 128 88 / 80.  (Plans of fresh matrices in
+// turn, 2^20, N = 128: 482 / 421.)
+// Eight waves a compute unit: 4 / 8 / 12 / 16 measured, in a session of their own, 430 / 400 / 400 / 397 us at 2^20, N = 128, 281 / 206 / 204 / 204 at N = 64, 82 / 80 / 88 / 85 at 2^18,
 // N = 128, and 354 / 349 / 355 / 359 at N = 512; they have about 350 (2^20) to 540 parts, of 150 to 200 cut windows.
 #pragma once
 #include <cstdint>
