@@ -107,10 +107,10 @@ int build_block_units(hspmm_plan *p, const StepStream &st, const uint32_t *rowOf
 // most), 1.45 times as fast on the mean.  Odd ones stay with the wide-tile kernels (0.9 to 1.2 there), and from 65 on all (0.7 to 1.2).  fp32 storage: every launch
 // of the gather kernels (207 of 60 matrices: 1.07 to 3.5 times as fast); those of the LDS-panel kernels, which are faster from 33 features on
 // and for the largest matrices, by expected time (134 taken: 1.49 on the mean, 0.88 at least; 26 up to 32 features left).
-// Not at N = 32 on more than 65 % of all blocks, where the wide-tile kernels take it (11 of 12 launches were 2 to 20 % slower here, of 22 below none), and
+// Not at N = 32 on more than 65 % of all blocks, where the wide-tile kernels take it (11 of 14 launches were 2 to 20 % slower here, of 20 below none), and
 // not above 32 features on rows of over 512 blocks of fp32 storage (nine with B off its alignment: 0.9).  A B that begins between two words has loads of
 // twice the time: the wide-tile kernels keep theirs (224 launches: 0.87 times as fast here), and above 32 features units of over 128 blocks stay (91:
-// 1.1, 26 behind, by up to 34 %); the others were 1.28 (up to 32 features) and 1.46 times as fast.
+// 1.1, 26 behind, by up to 34 %); the others were 1.28 (up to 32 features) and 1.48 times as fast.
 bool block_serves(const hspmm_plan *p, uint32_t N, bool on_word)
 {
     const Config &c = p->cfg;
