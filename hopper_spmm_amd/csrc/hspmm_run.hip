@@ -610,8 +610,9 @@ static int run_gather(hspmm_plan *p, const void *dB, void *dC, uint32_t N, uint3
         if (rc) return rc;
         if (fused && ka.n_split && (rc = ensure_arrive(p, s, size_t(ka.n_split) * ka.n_feat_blocks, mode, &ka.arrive))) return rc;
     }
-    ka.ranges = dp.d_ranges; ka.split = dp.d_split; ka.fix_slots = dp.d_fix_slots;
-    if (g.scheduled) {
+    if (!g.scheduled) {             // (else another thread may be making the partition)
+        ka.ranges = dp.d_ranges; ka.split = dp.d_split; ka.fix_slots = dp.d_fix_slots;
+    } else {
         ka.unitOffset = sc.d_unitOffset; ka.unitRow = sc.d_info; ka.ids = sc.d_ids; ka.bm_header = sc.d_header;
         ka.ranges = sc.d_ranges; ka.split = sc.d_split; ka.fix_slots = sc.d_fix_slots;
         ka.n_units = sc.n_units;
