@@ -102,7 +102,7 @@ int build_block_units(hspmm_plan *p, const StepStream &st, const uint32_t *rowOf
     return HSPMM_OK;
 }
 
-// Up to 32 features always: of 700 launches of 260 matrices (1024 to 16384 rows, 20 to 60 % of blocks kept, all N) three were slower than by
+// Of the rows of blocks that units_suit takes, up to 32 features: of 700 launches of 260 matrices (1024 to 16384 rows, 20 to 60 % of blocks kept, all N) three were slower than by
 // the gather kernels, by 1 to 11 %.  From 33 on, even numbers, by expected time: of 450 launches taken 11 are slower by more than 3 % (16 % at
 // most), 1.45 times as fast on the mean.  Odd ones stay with the wide-tile kernels (0.9 to 1.2 there), and from 65 on all (0.7 to 1.2).  fp32 storage: every launch
 // of the gather kernels (207 of 60 matrices: 1.07 to 3.5 times as fast); those of the LDS-panel kernels, which are faster from 33 features on
